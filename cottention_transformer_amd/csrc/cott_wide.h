@@ -1,0 +1,317 @@
+// Chunked causal scan for 16-bit tensors whose head dims lie outside the kernels of cott_mfma.h (wider than 128
+// columns, up to 256 contracted ones; value widths are cut into slices, so any multiple of 16).
+//
+//     out_c = ((A_c B_c^T) o mask) C_c + A_c S_c ;   S_{c+1} = S_c + B_c^T C_c          (chunks of 32 positions)
+//
+// One workgroup walks the sequence of one head for one 64-column slice of C and of the output.
+//   * Four compute wavefronts each own 16 columns of the state, all DI rows, in fp32 accumulators (64 registers at
+//     DI = 256).  The rows of neighbouring 16 x 16 tiles are interleaved as in colscan_kernel (tile 2ks+t, row 4g+q
+//     holds state row 32ks+8g+4t+q), which makes a lane's accumulators eight consecutive contraction steps: they are
+//     the operand of A_c S_c as they lie and the state never passes through LDS.
+//   * Four loader wavefronts move the tiles global -> registers -> LDS two chunks ahead, form the three live 16 x 16
+//     score tiles of the chunk (once per workgroup, handed to the compute wavefronts through LDS) and write the
+//     finished output tile to memory as 16-byte pieces of whole 128-byte row segments.
+//   * One barrier per chunk: the product of the scores with C_c is finished at the start of the next chunk.
+// Precision: the plain-FMA kernel that served these widths keeps state and scores in fp32.  So that nothing is lost,
+// both enter the matrix instructions as two 16-bit numbers, x = hi + lo (the second term costs a matrix instruction
+// but no LDS read, and LDS is what this kernel spends its time on).  bf16: 16 significant bits, full exponent range.
+// fp16: the state is scaled by a power of two per column first, so that neither its largest nor its small entries leave
+// the range, and the scores and C take part as bf16 pairs (C exactly).
+// What bounds it: B1 H16 N1024 D256 is 64 workgroups forward and 192 in the gradient launch, each a chain of 32
+// chunks of 1.75 us (57 us a launch, forward + gradients 112 us; the plain-FMA kernel took 18.0 ms).  64-column slices
+// rather than 128: the state then takes 64 registers and twice as many workgroups share the chip, and with 16 heads
+// workgroups are what is short.
+#pragma once
+#include "cott_mfma.h"
+
+namespace cott {
+
+constexpr int kWideChunk = 32;  // positions per chunk: with 64 the double-buffered 256-wide tiles do not fit LDS
+constexpr int kWideSlice = 64;  // output columns per workgroup
+
+struct WideOp {
+    const u16 *A, *B, *C;  // (BH,N,di), (BH,N,di), (BH,N,dj)
+    u16 *O;                // (BH,N,dj)
+    const float *sin;      // (BH,di,dj) fp32 state to start from, or null
+    float *sout;           // receives the state after the last position, or null
+    int di, dj, reversed, slices;
+};
+struct WideSet {
+    WideOp op[3];
+    int count, items;  // ops; workgroups per head = all slices of all ops
+    int xcds;
+};
+
+template <int DI>
+struct WideTiling {
+    static_assert(DI % 64 == 0, "contracted dim padded to a multiple of 64");
+    static constexpr int RS = DI + 16;          // LDS row stride (elements): 8 (mod 32) dwords, see Tiling
+    static constexpr int CS = kWideSlice + 16;
+    static constexpr int OS = kWideSlice + 8;
+    static constexpr int KS = DI / 32;
+    static constexpr int TILE = kWideChunk * RS, CTILE = kWideChunk * CS, OTILE = kWideChunk * OS;
+    static constexpr int PIECES = kWideChunk * DI / 8 / 256;  // 16-byte pieces of an A or B tile per loader thread
+    // A and B tiles, C tiles, output tiles (two buffers each), then the score operands [2 buffers][hi, lo][2 blocks][64]
+    static constexpr size_t LDS = (4 * TILE + 2 * CTILE + 2 * OTILE) * sizeof(u16) + 2 * 2 * 2 * 64 * sizeof(u32x4);
+};
+
+// fp32 -> two 16-bit numbers of type TR, hi + lo
+template <class TR>
+__device__ __forceinline__ void split2(float a, float b, uint32_t &hi, uint32_t &lo) {
+    hi = TR::pack2(a, b);
+    lo = TR::pack2(a - TR::to_float((u16)(hi & 0xffffu)), b - TR::to_float((u16)(hi >> 16)));
+}
+// eight fp16 numbers -> the same eight as bf16 hi + lo (exact: 8 + 8 significant bits hold the 11)
+__device__ __forceinline__ void fp16_as_bf16_pair(u32x4 v, u32x4 &hi, u32x4 &lo) {
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        uint32_t h, x;
+        split2<Bf16>(Fp16::to_float((u16)(v[e] & 0xffffu)), Fp16::to_float((u16)(v[e] >> 16)), h, x);
+        hi[e] = h;
+        lo[e] = x;
+    }
+}
+__device__ __forceinline__ bool any_nan(f32x4 v) {
+    return (v[0] != v[0]) | (v[1] != v[1]) | (v[2] != v[2]) | (v[3] != v[3]);
+}
+// v where it is a number, else the same element of w.  An infinite state or score entry splits into hi = inf and lo =
+// inf - inf; the sum formed from the hi parts alone then has the value the single-number arithmetic gives.
+__device__ __forceinline__ f32x4 number_or(f32x4 v, f32x4 w) {
+#pragma unroll
+    for (int e = 0; e < 4; ++e) v[e] = v[e] == v[e] ? v[e] : w[e];
+    return v;
+}
+
+template <class TR, int DI>
+__device__ __forceinline__ void wide_loader_role(const WideOp &op, int bh, int c0, int N, int nchunks, int tid, u16 *sA,
+                                                 u16 *sB, u16 *sC, const u16 *sO, u32x2 *sP) {
+    using T = WideTiling<DI>;
+    constexpr int PF = 2, PIECES = T::PIECES;
+    const int l = tid & 63, g = l >> 4, m = l & 15;
+    const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int di = op.di, dj = op.dj, reversed = op.reversed;
+    const uint32_t rows = (uint32_t)(N - 1);
+    const rsrc_t rA = make_rsrc_uniform(op.A + (size_t)bh * N * di, (rows * di + di) * 2u);
+    const rsrc_t rB = make_rsrc_uniform(op.B + (size_t)bh * N * di, (rows * di + di) * 2u);
+    const rsrc_t rC = make_rsrc_uniform(op.C + (size_t)bh * N * dj + c0, (rows * dj + (dj - c0)) * 2u);
+    const rsrc_t rO = make_rsrc_uniform(op.O + (size_t)bh * N * dj + c0, (rows * dj + (dj - c0)) * 2u);
+    u32x4 ra[PF][PIECES], rb[PF][PIECES], rc[PF];
+    const int ccol = (tid % (kWideSlice / 8)) * 8, crow = tid / (kWideSlice / 8);
+    auto first_row = [&](int p) __attribute__((always_inline)) { return (reversed ? nchunks - 1 - p : p) * kWideChunk; };
+    auto load_chunk = [&](int s, int p) __attribute__((always_inline)) {
+        const int row0 = first_row(min(p, nchunks - 1));
+#pragma unroll
+        for (int u = 0; u < PIECES; ++u) {
+            const int v = tid + 256 * u;
+            const uint32_t off = (uint32_t)((row0 + v / (DI / 8)) * di + (v % (DI / 8)) * 8) * 2u;
+            ra[s][u] = buf_load16(rA, off);
+            rb[s][u] = buf_load16(rB, off);
+        }
+        rc[s] = buf_load16(rC, (uint32_t)((row0 + crow) * dj + ccol) * 2u);
+    };
+    auto stage = [&](int s, int buf) __attribute__((always_inline)) {
+        const u32x4 z = {0u, 0u, 0u, 0u};
+#pragma unroll
+        for (int u = 0; u < PIECES; ++u) {
+            const int v = tid + 256 * u, col = (v % (DI / 8)) * 8, at = (v / (DI / 8)) * T::RS + col;
+            *reinterpret_cast<u32x4 *>(sA + buf * T::TILE + at) = col < di ? ra[s][u] : z;
+            *reinterpret_cast<u32x4 *>(sB + buf * T::TILE + at) = col < di ? rb[s][u] : z;
+        }
+        *reinterpret_cast<u32x4 *>(sC + buf * T::CTILE + crow * T::CS + ccol) = c0 + ccol < dj ? rc[s] : z;
+    };
+    // Score tile of this wavefront: key block kt against position block pb, transposed (a lane holds four consecutive
+    // keys of one position).  Sum over the past: (0,0) (1,0) (1,1); over the future: (0,0) (0,1) (1,1).
+    const int pb = reversed ? (w == 2) : (w >= 1), kt = reversed ? (w >= 1) : (w == 2);
+    auto scores = [&](int buf) __attribute__((always_inline)) {
+        if (w >= 3) return;
+        f32x4 p0 = {0.f, 0.f, 0.f, 0.f}, p1 = p0;
+        const u16 *keys = sB + buf * T::TILE + (16 * kt + m) * T::RS + 8 * g;
+        const u16 *pos = sA + buf * T::TILE + (16 * pb + m) * T::RS + 8 * g;
+#pragma unroll
+        for (int ks = 0; ks < T::KS; ++ks) {
+            const u32x4 a = *reinterpret_cast<const u32x4 *>(keys + 32 * ks);
+            const u32x4 b = *reinterpret_cast<const u32x4 *>(pos + 32 * ks);
+            if (ks & 1)
+                p1 = TR::mfma(a, b, p1);
+            else
+                p0 = TR::mfma(a, b, p0);
+        }
+        p0 += p1;
+        if (pb == kt) {
+#pragma unroll
+            for (int q = 0; q < 4; ++q) p0[q] = (reversed ? 4 * g + q >= m : 4 * g + q <= m) ? p0[q] : 0.f;
+        }
+        u32x2 hi, lo;
+        uint32_t h0, l0, h1, l1;
+        split2<Bf16>(p0[0], p0[1], h0, l0);
+        split2<Bf16>(p0[2], p0[3], h1, l1);
+        hi = u32x2{h0, h1};
+        lo = u32x2{l0, l1};
+        sP[((buf * 2 + 0) * 2 + pb) * 128 + 2 * l + kt] = hi;
+        sP[((buf * 2 + 1) * 2 + pb) * 128 + 2 * l + kt] = lo;
+    };
+    // output tile of chunk p, left in LDS by the compute wavefronts: one 16-byte piece per thread
+    auto store_out = [&](int p) __attribute__((always_inline)) {
+        const u32x4 v = *reinterpret_cast<const u32x4 *>(sO + (p & 1) * T::OTILE + crow * T::OS + ccol);
+        const int row = first_row(p) + crow;
+        if (c0 + ccol < dj && row < N)
+            __builtin_amdgcn_raw_buffer_store_b128(v, rO, (int)((uint32_t)(row * dj + ccol) * 2u), 0, 0);
+    };
+#pragma unroll
+    for (int s = 0; s < PF; ++s) load_chunk(s, s);
+    stage(0, 0);
+    load_chunk(0, PF);
+    __syncthreads();
+    run_rounds<PF>(0, nchunks, [&](int s, int p) __attribute__((always_inline)) {
+        const int s1 = (s + 1) % PF, buf = p & 1;
+        stage(s1, buf ^ 1);
+        load_chunk(s1, p + 1 + PF);
+        scores(buf);
+        if (p >= 2) store_out(p - 2);
+        chunk_barrier();
+    });
+    // the compute wavefronts finish the last chunk after the last barrier of the loop
+    if (nchunks >= 2) store_out(nchunks - 2);
+    chunk_barrier();
+    store_out(nchunks - 1);
+}
+
+template <class TR, int DI>
+__device__ __forceinline__ void wide_compute_role(const WideOp &op, int bh, int c0, int nchunks, int w, int l, const u16 *sA,
+                                                  const u16 *sB, const u16 *sC, u16 *sO, const u32x4 *sP) {
+    using T = WideTiling<DI>;
+    constexpr bool FP16 = std::is_same<TR, Fp16>::value;
+    constexpr int KS = T::KS;
+    const int g = l >> 4, m = l & 15;
+    const int di = op.di, dj = op.dj, j = c0 + 16 * w + m;  // this lane's state column
+    const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
+    f32x4 S[2 * KS];
+#pragma unroll
+    for (int it = 0; it < 2 * KS; ++it) S[it] = zero;
+    if (op.sin != nullptr && j < dj) {
+        const float *src = op.sin + (size_t)bh * di * dj + j;
+#pragma unroll
+        for (int it = 0; it < 2 * KS; ++it)
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                const int i = 32 * (it >> 1) + 8 * g + 4 * (it & 1) + q;
+                if (i < di) S[it][q] = src[(size_t)i * dj];
+            }
+    }
+    f32x4 o[2] = {zero, zero};       // A_c S_c of the chunk whose scores are still outstanding
+    u32x4 cf = {0u, 0u, 0u, 0u};     // ... and its C fragment, keys in the order of the score operands
+    auto finish = [&](int p) __attribute__((always_inline)) {
+        const int buf = p & 1;
+        u32x4 ch = cf, cl = cf;
+        if constexpr (FP16) fp16_as_bf16_pair(cf, ch, cl);
+#pragma unroll
+        for (int pb = 0; pb < 2; ++pb) {
+            const u32x4 ph = sP[((buf * 2 + 0) * 2 + pb) * 64 + l], pl = sP[((buf * 2 + 1) * 2 + pb) * 64 + l];
+            f32x4 hi = Bf16::mfma(ch, ph, o[pb]);
+            if constexpr (FP16) hi = Bf16::mfma(cl, ph, hi);
+            f32x4 r = Bf16::mfma(ch, pl, hi);
+            if (__any(any_nan(r))) r = number_or(r, hi);
+            const u32x2 packed = {TR::pack2(r[0], r[1]), TR::pack2(r[2], r[3])};
+            *reinterpret_cast<u32x2 *>(sO + buf * T::OTILE + (16 * pb + m) * T::OS + 16 * w + 4 * g) = packed;
+        }
+    };
+    __syncthreads();
+    run_rounds<2>(0, nchunks, [&](int, int p) __attribute__((always_inline)) {
+        const int buf = p & 1;
+        const u16 *tA = sA + buf * T::TILE, *tB = sB + buf * T::TILE, *tC = sC + buf * T::CTILE;
+        if (p > 0) finish(p - 1);
+        cf = cat(lds_col4(tC, T::CS, 4 * g, 16 * w, m), lds_col4(tC, T::CS, 16 + 4 * g, 16 * w, m));
+        const u32x4 cu = cat(lds_col4(tC, T::CS, 8 * g, 16 * w, m), lds_col4(tC, T::CS, 8 * g + 4, 16 * w, m));
+        float up = 1.f;
+        f32x4 down = {1.f, 1.f, 1.f, 1.f};
+        if constexpr (FP16) {  // scale of this lane's state column: its largest entry to [2^14, 2^15)
+            float mx = 0.f;
+#pragma unroll
+            for (int it = 0; it < 2 * KS; ++it)
+#pragma unroll
+                for (int q = 0; q < 4; ++q) mx = fmaxf(mx, __builtin_fabsf(S[it][q]));
+            mx = fmaxf(mx, __shfl_xor(mx, 16));
+            mx = fmaxf(mx, __shfl_xor(mx, 32));
+            // exponent kept to where both the scale and its inverse are normal numbers
+            int e = (int)(bitcast<uint32_t>(mx) >> 23) - 127;
+            e = e < -100 ? -100 : (e > 120 ? 120 : e);
+            up = bitcast<float>((uint32_t)(127 + 14 - e) << 23);
+#pragma unroll
+            for (int q = 0; q < 4; ++q) down[q] = bitcast<float>((uint32_t)(127 - 14 + __shfl(e, 4 * g + q)) << 23);
+        }
+        f32x4 ah[2] = {zero, zero}, al[2] = {zero, zero};
+#pragma unroll
+        for (int ks = 0; ks < KS; ++ks) {
+            u32x4 sh, sl;
+#pragma unroll
+            for (int t = 0; t < 2; ++t)
+#pragma unroll
+                for (int q = 0; q < 2; ++q) {
+                    uint32_t h, lo;
+                    split2<TR>(S[2 * ks + t][2 * q] * up, S[2 * ks + t][2 * q + 1] * up, h, lo);
+                    sh[2 * t + q] = h;
+                    sl[2 * t + q] = lo;
+                }
+#pragma unroll
+            for (int pb = 0; pb < 2; ++pb) {
+                const u32x4 a = *reinterpret_cast<const u32x4 *>(tA + (16 * pb + m) * T::RS + 32 * ks + 8 * g);
+                ah[pb] = TR::mfma(sh, a, ah[pb]);
+                al[pb] = TR::mfma(sl, a, al[pb]);
+            }
+#pragma unroll
+            for (int t = 0; t < 2; ++t) {
+                // rows of state tile 2ks+t: columns 32ks + 8i + 4t .. +3 of B, i = 0..3
+                const u16 *src = tB + (8 * g + (m >> 2)) * T::RS + 32 * ks + 8 * (m & 3) + 4 * t;
+                const u32x4 b = cat(lds_read_tr16(src), lds_read_tr16(src + 4 * T::RS));
+                S[2 * ks + t] = TR::mfma(b, cu, S[2 * ks + t]);
+            }
+        }
+#pragma unroll
+        for (int pb = 0; pb < 2; ++pb) {
+            f32x4 r = ah[pb] + al[pb];
+            if (__any(any_nan(r))) r = number_or(r, ah[pb]);
+            o[pb] = FP16 ? r * down : r;
+        }
+        chunk_barrier();
+    });
+    finish(nchunks - 1);
+    chunk_barrier();
+    if (op.sout != nullptr && j < dj) {
+        float *dst = op.sout + (size_t)bh * di * dj + j;
+#pragma unroll
+        for (int it = 0; it < 2 * KS; ++it)
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                const int i = 32 * (it >> 1) + 8 * g + 4 * (it & 1) + q;
+                if (i < di) dst[(size_t)i * dj] = S[it][q];
+            }
+    }
+}
+
+// 512 threads: wavefronts 0..3 compute, 4..7 load.  Grid: grid_for(BH, set.items, 1, set.xcds), so that the slices and ops
+// of a head run on one XCD and share its tiles through that L2.
+template <class TR, int DI>
+__global__ __launch_bounds__(512) void wide_scan_kernel(WideSet set, int BH, int N, int nchunks) {
+    using T = WideTiling<DI>;
+    __shared__ __attribute__((aligned(16))) unsigned char wide_smem[T::LDS];
+    u16 *sA = reinterpret_cast<u16 *>(wide_smem);
+    u16 *sB = sA + 2 * T::TILE, *sC = sB + 2 * T::TILE, *sO = sC + 2 * T::CTILE;
+    u32x4 *sP = reinterpret_cast<u32x4 *>(sO + 2 * T::OTILE);
+    const WorkItem wi = decode_workgroup(set.items, BH, set.xcds);
+    if (wi.grp >= 1) return;
+    int which = 0, slice = wi.prob;
+    while (which + 1 < set.count && slice >= set.op[which].slices) slice -= set.op[which++].slices;
+    const WideOp &op = set.op[which];
+    const int tid = threadIdx.x;
+    // the score tiles on the other side of the diagonal are never written: zero
+    for (int x = tid; x < 2 * 2 * 2 * 64; x += 512) sP[x] = u32x4{0u, 0u, 0u, 0u};
+    __syncthreads();
+    const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+    if (w < 4)
+        wide_compute_role<TR, DI>(op, wi.bh, slice * kWideSlice, nchunks, w, tid & 63, sA, sB, sC, sO, sP);
+    else
+        wide_loader_role<TR, DI>(op, wi.bh, slice * kWideSlice, N, nchunks, tid - 256, sA, sB, sC, sO,
+                                 reinterpret_cast<u32x2 *>(sP));
+}
+
+}  // namespace cott

@@ -1,0 +1,88 @@
+"""Causal ops of 16-bit heads outside the 32..128 column range (wide_scan_kernel) against the oracle.
+
+Tolerance: inputs are exact, products and sums are fp32, state and scores enter the products with 16 (bf16) or more
+significant bits, so what is left is the rounding of the output: at most half a unit in the last place of every element,
+2^-9 (bf16) and 2^-12 (fp16, away from its subnormals) of it, plus 2^-13 for the hi / lo split and the fp32 sums of
+outputs that cancel."""
+import pytest
+import torch
+
+from util import inputs, rel_l2, worst_block
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+BF, HF = torch.bfloat16, torch.float16
+BOUND = {BF: 2.0 ** -9 + 2.0 ** -13, HF: 2.0 ** -12 + 2.0 ** -13}
+
+
+@pytest.fixture(scope="module")
+def ct():
+    import cottention_transformer_amd as ct_
+    return ct_
+
+
+CASES = [
+    (1, 1, 1, 256, 256, BF),      # one position
+    (1, 2, 31, 256, 256, BF),     # less than a chunk
+    (1, 2, 32, 160, 160, HF),     # exactly one chunk; last slice half empty
+    (2, 3, 33, 192, 192, BF),     # one chunk and one position
+    (1, 9, 64, 256, 256, HF),     # two chunks, more heads than XCDs
+    (1, 2, 203, 224, 224, BF),    # odd number of chunks, padded contracted dim
+    (1, 2, 1000, 256, 256, BF),
+    (1, 2, 130, 256, 64, HF),     # the ops of a gradient call differ in padded width
+    (1, 2, 130, 64, 256, BF),
+    (1, 2, 96, 48, 144, BF),      # contracted dim far below its padding
+    (1, 1, 70, 144, 400, HF),     # seven slices; the gradients contract 400 columns (plain-FMA kernel)
+]
+IDS = lambda c: "x".join(map(str, c[:5])) + "-" + str(c[5]).split(".")[-1]
+
+
+@pytest.mark.parametrize("case", CASES, ids=IDS)
+def test_forward_and_gradients(ct, oracle, case):
+    b, h, n, dk, dv, dt = case
+    q, k, v, do = inputs(b, h, n, dk, dv, dt, seed=n)
+    dev = [t.to(DEV) for t in (q, k, v, do)]
+    for rev in (False, True):
+        got, ref = ct.causal_dot_product(*dev[:3], rev), oracle.causal(q, k, v, rev)
+        assert rel_l2(got, ref) <= BOUND[dt], rev
+        assert worst_block(got, ref, 32) <= 2 * BOUND[dt], rev
+    for name, got, ref in zip(("dQ", "dK", "dV"), ct.causal_backward(*dev), oracle.causal_bwd(q, k, v, do)):
+        assert rel_l2(got, ref) <= BOUND[dt], name
+
+
+@pytest.mark.parametrize("dt", [BF, HF], ids=["bf16", "fp16"])
+def test_states_in_and_out(ct, oracle, dt):
+    """A sequence in two calls, the state handed over, equals the sequence in one; the state is held in fp32."""
+    q, k, v, _ = inputs(1, 2, 150, 256, 160, dt, seed=7)
+    qd, kd, vd = (t.to(DEV) for t in (q, k, v))
+    o1, s1 = ct.causal_prefill(qd[:, :, :70], kd[:, :, :70], vd[:, :, :70])
+    o2, s2 = ct.causal_prefill(qd[:, :, 70:], kd[:, :, 70:], vd[:, :, 70:], state=s1)
+    assert rel_l2(torch.cat((o1, o2), 2), oracle.causal(q, k, v)) <= BOUND[dt]
+    # sums of 150 products in fp32: 150 * 2^-24 at the very most
+    assert rel_l2(s2, (k.double().transpose(2, 3) @ v.double()).numpy()) <= 150 * 2.0 ** -24
+
+
+@pytest.mark.parametrize("scale", [2.0 ** -12, 1.0, 2.0 ** 9], ids=["small", "unit", "large"])
+def test_fp16_state_range(ct, oracle, scale):
+    """Scores, state and their 16-bit halves leave fp16's range on both sides; the outputs (brought back by q) do not:
+    values of `scale`, keys of 1 / 16 .. 16 times `scale`."""
+    q, k, v, _ = inputs(1, 1, 300, 256, 256, HF, seed=3)
+    k, v, q = (k.float() * 16 * scale).half(), (v.float() * scale).half(), (q.float() * min(1.0, scale ** -2 * 2.0 ** 6)).half()
+    got, ref = ct.causal_dot_product(q.to(DEV), k.to(DEV), v.to(DEV)).double().cpu(), torch.from_numpy(oracle.causal(q, k, v))
+    assert torch.isfinite(got).all()
+    # half a unit of 2^-24, the spacing of fp16's subnormals, where the output is one
+    assert ((got - ref).abs() <= 2.0 ** -11 * ref.abs() + 2.0 ** -25 + 2.0 ** -13 * ref.pow(2).mean().sqrt()).all()
+
+
+@pytest.mark.parametrize("dt", [BF, HF], ids=["bf16", "fp16"])
+def test_an_infinite_value_stays_in_its_column(ct, dt):
+    """v[40, 5] infinite: from position 64 (the next chunk) on column 5 is no number a finite sum could give, every other
+    column what it is without it."""
+    q, k, v, _ = (t.to(DEV) for t in inputs(1, 1, 128, 256, 256, dt, seed=4))
+    want = ct.causal_dot_product(q, k, v)
+    v[0, 0, 40, 5] = float("inf")
+    got = ct.causal_dot_product(q, k, v)
+    other = [j for j in range(256) if j != 5]
+    assert torch.equal(got[..., other], want[..., other])
+    assert torch.isfinite(got[0, 0, :32, 5]).all()
+    assert not torch.isfinite(got[0, 0, 64:, 5]).any()

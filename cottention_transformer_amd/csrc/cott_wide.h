@@ -4,8 +4,9 @@
 //     out_c = ((A_c B_c^T) o mask) C_c + A_c S_c ;   S_{c+1} = S_c + B_c^T C_c          (chunks of 32 positions)
 //
 // One workgroup walks the sequence of one head for one 64-column slice of C and of the output.
-//   * Four compute wavefronts each own 16 columns of the state, all DI rows, in fp32 accumulators (64 registers at
-//     DI = 256).  The rows of neighbouring 16 x 16 tiles are interleaved as in colscan_kernel (tile 2ks+t, row 4g+q
+//   * Eight compute wavefronts each own 16 columns and half of the DI rows of the state in fp32 accumulators (32
+//     registers at DI = 256).  The two halves of a column exchange partial outputs through LDS: each finishes one of
+//     the chunk's two blocks of 16 positions.  The rows of neighbouring 16 x 16 tiles are interleaved as in colscan_kernel (tile 2ks+t, row 4g+q
 //     holds state row 32ks+8g+4t+q), which makes a lane's accumulators eight consecutive contraction steps: they are
 //     the operand of A_c S_c as they lie and the state never passes through LDS.
 //   * Four loader wavefronts move the tiles global -> registers -> LDS two chunks ahead, form the three live 16 x 16
@@ -18,8 +19,9 @@
 // fp16: the state is scaled by a power of two per column first, so that neither its largest nor its small entries leave
 // the range, and the scores and C take part as bf16 pairs (C exactly).
 // What bounds it: B1 H16 N1024 D256 is 64 workgroups forward and 192 in the gradient launch, each a chain of 32
-// chunks of 1.75 us (57 us a launch, forward + gradients 112 us; the plain-FMA kernel took 18.0 ms).  64-column slices
-// rather than 128: the state then takes 64 registers and twice as many workgroups share the chip, and with 16 heads
+// chunks of 1.55 us (50 us a launch; the plain-FMA kernel took 18.0 ms for forward + gradients).  Per chunk LDS is busy
+// 2100 of 3300 cycles, the matrix pipe 930, vector-ALU issue about 1700.  Four compute wavefronts that own all DI rows of
+// their columns took 57 us.  64-column slices rather than 128: twice as many workgroups share the chip, and with 16 heads
 // workgroups are what is short.
 #pragma once
 #include "cott_mfma.h"
@@ -28,6 +30,7 @@ namespace cott {
 
 constexpr int kWideChunk = 32;  // positions per chunk: with 64 the double-buffered 256-wide tiles do not fit LDS
 constexpr int kWideSlice = 64;  // output columns per workgroup
+constexpr int kWideCompute = 8, kWideLoad = 4;  // wavefronts of either role
 
 struct WideOp {
     const u16 *A, *B, *C;  // (BH,N,di), (BH,N,di), (BH,N,dj)
@@ -45,15 +48,24 @@ struct WideSet {
 template <int DI>
 struct WideTiling {
     static_assert(DI % 64 == 0, "contracted dim padded to a multiple of 64");
-    static constexpr int RS = DI + 16;          // LDS row stride (elements): 8 (mod 32) dwords, see Tiling
+    // LDS row stride (elements) of the A and B tiles: whole 256-byte spans, in which the 16-byte pieces of a row are
+    // permuted (wide_piece)
+    static constexpr int RS = (DI + 127) / 128 * 128;
     static constexpr int CS = kWideSlice + 16;
     static constexpr int OS = kWideSlice + 8;
     static constexpr int KS = DI / 32;
     static constexpr int TILE = kWideChunk * RS, CTILE = kWideChunk * CS, OTILE = kWideChunk * OS;
     static constexpr int PIECES = kWideChunk * DI / 8 / 256;  // 16-byte pieces of an A or B tile per loader thread
     // A and B tiles, C tiles, output tiles (two buffers each), then the score operands [2 buffers][hi, lo][2 blocks][64]
-    static constexpr size_t LDS = (4 * TILE + 2 * CTILE + 2 * OTILE) * sizeof(u16) + 2 * 2 * 2 * 64 * sizeof(u32x4);
+    // and the partial outputs [2 buffers][8 wavefronts][64]
+    static constexpr size_t LDS = (4 * TILE + 2 * CTILE + 2 * OTILE) * sizeof(u16) +
+                                  (2 * 2 * 2 * 64 + 2 * kWideCompute * 64) * sizeof(u32x4);
 };
+
+// Where 16-byte piece c of row r of an A or B tile lies within the row.  Read in the order of either access, 16 pieces
+// then fall on 16 different 16-byte bank groups: piece c of rows r .. r + 15 (operands along the contracted dim), and
+// pieces 4k .. 4k+3 of rows 4r' .. 4r'+3 (the transposing reads).
+__device__ __forceinline__ int wide_piece(int r, int c) { return c ^ (4 * (r & 3) + ((r >> 2) & 3)); }
 
 // fp32 -> two 16-bit numbers of type TR, hi + lo
 template <class TR>
@@ -72,7 +84,8 @@ __device__ __forceinline__ void fp16_as_bf16_pair(u32x4 v, u32x4 &hi, u32x4 &lo)
     }
 }
 __device__ __forceinline__ bool any_nan(f32x4 v) {
-    return (v[0] != v[0]) | (v[1] != v[1]) | (v[2] != v[2]) | (v[3] != v[3]);
+    const float s = (v[0] + v[1]) + (v[2] + v[3]);  // (also true where infinities cancel: number_or then changes nothing)
+    return s != s;
 }
 // v where it is a number, else the same element of w.  An infinite state or score entry splits into hi = inf and lo =
 // inf - inf; the sum formed from the hi parts alone then has the value the single-number arithmetic gives.
@@ -113,7 +126,8 @@ __device__ __forceinline__ void wide_loader_role(const WideOp &op, int bh, int c
         const u32x4 z = {0u, 0u, 0u, 0u};
 #pragma unroll
         for (int u = 0; u < PIECES; ++u) {
-            const int v = tid + 256 * u, col = (v % (DI / 8)) * 8, at = (v / (DI / 8)) * T::RS + col;
+            const int v = tid + 256 * u, col = (v % (DI / 8)) * 8, row = v / (DI / 8);
+            const int at = row * T::RS + 8 * wide_piece(row, col / 8);
             *reinterpret_cast<u32x4 *>(sA + buf * T::TILE + at) = col < di ? ra[s][u] : z;
             *reinterpret_cast<u32x4 *>(sB + buf * T::TILE + at) = col < di ? rb[s][u] : z;
         }
@@ -122,25 +136,27 @@ __device__ __forceinline__ void wide_loader_role(const WideOp &op, int bh, int c
     // Score tile of this wavefront: key block kt against position block pb, transposed (a lane holds four consecutive
     // keys of one position).  Sum over the past: (0,0) (1,0) (1,1); over the future: (0,0) (0,1) (1,1).
     const int pb = reversed ? (w == 2) : (w >= 1), kt = reversed ? (w >= 1) : (w == 2);
+    // key 4g+q of the tile counts for position m where side + dir q >= 0: on the diagonal the keys of its side, else all
+    const int dir = pb != kt ? 0 : (reversed ? 1 : -1), side = dir * (4 * g - m);
+    int soff[4];  // piece 4ks + g of row m (and of row 16 + m), ks = 0..3
+#pragma unroll
+    for (int ks = 0; ks < 4; ++ks) soff[ks] = m * T::RS + 8 * wide_piece(m, 4 * ks + g);
     auto scores = [&](int buf) __attribute__((always_inline)) {
         if (w >= 3) return;
         f32x4 p0 = {0.f, 0.f, 0.f, 0.f}, p1 = p0;
-        const u16 *keys = sB + buf * T::TILE + (16 * kt + m) * T::RS + 8 * g;
-        const u16 *pos = sA + buf * T::TILE + (16 * pb + m) * T::RS + 8 * g;
+        const u16 *keys = sB + buf * T::TILE + 16 * kt * T::RS, *pos = sA + buf * T::TILE + 16 * pb * T::RS;
 #pragma unroll
         for (int ks = 0; ks < T::KS; ++ks) {
-            const u32x4 a = *reinterpret_cast<const u32x4 *>(keys + 32 * ks);
-            const u32x4 b = *reinterpret_cast<const u32x4 *>(pos + 32 * ks);
+            const u32x4 a = *reinterpret_cast<const u32x4 *>(keys + soff[ks & 3] + 128 * (ks >> 2));
+            const u32x4 b = *reinterpret_cast<const u32x4 *>(pos + soff[ks & 3] + 128 * (ks >> 2));
             if (ks & 1)
                 p1 = TR::mfma(a, b, p1);
             else
                 p0 = TR::mfma(a, b, p0);
         }
         p0 += p1;
-        if (pb == kt) {
 #pragma unroll
-            for (int q = 0; q < 4; ++q) p0[q] = (reversed ? 4 * g + q >= m : 4 * g + q <= m) ? p0[q] : 0.f;
-        }
+        for (int q = 0; q < 4; ++q) p0[q] = side + dir * q >= 0 ? p0[q] : 0.f;
         u32x2 hi, lo;
         uint32_t h0, l0, h1, l1;
         split2<Bf16>(p0[0], p0[1], h0, l0);
@@ -150,12 +166,12 @@ __device__ __forceinline__ void wide_loader_role(const WideOp &op, int bh, int c
         sP[((buf * 2 + 0) * 2 + pb) * 128 + 2 * l + kt] = hi;
         sP[((buf * 2 + 1) * 2 + pb) * 128 + 2 * l + kt] = lo;
     };
-    // output tile of chunk p, left in LDS by the compute wavefronts: one 16-byte piece per thread
+    // output tile of chunk p, left in LDS by the compute wavefronts: one 16-byte piece per thread.  Unconditional like the
+    // loads (see run_rounds): before the first tile and past the real columns the offset is out of range instead.
     auto store_out = [&](int p) __attribute__((always_inline)) {
         const u32x4 v = *reinterpret_cast<const u32x4 *>(sO + (p & 1) * T::OTILE + crow * T::OS + ccol);
-        const int row = first_row(p) + crow;
-        if (c0 + ccol < dj && row < N)
-            __builtin_amdgcn_raw_buffer_store_b128(v, rO, (int)((uint32_t)(row * dj + ccol) * 2u), 0, 0);
+        const uint32_t off = (uint32_t)((first_row(p) + crow) * dj + ccol) * 2u;
+        __builtin_amdgcn_raw_buffer_store_b128(v, rO, (int)(p >= 0 && c0 + ccol < dj ? off : kOobOffset), 0, 0);
     };
 #pragma unroll
     for (int s = 0; s < PF; ++s) load_chunk(s, s);
@@ -163,27 +179,29 @@ __device__ __forceinline__ void wide_loader_role(const WideOp &op, int bh, int c
     load_chunk(0, PF);
     __syncthreads();
     run_rounds<PF>(0, nchunks, [&](int s, int p) __attribute__((always_inline)) {
-        const int s1 = (s + 1) % PF, buf = p & 1;
+        const int s1 = (s + 1) % PF, buf = s;  // (PF = 2 and the first chunk is 0: the LDS buffer is the stage)
         stage(s1, buf ^ 1);
         load_chunk(s1, p + 1 + PF);
         scores(buf);
-        if (p >= 2) store_out(p - 2);
+        store_out(p - 2);
         chunk_barrier();
     });
     // the compute wavefronts finish the last chunk after the last barrier of the loop
-    if (nchunks >= 2) store_out(nchunks - 2);
+    store_out(nchunks - 2);
     chunk_barrier();
     store_out(nchunks - 1);
 }
 
+// Wavefront w of kWideCompute: state columns 16 (w & 3) .. + 15 of the slice, row half w >> 2.
 template <class TR, int DI>
 __device__ __forceinline__ void wide_compute_role(const WideOp &op, int bh, int c0, int nchunks, int w, int l, const u16 *sA,
-                                                  const u16 *sB, const u16 *sC, u16 *sO, const u32x4 *sP) {
+                                                  const u16 *sB, const u16 *sC, u16 *sO, const u32x4 *sP, f32x4 *sX) {
     using T = WideTiling<DI>;
     constexpr bool FP16 = std::is_same<TR, Fp16>::value;
-    constexpr int KS = T::KS;
+    constexpr int KS = T::KS / 2;
     const int g = l >> 4, m = l & 15;
-    const int di = op.di, dj = op.dj, j = c0 + 16 * w + m;  // this lane's state column
+    const int half = w >> 2, cw = 16 * (w & 3), i0 = half * (DI / 2);
+    const int di = op.di, dj = op.dj, j = c0 + cw + m;  // this lane's state column
     const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
     f32x4 S[2 * KS];
 #pragma unroll
@@ -194,37 +212,41 @@ __device__ __forceinline__ void wide_compute_role(const WideOp &op, int bh, int 
         for (int it = 0; it < 2 * KS; ++it)
 #pragma unroll
             for (int q = 0; q < 4; ++q) {
-                const int i = 32 * (it >> 1) + 8 * g + 4 * (it & 1) + q;
+                const int i = i0 + 32 * (it >> 1) + 8 * g + 4 * (it & 1) + q;
                 if (i < di) S[it][q] = src[(size_t)i * dj];
             }
     }
-    f32x4 o[2] = {zero, zero};       // A_c S_c of the chunk whose scores are still outstanding
-    u32x4 cf = {0u, 0u, 0u, 0u};     // ... and its C fragment, keys in the order of the score operands
-    auto finish = [&](int p) __attribute__((always_inline)) {
-        const int buf = p & 1;
+    f32x4 o = zero;                // own part of A_c S_c, block `half` of the chunk whose scores are outstanding
+    u32x4 cf = {0u, 0u, 0u, 0u};   // ... and its C fragment, keys in the order of the score operands
+    int aoff[KS], boff[KS][2];  // A: piece 4ks + g of row m; B: rows 8g + m/4 (and + 4), piece 4ks + m%4, of this row half
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) {
+        const int c = i0 / 8 + 4 * ks, r = 8 * g + (m >> 2);
+        aoff[ks] = m * T::RS + 8 * wide_piece(m, c + g);
+        boff[ks][0] = r * T::RS + 8 * wide_piece(r, c + (m & 3));
+        boff[ks][1] = (r + 4) * T::RS + 8 * wide_piece(r + 4, c + (m & 3));
+    }
+    auto finish = [&](int buf) __attribute__((always_inline)) {
         u32x4 ch = cf, cl = cf;
         if constexpr (FP16) fp16_as_bf16_pair(cf, ch, cl);
-#pragma unroll
-        for (int pb = 0; pb < 2; ++pb) {
-            const u32x4 ph = sP[((buf * 2 + 0) * 2 + pb) * 64 + l], pl = sP[((buf * 2 + 1) * 2 + pb) * 64 + l];
-            f32x4 hi = Bf16::mfma(ch, ph, o[pb]);
-            if constexpr (FP16) hi = Bf16::mfma(cl, ph, hi);
-            f32x4 r = Bf16::mfma(ch, pl, hi);
-            if (__any(any_nan(r))) r = number_or(r, hi);
-            const u32x2 packed = {TR::pack2(r[0], r[1]), TR::pack2(r[2], r[3])};
-            *reinterpret_cast<u32x2 *>(sO + buf * T::OTILE + (16 * pb + m) * T::OS + 16 * w + 4 * g) = packed;
-        }
+        const u32x4 ph = sP[((buf * 2 + 0) * 2 + half) * 64 + l], pl = sP[((buf * 2 + 1) * 2 + half) * 64 + l];
+        const f32x4 other = sX[(buf * kWideCompute + (w ^ 4)) * 64 + l];
+        f32x4 hi = Bf16::mfma(ch, ph, o + other);
+        if constexpr (FP16) hi = Bf16::mfma(cl, ph, hi);
+        f32x4 r = Bf16::mfma(ch, pl, hi);
+        if (__any(any_nan(r))) r = number_or(r, hi);
+        const u32x2 packed = {TR::pack2(r[0], r[1]), TR::pack2(r[2], r[3])};
+        *reinterpret_cast<u32x2 *>(sO + buf * T::OTILE + (16 * half + m) * T::OS + cw + 4 * g) = packed;
     };
     __syncthreads();
-    run_rounds<2>(0, nchunks, [&](int, int p) __attribute__((always_inline)) {
-        const int buf = p & 1;
+    run_rounds<2>(0, nchunks, [&](int buf, int p) __attribute__((always_inline)) {
         const u16 *tA = sA + buf * T::TILE, *tB = sB + buf * T::TILE, *tC = sC + buf * T::CTILE;
-        if (p > 0) finish(p - 1);
-        cf = cat(lds_col4(tC, T::CS, 4 * g, 16 * w, m), lds_col4(tC, T::CS, 16 + 4 * g, 16 * w, m));
-        const u32x4 cu = cat(lds_col4(tC, T::CS, 8 * g, 16 * w, m), lds_col4(tC, T::CS, 8 * g + 4, 16 * w, m));
+        if (p > 0) finish(buf ^ 1);
+        cf = cat(lds_col4(tC, T::CS, 4 * g, cw, m), lds_col4(tC, T::CS, 16 + 4 * g, cw, m));
+        const u32x4 cu = cat(lds_col4(tC, T::CS, 8 * g, cw, m), lds_col4(tC, T::CS, 8 * g + 4, cw, m));
         float up = 1.f;
         f32x4 down = {1.f, 1.f, 1.f, 1.f};
-        if constexpr (FP16) {  // scale of this lane's state column: its largest entry to [2^14, 2^15)
+        if constexpr (FP16) {  // scale of this lane's half column: its largest entry to [2^14, 2^15)
             float mx = 0.f;
 #pragma unroll
             for (int it = 0; it < 2 * KS; ++it)
@@ -254,27 +276,35 @@ __device__ __forceinline__ void wide_compute_role(const WideOp &op, int bh, int 
                 }
 #pragma unroll
             for (int pb = 0; pb < 2; ++pb) {
-                const u32x4 a = *reinterpret_cast<const u32x4 *>(tA + (16 * pb + m) * T::RS + 32 * ks + 8 * g);
+                const u32x4 a = *reinterpret_cast<const u32x4 *>(tA + 16 * pb * T::RS + aoff[ks]);
                 ah[pb] = TR::mfma(sh, a, ah[pb]);
                 al[pb] = TR::mfma(sl, a, al[pb]);
             }
 #pragma unroll
             for (int t = 0; t < 2; ++t) {
                 // rows of state tile 2ks+t: columns 32ks + 8i + 4t .. +3 of B, i = 0..3
-                const u16 *src = tB + (8 * g + (m >> 2)) * T::RS + 32 * ks + 8 * (m & 3) + 4 * t;
-                const u32x4 b = cat(lds_read_tr16(src), lds_read_tr16(src + 4 * T::RS));
+                const u32x4 b = cat(lds_read_tr16(tB + boff[ks][0] + 4 * t), lds_read_tr16(tB + boff[ks][1] + 4 * t));
                 S[2 * ks + t] = TR::mfma(b, cu, S[2 * ks + t]);
             }
         }
 #pragma unroll
+        for (int pb = 0; pb < 2; ++pb) al[pb] += ah[pb];
+        if (__any(any_nan(al[0]) | any_nan(al[1]))) {
+            al[0] = number_or(al[0], ah[0]);
+            al[1] = number_or(al[1], ah[1]);
+        }
+#pragma unroll
         for (int pb = 0; pb < 2; ++pb) {
-            f32x4 r = ah[pb] + al[pb];
-            if (__any(any_nan(r))) r = number_or(r, ah[pb]);
-            o[pb] = FP16 ? r * down : r;
+            f32x4 r = al[pb];
+            if constexpr (FP16) r *= down;
+            if (pb == half)
+                o = r;
+            else
+                sX[(buf * kWideCompute + w) * 64 + l] = r;
         }
         chunk_barrier();
     });
-    finish(nchunks - 1);
+    finish((nchunks - 1) & 1);
     chunk_barrier();
     if (op.sout != nullptr && j < dj) {
         float *dst = op.sout + (size_t)bh * di * dj + j;
@@ -282,21 +312,22 @@ __device__ __forceinline__ void wide_compute_role(const WideOp &op, int bh, int 
         for (int it = 0; it < 2 * KS; ++it)
 #pragma unroll
             for (int q = 0; q < 4; ++q) {
-                const int i = 32 * (it >> 1) + 8 * g + 4 * (it & 1) + q;
+                const int i = i0 + 32 * (it >> 1) + 8 * g + 4 * (it & 1) + q;
                 if (i < di) dst[(size_t)i * dj] = S[it][q];
             }
     }
 }
 
-// 512 threads: wavefronts 0..3 compute, 4..7 load.  Grid: grid_for(BH, set.items, 1, set.xcds), so that the slices and ops
+// 768 threads: wavefronts 0..7 compute, 8..11 load.  Grid: grid_for(BH, set.items, 1, set.xcds), so that the slices and ops
 // of a head run on one XCD and share its tiles through that L2.
 template <class TR, int DI>
-__global__ __launch_bounds__(512) void wide_scan_kernel(WideSet set, int BH, int N, int nchunks) {
+__global__ __launch_bounds__(64 * (kWideCompute + kWideLoad)) void wide_scan_kernel(WideSet set, int BH, int N, int nchunks) {
     using T = WideTiling<DI>;
     __shared__ __attribute__((aligned(16))) unsigned char wide_smem[T::LDS];
     u16 *sA = reinterpret_cast<u16 *>(wide_smem);
     u16 *sB = sA + 2 * T::TILE, *sC = sB + 2 * T::TILE, *sO = sC + 2 * T::CTILE;
     u32x4 *sP = reinterpret_cast<u32x4 *>(sO + 2 * T::OTILE);
+    f32x4 *sX = reinterpret_cast<f32x4 *>(sP + 2 * 2 * 2 * 64);
     const WorkItem wi = decode_workgroup(set.items, BH, set.xcds);
     if (wi.grp >= 1) return;
     int which = 0, slice = wi.prob;
@@ -304,13 +335,13 @@ __global__ __launch_bounds__(512) void wide_scan_kernel(WideSet set, int BH, int
     const WideOp &op = set.op[which];
     const int tid = threadIdx.x;
     // the score tiles on the other side of the diagonal are never written: zero
-    for (int x = tid; x < 2 * 2 * 2 * 64; x += 512) sP[x] = u32x4{0u, 0u, 0u, 0u};
+    for (int x = tid; x < 2 * 2 * 2 * 64; x += 64 * (kWideCompute + kWideLoad)) sP[x] = u32x4{0u, 0u, 0u, 0u};
     __syncthreads();
     const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
-    if (w < 4)
-        wide_compute_role<TR, DI>(op, wi.bh, slice * kWideSlice, nchunks, w, tid & 63, sA, sB, sC, sO, sP);
+    if (w < kWideCompute)
+        wide_compute_role<TR, DI>(op, wi.bh, slice * kWideSlice, nchunks, w, tid & 63, sA, sB, sC, sO, sP, sX);
     else
-        wide_loader_role<TR, DI>(op, wi.bh, slice * kWideSlice, N, nchunks, tid - 256, sA, sB, sC, sO,
+        wide_loader_role<TR, DI>(op, wi.bh, slice * kWideSlice, N, nchunks, tid - 64 * kWideCompute, sA, sB, sC, sO,
                                  reinterpret_cast<u32x2 *>(sP));
 }
 

@@ -12,7 +12,7 @@ template <class TR, int DI>
 hipError_t launch_set(const WideSet &set, int BH, int N, int prof_id, hipStream_t stream) {
     ProfScope ps(prof_id, stream);
     const int nchunks = (N + kWideChunk - 1) / kWideChunk;
-    wide_scan_kernel<TR, DI><<<dim3(grid_for(BH, set.items, 1, set.xcds)), dim3(512), 0, stream>>>(set, BH, N, nchunks);
+    wide_scan_kernel<TR, DI><<<dim3(grid_for(BH, set.items, 1, set.xcds)), dim3(64 * (kWideCompute + kWideLoad)), 0, stream>>>(set, BH, N, nchunks);
     return hipGetLastError();
 }
 

@@ -228,6 +228,8 @@ struct DecodePrep {
     int R, H, on;
 };
 
+// 1 << strip_log2 wavefronts per head, each with its own columns of the state (1 << row_log2 lanes to a row, at least 8):
+// few heads are a serial chain of row batches in too few wavefronts otherwise.
 // NT bit 0: non-temporal state loads, bit 1: non-temporal state stores (a state far larger than the last-level
 // cache is not found there again by the next step).
 template <class ST, class SF, bool PREP, int NT = 0>
@@ -235,13 +237,13 @@ __global__ __launch_bounds__(256) void decode_wave_kernel(SF *__restrict__ S, co
                                                           const typename ST::elem *__restrict__ k,
                                                           const typename ST::elem *__restrict__ v,
                                                           typename ST::elem *__restrict__ o, int BH, int dk, int dv,
-                                                          DecodePrep prep) {
+                                                          int strip_log2, int row_log2, DecodePrep prep) {
     typedef SF __attribute__((ext_vector_type(4))) sf4;
     constexpr int U = 16;
     extern __shared__ __attribute__((aligned(32))) unsigned char smem_raw[];
     const int lane = threadIdx.x & 63;
     const int wv = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
-    const int bh = blockIdx.x * 4 + wv;
+    const int unit = blockIdx.x * (int)(blockDim.x >> 6) + wv, bh = unit >> strip_log2;
     if (bh >= BH) return;
     SF *sq = reinterpret_cast<SF *>(smem_raw) + (size_t)wv * 2 * dk;  // this wavefront's [q | k]
     SF *sk = sq + dk;
@@ -251,8 +253,9 @@ __global__ __launch_bounds__(256) void decode_wave_kernel(SF *__restrict__ S, co
     v += (size_t)bh * dv;
     o += (size_t)bh * dv;
     const int nv = dv / 4;       // 8, 16, 32 or 64
-    const int rpw = 64 / nv;     // rows covered by one wavefront-wide load
-    const int mc = lane % nv, mr = lane / nv;
+    const int lw = 1 << row_log2;   // lanes per row: this wavefront's strip of the columns
+    const int rpw = 64 >> row_log2; // rows covered by one wavefront-wide load
+    const int mc = ((unit & ((1 << strip_log2) - 1)) << row_log2) + (lane & (lw - 1)), mr = lane >> row_log2;
     sf4 *col = reinterpret_cast<sf4 *>(S) + mc;
     sf4 acc = {0, 0, 0, 0};
     sf4 vv = {0, 0, 0, 0};
@@ -334,7 +337,7 @@ __global__ __launch_bounds__(256) void decode_wave_kernel(SF *__restrict__ S, co
             }
         }
     }
-    for (int off = nv; off < 64; off <<= 1) {
+    for (int off = lw; off < 64; off <<= 1) {
         acc.x += __shfl_xor(acc.x, off);
         acc.y += __shfl_xor(acc.y, off);
         acc.z += __shfl_xor(acc.z, off);

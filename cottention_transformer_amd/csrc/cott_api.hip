@@ -1286,6 +1286,49 @@ int cott_decode_step_prep(void *state, const void *q, const void *k, const void 
     return COTT_OK;
 }
 
+size_t cott_decode_block_scratch_bytes(int B, int H, int D, int dtype) {
+    if (B < 1 || H < 1 || D < 1 || (dtype != COTT_BF16 && dtype != COTT_F16)) return 0;
+    return (size_t)4 * B * H * D * 2;
+}
+
+int cott_decode_block(const void *x, const void *wq, const void *wk, const void *wv, const void *wo, void *state, void *y,
+                      const float *sig, float cnt, const float *rot_table, long long position, int rotary_dim,
+                      int table_rows, int B, int H, int D, int dtype, void *scratch, size_t scratch_bytes, void *stream) {
+    const char *fn = "cott_decode_block";
+    if (dtype != COTT_BF16 && dtype != COTT_F16) return fail(COTT_ERR_UNSUPPORTED, "%s: needs bf16 / fp16 tensors", fn);
+    if (B < 0 || H < 1 || D < 1) return fail(COTT_ERR_INVALID, "%s: bad size", fn);
+    if (D != 32 && D != 64 && D != 128 && D != 256)
+        return fail(COTT_ERR_UNSUPPORTED, "%s: needs D in {32, 64, 128, 256} (got %d)", fn, D);
+    const long E = (long)H * D;
+    if (B > cott::kTokenRows || E > (1L << 20))
+        return fail(COTT_ERR_UNSUPPORTED, "%s: at most %d sequences of at most 2^20 columns", fn, cott::kTokenRows);
+    if (B == 0) return COTT_OK;
+    if (!x || !wq || !wk || !wv || !wo || !state || !y) return fail(COTT_ERR_INVALID, "%s: null tensor pointer", fn);
+    if (!aligned16(x) || !aligned16(wq) || !aligned16(wk) || !aligned16(wv) || !aligned16(wo) || !aligned16(state) || !aligned16(y))
+        return fail(COTT_ERR_INVALID, "%s: tensor pointers must be 16-byte aligned", fn);
+    const size_t need = cott_decode_block_scratch_bytes(B, H, D, dtype);
+    if (scratch == nullptr || scratch_bytes < need || !aligned16(scratch))
+        return fail(COTT_ERR_WORKSPACE, "%s: scratch of %zu bytes (16-byte aligned) required, got %zu", fn, need,
+                    scratch ? scratch_bytes : (size_t)0);
+    if (rot_table != nullptr) {
+        if (rotary_dim < 2 || rotary_dim % 2 != 0 || rotary_dim > D)
+            return fail(COTT_ERR_INVALID, "%s: rotary_dim must be even and in [2, D] (got %d)", fn, rotary_dim);
+        if (table_rows < 1) return fail(COTT_ERR_INVALID, "%s: empty rotary table", fn);
+    }
+    hipStream_t st = static_cast<hipStream_t>(stream);
+    char *q = static_cast<char *>(scratch), *k = q + need / 4, *v = k + need / 4, *o = v + need / 4;
+    const void *const win[3] = {wq, wk, wv}, *const wout[3] = {wo, nullptr, nullptr};
+    void *const yin[3] = {q, k, v}, *const yout[3] = {y, nullptr, nullptr};
+    hipError_t e = cott::launch_token_linear(dtype, x, win, yin, 3, B, (int)E, (int)E, st);
+    if (e != hipSuccess) return fail(COTT_ERR_HIP, "%s: HIP launch failed: %s", fn, hipGetErrorString(e));
+    if (int rc = cott_decode_step_prep(state, q, k, v, o, sig, cnt, rot_table, position, rotary_dim, table_rows, B, H, D, D,
+                                       dtype, stream))
+        return rc;
+    e = cott::launch_token_linear(dtype, o, wout, yout, 1, B, (int)E, (int)E, st);
+    if (e != hipSuccess) return fail(COTT_ERR_HIP, "%s: HIP launch failed: %s", fn, hipGetErrorString(e));
+    return COTT_OK;
+}
+
 namespace {
 int check_prep(const char *fn, int B, int H, int N, int Dk, int Dv, int d0, int d1) {
     if (elem_size(d0) == 0 || elem_size(d1) == 0) return fail(COTT_ERR_INVALID, "%s: unknown dtype", fn);

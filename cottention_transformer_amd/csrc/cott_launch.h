@@ -122,4 +122,10 @@ hipError_t launch_decode_prep(int dtype, void *state, const void *q, const void 
                               int dk, int dv, const float *sig, float cnt, const float *rot, long long pos, int R,
                               float eps, hipStream_t stream);
 
+// y[i] = x w[i]^T for i < count <= 3: x (rows, in), w (out, in), y (rows, out), all 16-bit of one type, 16-byte aligned;
+// rows <= 16, in a multiple of 32, out of 16, 32 * in bytes and rows * in * 2 below 2^31.
+constexpr int kTokenRows = 16;
+hipError_t launch_token_linear(int dtype, const void *x, const void *const w[3], void *const y[3], int count, int rows, int in,
+                               int out, hipStream_t stream);
+
 }  // namespace cott

@@ -17,7 +17,7 @@ from torch import nn
 from . import ops
 from .autograd import (CustomAttention, CustomAttentionMergedHeads, NonCausalAttention,
                        NonCausalAttentionMergedHeads, PreparedCausalAttention, PreparedNonCausalAttention, PrepareInputs,
-                       _autocast_target, project)
+                       _autocast_target, _is_plain_linear, project)
 
 
 def _autocast_on():
@@ -97,17 +97,43 @@ class GPTCosAttention(nn.Module):
         if self.state is None:
             self.state = torch.zeros(b, h, d, value.shape[-1], device=query.device,
                                      dtype=torch.float64 if query.dtype == torch.float64 else torch.float32)
-        cached = getattr(self, "_sig_cache", None)
-        if cached is None or cached[0] != self.norm_const._version or cached[1].device != query.device:
-            cached = (self.norm_const._version, self.norm_const.detach().sigmoid().reshape(h).float().to(query.device))
-            self._sig_cache = cached
-        table = self.embed_positions
-        if table.device != query.device:
-            table = self.embed_positions = table.to(query.device)
-        out = ops.decode_step_prepared(self.state, query, key, value, sig=cached[1], cnt=float(self.cur_s),
+        sig, table = self._decode_side_inputs(query.device)
+        out = ops.decode_step_prepared(self.state, query, key, value, sig=sig, cnt=float(self.cur_s),
                                        rotary=(table, self.cur_s - 1))
         self.cur_s += 1
         return out.reshape(b, 1, h * value.shape[-1])
+
+    def _decode_side_inputs(self, device):
+        """sigmoid(norm_const) per head (recomputed when the parameter was written to) and the rotary table on `device`."""
+        cached = getattr(self, "_sig_cache", None)
+        if cached is None or cached[0] != self.norm_const._version or cached[1].device != device:
+            cached = (self.norm_const._version,
+                      self.norm_const.detach().sigmoid().reshape(self.num_attention_heads).float().to(device))
+            self._sig_cache = cached
+        table = self.embed_positions
+        if table.device != device:
+            table = self.embed_positions = table.to(device)
+        return cached[1], table
+
+    def _decode_block_ready(self, hidden_states):
+        """Whether one new token can take ops.decode_block: nothing to differentiate (neither backwards nor forwards), no
+        autocast, 16-bit hidden states of few sequences, and four plain projections without bias whose weights are
+        ordinary contiguous parameters of the same type."""
+        dt = hidden_states.dtype
+        if (torch.is_grad_enabled() or torch.autograd.forward_ad._current_level >= 0 or _autocast_on()
+                or dt not in (torch.bfloat16, torch.float16) or not hidden_states.is_cuda
+                or type(hidden_states) is not torch.Tensor or hidden_states.shape[0] > ops.DECODE_BLOCK_ROWS
+                or hidden_states.dim() != 3 or hidden_states.shape[0] == 0):
+            return False
+        e, dev = self.embed_dim, hidden_states.device
+        for lin in (self.q_proj, self.k_proj, self.v_proj, self.out_proj):
+            if not _is_plain_linear(lin) or lin.bias is not None:
+                return False
+            w = lin.weight
+            if (type(w) is not nn.Parameter or w.dtype != dt or w.device != dev or w.shape != (e, e)
+                    or not w.is_contiguous() or w.data_ptr() % 16 != 0):
+                return False
+        return hidden_states.shape[2] == e and hidden_states.data_ptr() % 16 == 0
 
     def _unmasked_side_inputs(self, b, s, device):
         """Keep mask (all true) and running count of kept keys (1, 2, ..., s) of a batch without padding: constants,
@@ -192,12 +218,23 @@ class GPTCosAttention(nn.Module):
 
     def forward(self, hidden_states, layer_past=None, attention_mask=None, position_ids=None, head_mask=None,
                 use_cache=False, output_attentions=False):
+        one_token = (self.fast_inference and hidden_states.shape[1] == 1 and position_ids is None and layer_past is None
+                     and use_cache is not True and not output_attentions and attention_mask is None
+                     and self.head_dim in (32, 64, 128, 256) and self.rotary_dim is not None
+                     and self.rotary_dim % 2 == 0 and self.rotary_dim <= self.head_dim)
+        if one_token and self._decode_block_ready(hidden_states):
+            b, dev = hidden_states.shape[0], hidden_states.device
+            if self.state is None:
+                self.state = torch.zeros(b, self.num_attention_heads, self.head_dim, self.head_dim, device=dev)
+            sig, table = self._decode_side_inputs(dev)
+            out = ops.decode_block(hidden_states[:, 0], self.q_proj.weight, self.k_proj.weight, self.v_proj.weight,
+                                   self.out_proj.weight, self.state, sig=sig, cnt=float(self.cur_s),
+                                   rotary=(table, self.cur_s - 1))
+            self.cur_s += 1
+            return (self.resid_dropout(out[:, None]), None)
         query, key, value = (self._split_heads(t)                       # (B,S,H,D)
                              for t in project(hidden_states, self.q_proj, self.k_proj, self.v_proj))
-        if (self.fast_inference and hidden_states.shape[1] == 1 and position_ids is None and layer_past is None
-                and use_cache is not True and not output_attentions and attention_mask is None
-                and self.head_dim in (32, 64, 128, 256) and self.rotary_dim is not None
-                and self.rotary_dim % 2 == 0 and self.rotary_dim <= self.head_dim):
+        if one_token:
             attn_output = self._decode_one(query, key, value)
             if not _autocast_on():
                 attn_output = attn_output.to(hidden_states.dtype)

@@ -527,6 +527,45 @@ def decode_step_prepared(state, q, k, v, sig=None, cnt=0.0, rotary=None, out=Non
     return out
 
 
+DECODE_BLOCK_ROWS = 16  # sequences up to which decode_block is built (kTokenRows, csrc/cott_launch.h)
+
+
+def decode_block(x, wq, wk, wv, wo, state, sig=None, cnt=0.0, rotary=None):
+    """One new token of up to DECODE_BLOCK_ROWS sequences through a whole attention block without biases, three launches:
+    q, k, v = x wq^T, x wk^T, x wv^T, then decode_step_prepared on them (state (B,H,D,D) fp32, updated in place), then
+    the returned y = o wo^T.  x: (B,E) bf16 / fp16; weights (E,E), contiguous and 16-byte aligned, in x's type;
+    sig, cnt, rotary as in decode_step_prepared."""
+    _require_gpu(x=x, wq=wq, wk=wk, wv=wv, wo=wo, state=state)
+    code = _dtype_code(x)
+    if x.dim() != 2 or state.dim() != 4:
+        raise RuntimeError("decode_block: x (B,E), state (B,H,D,D)")
+    b, e = x.shape
+    h, d = state.shape[1:3]
+    if state.shape != (b, h, d, d) or h * d != e or state.dtype != torch.float32 or not state.is_contiguous():
+        raise RuntimeError(f"decode_block: state must be a contiguous float32 (B,H,D,D) tensor with H * D = {e}")
+    for w in (wq, wk, wv, wo):
+        if w.shape != (e, e) or w.dtype != x.dtype or not w.is_contiguous():
+            raise RuntimeError(f"decode_block: weights must be contiguous {(e, e)} tensors of type {x.dtype}")
+    if sig is not None and (sig.shape != (h,) or sig.dtype != torch.float32 or sig.device != x.device or not sig.is_contiguous()):
+        raise RuntimeError(f"decode_block: sig must be a contiguous float32 tensor of shape {(h,)} on x's device")
+    table, pos, rdim, rows = None, 0, 0, 0
+    if rotary is not None:
+        table, pos = rotary
+        if table.dim() != 2 or table.dtype != torch.float32 or table.device != x.device or not table.is_contiguous():
+            raise RuntimeError("rotary table must be a contiguous float32 (positions, rotary_dim) tensor on the inputs' device")
+        rows, rdim = table.shape
+    x = x.contiguous()
+    scratch = torch.empty((4, b, e), dtype=x.dtype, device=x.device)
+    y = torch.empty((b, e), dtype=x.dtype, device=x.device)
+    with _on(x.device):
+        rc = _loader.lib().cott_decode_block(x.data_ptr(), wq.data_ptr(), wk.data_ptr(), wv.data_ptr(), wo.data_ptr(),
+                                             state.data_ptr(), y.data_ptr(), _ptr(sig), float(cnt), _ptr(table), int(pos),
+                                             rdim, rows, b, h, d, code, scratch.data_ptr(), scratch.numel() * 2,
+                                             _stream(x.device))
+    _check(rc, "cott_decode_block")
+    return y
+
+
 def _prep_side_inputs(b, h, n, keep, cnt, sig, device):
     if keep is not None:
         if keep.shape != (b, n):

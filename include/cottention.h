@@ -214,6 +214,16 @@ COTT_API int cott_decode_step_prep(void *state, const void *q, const void *k, co
                           int rotary_dim, int table_rows,
                           int B, int H, int Dk, int Dv, int dtype, void *stream);
 
+/* One new token through a whole attention block without biases (GPT_Trainer/GPTCosAttention.py:443-445, 229-272, 501):
+ * q, k, v = x wq^T, x wk^T, x wv^T; cott_decode_step_prep on them; y = o wo^T.  Three launches.  x, y: (B, H * D), the
+ * weights (H * D, H * D) as nn.Linear keeps them, state (B,H,D,D) fp32 updated in place; bf16 / fp16, B <= 16, D in
+ * {32,64,128,256}; q, k, v, o are rounded to `dtype` in the scratch memory, as separate calls leave them. */
+COTT_API size_t cott_decode_block_scratch_bytes(int B, int H, int D, int dtype);
+COTT_API int cott_decode_block(const void *x, const void *wq, const void *wk, const void *wv, const void *wo,
+                      void *state, void *y, const float *sig, float cnt,
+                      const float *rot_table, long long position, int rotary_dim, int table_rows,
+                      int B, int H, int D, int dtype, void *scratch, size_t scratch_bytes, void *stream);
+
 /* ---- fused input preparation (the elementwise work the module does before the attention op) --
  *   q_out = keep * q / max(|q|_2, 1e-12)     (rows of Dk; same for k)
  *   v_out = keep * v / max(cnt^sig[h], 1)    (rows of Dv)

@@ -170,6 +170,32 @@ bool pair_eligible(const Op *ops, int n, int dtype, bool causal) {
     return true;
 }
 
+// Chunks up to which a set runs as ONE group per head even where that leaves most of the chip idle: cutting the sequence
+// costs a group-state and a prefix launch (together about 8 us on the device and as much host time) and saves chunks of
+// 0.55 us (16-bit, 64 x 64 tiles) to 3 us (fp32 on split operands).  Times in us, cut / one group, launches back to back:
+//   forward, 16-bit D64: 2 heads N128 8.8 / 4.2, N768 10.3 / 9.3, N1023 10.8 / 11.5; 12 heads N1023 12.1 / 11.7; 64 heads
+//   17.7 / 13.1.  D128: 2 heads N256 11.4 / 8.1, N512 12.2 / 12.4; 12 heads N512 17.1 / 12.7, N768 17.2 / 17.4; 16 heads
+//   N768 19.0 / 17.5.
+//   gradients, 16-bit D64: 2 heads N128 10.5 / 4.9; 12 heads N256 12.0 / 6.6, N512 14.5 / 9.5; D32 12 heads N768 10.6 / 8.5;
+//   D128: 2 heads N512 14.0 / 13.1, N768 16.2 / 18.1; 12 heads N768 23.9 / 18.5.
+//   fp32 D64: 2 heads N128 12.8 / 7.9 forward, N256 13.1 / 11.3, N512 13.5 / 18.3; gradients of 16 heads N512 19.7 / 19.0.
+//   fp32 D32 (fp32 matrix pipe): gradients N128 11.5 / 9.4, N256 11.9 / 16.8; D128: always cut (N128 30.9 / 35.5).
+//   non-causal, 16-bit D64: 2 heads N512 7.9 / 6.6 forward, 8.4 / 8.2 gradients, N768 8.4 / 8.7; 12 heads N768 9.2 / 8.9, 11.3 /
+//   10.7.  D128: 2 heads N256 9.4 / 7.4, 10.2 / 9.7; 12 heads N512 13.0 / 11.7, 17.6 / 16.0; 32 heads N768 18.1 / 16.6 forward.
+//   (the fp32 non-causal form goes through the workspace in any case)
+int one_group_chunks(long BH, int nops, int di, int dj, int dtype, bool causal) {
+    const int pi = cott::mfma_pad(di), pj = cott::mfma_pad(dj);
+    if (dtype == COTT_F32) {
+        if (!causal) return 0;
+        if (pi == 64 && pj == 64) return nops == 3 && BH >= 16 ? 8 : 4;
+        return pi <= 64 && pj <= 64 ? 2 : 0;
+    }
+    const bool wide = pi > 64 || pj > 64, forward = nops == 1;
+    if (!causal) return wide ? (forward && BH >= 32 ? 12 : BH >= 8 ? 8 : 4) : (BH >= 8 ? 12 : 8);
+    if (wide) return forward ? (BH >= 16 ? 12 : BH >= 8 ? 8 : 4) : (BH >= 8 ? 12 : 8);
+    return forward ? (BH >= 8 ? 16 : 12) : (BH >= 8 || pi + pj == 64 ? 12 : 8);
+}
+
 SetPlan plan_set(long BH, int N, int nops, int di, int dj, bool causal, int dtype, bool no_split = false,
                  bool has_ext = false) {
     SetPlan p;
@@ -256,6 +282,17 @@ SetPlan plan_set(long BH, int N, int nops, int di, int dj, bool causal, int dtyp
         const bool groups = g_of[1] > 2 ? cpg_of[1] >= (wide ? 16 : 32) : (cpg_of[1] >= 64 && 2 * BH * 20 <= tgt * 17);
         best_h = groups ? 1 : 2;
         best_g = groups ? (int)g_of[1] : 1;
+    }
+    // Short sequences of few heads: one group, however few workgroups that is.  Column halves where there is room for
+    // them, but not of three causal gradient problems of tiles up to 64 x 64 (whole and separate, they are lighter than a
+    // pair workgroup, see use_pair) nor halves below 64 columns beside 128-wide rows (the input preparation inside the
+    // forward is not built for those).
+    if (pol < 0 && p.nchunks <= one_group_chunks(BH, nops, di, dj, dtype, causal)) {
+        best_g = 1;
+        best_h = can_split && BH * nops * 2 <= tgt && !(causal && nops == 3 && small_tiles) &&
+                         !(cott::mfma_pad(di) == 128 && dj < 128)
+                     ? 2
+                     : 1;
     }
     // Non-causal forward of small heads, more heads than CUs but at most half of the workgroups that can be resident
     // (three per CU): the one-workgroup-per-head kernel runs its two passes over a short sequence, and twice as many

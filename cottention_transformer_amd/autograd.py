@@ -283,6 +283,12 @@ class InputProjections(torch.autograd.Function):
         return tuple(grads)
 
 
+def linear_hooks_installed():
+    """Whether hooks are registered for every module of the process."""
+    m = torch.nn.modules.module
+    return bool(getattr(m, "_global_forward_hooks", None) or getattr(m, "_global_forward_pre_hooks", None))
+
+
 def _is_plain_linear(lin):
     """Whether calling the layer is nothing but x w^T + b with the parameters it holds: exactly torch.nn.Linear, no
     forward (pre-)hooks and no parametrization.  Adapters, quantised linears and hooked layers must be CALLED."""
@@ -290,8 +296,7 @@ def _is_plain_linear(lin):
         return False
     if lin._forward_hooks or lin._forward_pre_hooks or getattr(lin, "_forward_hooks_with_kwargs", None):
         return False
-    if getattr(torch.nn.modules.module, "_global_forward_hooks", None) or getattr(
-            torch.nn.modules.module, "_global_forward_pre_hooks", None):
+    if linear_hooks_installed():
         return False
     return not torch.nn.utils.parametrize.is_parametrized(lin)
 

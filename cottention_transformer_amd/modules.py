@@ -17,7 +17,10 @@ from torch import nn
 from . import ops
 from .autograd import (CustomAttention, CustomAttentionMergedHeads, NonCausalAttention,
                        NonCausalAttentionMergedHeads, PreparedCausalAttention, PreparedNonCausalAttention, PrepareInputs,
-                       _autocast_target, _is_plain_linear, project)
+                       _autocast_target, linear_hooks_installed, project)
+
+
+_DECODE_BLOCK_TYPES = (torch.bfloat16, torch.float16)
 
 
 def _autocast_on():
@@ -115,25 +118,34 @@ class GPTCosAttention(nn.Module):
             table = self.embed_positions = table.to(device)
         return cached[1], table
 
-    def _decode_block_ready(self, hidden_states):
-        """Whether one new token can take ops.decode_block: nothing to differentiate (neither backwards nor forwards), no
-        autocast, 16-bit hidden states of few sequences, and four plain projections without bias whose weights are
-        ordinary contiguous parameters of the same type."""
+    def _decode_block_weights(self, hidden_states):
+        """The four projection weights when one new token can take ops.decode_block, else None.  It can when there is
+        nothing to differentiate (neither backwards nor forwards), no autocast, 16-bit hidden states of few sequences, and
+        four plain projections without bias whose weights are ordinary contiguous parameters of the same type.  Runs for
+        every token, so it reads the modules' dictionaries directly (nn.Module.__getattr__ is most of the cost
+        otherwise)."""
         dt = hidden_states.dtype
-        if (torch.is_grad_enabled() or torch.autograd.forward_ad._current_level >= 0 or _autocast_on()
-                or dt not in (torch.bfloat16, torch.float16) or not hidden_states.is_cuda
-                or type(hidden_states) is not torch.Tensor or hidden_states.shape[0] > ops.DECODE_BLOCK_ROWS
-                or hidden_states.dim() != 3 or hidden_states.shape[0] == 0):
-            return False
+        shape = hidden_states.shape
+        if (torch.is_grad_enabled() or dt not in _DECODE_BLOCK_TYPES or type(hidden_states) is not torch.Tensor
+                or len(shape) != 3 or not 0 < shape[0] <= ops.DECODE_BLOCK_ROWS or not hidden_states.is_cuda
+                or torch.autograd.forward_ad._current_level >= 0 or _autocast_on() or linear_hooks_installed()):
+            return None
         e, dev = self.embed_dim, hidden_states.device
-        for lin in (self.q_proj, self.k_proj, self.v_proj, self.out_proj):
-            if not _is_plain_linear(lin) or lin.bias is not None:
-                return False
-            w = lin.weight
-            if (type(w) is not nn.Parameter or w.dtype != dt or w.device != dev or w.shape != (e, e)
-                    or not w.is_contiguous() or w.data_ptr() % 16 != 0):
-                return False
-        return hidden_states.shape[2] == e and hidden_states.data_ptr() % 16 == 0
+        if shape[2] != e or hidden_states.data_ptr() % 16 != 0:
+            return None
+        weights = []
+        modules = self._modules
+        for name in ("q_proj", "k_proj", "v_proj", "out_proj"):
+            lin = modules.get(name)
+            if type(lin) is not nn.Linear or lin._forward_hooks or lin._forward_pre_hooks or "parametrizations" in lin._modules:
+                return None
+            params = lin._parameters
+            w = params.get("weight")
+            if (type(w) is not nn.Parameter or params.get("bias") is not None or w.dtype != dt or w.device != dev
+                    or w.shape != (e, e) or not w.is_contiguous() or w.data_ptr() % 16 != 0):
+                return None
+            weights.append(w)
+        return weights
 
     def _unmasked_side_inputs(self, b, s, device):
         """Keep mask (all true) and running count of kept keys (1, 2, ..., s) of a batch without padding: constants,
@@ -222,13 +234,13 @@ class GPTCosAttention(nn.Module):
                      and use_cache is not True and not output_attentions and attention_mask is None
                      and self.head_dim in (32, 64, 128, 256) and self.rotary_dim is not None
                      and self.rotary_dim % 2 == 0 and self.rotary_dim <= self.head_dim)
-        if one_token and self._decode_block_ready(hidden_states):
+        weights = self._decode_block_weights(hidden_states) if one_token else None
+        if weights is not None:
             b, dev = hidden_states.shape[0], hidden_states.device
             if self.state is None:
                 self.state = torch.zeros(b, self.num_attention_heads, self.head_dim, self.head_dim, device=dev)
             sig, table = self._decode_side_inputs(dev)
-            out = ops.decode_block(hidden_states[:, 0], self.q_proj.weight, self.k_proj.weight, self.v_proj.weight,
-                                   self.out_proj.weight, self.state, sig=sig, cnt=float(self.cur_s),
+            out = ops.decode_block(hidden_states[:, 0], *weights, self.state, sig=sig, cnt=float(self.cur_s),
                                    rotary=(table, self.cur_s - 1))
             self.cur_s += 1
             return (self.resid_dropout(out[:, None]), None)

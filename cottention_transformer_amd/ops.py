@@ -536,16 +536,17 @@ def decode_block(x, wq, wk, wv, wo, state, sig=None, cnt=0.0, rotary=None):
     the returned y = o wo^T.  x: (B,E) bf16 / fp16; weights (E,E), contiguous and 16-byte aligned, in x's type;
     sig, cnt, rotary as in decode_step_prepared."""
     _require_gpu(x=x, wq=wq, wk=wk, wv=wv, wo=wo, state=state)
+    dt = x.dtype
     code = _dtype_code(x)
     if x.dim() != 2 or state.dim() != 4:
         raise RuntimeError("decode_block: x (B,E), state (B,H,D,D)")
     b, e = x.shape
-    h, d = state.shape[1:3]
-    if state.shape != (b, h, d, d) or h * d != e or state.dtype != torch.float32 or not state.is_contiguous():
+    sb, h, d, d2 = state.shape
+    if sb != b or d2 != d or h * d != e or state.dtype != torch.float32 or not state.is_contiguous():
         raise RuntimeError(f"decode_block: state must be a contiguous float32 (B,H,D,D) tensor with H * D = {e}")
     for w in (wq, wk, wv, wo):
-        if w.shape != (e, e) or w.dtype != x.dtype or not w.is_contiguous():
-            raise RuntimeError(f"decode_block: weights must be contiguous {(e, e)} tensors of type {x.dtype}")
+        if w.shape != (e, e) or w.dtype != dt or not w.is_contiguous():
+            raise RuntimeError(f"decode_block: weights must be contiguous {(e, e)} tensors of type {dt}")
     if sig is not None and (sig.shape != (h,) or sig.dtype != torch.float32 or sig.device != x.device or not sig.is_contiguous()):
         raise RuntimeError(f"decode_block: sig must be a contiguous float32 tensor of shape {(h,)} on x's device")
     table, pos, rdim, rows = None, 0, 0, 0

@@ -50,7 +50,7 @@ class CustomAttention(torch.autograd.Function):
             ctx.save_for_backward(Q, K, V, *(() if states is None else (states,)))
             return out
         ctx.save_for_backward(Q, K, V)  # saved before any autocast conversion (Custom_Kernel.py:16)
-        return ops.causal_dot_product(Q.to(dt), K.to(dt), V.to(dt), False)
+        return ops.causal_dot_product_as(Q, K, V, dt)
 
     @staticmethod
     def backward(ctx, grad_output):

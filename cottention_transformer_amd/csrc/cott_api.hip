@@ -137,6 +137,7 @@ struct Op {
     void *sout = nullptr;
     unsigned char lay[4] = {0, 0, 0, 0};  // A, B, C, O given as (B,N,H,width) instead of (BH,N,width)
     int H = 1;
+    bool f32_in = false;  // A, B, C are fp32 tensors of an op in bf16 (cott_causal_fwd_f32in)
     // states handed from a forward to a backward pass (cott_causal_fwd_save / cott_causal_bwd_saved)
     void *save = nullptr;       // (BH, save_n, pad(di) * pad(dj)) fp32 in 16 x 16 tiles: written by a forward op
     const void *ext = nullptr;  // the same array, read by the backward op that sums over the past (dQ)
@@ -544,7 +545,7 @@ int run_ops(const char *fn, bool causal, const Op *ops, int n, long BH, int N, i
                 cott::OpDesc &d = a.op[a.count++];
                 d.A = o.A;
                 d.B = o.B;
-                d.C = static_cast<const char *>(o.C) + (size_t)h * djh * esz;
+                d.C = static_cast<const char *>(o.C) + (size_t)h * djh * (o.f32_in ? sizeof(float) : esz);
                 d.O = static_cast<char *>(o.O) + (size_t)h * djh * esz;
                 d.di = o.di;
                 d.dj = djh;
@@ -587,6 +588,7 @@ int run_ops(const char *fn, bool causal, const Op *ops, int n, long BH, int N, i
         a.nchunks = p.nchunks; a.cpg = p.cpg; a.G = p.G; a.sub = p.sub;
         a.cus = device_cus();
         a.xcds = device_xcds();
+        a.f32_in = ops[i].f32_in;
         a.scan_prof_id = n > 1 ? cott::K_SCAN_GRAD : cott::K_SCAN;
         a.stream = stream;
         hipError_t e;
@@ -672,6 +674,31 @@ int cott_causal_fwd(const void *q, const void *k, const void *v, void *o, int B,
         return fail(COTT_ERR_INVALID, "%s: tensor pointers must be 16-byte aligned", fn);
     const Op op{q, k, v, o, Dk, Dv, reversed ? 1 : 0};
     return run_ops(fn, true, &op, 1, (long)B * H, N, dtype, workspace, workspace_bytes, static_cast<hipStream_t>(stream));
+}
+
+int cott_causal_fwd_f32in_supported(int B, int H, int N, int Dk, int Dv) {
+    if (B < 0 || H < 0 || N < 0 || Dk % 16 != 0 || Dk < 32 || (long)B * H > (1L << 22)) return 0;
+    if (!use_mfma(COTT_BF16, Dk, Dv, N) || !use_mfma(COTT_F32, Dk, Dv, N)) return 0;
+    if ((long)B * H * N == 0) return 1;
+    const SetPlan p = plan_set((long)B * H, N, 1, Dk, Dv, true, COTT_BF16);
+    const int pk = cott::mfma_pad(Dk), pv = cott::mfma_pad(Dv / p.halves);
+    return p.G == 1 && pk <= 64 && pk * pv <= 128 * 64;
+}
+
+int cott_causal_fwd_f32in(const float *q, const float *k, const float *v, void *o, int B, int H, int N, int Dk, int Dv,
+                          void *stream) {
+    const char *fn = "cott_causal_fwd_f32in";
+    if (int rc = check_common(fn, B, H, N, Dk, Dv, COTT_F32)) return rc;
+    if (!cott_causal_fwd_f32in_supported(B, H, N, Dk, Dv))
+        return fail(COTT_ERR_UNSUPPORTED, "%s: not built for this shape (cott_causal_fwd_f32in_supported); convert the tensors "
+                    "and use cott_causal_fwd", fn);
+    if ((long)B * H * N == 0) return COTT_OK;
+    if (!q || !k || !v || !o) return fail(COTT_ERR_INVALID, "%s: null tensor pointer", fn);
+    if (!aligned16(q) || !aligned16(k) || !aligned16(v) || !aligned16(o))
+        return fail(COTT_ERR_INVALID, "%s: tensor pointers must be 16-byte aligned", fn);
+    Op op{q, k, v, o, Dk, Dv, 0};
+    op.f32_in = true;
+    return run_ops(fn, true, &op, 1, (long)B * H, N, COTT_BF16, nullptr, 0, static_cast<hipStream_t>(stream));
 }
 
 int cott_causal_fwd_may_alias_v(int B, int H, int N, int Dk, int Dv, int dtype) {

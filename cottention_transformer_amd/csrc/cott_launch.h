@@ -49,6 +49,9 @@ struct SetArgs {
     // non-temporal loads in the group-state pass / in the scan: for tensors far larger than the caches, when no
     // two problems of the set read the same operand
     bool stream_state = false, stream_scan = false;
+    // the operands of a forward pass (16-bit op, G = 1, contracted dim padded to at most 64) are fp32 tensors, rounded
+    // inside the kernel
+    bool f32_in = false;
     int cus = 256, xcds = 8;  // CUs and XCDs of the device (placement and occupancy choices)
     // Input preparation inside the causal forward (16-bit, one group per head): q, k, v of the ops are the raw
     // projections; see PrepSide in cott_mfma.h for the meaning of the fields.  prep_on = false: none.

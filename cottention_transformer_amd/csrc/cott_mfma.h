@@ -579,32 +579,37 @@ struct StagedOut {
     const u16 *sO;  // [2 buffers][2 tiles][64 * OS]
 };
 
+// Loader threads: the staged tile(s) of chunk p (scan order) to memory as 16-byte row segments; rows past N are dropped by
+// the range check
+template <int DJ, int LT>
+__device__ __forceinline__ void write_staged(const StagedOut &so, const ScanRange &r, int p, int tid) {
+    constexpr int OS = DJ + 8, SO = kChunk * OS;  // Tiling::OS
+    const int row0 = (r.reversed ? r.nchunks - 1 - p : p) * kChunk;
+#pragma unroll
+    for (int t = 0; t < 2; ++t) {
+        if (so.O[t] == nullptr) continue;
+        const rsrc_t rO = make_rsrc(so.O[t], ((uint32_t)(r.N - 1) * so.ld[t] + so.dj[t]) * 2u);
+        const u16 *tile = so.sO + (((p - r.p0) & 1) * 2 + t) * SO;
+#pragma unroll
+        for (int u = 0; u < 8 * DJ / LT; ++u) {
+            const int v = tid + LT * u;
+            const int row = v / (DJ / 8), col = (v % (DJ / 8)) * 8;
+            const u32x4 val = *reinterpret_cast<const u32x4 *>(tile + row * OS + col);
+            const uint32_t off = (col < so.dj[t]) ? (uint32_t)((row0 + row) * so.ld[t] + col) * 2u : kOobOffset;
+            __builtin_amdgcn_raw_buffer_store_b128(val, rO, (int)off, 0, 0);
+        }
+    }
+}
+
 template <int DI, int DJ, int PF, int LT, bool STREAM = false>
 __device__ __forceinline__ void loader_role(const u16 *B_head, const u16 *C_head, int di, int dj, int ldb, int ldc,
                                             const ScanRange &r, int tid, u16 *sB, u16 *sC,
                                             const StagedOut *so = nullptr) {
     using TL = Tiling<DI, DJ>;
-    constexpr int SB = kChunk * TL::BS, SC = kChunk * TL::CS, SO = kChunk * TL::OS;
+    constexpr int SB = kChunk * TL::BS, SC = kChunk * TL::CS;
     const rsrc_t rB = make_rsrc(B_head, ((uint32_t)(r.N - 1) * ldb + di) * 2u);
     const rsrc_t rC = make_rsrc(C_head, ((uint32_t)(r.N - 1) * ldc + dj) * 2u);
-    // the staged tile(s) of chunk p (scan order): 16-byte row segments, rows past N dropped by the range check
-    auto write_out = [&](int p) __attribute__((always_inline)) {
-        const int row0 = (r.reversed ? r.nchunks - 1 - p : p) * kChunk;
-#pragma unroll
-        for (int t = 0; t < 2; ++t) {
-            if (so->O[t] == nullptr) continue;
-            const rsrc_t rO = make_rsrc(so->O[t], ((uint32_t)(r.N - 1) * so->ld[t] + so->dj[t]) * 2u);
-            const u16 *tile = so->sO + (((p - r.p0) & 1) * 2 + t) * SO;
-#pragma unroll
-            for (int u = 0; u < 8 * DJ / LT; ++u) {
-                const int v = tid + LT * u;
-                const int row = v / (DJ / 8), col = (v % (DJ / 8)) * 8;
-                const u32x4 val = *reinterpret_cast<const u32x4 *>(tile + row * TL::OS + col);
-                const uint32_t off = (col < so->dj[t]) ? (uint32_t)((row0 + row) * so->ld[t] + col) * 2u : kOobOffset;
-                __builtin_amdgcn_raw_buffer_store_b128(val, rO, (int)off, 0, 0);
-            }
-        }
-    };
+    auto write_out = [&](int p) __attribute__((always_inline)) { write_staged<DJ, LT>(*so, r, p, tid); };
     u32x4 rb[PF][8 * DI / LT], rc[PF][8 * DJ / LT];
     auto load_chunk = [&](int s, int p) __attribute__((always_inline)) {
         const int pc = min(p, r.p1 - 1);
@@ -629,6 +634,69 @@ __device__ __forceinline__ void loader_role(const u16 *B_head, const u16 *C_head
         chunk_barrier();
     });
     if (so != nullptr && r.p1 > r.p0) write_out(r.p1 - 1);
+}
+
+// Loader role for fp32 operands of a 16-bit op: the A, B and C rows are rounded to TR on their way into the tiles (A too,
+// from where the output wavefronts take it), exactly as a conversion of the whole tensors beforehand would round them.
+template <class TR, int DI, int DJ, int PF, int LT>
+__device__ __forceinline__ void loader_role_f32(const float *A_head, const float *B_head, const float *C_head, int di, int dj,
+                                                int lda, int ldb, int ldc, const ScanRange &r, int tid, u16 *sA, u16 *sB,
+                                                u16 *sC, const StagedOut *so) {
+    using TL = Tiling<DI, DJ>;
+    constexpr int SB = kChunk * TL::BS, SC = kChunk * TL::CS, NI = 8 * DI / LT, NJ = 8 * DJ / LT;
+    const rsrc_t rA = make_rsrc(A_head, ((uint32_t)(r.N - 1) * lda + di) * 4u);
+    const rsrc_t rB = make_rsrc(B_head, ((uint32_t)(r.N - 1) * ldb + di) * 4u);
+    const rsrc_t rC = make_rsrc(C_head, ((uint32_t)(r.N - 1) * ldc + dj) * 4u);
+    u32x4 ra[PF][2 * NI], rb[PF][2 * NI], rc[PF][2 * NJ];  // a piece of eight columns is two loads
+    auto load_rows = [&](u32x4 *dst, rsrc_t rs, auto width, int row0, int ld) __attribute__((always_inline)) {
+        constexpr int D = decltype(width)::value;
+#pragma unroll
+        for (int u = 0; u < 8 * D / LT; ++u) {
+            const int v = tid + LT * u;
+            const uint32_t off = (uint32_t)((row0 + v / (D / 8)) * ld + (v % (D / 8)) * 8) * 4u;
+            dst[2 * u] = buf_load16(rs, off);
+            dst[2 * u + 1] = buf_load16(rs, off + 16u);
+        }
+    };
+    auto store_rows = [&](u16 *tile, const u32x4 *src, auto width, int stride, int d) __attribute__((always_inline)) {
+        constexpr int D = decltype(width)::value;
+#pragma unroll
+        for (int u = 0; u < 8 * D / LT; ++u) {
+            const int v = tid + LT * u, col = (v % (D / 8)) * 8;
+            u32x4 x;
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+                x[e] = TR::pack2(bitcast<float>(src[2 * u + e / 2][2 * (e & 1)]), bitcast<float>(src[2 * u + e / 2][2 * (e & 1) + 1]));
+            *reinterpret_cast<u32x4 *>(tile + (v / (D / 8)) * stride + col) = col < d ? x : u32x4{0u, 0u, 0u, 0u};
+        }
+    };
+    constexpr std::integral_constant<int, DI> WI{};
+    constexpr std::integral_constant<int, DJ> WJ{};
+    auto load_chunk = [&](int s, int p) __attribute__((always_inline)) {
+        const int pc = min(p, r.p1 - 1);
+        const int row0 = (r.reversed ? r.nchunks - 1 - pc : pc) * kChunk;
+        load_rows(ra[s], rA, WI, row0, lda);
+        load_rows(rb[s], rB, WI, row0, ldb);
+        load_rows(rc[s], rC, WJ, row0, ldc);
+    };
+    auto stage = [&](int s, int buf) __attribute__((always_inline)) {
+        store_rows(sA + buf * SB, ra[s], WI, TL::BS, di);
+        store_rows(sB + buf * SB, rb[s], WI, TL::BS, di);
+        store_rows(sC + buf * SC, rc[s], WJ, TL::CS, dj);
+    };
+#pragma unroll
+    for (int s = 0; s < PF; ++s) load_chunk(s, r.p0 + s);
+    stage(0, 0);
+    load_chunk(0, r.p0 + PF);
+    __syncthreads();
+    run_rounds<PF>(r.p0, r.p1, [&](int s, int p) __attribute__((always_inline)) {
+        const int s1 = (s + 1) % PF, buf = (p - r.p0) & 1;
+        stage(s1, buf ^ 1);
+        load_chunk(s1, p + 1 + PF);
+        if (so != nullptr && p > r.p0) write_staged<DJ, LT>(*so, r, p - 1, tid);
+        chunk_barrier();
+    });
+    if (so != nullptr && r.p1 > r.p0) write_staged<DJ, LT>(*so, r, r.p1 - 1, tid);
 }
 
 // Loader role with the input preparation folded in (see PrepSide): same pipeline as loader_role, for THREE tiles:
@@ -1111,10 +1179,13 @@ __device__ __forceinline__ void one_block_variant(int block, bool future, F &&f)
 
 // One problem per workgroup: OW output wavefronts (IB = 4/OW blocks each), 4 state, LW loader.
 // PREP: q, k, v are the raw projections and are prepared inside the kernel (PrepSide; forward direction, G = 1).
+// F32IN: A, B and C are fp32 tensors (the pointers of the set are to floats), rounded by the loader wavefronts (G = 1).  The
+// forward pass of a trainer that feeds fp32 tensors under autocast, B8 H16 N2048 D64: 43 us (224 MiB, 5.5 TB/s), where three
+// conversions of 18 us and the forward on their results took 93; training step 258 -> 208 us.
 // WST: every output wavefront passes its tiles through a small staging tile of its own in LDS and stores them as
 // 16-byte pieces that make up whole 128-byte row segments (where a workgroup-wide staged tile, STAGED, has no room).
 template <class TR, int DI, int DJ, int PF, int OW, int LW, bool STAGED = false, bool STREAM = false, bool PREP = false,
-          bool WST = false>
+          bool WST = false, bool F32IN = false>
 __global__ __launch_bounds__(64 * (OW + 4 + LW)) void scan_kernel(ProblemSet set, int BH, int N, int nchunks,
                                                                   int cpg, int G, PrepSide prep) {
     using TL = Tiling<DI, DJ>;
@@ -1130,7 +1201,8 @@ __global__ __launch_bounds__(64 * (OW + 4 + LW)) void scan_kernel(ProblemSet set
     // STAGED: output tiles go through LDS and leave as 16-byte row segments from the loader wavefronts (StagedOut;
     // the layout has room for two tiles per buffer, this kernel uses the first)
     __shared__ __attribute__((aligned(16))) u16 sO[STAGED ? 2 * 2 * kChunk * TL::OS : 8];
-    __shared__ __attribute__((aligned(16))) u16 sA[PREP ? 2 * SB : 8];  // PREP: the prepared A rows, staged like sB
+    constexpr bool ALDS = PREP || F32IN;  // the A rows are staged too, like sB
+    __shared__ __attribute__((aligned(16))) u16 sA[ALDS ? 2 * SB : 8];
     static_assert(!WST || (!STAGED && 4 / OW == 2 && DJ % 64 == 0), "wave-staged stores: two blocks per wavefront");
     __shared__ __attribute__((aligned(16))) u16 sWst[WST ? OW * 32 * kWaveStageStride : 8];
     const int l = threadIdx.x & 63;
@@ -1156,7 +1228,13 @@ __global__ __launch_bounds__(64 * (OW + 4 + LW)) void scan_kernel(ProblemSet set
         so.dj[1] = 0;
         so.ld[1] = 0;
         so.sO = sO;
-        if constexpr (PREP)
+        if constexpr (F32IN)
+            loader_role_f32<TR, DI, DJ, PF, LT>(reinterpret_cast<const float *>(pr.A) + head_base(pr.bsA, pr.hsA, pr.H, wi.bh),
+                                                reinterpret_cast<const float *>(pr.B) + head_base(pr.bsB, pr.hsB, pr.H, wi.bh),
+                                                reinterpret_cast<const float *>(pr.C) + head_base(pr.bsC, pr.hsC, pr.H, wi.bh),
+                                                di, dj, pr.lda, pr.ldb, ldc, r, (int)threadIdx.x - 64 * (OW + 4), sA, sB, sC,
+                                                STAGED ? &so : nullptr);
+        else if constexpr (PREP)
             loader_role_prep<TR, DI, DJ, PF, LT>(pr.A + head_base(pr.bsA, pr.hsA, pr.H, wi.bh),
                                                  pr.B + head_base(pr.bsB, pr.hsB, pr.H, wi.bh),
                                                  pr.C + head_base(pr.bsC, pr.hsC, pr.H, wi.bh), di, dj, pr.lda, pr.ldb, ldc,
@@ -1190,23 +1268,23 @@ __global__ __launch_bounds__(64 * (OW + 4 + LW)) void scan_kernel(ProblemSet set
             u16 *sW = sWst + (WST ? wv * 32 * kWaveStageStride : 0);
             if (future) {
                 if (wv == 0)
-                    output_role<TR, DI, DJ, PF, 2, STREAM, PREP, 1, false, WST>(A_head, O_head, di, dj, pr.lda, pr.ldo, r, 0, l,
+                    output_role<TR, DI, DJ, PF, 2, STREAM, ALDS, 1, false, WST>(A_head, O_head, di, dj, pr.lda, pr.ldo, r, 0, l,
                                                                                       sB, sC, sS, STAGED ? sO : nullptr, sA, sW);
                 else
-                    output_role<TR, DI, DJ, PF, 2, STREAM, PREP, 2, false, WST>(A_head, O_head, di, dj, pr.lda, pr.ldo, r, 0, l,
+                    output_role<TR, DI, DJ, PF, 2, STREAM, ALDS, 2, false, WST>(A_head, O_head, di, dj, pr.lda, pr.ldo, r, 0, l,
                                                                                       sB, sC, sS, STAGED ? sO : nullptr, sA, sW);
             } else {
                 if (wv == 0)
-                    output_role<TR, DI, DJ, PF, 2, STREAM, PREP, 3, false, WST>(A_head, O_head, di, dj, pr.lda, pr.ldo, r, 0, l,
+                    output_role<TR, DI, DJ, PF, 2, STREAM, ALDS, 3, false, WST>(A_head, O_head, di, dj, pr.lda, pr.ldo, r, 0, l,
                                                                                       sB, sC, sS, STAGED ? sO : nullptr, sA, sW);
                 else
-                    output_role<TR, DI, DJ, PF, 2, STREAM, PREP, 4, false, WST>(A_head, O_head, di, dj, pr.lda, pr.ldo, r, 0, l,
+                    output_role<TR, DI, DJ, PF, 2, STREAM, ALDS, 4, false, WST>(A_head, O_head, di, dj, pr.lda, pr.ldo, r, 0, l,
                                                                                       sB, sC, sS, STAGED ? sO : nullptr, sA, sW);
             }
         } else {
             // one block per wavefront: the variant that knows its block and the side of the diagonal that counts
             one_block_variant(wv, (pr.mask_rev != 0) != (pr.comp != 0), [&](auto tag) {
-                output_role<TR, DI, DJ, PF, 1, STREAM, PREP, 5 + decltype(tag)::value>(
+                output_role<TR, DI, DJ, PF, 1, STREAM, ALDS, 5 + decltype(tag)::value>(
                     A_head, O_head, di, dj, pr.lda, pr.ldo, r, wv, l, sB, sC, sS, STAGED ? sO : nullptr, sA);
             });
         }

@@ -165,6 +165,30 @@ def causal_dot_product(q, k, v, reversed=False, merged_heads=False, into_v=False
     return o
 
 
+_f32in_cache = {}
+
+
+def causal_dot_product_as(q, k, v, dtype):
+    """causal_dot_product(q.to(dtype), k.to(dtype), v.to(dtype)): the rule of an autocast forward pass
+    (Cuda_Kernel/combined_kernel_general.cu:377-389).  fp32 tensors computed in bf16 are rounded inside the kernel where that
+    is built (cott_causal_fwd_f32in_supported), bit for bit as the conversions round them."""
+    if dtype is torch.bfloat16 and q.dtype == k.dtype == v.dtype == torch.float32 and q.is_cuda:
+        _require_gpu(Q=q, K=k, V=v)
+        b, h, n, dk, dv = shape = _shapes(q, k, v)
+        ok = _f32in_cache.get(shape)
+        if ok is None:
+            ok = _remember(_f32in_cache, shape, bool(_loader.lib().cott_causal_fwd_f32in_supported(*shape)))
+        q, k, v = q.contiguous(), k.contiguous(), v.contiguous()
+        if ok and not (q.data_ptr() | k.data_ptr() | v.data_ptr()) & 15:
+            o = torch.empty((b, h, n, dv), dtype=dtype, device=q.device)
+            with _on(q.device):
+                rc = _loader.lib().cott_causal_fwd_f32in(q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(), b, h, n, dk,
+                                                         dv, _stream(q.device))
+            _check(rc, "cott_causal_fwd_f32in")
+            return o
+    return causal_dot_product(q.to(dtype), k.to(dtype), v.to(dtype))
+
+
 _saved_plan_cache = {}
 
 

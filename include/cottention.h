@@ -56,6 +56,13 @@ COTT_API size_t cott_causal_workspace_bytes(int B, int H, int N, int Dk, int Dv,
 COTT_API int cott_causal_fwd(const void *q, const void *k, const void *v, void *o,
                     int B, int H, int N, int Dk, int Dv, int dtype, int reversed,
                     void *workspace, size_t workspace_bytes, void *stream);
+/* cott_causal_fwd in bf16 on fp32 tensors, which the kernel rounds as it reads them (o is bf16): the forward pass of an
+ * autocast step (Cuda_Kernel/combined_kernel_general.cu:377-389) without converted copies of q, k and v.  Built where
+ * cott_causal_fwd_f32in_supported answers 1 (heads that are one sequence group, Dk <= 64); needs no workspace. */
+COTT_API int cott_causal_fwd_f32in_supported(int B, int H, int N, int Dk, int Dv);
+COTT_API int cott_causal_fwd_f32in(const float *q, const float *k, const float *v, void *o,
+                      int B, int H, int N, int Dk, int Dv, void *stream);
+
 /* inplace=True of forward_<T> (combined_kernel_general.cu:403-404: the output tensor IS V).  Returns 1 when
  * cott_causal_fwd may be called with o == v for this shape and dtype (every workgroup has read the rows and
  * columns of v it needs before it, or any other workgroup, writes them as o): the MFMA kernels, i.e. bf16 / fp16 /

@@ -1,0 +1,43 @@
+"""Autocast forward on fp32 tensors: rounded inside the kernel, bit for bit what the op gives on converted tensors."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+F32, BF = torch.float32, torch.bfloat16
+
+
+@pytest.fixture(scope="module")
+def ct():
+    import cottention_transformer_amd as ct_
+    return ct_
+
+
+# widths below their padding, ragged lengths, one chunk, column halves, more workgroups than CUs (two output wavefronts)
+@pytest.mark.parametrize("case", [(1, 2, 128, 64, 64), (1, 1, 1, 32, 32), (1, 5, 63, 48, 32), (2, 20, 300, 64, 96), (20, 16, 100, 64, 64),
+                                  (20, 16, 65, 48, 128), (8, 16, 1023, 64, 64), (3, 50, 130, 32, 64)],
+                         ids=lambda c: "x".join(map(str, c)))
+def test_equals_converted_tensors(ct, case):
+    from cottention_transformer_amd import _loader, ops
+    b, h, n, dk, dv = case
+    assert _loader.lib().cott_causal_fwd_f32in_supported(*case) == 1
+    g = torch.Generator().manual_seed(n)
+    q, k, v = (torch.randn(b, h, n, d, generator=g).to(DEV) for d in (dk, dk, dv))
+    got, want = ops.causal_dot_product_as(q, k, v, BF), ops.causal_dot_product(q.to(BF), k.to(BF), v.to(BF))
+    assert got.dtype == BF and torch.equal(got, want)
+
+
+def test_other_calls_convert(ct):
+    """Sequence groups, wide rows, unaligned and mixed tensors take the conversion; CustomAttention's result is the same."""
+    from cottention_transformer_amd import _loader, ops
+    assert _loader.lib().cott_causal_fwd_f32in_supported(1, 2, 4096, 64, 64) == 0
+    assert _loader.lib().cott_causal_fwd_f32in_supported(8, 16, 256, 128, 128) == 0
+    q, k, v = (torch.randn(1, 2, 129 * 64, device=DEV)[..., 64:].contiguous().view(1, 2, 128, 64) for _ in range(3))
+    odd = torch.randn(2 * 128 * 64 + 1, device=DEV)[1:].view(1, 2, 128, 64)  # 4 bytes past an aligned address
+    for x in (q, odd, q.half().float(), q.double().float().to(BF)):
+        got = ops.causal_dot_product_as(x, k, v, BF)
+        assert torch.equal(got, ops.causal_dot_product(x.to(BF).clone(), k.to(BF), v.to(BF)))
+    with torch.autocast("cuda", dtype=BF):
+        out = ct.CustomAttention.apply(q.requires_grad_(True), k, v)
+    assert torch.equal(out, ops.causal_dot_product(q.detach().to(BF), k.to(BF), v.to(BF)))
+    assert torch.autograd.grad(out.float().sum(), q)[0].dtype == F32

@@ -36,6 +36,8 @@ SIGNATURES = {
     "cott_causal_fwd_may_alias_v": (_i, [_i] * 6),
     "cott_causal_bwd_workspace_bytes": (_sz, [_i] * 6),
     "cott_causal_bwd": (_i, [_vp] * 7 + [_i] * 6 + [_vp, _sz, _vp]),
+    "cott_causal_bwd_g16_supported": (_i, [_i] * 5),
+    "cott_causal_bwd_g16": (_i, [_vp] * 7 + [_i] * 5 + [_vp, _sz, _vp]),
     "cott_causal_saved_plan": (_i, [_i] * 6 + [ctypes.POINTER(_i)] * 3 + [ctypes.POINTER(_sz)]),
     "cott_causal_fwd_save": (_i, [_vp] * 5 + [_i] * 8 + [_vp, _sz, _vp]),
     "cott_causal_bwd_saved": (_i, [_vp] * 8 + [_i] * 8 + [_vp, _sz, _vp]),

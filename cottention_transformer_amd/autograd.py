@@ -59,8 +59,10 @@ class CustomAttention(torch.autograd.Function):
             raise ValueError("Only float32, float64, float16, and bfloat16 are supported")
         # One fused call in the saved tensors' dtype replaces the three launches of
         # Custom_Kernel.py:106-108 (same operand permutations inside the library).
-        g = grad_output.contiguous().to(Q.dtype)
-        grads = ops.causal_backward(Q, K.to(Q.dtype), V.to(Q.dtype), g, saved=states[0] if states else None)
+        if states:
+            grads = ops.causal_backward(Q, K, V, grad_output.contiguous().to(Q.dtype), saved=states[0])
+        else:
+            grads = ops.causal_backward_from(Q, K.to(Q.dtype), V.to(Q.dtype), grad_output)
         if ctx.grad_dtypes is not None:
             grads = tuple(x.to(t) for x, t in zip(grads, ctx.grad_dtypes))
         return grads

@@ -137,6 +137,7 @@ struct Op {
     void *sout = nullptr;
     unsigned char lay[4] = {0, 0, 0, 0};  // A, B, C, O given as (B,N,H,width) instead of (BH,N,width)
     int H = 1;
+    int bf16_operands = 0;  // fp32 op on split operands: bit 0 / 1 / 2 = A / B / C is a bf16 tensor
     bool f32_in = false;  // A, B, C are fp32 tensors of an op in bf16 (cott_causal_fwd_f32in)
     // states handed from a forward to a backward pass (cott_causal_fwd_save / cott_causal_bwd_saved)
     void *save = nullptr;       // (BH, save_n, pad(di) * pad(dj)) fp32 in 16 x 16 tiles: written by a forward op
@@ -561,6 +562,7 @@ int run_ops(const char *fn, bool causal, const Op *ops, int n, long BH, int N, i
                 d.lds = o.dj;
                 for (int x = 0; x < 4; ++x) d.lay[x] = o.lay[x];
                 d.H = o.H;
+                d.bf16_operands = o.bf16_operands;
                 if (o.save != nullptr) {
                     if (!causal || o.reversed || dtype == COTT_F32)
                         return fail(COTT_ERR_UNSUPPORTED, "%s: states are saved by a forward-direction 16-bit causal op", fn);
@@ -989,6 +991,32 @@ int cott_causal_bwd(const void *q, const void *k, const void *v, const void *d_o
     Op ops[3];
     grad_ops(ops, q, k, v, d_o, dq, dk, dv, Dk, Dv, true);
     return run_ops(fn, true, ops, 3, (long)B * H, N, dtype, workspace, workspace_bytes, static_cast<hipStream_t>(stream));
+}
+
+int cott_causal_bwd_g16_supported(int B, int H, int N, int Dk, int Dv) {
+    if (B < 0 || H < 0 || N < 0 || Dk < 1 || Dv < 1 || (long)B * H > (1L << 22)) return 0;
+    // all three gradients on split operands: padded head dims 64 x 64
+    return use_mfma(COTT_F32, Dk, Dv, N) && cott::mfma_pad(Dk) == 64 && cott::mfma_pad(Dv) == 64 &&
+           exp_int("COTT_F32_SPLIT", 1) != 0;
+}
+
+int cott_causal_bwd_g16(const float *q, const float *k, const float *v, const void *d_o, float *dq, float *dk, float *dv, int B,
+                        int H, int N, int Dk, int Dv, void *workspace, size_t workspace_bytes, void *stream) {
+    const char *fn = "cott_causal_bwd_g16";
+    if (int rc = check_common(fn, B, H, N, Dk, Dv, COTT_F32)) return rc;
+    if (int rc = check_common(fn, B, H, N, Dv, Dk, COTT_F32)) return rc;
+    if (!cott_causal_bwd_g16_supported(B, H, N, Dk, Dv))
+        return fail(COTT_ERR_UNSUPPORTED, "%s: needs head dims of 48 or 64 (cott_causal_bwd_g16_supported); convert d_o and use "
+                    "cott_causal_bwd", fn);
+    if ((long)B * H * N == 0) return COTT_OK;
+    if (!q || !k || !v || !d_o || !dq || !dk || !dv) return fail(COTT_ERR_INVALID, "%s: null tensor pointer", fn);
+    if (!aligned16(q) || !aligned16(k) || !aligned16(v) || !aligned16(d_o) || !aligned16(dq) || !aligned16(dk) ||
+        !aligned16(dv))
+        return fail(COTT_ERR_INVALID, "%s: tensor pointers must be 16-byte aligned", fn);
+    Op ops[3];
+    grad_ops(ops, q, k, v, d_o, dq, dk, dv, Dk, Dv, true);
+    for (Op &o : ops) o.bf16_operands = (o.A == d_o ? 1 : 0) | (o.B == d_o ? 2 : 0) | (o.C == d_o ? 4 : 0);
+    return run_ops(fn, true, ops, 3, (long)B * H, N, COTT_F32, workspace, workspace_bytes, static_cast<hipStream_t>(stream));
 }
 
 namespace {

@@ -20,6 +20,8 @@ struct OpDesc {
     // of a position next to each other, as the projections of a transformer block produce and consume them.
     unsigned char lay[4] = {0, 0, 0, 0};
     int H = 1;  // heads per batch element; needed when any layout flag is set
+    // fp32 ops on split operands only: bit 0 / 1 / 2 = A / B / C is a bf16 tensor (its lo parts are zero)
+    int bf16_operands = 0;
     // Complement form (16-bit causal MFMA kernels, sets with sequence groups only): the op is walked against its
     // own direction so that it reads the same tiles at the same time as the other ops of its set.
     int comp = 0;

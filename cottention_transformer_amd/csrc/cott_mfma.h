@@ -73,6 +73,7 @@ struct ProblemT {
     // scan_pair_kernel only: a second problem G(A2, C, B) -> O2 served by the same workgroup (null = none)
     const E *A2;
     E *O2;
+    int bf16_operands;  // fp32 ops on split operands: bit 0 / 1 / 2 = A / B / C points to bf16 rows (strides in elements)
 };
 
 template <class E>

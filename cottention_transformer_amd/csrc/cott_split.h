@@ -63,26 +63,47 @@ __device__ __forceinline__ f32x4 mfma3(u32x4 ah, u32x4 al, u32x4 bh, u32x4 bl, f
     return Bf16::mfma(ah, bh, c);
 }
 
-// [64][D] fp32 tile, global -> registers: thread t of NT owns the 32-byte pieces t, t + NT, ... (eight columns of a row)
-template <int D, int NT, bool STREAM>
-__device__ __forceinline__ void load_tile_f(u32x4 (*r)[2], rsrc_t rs, int row0, int ld, int tid) {
+// One operand of a problem: the rows of one head, fp32, or bf16 (an upstream gradient as the consumer of a bf16 output left
+// it: exact as a hi part, so the tiles are those of the converted tensor; B8 H16 N2048 D64, training
+// step 208 -> 183 us).
+struct SplitRows {
+    rsrc_t rs;
+    uint32_t esz;  // bytes per element
+    bool half;
+};
+__device__ __forceinline__ SplitRows split_rows(const float *base, size_t head, int half, int N, int ld, int d) {
+    SplitRows s;
+    s.half = half != 0;
+    s.esz = s.half ? 2u : 4u;
+    s.rs = make_rsrc_uniform(reinterpret_cast<const char *>(base) + head * s.esz, ((uint32_t)(N - 1) * ld + d) * s.esz);
+    return s;
+}
+// [64][D] tile, global -> registers: thread t of NT owns pieces t, t + NT, ... (eight columns of a row: two 16-byte loads,
+// of bf16 rows one and one out of range, so that the number of loads in flight is the same)
+template <int D, int NT>
+__device__ __forceinline__ void load_tile_f(u32x4 (*r)[2], const SplitRows &src, int row0, int ld, int tid) {
 #pragma unroll
     for (int u = 0; u < 8 * D / NT; ++u) {
         const int v = tid + NT * u;
-        const uint32_t off = (uint32_t)((row0 + v / (D / 8)) * ld + (v % (D / 8)) * 8) * 4u;
-        r[u][0] = buf_load16<STREAM>(rs, off);
-        r[u][1] = buf_load16<STREAM>(rs, off + 16u);
+        const uint32_t off = (uint32_t)((row0 + v / (D / 8)) * ld + (v % (D / 8)) * 8) * src.esz;
+        r[u][0] = buf_load16(src.rs, off);
+        r[u][1] = buf_load16(src.rs, src.half ? kOobOffset : off + 16u);
     }
 }
 // registers -> the hi tile and the lo tile in LDS; columns past the runtime width d become zero
 template <int D, int STRIDE, int NT>
-__device__ __forceinline__ void store_tile_split(u16 *th, u16 *tl, const u32x4 (*r)[2], int d, int tid) {
+__device__ __forceinline__ void store_tile_split(u16 *th, u16 *tl, const u32x4 (*r)[2], const SplitRows &src, int d, int tid) {
 #pragma unroll
     for (int u = 0; u < 8 * D / NT; ++u) {
         const int v = tid + NT * u;
         const int col = (v % (D / 8)) * 8;
         u32x4 hi = {0u, 0u, 0u, 0u}, lo = hi;
-        if (col < d) split8(r[u][0], r[u][1], hi, lo);
+        if (col < d) {
+            if (src.half)
+                hi = r[u][0];
+            else
+                split8(r[u][0], r[u][1], hi, lo);
+        }
         *reinterpret_cast<u32x4 *>(th + (v / (D / 8)) * STRIDE + col) = hi;
         *reinterpret_cast<u32x4 *>(tl + (v / (D / 8)) * STRIDE + col) = lo;
     }
@@ -108,8 +129,8 @@ __global__ __launch_bounds__(kThreads) void group_state_split_kernel(ProblemSetF
     const ProblemF &pr = set.p[set.act[wi.prob / sub]];
     const int piece = wi.prob % sub;
     const int di = pr.di, dj = pr.dj, ldb = pr.ldb, ldc = pr.ldc, reversed = pr.reversed;
-    const rsrc_t rB = make_rsrc(pr.B + head_base(pr.bsB, pr.hsB, pr.H, wi.bh), ((uint32_t)(N - 1) * ldb + di) * 4u);
-    const rsrc_t rC = make_rsrc(pr.C + head_base(pr.bsC, pr.hsC, pr.H, wi.bh), ((uint32_t)(N - 1) * ldc + dj) * 4u);
+    const SplitRows rB = split_rows(pr.B, head_base(pr.bsB, pr.hsB, pr.H, wi.bh), pr.bf16_operands & 2, N, ldb, di);
+    const SplitRows rC = split_rows(pr.C, head_base(pr.bsC, pr.hsC, pr.H, wi.bh), pr.bf16_operands & 4, N, ldc, dj);
     const int cps = (cpg + sub - 1) / sub;  // chunks per piece
     const int p0 = wi.grp * cpg + piece * cps;
     const int p1 = min(p0 + cps, min((wi.grp + 1) * cpg, nchunks));
@@ -126,12 +147,12 @@ __global__ __launch_bounds__(kThreads) void group_state_split_kernel(ProblemSetF
     auto load_chunk = [&](int s, int p) __attribute__((always_inline)) {
         const int pc = min(p, p1 - 1);
         const int row0 = (reversed ? nchunks - 1 - pc : pc) * kChunk;
-        load_tile_f<DI, kThreads, false>(rb[s], rB, row0, ldb, tid);
-        load_tile_f<DJ, kThreads, false>(rc[s], rC, row0, ldc, tid);
+        load_tile_f<DI, kThreads>(rb[s], rB, row0, ldb, tid);
+        load_tile_f<DJ, kThreads>(rc[s], rC, row0, ldc, tid);
     };
     auto stage = [&](int s, int buf) __attribute__((always_inline)) {
-        store_tile_split<DI, TL::BS, kThreads>(sBh + buf * SB, sBl + buf * SB, rb[s], di, tid);
-        store_tile_split<DJ, TL::CS, kThreads>(sCh + buf * SC, sCl + buf * SC, rc[s], dj, tid);
+        store_tile_split<DI, TL::BS, kThreads>(sBh + buf * SB, sBl + buf * SB, rb[s], rB, di, tid);
+        store_tile_split<DJ, TL::CS, kThreads>(sCh + buf * SC, sCl + buf * SC, rc[s], rC, dj, tid);
     };
     // S[i][j] += sum over the 64 positions of B[tok][i] C[tok][j] for the tiles this wavefront owns (see state_update)
     auto update = [&](int buf) __attribute__((always_inline)) {
@@ -179,28 +200,25 @@ __global__ __launch_bounds__(kThreads) void group_state_split_kernel(ProblemSetF
 // Loader role: LT threads move the A, B and C tiles of fp32 rows global -> registers -> hi / lo tiles in LDS, PF
 // chunks ahead.  One barrier per chunk.
 template <int DI, int DJ, int PF, int LT>
-__device__ __forceinline__ void split_loader_role(const float *A_head, const float *B_head, const float *C_head, int di, int dj,
+__device__ __forceinline__ void split_loader_role(const SplitRows &rA, const SplitRows &rB, const SplitRows &rC, int di, int dj,
                                                   int lda, int ldb, int ldc, const ScanRange &r, int tid, u16 *sA, u16 *sB,
                                                   u16 *sC) {
     using TL = Tiling<DI, DJ>;
     using CT = ColTiling<DI, DJ>;
     static_assert((8 * DI) % LT == 0 && (8 * DJ) % LT == 0, "tile pieces divide over the loader threads");
-    const rsrc_t rA = make_rsrc(A_head, ((uint32_t)(r.N - 1) * lda + di) * 4u);
-    const rsrc_t rB = make_rsrc(B_head, ((uint32_t)(r.N - 1) * ldb + di) * 4u);
-    const rsrc_t rC = make_rsrc(C_head, ((uint32_t)(r.N - 1) * ldc + dj) * 4u);
     u32x4 ra[PF][8 * DI / LT][2], rb[PF][8 * DI / LT][2], rc[PF][8 * DJ / LT][2];
     auto load_chunk = [&](int s, int p) __attribute__((always_inline)) {
         const int pc = min(p, r.p1 - 1);
         const int row0 = (r.reversed ? r.nchunks - 1 - pc : pc) * kChunk;
-        load_tile_f<DI, LT, false>(ra[s], rA, row0, lda, tid);
-        load_tile_f<DI, LT, false>(rb[s], rB, row0, ldb, tid);
-        load_tile_f<DJ, LT, false>(rc[s], rC, row0, ldc, tid);
+        load_tile_f<DI, LT>(ra[s], rA, row0, lda, tid);
+        load_tile_f<DI, LT>(rb[s], rB, row0, ldb, tid);
+        load_tile_f<DJ, LT>(rc[s], rC, row0, ldc, tid);
     };
     // LDS: [hi | lo] x [2 buffers] per operand
     auto stage = [&](int s, int buf) __attribute__((always_inline)) {
-        store_tile_split<DI, TL::BS, LT>(sA + buf * CT::SA, sA + (2 + buf) * CT::SA, ra[s], di, tid);
-        store_tile_split<DI, TL::BS, LT>(sB + buf * CT::SA, sB + (2 + buf) * CT::SA, rb[s], di, tid);
-        store_tile_split<DJ, TL::CS, LT>(sC + buf * CT::SC, sC + (2 + buf) * CT::SC, rc[s], dj, tid);
+        store_tile_split<DI, TL::BS, LT>(sA + buf * CT::SA, sA + (2 + buf) * CT::SA, ra[s], rA, di, tid);
+        store_tile_split<DI, TL::BS, LT>(sB + buf * CT::SA, sB + (2 + buf) * CT::SA, rb[s], rB, di, tid);
+        store_tile_split<DJ, TL::CS, LT>(sC + buf * CT::SC, sC + (2 + buf) * CT::SC, rc[s], rC, dj, tid);
     };
 #pragma unroll
     for (int s = 0; s < PF; ++s) load_chunk(s, r.p0 + s);
@@ -512,9 +530,10 @@ __global__ __launch_bounds__(512) void split_scan_kernel(ProblemSetF set, int BH
     r.mask_rev = pr.mask_rev;
     r.comp = 0;
     if (wv >= 4) {
-        split_loader_role<DI, DJ, PF, 256>(pr.A + head_base(pr.bsA, pr.hsA, pr.H, wi.bh), pr.B + head_base(pr.bsB, pr.hsB, pr.H, wi.bh),
-                                           pr.C + head_base(pr.bsC, pr.hsC, pr.H, wi.bh), di, dj, pr.lda, pr.ldb, pr.ldc, r,
-                                           (int)threadIdx.x - 256, sA, sB, sC);
+        const SplitRows rA = split_rows(pr.A, head_base(pr.bsA, pr.hsA, pr.H, wi.bh), pr.bf16_operands & 1, N, pr.lda, di);
+        const SplitRows rB = split_rows(pr.B, head_base(pr.bsB, pr.hsB, pr.H, wi.bh), pr.bf16_operands & 2, N, pr.ldb, di);
+        const SplitRows rC = split_rows(pr.C, head_base(pr.bsC, pr.hsC, pr.H, wi.bh), pr.bf16_operands & 4, N, pr.ldc, dj);
+        split_loader_role<DI, DJ, PF, 256>(rA, rB, rC, di, dj, pr.lda, pr.ldb, pr.ldc, r, (int)threadIdx.x - 256, sA, sB, sC);
         return;
     }
     ColStateIO io;

@@ -435,6 +435,33 @@ def causal_backward(q, k, v, grad_out, merged_heads=False, saved=None):
     return dq, dk_, dv_
 
 
+_g16_cache = {}
+
+
+def causal_backward_from(q, k, v, grad_out):
+    """causal_backward(q, k, v, grad_out.to(q.dtype)): the backward of an autocast step saves fp32 tensors and is handed the
+    gradient of a bf16 output (Cuda_Kernel/Custom_Kernel.py:38).  Where that is built (cott_causal_bwd_g16_supported) the
+    kernels read the bf16 gradient as it is, with the results of the converted one."""
+    if (grad_out.dtype is torch.bfloat16 and q.dtype == k.dtype == v.dtype == torch.float32 and grad_out.is_cuda
+            and tuple(grad_out.shape) == tuple(v.shape)):
+        _require_gpu(Q=q, K=k, V=v, prev_grad=grad_out)
+        b, h, n, dk, dv = shape = _shapes(q, k, v)
+        ok = _g16_cache.get(shape)
+        if ok is None:
+            ok = _remember(_g16_cache, shape, bool(_loader.lib().cott_causal_bwd_g16_supported(*shape)))
+        q, k, v, g = q.contiguous(), k.contiguous(), v.contiguous(), grad_out.contiguous()
+        if ok and not (q.data_ptr() | k.data_ptr() | v.data_ptr() | g.data_ptr()) & 15:
+            dq, dk_, dv_ = torch.empty_like(q), torch.empty_like(k), torch.empty_like(v)
+            with _on(q.device):
+                ws, ws_ptr = _workspace(_ws_bytes("cott_causal_bwd_workspace_bytes", *shape, _loader.F32), q.device)
+                rc = _loader.lib().cott_causal_bwd_g16(q.data_ptr(), k.data_ptr(), v.data_ptr(), g.data_ptr(), dq.data_ptr(),
+                                                       dk_.data_ptr(), dv_.data_ptr(), *shape, ws_ptr,
+                                                       ws.numel() if ws is not None else 0, _stream(q.device))
+            _check(rc, "cott_causal_bwd_g16")
+            return dq, dk_, dv_
+    return causal_backward(q, k, v, grad_out.contiguous().to(q.dtype))
+
+
 def noncausal_dot_product(q, k, v, merged_heads=False):
     """o = q (k^T v) per (batch, head): BERT_Trainer/BertCosAttention.py:249.  merged_heads: o as (B,N,H,Dv)
     (the context-layer permute of :317 without its copy; see merged_heads_supported)."""

@@ -112,6 +112,14 @@ COTT_API int cott_causal_bwd(const void *q, const void *k, const void *v, const 
                     int B, int H, int N, int Dk, int Dv, int dtype,
                     void *workspace, size_t workspace_bytes, void *stream);
 
+/* cott_causal_bwd of fp32 tensors with the upstream gradient in bf16, as the consumer of a bf16 forward output leaves it
+ * (an autocast step, Cuda_Kernel/Custom_Kernel.py:38): the gradients are those of the converted d_o, without the copy.
+ * Built where cott_causal_bwd_g16_supported answers 1; the workspace is cott_causal_bwd_workspace_bytes(..., COTT_F32). */
+COTT_API int cott_causal_bwd_g16_supported(int B, int H, int N, int Dk, int Dv);
+COTT_API int cott_causal_bwd_g16(const float *q, const float *k, const float *v, const void *d_o,
+                      float *dq, float *dk, float *dv, int B, int H, int N, int Dk, int Dv,
+                      void *workspace, size_t workspace_bytes, void *stream);
+
 /* ---- causal forward / backward with states saved for the backward pass -----------------------
  * dq sums over the past, dk and dv over the future.  Started from the sum of k^T v over the whole sequence (or, when
  * heads are cut into sequence groups, over everything before a group's end) dq can be computed walking the sequence

@@ -1,4 +1,5 @@
-"""Autocast forward on fp32 tensors: rounded inside the kernel, bit for bit what the op gives on converted tensors."""
+"""Autocast steps on fp32 tensors: the forward rounds them inside the kernel, the backward reads the bf16 gradient; both bit for
+bit what the ops give on converted tensors."""
 import pytest
 import torch
 
@@ -41,3 +42,30 @@ def test_other_calls_convert(ct):
         out = ct.CustomAttention.apply(q.requires_grad_(True), k, v)
     assert torch.equal(out, ops.causal_dot_product(q.detach().to(BF), k.to(BF), v.to(BF)))
     assert torch.autograd.grad(out.float().sum(), q)[0].dtype == F32
+
+
+# one group and several (the group-state pass reads d_o too), ragged, widths below their padding
+@pytest.mark.parametrize("case", [(1, 2, 128, 64, 64), (1, 1, 1, 48, 64), (1, 2, 700, 64, 48), (2, 20, 100, 48, 48), (1, 3, 4097, 64, 64)],
+                         ids=lambda c: "x".join(map(str, c)))
+def test_backward_of_a_bf16_gradient(ct, case):
+    from cottention_transformer_amd import _loader, ops
+    b, h, n, dk, dv = case
+    assert _loader.lib().cott_causal_bwd_g16_supported(*case) == 1
+    g = torch.Generator().manual_seed(n)
+    q, k, v, do = (torch.randn(b, h, n, d, generator=g).to(DEV) for d in (dk, dk, dv, dv))
+    do = do.to(BF)
+    for layout in (do, do.transpose(1, 2).contiguous().transpose(1, 2)):
+        for got, want in zip(ops.causal_backward_from(q, k, v, layout), ops.causal_backward(q, k, v, do.float())):
+            assert got.dtype == F32 and torch.equal(got, want)
+
+
+def test_backward_of_other_gradients_converts(ct):
+    from cottention_transformer_amd import _loader, ops
+    assert _loader.lib().cott_causal_bwd_g16_supported(1, 2, 128, 64, 128) == 0
+    q, k, v = (torch.randn(1, 2, 70, d, device=DEV) for d in (32, 32, 64))
+    do = torch.randn(1, 2, 70, 64, device=DEV)
+    for g in (do, do.to(BF), do.half()):
+        for got, want in zip(ops.causal_backward_from(q, k, v, g), ops.causal_backward(q, k, v, g.float())):
+            assert torch.equal(got, want)
+    with pytest.raises(RuntimeError, match="prev_grad must have shape"):
+        ops.causal_backward_from(q, k, v, do[:, :, :5].to(BF))

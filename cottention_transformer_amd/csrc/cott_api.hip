@@ -444,11 +444,28 @@ int form_sets(const Op *ops, int n, long BH, int N, int dtype, bool causal, int 
     return nsets;
 }
 
+// Ops outside the range of use_mfma: whether they run on the wide-head scan (cott_wide.h).  16-bit causal ops of heads wider
+// than 128 columns, mostly: three gradients and forward at B1 H16 N1024 D256 in 0.10 ms against 18.0 on the plain-FMA
+// kernel, which keeps the non-causal form, fp32 / fp64 tensors and widths the matrix kernels cannot tile.
+bool use_wide(const Op *ops, int n, int dtype, bool causal) {
+    bool wide = causal && n <= 3 && (dtype == COTT_F16 || dtype == COTT_BF16);
+    for (int i = 0; i < n; ++i) wide = wide && cott::wide_fits(ops[i].di, ops[i].dj);
+    return wide;
+}
+
 // Workspace needed by run_ops for the same arguments.
 size_t ops_workspace(const Op *ops, int n, long BH, int N, int dtype, bool causal) {
     if (BH <= 0 || N <= 0) return 0;
     for (int i = 0; i < n; ++i)
-        if (!use_mfma(dtype, ops[i].di, ops[i].dj, N)) return 0;
+        if (!use_mfma(dtype, ops[i].di, ops[i].dj, N)) {
+            if (!use_wide(ops, n, dtype, causal)) return 0;
+            int di[3], dj[3];
+            for (int j = 0; j < n; ++j) {
+                di[j] = ops[j].di;
+                dj[j] = ops[j].dj;
+            }
+            return cott::wide_workspace(di, dj, n, BH, N, device_cus(), device_xcds());
+        }
     size_t total = 0;
     int sets[8][8], counts[8];
     const int nsets = form_sets(ops, n, BH, N, dtype, causal, sets, counts);
@@ -483,11 +500,7 @@ int run_ops(const char *fn, bool causal, const Op *ops, int n, long BH, int N, i
     if (interleaved && !(mfma && (dtype == COTT_BF16 || dtype == COTT_F16)))
         return fail(COTT_ERR_UNSUPPORTED, "%s: (B,N,H,D) operands need bf16 / fp16 and head dims 32..128 in steps of 16", fn);
     if (!mfma) {
-        // 16-bit causal ops of heads wider than 128 columns run on the matrix cores too (cott_wide.h): three gradients
-        // and forward at B1 H16 N1024 D256 in 0.11 ms against 18.0 on the plain-FMA kernel, which keeps the
-        // non-causal form, fp32 / fp64 tensors and widths the matrix kernels cannot tile.
-        bool wide = causal && (dtype == COTT_F16 || dtype == COTT_BF16);
-        for (int i = 0; i < n; ++i) wide = wide && cott::wide_fits(ops[i].di, ops[i].dj);
+        const bool wide = use_wide(ops, n, dtype, causal);
         cott::OpDesc wide_ops[3];
         for (int i = 0; i < n; ++i) {
             if (!cott::generic_fits(dtype, ops[i].di))
@@ -503,8 +516,8 @@ int run_ops(const char *fn, bool causal, const Op *ops, int n, long BH, int N, i
             if (e != hipSuccess) return fail(COTT_ERR_HIP, "%s: HIP launch failed: %s", fn, hipGetErrorString(e));
         }
         if (wide) {
-            hipError_t e = cott::launch_wide(dtype, wide_ops, n, (int)BH, N, device_xcds(),
-                                             n > 1 ? cott::K_SCAN_GRAD : cott::K_SCAN, stream);
+            hipError_t e = cott::launch_wide(dtype, wide_ops, n, (int)BH, N, device_cus(), device_xcds(), ws,
+                                             ws != nullptr && aligned16(ws) ? ws_bytes : 0, n > 1 ? cott::K_SCAN_GRAD : cott::K_SCAN, stream);
             if (e != hipSuccess) return fail(COTT_ERR_HIP, "%s: HIP launch failed: %s", fn, hipGetErrorString(e));
         }
         return COTT_OK;

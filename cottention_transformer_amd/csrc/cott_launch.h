@@ -110,7 +110,10 @@ bool generic_fits(int dtype, int di);
 // Causal ops on 16-bit tensors whose head dims lie outside the MFMA path's range (cott_wide.h): every op needs
 // wide_fits(); full tensors (ldc == dj), no layout flags.
 inline bool wide_fits(int di, int dj) { return di % 16 == 0 && dj % 16 == 0 && di >= 32 && di <= 256 && dj >= 16; }
-hipError_t launch_wide(int dtype, const OpDesc *ops, int n, int BH, int N, int xcds, int prof_id, hipStream_t stream);
+// The workspace (16-byte aligned) may be smaller than wide_workspace() or null: sequences are then walked whole.
+size_t wide_workspace(const int *di, const int *dj, int n, long BH, int N, int cus, int xcds);
+hipError_t launch_wide(int dtype, const OpDesc *ops, int n, int BH, int N, int cus, int xcds, void *ws, size_t ws_bytes,
+                       int prof_id, hipStream_t stream);
 
 // Fused input preparation (backward = false) or its backward; see cott_prep.hip.
 hipError_t launch_prep(bool backward, const void *const x[3], const void *const g[3], void *const y[3],

@@ -64,8 +64,8 @@ __device__ __forceinline__ f32x4 mfma3(u32x4 ah, u32x4 al, u32x4 bh, u32x4 bl, f
 }
 
 // One operand of a problem: the rows of one head, fp32, or bf16 (an upstream gradient as the consumer of a bf16 output left
-// it: exact as a hi part, so the tiles are those of the converted tensor; B8 H16 N2048 D64, training
-// step 208 -> 183 us).
+// it: exact as a hi part, so the tiles are those of the converted tensor; B8 H16 N2048 D64,
+// training step 208 -> 183 us).
 struct SplitRows {
     rsrc_t rs;
     uint32_t esz;  // bytes per element

@@ -18,11 +18,11 @@
 // but no LDS read, and LDS is what this kernel spends its time on).  bf16: 16 significant bits, full exponent range.
 // fp16: the state is scaled by a power of two per column first, so that neither its largest nor its small entries leave
 // the range, and the scores and C take part as bf16 pairs (C exactly).
-// What bounds it: B1 H16 N1024 D256 is 64 workgroups forward and 192 in the gradient launch, each a chain of 32
-// chunks of 1.55 us (50 us a launch; the plain-FMA kernel took 18.0 ms for forward + gradients).  Per chunk LDS is busy
-// 2100 of 3300 cycles, the matrix pipe 930, vector-ALU issue about 1700.  Four compute wavefronts that own all DI rows of
-// their columns took 57 us.  64-column slices rather than 128: twice as many workgroups share the chip, and with 16 heads
-// workgroups are what is short.
+// What bounds it: the chain of chunks, 1.55 us each at DI = 256 (LDS busy 2100 of 3300 cycles, the matrix pipe 930,
+// vector-ALU issue about 1700); four compute wavefronts that own all DI rows of their columns took 1.75 us.  64-column slices
+// rather than 128: twice as many workgroups share the chip, and with few heads workgroups are what is short; the rest of the
+// chip is filled by sequence groups (wide_groups).  B1 H16 N1024 D256: forward 28 us, gradients (192 workgroups, whole
+// sequences) 50 us, where the plain-FMA kernel took 18.0 ms for both.
 #pragma once
 #include "cott_mfma.h"
 
@@ -41,8 +41,18 @@ struct WideOp {
 };
 struct WideSet {
     WideOp op[3];
-    int count, items;  // ops; workgroups per head = all slices of all ops
+    int count, items;  // ops; workgroups per head and group = all slices of all ops
     int xcds;
+    // Few heads: the sequence is cut into G groups of cpg chunks (in walking order).  wide_scan_kernel<..., SUMS> leaves the
+    // sum of B^T C over each group but the last in slots [head][item][group] of wide_slot_vectors() float4; a group of the
+    // scan starts from the sum of the slots before it (and sin).
+    int G, cpg;
+    f32x4 *slots;
+};
+// One slice's state in the order of its owners: [wavefront][tile][lane].
+__host__ __device__ constexpr int wide_slot_vectors(int DI) { return DI * kWideSlice / 4; }
+struct WideRange {
+    int N, nchunks, p0, p1;  // chunks p0 .. p1-1 in walking order
 };
 
 template <int DI>
@@ -95,14 +105,15 @@ __device__ __forceinline__ f32x4 number_or(f32x4 v, f32x4 w) {
     return v;
 }
 
-template <class TR, int DI>
-__device__ __forceinline__ void wide_loader_role(const WideOp &op, int bh, int c0, int N, int nchunks, int tid, u16 *sA,
+template <class TR, int DI, bool SUMS>
+__device__ __forceinline__ void wide_loader_role(const WideOp &op, int bh, int c0, const WideRange &rg, int tid, u16 *sA,
                                                  u16 *sB, u16 *sC, const u16 *sO, u32x2 *sP) {
     using T = WideTiling<DI>;
     constexpr int PF = 2, PIECES = T::PIECES;
     const int l = tid & 63, g = l >> 4, m = l & 15;
     const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int di = op.di, dj = op.dj, reversed = op.reversed;
+    const int N = rg.N, p0 = rg.p0, p1 = rg.p1;
     const uint32_t rows = (uint32_t)(N - 1);
     const rsrc_t rA = make_rsrc_uniform(op.A + (size_t)bh * N * di, (rows * di + di) * 2u);
     const rsrc_t rB = make_rsrc_uniform(op.B + (size_t)bh * N * di, (rows * di + di) * 2u);
@@ -110,14 +121,14 @@ __device__ __forceinline__ void wide_loader_role(const WideOp &op, int bh, int c
     const rsrc_t rO = make_rsrc_uniform(op.O + (size_t)bh * N * dj + c0, (rows * dj + (dj - c0)) * 2u);
     u32x4 ra[PF][PIECES], rb[PF][PIECES], rc[PF];
     const int ccol = (tid % (kWideSlice / 8)) * 8, crow = tid / (kWideSlice / 8);
-    auto first_row = [&](int p) __attribute__((always_inline)) { return (reversed ? nchunks - 1 - p : p) * kWideChunk; };
+    auto first_row = [&](int p) __attribute__((always_inline)) { return (reversed ? rg.nchunks - 1 - p : p) * kWideChunk; };
     auto load_chunk = [&](int s, int p) __attribute__((always_inline)) {
-        const int row0 = first_row(min(p, nchunks - 1));
+        const int row0 = first_row(min(p, p1 - 1));
 #pragma unroll
         for (int u = 0; u < PIECES; ++u) {
             const int v = tid + 256 * u;
             const uint32_t off = (uint32_t)((row0 + v / (DI / 8)) * di + (v % (DI / 8)) * 8) * 2u;
-            ra[s][u] = buf_load16(rA, off);
+            if constexpr (!SUMS) ra[s][u] = buf_load16(rA, off);
             rb[s][u] = buf_load16(rB, off);
         }
         rc[s] = buf_load16(rC, (uint32_t)((row0 + crow) * dj + ccol) * 2u);
@@ -128,7 +139,7 @@ __device__ __forceinline__ void wide_loader_role(const WideOp &op, int bh, int c
         for (int u = 0; u < PIECES; ++u) {
             const int v = tid + 256 * u, col = (v % (DI / 8)) * 8, row = v / (DI / 8);
             const int at = row * T::RS + 8 * wide_piece(row, col / 8);
-            *reinterpret_cast<u32x4 *>(sA + buf * T::TILE + at) = col < di ? ra[s][u] : z;
+            if constexpr (!SUMS) *reinterpret_cast<u32x4 *>(sA + buf * T::TILE + at) = col < di ? ra[s][u] : z;
             *reinterpret_cast<u32x4 *>(sB + buf * T::TILE + at) = col < di ? rb[s][u] : z;
         }
         *reinterpret_cast<u32x4 *>(sC + buf * T::CTILE + crow * T::CS + ccol) = c0 + ccol < dj ? rc[s] : z;
@@ -169,33 +180,39 @@ __device__ __forceinline__ void wide_loader_role(const WideOp &op, int bh, int c
     // output tile of chunk p, left in LDS by the compute wavefronts: one 16-byte piece per thread.  Unconditional like the
     // loads (see run_rounds): before the first tile and past the real columns the offset is out of range instead.
     auto store_out = [&](int p) __attribute__((always_inline)) {
-        const u32x4 v = *reinterpret_cast<const u32x4 *>(sO + (p & 1) * T::OTILE + crow * T::OS + ccol);
+        const u32x4 v = *reinterpret_cast<const u32x4 *>(sO + ((p - p0) & 1) * T::OTILE + crow * T::OS + ccol);
         const uint32_t off = (uint32_t)((first_row(p) + crow) * dj + ccol) * 2u;
-        __builtin_amdgcn_raw_buffer_store_b128(v, rO, (int)(p >= 0 && c0 + ccol < dj ? off : kOobOffset), 0, 0);
+        __builtin_amdgcn_raw_buffer_store_b128(v, rO, (int)(p >= p0 && c0 + ccol < dj ? off : kOobOffset), 0, 0);
     };
 #pragma unroll
-    for (int s = 0; s < PF; ++s) load_chunk(s, s);
+    for (int s = 0; s < PF; ++s) load_chunk(s, p0 + s);
     stage(0, 0);
-    load_chunk(0, PF);
+    load_chunk(0, p0 + PF);
     __syncthreads();
-    run_rounds<PF>(0, nchunks, [&](int s, int p) __attribute__((always_inline)) {
-        const int s1 = (s + 1) % PF, buf = s;  // (PF = 2 and the first chunk is 0: the LDS buffer is the stage)
+    run_rounds<PF>(p0, p1, [&](int s, int p) __attribute__((always_inline)) {
+        const int s1 = (s + 1) % PF, buf = s;  // (PF = 2: the LDS buffer is the register stage)
         stage(s1, buf ^ 1);
         load_chunk(s1, p + 1 + PF);
-        scores(buf);
-        store_out(p - 2);
+        if constexpr (!SUMS) {
+            scores(buf);
+            store_out(p - 2);
+        }
         chunk_barrier();
     });
-    // the compute wavefronts finish the last chunk after the last barrier of the loop
-    store_out(nchunks - 2);
-    chunk_barrier();
-    store_out(nchunks - 1);
+    if constexpr (!SUMS) {
+        // the compute wavefronts finish the last chunk after the last barrier of the loop
+        store_out(p1 - 2);
+        chunk_barrier();
+        store_out(p1 - 1);
+    }
 }
 
 // Wavefront w of kWideCompute: state columns 16 (w & 3) .. + 15 of the slice, row half w >> 2.
-template <class TR, int DI>
-__device__ __forceinline__ void wide_compute_role(const WideOp &op, int bh, int c0, int nchunks, int w, int l, const u16 *sA,
-                                                  const u16 *sB, const u16 *sC, u16 *sO, const u32x4 *sP, f32x4 *sX) {
+// slots: those of this head and item; `grp` of them precede this group (SUMS: slot `grp` receives the sum).
+template <class TR, int DI, bool SUMS>
+__device__ __forceinline__ void wide_compute_role(const WideOp &op, int bh, int c0, const WideRange &rg, f32x4 *slots, int grp,
+                                                  bool last_group, int w, int l, const u16 *sA, const u16 *sB,
+                                                  const u16 *sC, u16 *sO, const u32x4 *sP, f32x4 *sX) {
     using T = WideTiling<DI>;
     constexpr bool FP16 = std::is_same<TR, Fp16>::value;
     constexpr int KS = T::KS / 2;
@@ -206,7 +223,8 @@ __device__ __forceinline__ void wide_compute_role(const WideOp &op, int bh, int 
     f32x4 S[2 * KS];
 #pragma unroll
     for (int it = 0; it < 2 * KS; ++it) S[it] = zero;
-    if (op.sin != nullptr && j < dj) {
+    const int own = w * 2 * KS * 64 + l;
+    if (!SUMS && op.sin != nullptr && j < dj) {
         const float *src = op.sin + (size_t)bh * di * dj + j;
 #pragma unroll
         for (int it = 0; it < 2 * KS; ++it)
@@ -215,6 +233,15 @@ __device__ __forceinline__ void wide_compute_role(const WideOp &op, int bh, int 
                 const int i = i0 + 32 * (it >> 1) + 8 * g + 4 * (it & 1) + q;
                 if (i < di) S[it][q] = src[(size_t)i * dj];
             }
+    }
+    if constexpr (!SUMS) {
+        for (int gp = 0; gp < grp; ++gp) {
+            f32x4 t[2 * KS];
+#pragma unroll
+            for (int it = 0; it < 2 * KS; ++it) t[it] = slots[(size_t)gp * wide_slot_vectors(DI) + own + 64 * it];
+#pragma unroll
+            for (int it = 0; it < 2 * KS; ++it) S[it] += t[it];
+        }
     }
     f32x4 o = zero;                // own part of A_c S_c, block `half` of the chunk whose scores are outstanding
     u32x4 cf = {0u, 0u, 0u, 0u};   // ... and its C fragment, keys in the order of the score operands
@@ -239,14 +266,16 @@ __device__ __forceinline__ void wide_compute_role(const WideOp &op, int bh, int 
         *reinterpret_cast<u32x2 *>(sO + buf * T::OTILE + (16 * half + m) * T::OS + cw + 4 * g) = packed;
     };
     __syncthreads();
-    run_rounds<2>(0, nchunks, [&](int buf, int p) __attribute__((always_inline)) {
+    run_rounds<2>(rg.p0, rg.p1, [&](int buf, int p) __attribute__((always_inline)) {
         const u16 *tA = sA + buf * T::TILE, *tB = sB + buf * T::TILE, *tC = sC + buf * T::CTILE;
-        if (p > 0) finish(buf ^ 1);
-        cf = cat(lds_col4(tC, T::CS, 4 * g, cw, m), lds_col4(tC, T::CS, 16 + 4 * g, cw, m));
+        if constexpr (!SUMS) {
+            if (p > rg.p0) finish(buf ^ 1);
+        }
+        if constexpr (!SUMS) cf = cat(lds_col4(tC, T::CS, 4 * g, cw, m), lds_col4(tC, T::CS, 16 + 4 * g, cw, m));
         const u32x4 cu = cat(lds_col4(tC, T::CS, 8 * g, cw, m), lds_col4(tC, T::CS, 8 * g + 4, cw, m));
         float up = 1.f;
         f32x4 down = {1.f, 1.f, 1.f, 1.f};
-        if constexpr (FP16) {  // scale of this lane's half column: its largest entry to [2^14, 2^15)
+        if constexpr (FP16 && !SUMS) {  // scale of this lane's half column: its largest entry to [2^14, 2^15)
             float mx = 0.f;
 #pragma unroll
             for (int it = 0; it < 2 * KS; ++it)
@@ -264,21 +293,23 @@ __device__ __forceinline__ void wide_compute_role(const WideOp &op, int bh, int 
         f32x4 ah[2] = {zero, zero}, al[2] = {zero, zero};
 #pragma unroll
         for (int ks = 0; ks < KS; ++ks) {
-            u32x4 sh, sl;
+            if constexpr (!SUMS) {
+                u32x4 sh, sl;
 #pragma unroll
-            for (int t = 0; t < 2; ++t)
+                for (int t = 0; t < 2; ++t)
 #pragma unroll
-                for (int q = 0; q < 2; ++q) {
-                    uint32_t h, lo;
-                    split2<TR>(S[2 * ks + t][2 * q] * up, S[2 * ks + t][2 * q + 1] * up, h, lo);
-                    sh[2 * t + q] = h;
-                    sl[2 * t + q] = lo;
+                    for (int q = 0; q < 2; ++q) {
+                        uint32_t h, lo;
+                        split2<TR>(S[2 * ks + t][2 * q] * up, S[2 * ks + t][2 * q + 1] * up, h, lo);
+                        sh[2 * t + q] = h;
+                        sl[2 * t + q] = lo;
+                    }
+#pragma unroll
+                for (int pb = 0; pb < 2; ++pb) {
+                    const u32x4 a = *reinterpret_cast<const u32x4 *>(tA + 16 * pb * T::RS + aoff[ks]);
+                    ah[pb] = TR::mfma(sh, a, ah[pb]);
+                    al[pb] = TR::mfma(sl, a, al[pb]);
                 }
-#pragma unroll
-            for (int pb = 0; pb < 2; ++pb) {
-                const u32x4 a = *reinterpret_cast<const u32x4 *>(tA + 16 * pb * T::RS + aoff[ks]);
-                ah[pb] = TR::mfma(sh, a, ah[pb]);
-                al[pb] = TR::mfma(sl, a, al[pb]);
             }
 #pragma unroll
             for (int t = 0; t < 2; ++t) {
@@ -287,26 +318,33 @@ __device__ __forceinline__ void wide_compute_role(const WideOp &op, int bh, int 
                 S[2 * ks + t] = TR::mfma(b, cu, S[2 * ks + t]);
             }
         }
+        if constexpr (!SUMS) {
 #pragma unroll
-        for (int pb = 0; pb < 2; ++pb) al[pb] += ah[pb];
-        if (__any(any_nan(al[0]) | any_nan(al[1]))) {
-            al[0] = number_or(al[0], ah[0]);
-            al[1] = number_or(al[1], ah[1]);
-        }
+            for (int pb = 0; pb < 2; ++pb) al[pb] += ah[pb];
+            if (__any(any_nan(al[0]) | any_nan(al[1]))) {
+                al[0] = number_or(al[0], ah[0]);
+                al[1] = number_or(al[1], ah[1]);
+            }
 #pragma unroll
-        for (int pb = 0; pb < 2; ++pb) {
-            f32x4 r = al[pb];
-            if constexpr (FP16) r *= down;
-            if (pb == half)
-                o = r;
-            else
-                sX[(buf * kWideCompute + w) * 64 + l] = r;
+            for (int pb = 0; pb < 2; ++pb) {
+                f32x4 r = al[pb];
+                if constexpr (FP16) r *= down;
+                if (pb == half)
+                    o = r;
+                else
+                    sX[(buf * kWideCompute + w) * 64 + l] = r;
+            }
         }
         chunk_barrier();
     });
-    finish((nchunks - 1) & 1);
+    if constexpr (SUMS) {
+#pragma unroll
+        for (int it = 0; it < 2 * KS; ++it) slots[(size_t)grp * wide_slot_vectors(DI) + own + 64 * it] = S[it];
+        return;
+    }
+    finish((rg.p1 - 1 - rg.p0) & 1);
     chunk_barrier();
-    if (op.sout != nullptr && j < dj) {
+    if (op.sout != nullptr && last_group && j < dj) {
         float *dst = op.sout + (size_t)bh * di * dj + j;
 #pragma unroll
         for (int it = 0; it < 2 * KS; ++it)
@@ -318,9 +356,9 @@ __device__ __forceinline__ void wide_compute_role(const WideOp &op, int bh, int 
     }
 }
 
-// 768 threads: wavefronts 0..7 compute, 8..11 load.  Grid: grid_for(BH, set.items, 1, set.xcds), so that the slices and ops
-// of a head run on one XCD and share its tiles through that L2.
-template <class TR, int DI>
+// 768 threads: wavefronts 0..7 compute, 8..11 load.  Grid: grid_for(BH, set.items, groups, set.xcds), groups = G, or G - 1 for
+// the sums, so that the slices and ops of a head and group run on one XCD and share its tiles through that L2.
+template <class TR, int DI, bool SUMS>
 __global__ __launch_bounds__(64 * (kWideCompute + kWideLoad)) void wide_scan_kernel(WideSet set, int BH, int N, int nchunks) {
     using T = WideTiling<DI>;
     __shared__ __attribute__((aligned(16))) unsigned char wide_smem[T::LDS];
@@ -329,20 +367,24 @@ __global__ __launch_bounds__(64 * (kWideCompute + kWideLoad)) void wide_scan_ker
     u32x4 *sP = reinterpret_cast<u32x4 *>(sO + 2 * T::OTILE);
     f32x4 *sX = reinterpret_cast<f32x4 *>(sP + 2 * 2 * 2 * 64);
     const WorkItem wi = decode_workgroup(set.items, BH, set.xcds);
-    if (wi.grp >= 1) return;
+    if (wi.grp >= (SUMS ? set.G - 1 : set.G)) return;
     int which = 0, slice = wi.prob;
     while (which + 1 < set.count && slice >= set.op[which].slices) slice -= set.op[which++].slices;
     const WideOp &op = set.op[which];
+    const WideRange rg = {N, nchunks, wi.grp * set.cpg, min((wi.grp + 1) * set.cpg, nchunks)};
+    f32x4 *slots = set.slots + ((size_t)wi.bh * set.items + wi.prob) * (set.G - 1) * wide_slot_vectors(DI);
     const int tid = threadIdx.x;
-    // the score tiles on the other side of the diagonal are never written: zero
-    for (int x = tid; x < 2 * 2 * 2 * 64; x += 64 * (kWideCompute + kWideLoad)) sP[x] = u32x4{0u, 0u, 0u, 0u};
-    __syncthreads();
+    if constexpr (!SUMS) {  // the score tiles on the other side of the diagonal are never written: zero
+        for (int x = tid; x < 2 * 2 * 2 * 64; x += 64 * (kWideCompute + kWideLoad)) sP[x] = u32x4{0u, 0u, 0u, 0u};
+        __syncthreads();
+    }
     const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
     if (w < kWideCompute)
-        wide_compute_role<TR, DI>(op, wi.bh, slice * kWideSlice, nchunks, w, tid & 63, sA, sB, sC, sO, sP, sX);
+        wide_compute_role<TR, DI, SUMS>(op, wi.bh, slice * kWideSlice, rg, slots, wi.grp, wi.grp == set.G - 1, w, tid & 63, sA, sB,
+                                        sC, sO, sP, sX);
     else
-        wide_loader_role<TR, DI>(op, wi.bh, slice * kWideSlice, N, nchunks, tid - 64 * kWideCompute, sA, sB, sC, sO,
-                                 reinterpret_cast<u32x2 *>(sP));
+        wide_loader_role<TR, DI, SUMS>(op, wi.bh, slice * kWideSlice, rg, tid - 64 * kWideCompute, sA, sB, sC, sO,
+                                       reinterpret_cast<u32x2 *>(sP));
 }
 
 }  // namespace cott

@@ -8,16 +8,45 @@ namespace {
 
 int wide_pad(int di) { return di <= 128 ? 128 : (di <= 192 ? 192 : 256); }
 
+// Groups a sequence is cut into: as many as keep the launch at one workgroup per CU (the (head, group) units are dealt round
+// the XCDs, and the fullest XCD has to hold its units' workgroups at once), of eight chunks at least, at most 16 (a group
+// reads the slots of all groups before it).  Sequences below 24 chunks stay whole (2 heads N512 D256, forward 25 us; two
+// launches of a few us each would have to save more).  Whole / groups, us: forward 16 heads D256 N768 35.9 / 25.2, N1024
+// 46.6 / 29.0, N4096 171 / 83; 2 heads N4096 166 / 36, N16384 664 / 76; gradients 2 heads N1024 47 / 28, N4096 172 / 47.  More
+// groups than an XCD holds at once: gradients of 2 heads N4096 in 10 groups 67 us, in 8 47.
+int wide_groups(long BH, int items, int nchunks, int cus, int xcds) {
+    if (nchunks < 24) return 1;
+    long g = cus / xcds / items * xcds / BH;
+    if (g > nchunks / 8) g = nchunks / 8;
+    if (g > 16) g = 16;
+    if (g < 2) return 1;
+    const int cpg = (int)((nchunks + g - 1) / g);
+    return (nchunks + cpg - 1) / cpg;
+}
+
+int wide_chunks(int N) { return (N + kWideChunk - 1) / kWideChunk; }
+
+// Slots of one launch: BH heads, `items` slices, all groups but the last.
+size_t wide_slot_bytes(long BH, int items, int G, int pad) {
+    return (size_t)BH * items * (G - 1) * wide_slot_vectors(pad) * sizeof(f32x4);
+}
+
 template <class TR, int DI>
 hipError_t launch_set(const WideSet &set, int BH, int N, int prof_id, hipStream_t stream) {
+    const int nchunks = wide_chunks(N);
+    const dim3 block(64 * (kWideCompute + kWideLoad));
+    if (set.G > 1) {
+        ProfScope ps(K_GROUP_STATE, stream);
+        wide_scan_kernel<TR, DI, true><<<dim3(grid_for(BH, set.items, set.G - 1, set.xcds)), block, 0, stream>>>(set, BH, N, nchunks);
+    }
     ProfScope ps(prof_id, stream);
-    const int nchunks = (N + kWideChunk - 1) / kWideChunk;
-    wide_scan_kernel<TR, DI><<<dim3(grid_for(BH, set.items, 1, set.xcds)), dim3(64 * (kWideCompute + kWideLoad)), 0, stream>>>(set, BH, N, nchunks);
+    wide_scan_kernel<TR, DI, false><<<dim3(grid_for(BH, set.items, set.G, set.xcds)), block, 0, stream>>>(set, BH, N, nchunks);
     return hipGetLastError();
 }
 
 template <class TR>
-hipError_t launch_typed(const OpDesc *ops, int n, int BH, int N, int xcds, int prof_id, hipStream_t stream) {
+hipError_t launch_typed(const OpDesc *ops, int n, int BH, int N, int cus, int xcds, char *ws, size_t ws_bytes, int prof_id,
+                        hipStream_t stream) {
     // one launch per padded width of the contracted dim (the gradients of square heads are one)
     for (int pad = 128; pad <= 256; pad += 64) {
         WideSet set{};
@@ -39,6 +68,16 @@ hipError_t launch_typed(const OpDesc *ops, int n, int BH, int N, int xcds, int p
             set.items += w.slices;
         }
         if (set.count == 0) continue;
+        const int nchunks = wide_chunks(N);
+        set.G = wide_groups(BH, set.items, nchunks, cus, xcds);
+        const size_t need = wide_slot_bytes(BH, set.items, set.G, pad);
+        if (need > ws_bytes) set.G = 1;  // (a caller without the workspace gets the same results from whole sequences)
+        set.cpg = (nchunks + set.G - 1) / set.G;
+        if (set.G > 1) {
+            set.slots = reinterpret_cast<f32x4 *>(ws);
+            ws += need;
+            ws_bytes -= need;
+        }
         const hipError_t e = pad == 128   ? launch_set<TR, 128>(set, BH, N, prof_id, stream)
                              : pad == 192 ? launch_set<TR, 192>(set, BH, N, prof_id, stream)
                                           : launch_set<TR, 256>(set, BH, N, prof_id, stream);
@@ -49,9 +88,22 @@ hipError_t launch_typed(const OpDesc *ops, int n, int BH, int N, int xcds, int p
 
 }  // namespace
 
-hipError_t launch_wide(int dtype, const OpDesc *ops, int n, int BH, int N, int xcds, int prof_id, hipStream_t stream) {
-    if (dtype == COTT_BF16) return launch_typed<Bf16>(ops, n, BH, N, xcds, prof_id, stream);
-    if (dtype == COTT_F16) return launch_typed<Fp16>(ops, n, BH, N, xcds, prof_id, stream);
+size_t wide_workspace(const int *di, const int *dj, int n, long BH, int N, int cus, int xcds) {
+    size_t total = 0;
+    for (int pad = 128; pad <= 256; pad += 64) {
+        int items = 0;
+        for (int i = 0; i < n; ++i)
+            if (wide_pad(di[i]) == pad) items += (dj[i] + kWideSlice - 1) / kWideSlice;
+        if (items > 0) total += wide_slot_bytes(BH, items, wide_groups(BH, items, wide_chunks(N), cus, xcds), pad);
+    }
+    return total;
+}
+
+hipError_t launch_wide(int dtype, const OpDesc *ops, int n, int BH, int N, int cus, int xcds, void *ws, size_t ws_bytes,
+                       int prof_id, hipStream_t stream) {
+    char *w = static_cast<char *>(ws);
+    if (dtype == COTT_BF16) return launch_typed<Bf16>(ops, n, BH, N, cus, xcds, w, ws_bytes, prof_id, stream);
+    if (dtype == COTT_F16) return launch_typed<Fp16>(ops, n, BH, N, cus, xcds, w, ws_bytes, prof_id, stream);
     return hipErrorInvalidValue;
 }
 

@@ -32,6 +32,10 @@ CASES = [
     (1, 2, 130, 256, 64, HF),     # the ops of a gradient call differ in padded width
     (1, 2, 130, 64, 256, BF),
     (1, 2, 96, 48, 144, BF),      # contracted dim far below its padding
+    (1, 2, 737, 256, 256, BF),    # 24 chunks: the shortest sequence cut into groups
+    (1, 2, 736, 256, 256, HF),    # ... and the longest that is not
+    (1, 3, 2050, 64, 192, HF),    # groups of unequal length
+    (1, 1, 4100, 160, 160, BF),   # sixteen groups forward
     (1, 1, 70, 144, 400, HF),     # seven slices; the gradients contract 400 columns (plain-FMA kernel)
 ]
 IDS = lambda c: "x".join(map(str, c[:5])) + "-" + str(c[5]).split(".")[-1]
@@ -86,3 +90,26 @@ def test_an_infinite_value_stays_in_its_column(ct, dt):
     assert torch.equal(got[..., other], want[..., other])
     assert torch.isfinite(got[0, 0, :32, 5]).all()
     assert not torch.isfinite(got[0, 0, 64:, 5]).any()
+
+
+def test_groups_need_no_workspace(ct):
+    """Called without the workspace it asks for, the library walks the sequence whole."""
+    from cottention_transformer_amd import _loader
+    q, k, v, _ = (t.to(DEV) for t in inputs(1, 2, 2000, 192, 192, BF, seed=6))
+    want, out, L = ct.causal_dot_product(q, k, v), torch.empty_like(v), _loader.lib()
+    assert L.cott_causal_workspace_bytes(1, 2, 2000, 192, 192, _loader.BF16) > 0
+    rc = L.cott_causal_fwd(q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), 1, 2, 2000, 192, 192, _loader.BF16, 0, None, 0,
+                           torch.cuda.current_stream().cuda_stream)
+    assert rc == _loader.OK
+    # both within half a unit of the same number
+    assert rel_l2(out, want.double().cpu().numpy()) <= 2 * BOUND[BF]
+
+
+def test_states_in_and_out_of_groups(ct, oracle):
+    q, k, v, _ = inputs(1, 1, 4000, 256, 144, HF, seed=8)
+    qd, kd, vd = (t.to(DEV) for t in (q, k, v))
+    o1, s1 = ct.causal_prefill(qd[:, :, :1900], kd[:, :, :1900], vd[:, :, :1900])
+    o2, s2 = ct.causal_prefill(qd[:, :, 1900:], kd[:, :, 1900:], vd[:, :, 1900:], state=s1)
+    assert rel_l2(torch.cat((o1, o2), 2), oracle.causal(q, k, v)) <= BOUND[HF]
+    # 4000 products summed in fp32, errors of either sign: sqrt(4000) * 2^-24 in the mean
+    assert rel_l2(s2, (k.double().transpose(2, 3) @ v.double()).numpy()) <= 64 * 2.0 ** -24

@@ -1,0 +1,50 @@
+"""Host-side rules that choose a launch form, swept without a GPU: workspaces stay within what the entry points without a
+caller's workspace hold, and every call that was accepted has a plan."""
+import itertools
+
+import pytest
+
+from cottention_transformer_amd import _loader
+
+BF16, F16 = _loader.BF16, _loader.F16
+
+
+@pytest.fixture(params=[(256, 8), (64, 2), (38, 1), (304, 8)], ids=lambda g: f"{g[0]}cus-{g[1]}xcds")
+def lib(request):
+    L = _loader.lib()
+    assert L.cott_plan_geometry(*request.param) == _loader.OK
+    yield L, request.param
+    assert L.cott_plan_geometry(0, 0) == _loader.OK
+
+
+def test_wide_head_workspace_fits_the_builtin_scratch(lib):
+    L, (cus, _) = lib
+    for h, n, dk, dv in itertools.product((1, 2, 3, 8, 16, 40, 300), (1, 735, 737, 1024, 5000, 65536), (48, 144, 192, 256), (16, 144, 256, 400)):
+        if dk <= 128 and 32 <= dv <= 128:
+            continue
+        for dt in (BF16, F16):
+            fwd = L.cott_causal_workspace_bytes(1, h, n, dk, dv, dt)
+            # at most one workgroup per CU, each of whose groups but the last leaves one slot of at most 64 KiB
+            assert fwd <= cus * 65536 and fwd <= 48 << 20
+            if n <= 736:
+                assert fwd == 0
+
+
+def test_short_sequences_take_no_workspace(lib):
+    L, _ = lib
+    for h, d in itertools.product((1, 2, 7, 12, 16, 32, 64), (32, 48, 64, 80, 128)):
+        for n in (1, 63, 64, 128, 256):
+            assert L.cott_causal_workspace_bytes(1, h, n, d, d, BF16) == 0
+            assert L.cott_causal_bwd_workspace_bytes(1, h, n, d, d, BF16) == 0
+            assert L.cott_noncausal_workspace_bytes(1, h, n, d, d, BF16) == 0
+            # no workspace: one group, which is also what the forward with the preparation inside needs
+            assert L.cott_noncausal_fwd_prep_supported(1, h, n, d, d, BF16) == 1
+            assert L.cott_causal_fwd_f32in_supported(1, h, n, d, d) == (1 if d <= 64 else 0)
+
+
+def test_preparation_inside_the_forward_keeps_its_shapes(lib):
+    """128-wide q / k rows need value tiles of 64 columns: short sequences are not cut into narrower halves."""
+    L, _ = lib
+    for h, n, dv in itertools.product((1, 2, 8, 16, 32), (1, 64, 256, 500, 768), (64, 80, 128)):
+        if n <= 256:
+            assert L.cott_causal_fwd_prep_supported(1, h, n, 128, dv, BF16, 64) == 1

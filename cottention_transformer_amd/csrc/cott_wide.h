@@ -13,16 +13,17 @@
 //     score tiles of the chunk (once per workgroup, handed to the compute wavefronts through LDS) and write the
 //     finished output tile to memory as 16-byte pieces of whole 128-byte row segments.
 //   * One barrier per chunk: the product of the scores with C_c is finished at the start of the next chunk.
-// Precision: the plain-FMA kernel that served these widths keeps state and scores in fp32.  So that nothing is lost,
-// both enter the matrix instructions as two 16-bit numbers, x = hi + lo (the second term costs a matrix instruction
-// but no LDS read, and LDS is what this kernel spends its time on).  bf16: 16 significant bits, full exponent range.
-// fp16: the state is scaled by a power of two per column first, so that neither its largest nor its small entries leave
-// the range, and the scores and C take part as bf16 pairs (C exactly).
-// What bounds it: the chain of chunks, 1.55 us each at DI = 256 (LDS busy 2100 of 3300 cycles, the matrix pipe 930,
-// vector-ALU issue about 1700); four compute wavefronts that own all DI rows of their columns took 1.75 us.  64-column slices
-// rather than 128: twice as many workgroups share the chip, and with few heads workgroups are what is short; the rest of the
-// chip is filled by sequence groups (wide_groups).  B1 H16 N1024 D256: forward 28 us, gradients (192 workgroups, whole
-// sequences) 50 us, where the plain-FMA kernel took 18.0 ms for both.
+// Precision: the plain-FMA kernel that served these widths keeps state and scores in fp32, with 24 significant bits.
+// Here both enter the matrix instructions as the sum of three 16-bit numbers that holds all of them (split3), so that
+// every product is that of the fp32 number and what is left is the order of the fp32 sums.  fp16: the state is scaled by
+// a power of two per column first, so that neither its largest nor its small entries leave the range, and the scores and
+// C take part as bf16 triples and pairs (C exactly).
+// What bounds it: the chain of chunks, 1.5 us each at DI = 256, and in it the vector instructions of the splits (with two
+// terms, 16 significant bits, it took 1.27 us).  64-column slices rather than 128: twice as many workgroups share the chip,
+// and with few heads workgroups are what is short; the rest of the chip is filled by sequence groups (wide_groups).  B1 H16
+// N1024 D256: forward 30 us, gradients (192 workgroups, whole sequences) 57 us, where the plain-FMA kernel took 18.0 ms for
+// both.  Share of the outputs that are not the 16-bit number nearest to the exact result, same shape: 1.5e-4 (bf16) and
+// 1.2e-3 (fp16), plain-FMA kernel 2.9e-4 and 3.2e-3, two terms 2.4e-3 and 5.5e-3.
 #pragma once
 #include "cott_mfma.h"
 
@@ -66,10 +67,11 @@ struct WideTiling {
     static constexpr int KS = DI / 32;
     static constexpr int TILE = kWideChunk * RS, CTILE = kWideChunk * CS, OTILE = kWideChunk * OS;
     static constexpr int PIECES = kWideChunk * DI / 8 / 256;  // 16-byte pieces of an A or B tile per loader thread
-    // A and B tiles, C tiles, output tiles (two buffers each), then the score operands [2 buffers][hi, lo][2 blocks][64]
-    // and the partial outputs [2 buffers][8 wavefronts][64]
+    // A and B tiles, C tiles, output tiles (two buffers each), then the score operands [2 buffers][hi, mid, lo][2 blocks]
+    // [64] and the partial outputs [2 buffers][8 wavefronts][64]
+    static constexpr int SCORES = 2 * 3 * 2 * 64;
     static constexpr size_t LDS = (4 * TILE + 2 * CTILE + 2 * OTILE) * sizeof(u16) +
-                                  (2 * 2 * 2 * 64 + 2 * kWideCompute * 64) * sizeof(u32x4);
+                                  (SCORES + 2 * kWideCompute * 64) * sizeof(u32x4);
 };
 
 // Where 16-byte piece c of row r of an A or B tile lies within the row.  Read in the order of either access, 16 pieces
@@ -77,27 +79,38 @@ struct WideTiling {
 // pieces 4k .. 4k+3 of rows 4r' .. 4r'+3 (the transposing reads).
 __device__ __forceinline__ int wide_piece(int r, int c) { return c ^ (4 * (r & 3) + ((r >> 2) & 3)); }
 
-// fp32 -> two 16-bit numbers of type TR, hi + lo
+// Two fp32 numbers cut to 16-bit ones of type TR towards zero (so that no finite number becomes infinite).
 template <class TR>
-__device__ __forceinline__ void split2(float a, float b, uint32_t &hi, uint32_t &lo) {
-    hi = TR::pack2(a, b);
-    lo = TR::pack2(a - TR::to_float((u16)(hi & 0xffffu)), b - TR::to_float((u16)(hi >> 16)));
+__device__ __forceinline__ uint32_t cut2(float a, float b) {
+    if constexpr (std::is_same<TR, Fp16>::value)
+        return bitcast<uint32_t>(__builtin_amdgcn_cvt_pkrtz(a, b));
+    else
+        return (bitcast<uint32_t>(a) >> 16) | (bitcast<uint32_t>(b) & 0xffff0000u);
+}
+// fp32 -> three 16-bit numbers of type TR, hi + mid + lo.  Each takes the leading bits of what the ones before it leave: 8
+// of bf16 (3 x 8 = 24, exact wherever the last one is a normal number), 11 of fp16 (exact down to 2^-24).
+template <class TR>
+__device__ __forceinline__ void split3(float a, float b, uint32_t &hi, uint32_t &mid, uint32_t &lo) {
+    hi = cut2<TR>(a, b);
+    a -= TR::to_float((u16)(hi & 0xffffu));
+    b -= TR::to_float((u16)(hi >> 16));
+    mid = cut2<TR>(a, b);
+    lo = cut2<TR>(a - TR::to_float((u16)(mid & 0xffffu)), b - TR::to_float((u16)(mid >> 16)));
 }
 // eight fp16 numbers -> the same eight as bf16 hi + lo (exact: 8 + 8 significant bits hold the 11)
 __device__ __forceinline__ void fp16_as_bf16_pair(u32x4 v, u32x4 &hi, u32x4 &lo) {
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
-        uint32_t h, x;
-        split2<Bf16>(Fp16::to_float((u16)(v[e] & 0xffffu)), Fp16::to_float((u16)(v[e] >> 16)), h, x);
-        hi[e] = h;
-        lo[e] = x;
+        const float a = Fp16::to_float((u16)(v[e] & 0xffffu)), b = Fp16::to_float((u16)(v[e] >> 16));
+        hi[e] = cut2<Bf16>(a, b);
+        lo[e] = cut2<Bf16>(a - Bf16::to_float((u16)(hi[e] & 0xffffu)), b - Bf16::to_float((u16)(hi[e] >> 16)));
     }
 }
 __device__ __forceinline__ bool any_nan(f32x4 v) {
     const float s = (v[0] + v[1]) + (v[2] + v[3]);  // (also true where infinities cancel: number_or then changes nothing)
     return s != s;
 }
-// v where it is a number, else the same element of w.  An infinite state or score entry splits into hi = inf and lo =
+// v where it is a number, else the same element of w.  An infinite state or score entry splits into hi = inf and two times
 // inf - inf; the sum formed from the hi parts alone then has the value the single-number arithmetic gives.
 __device__ __forceinline__ f32x4 number_or(f32x4 v, f32x4 w) {
 #pragma unroll
@@ -168,14 +181,11 @@ __device__ __forceinline__ void wide_loader_role(const WideOp &op, int bh, int c
         p0 += p1;
 #pragma unroll
         for (int q = 0; q < 4; ++q) p0[q] = side + dir * q >= 0 ? p0[q] : 0.f;
-        u32x2 hi, lo;
-        uint32_t h0, l0, h1, l1;
-        split2<Bf16>(p0[0], p0[1], h0, l0);
-        split2<Bf16>(p0[2], p0[3], h1, l1);
-        hi = u32x2{h0, h1};
-        lo = u32x2{l0, l1};
-        sP[((buf * 2 + 0) * 2 + pb) * 128 + 2 * l + kt] = hi;
-        sP[((buf * 2 + 1) * 2 + pb) * 128 + 2 * l + kt] = lo;
+        uint32_t part[3][2];
+        split3<Bf16>(p0[0], p0[1], part[0][0], part[1][0], part[2][0]);
+        split3<Bf16>(p0[2], p0[3], part[0][1], part[1][1], part[2][1]);
+#pragma unroll
+        for (int x = 0; x < 3; ++x) sP[((buf * 3 + x) * 2 + pb) * 128 + 2 * l + kt] = u32x2{part[x][0], part[x][1]};
     };
     // output tile of chunk p, left in LDS by the compute wavefronts: one 16-byte piece per thread.  Unconditional like the
     // loads (see run_rounds): before the first tile and past the real columns the offset is out of range instead.
@@ -256,11 +266,19 @@ __device__ __forceinline__ void wide_compute_role(const WideOp &op, int bh, int 
     auto finish = [&](int buf) __attribute__((always_inline)) {
         u32x4 ch = cf, cl = cf;
         if constexpr (FP16) fp16_as_bf16_pair(cf, ch, cl);
-        const u32x4 ph = sP[((buf * 2 + 0) * 2 + half) * 64 + l], pl = sP[((buf * 2 + 1) * 2 + half) * 64 + l];
+        u32x4 p[3];
+#pragma unroll
+        for (int x = 0; x < 3; ++x) p[x] = sP[((buf * 3 + x) * 2 + half) * 64 + l];
         const f32x4 other = sX[(buf * kWideCompute + (w ^ 4)) * 64 + l];
-        f32x4 hi = Bf16::mfma(ch, ph, o + other);
-        if constexpr (FP16) hi = Bf16::mfma(cl, ph, hi);
-        f32x4 r = Bf16::mfma(ch, pl, hi);
+        f32x4 hi = Bf16::mfma(ch, p[0], o + other), rest = zero;
+        if constexpr (FP16) {
+            hi = Bf16::mfma(cl, p[0], hi);
+            rest = Bf16::mfma(cl, p[2], rest);
+            rest = Bf16::mfma(cl, p[1], rest);
+        }
+        rest = Bf16::mfma(ch, p[2], rest);
+        rest = Bf16::mfma(ch, p[1], rest);
+        f32x4 r = hi + rest;
         if (__any(any_nan(r))) r = number_or(r, hi);
         const u32x2 packed = {TR::pack2(r[0], r[1]), TR::pack2(r[2], r[3])};
         *reinterpret_cast<u32x2 *>(sO + buf * T::OTILE + (16 * half + m) * T::OS + cw + 4 * g) = packed;
@@ -294,14 +312,15 @@ __device__ __forceinline__ void wide_compute_role(const WideOp &op, int bh, int 
 #pragma unroll
         for (int ks = 0; ks < KS; ++ks) {
             if constexpr (!SUMS) {
-                u32x4 sh, sl;
+                u32x4 sh, sm, sl;
 #pragma unroll
                 for (int t = 0; t < 2; ++t)
 #pragma unroll
                     for (int q = 0; q < 2; ++q) {
-                        uint32_t h, lo;
-                        split2<TR>(S[2 * ks + t][2 * q] * up, S[2 * ks + t][2 * q + 1] * up, h, lo);
+                        uint32_t h, mid, lo;
+                        split3<TR>(S[2 * ks + t][2 * q] * up, S[2 * ks + t][2 * q + 1] * up, h, mid, lo);
                         sh[2 * t + q] = h;
+                        sm[2 * t + q] = mid;
                         sl[2 * t + q] = lo;
                     }
 #pragma unroll
@@ -309,6 +328,7 @@ __device__ __forceinline__ void wide_compute_role(const WideOp &op, int bh, int 
                     const u32x4 a = *reinterpret_cast<const u32x4 *>(tA + 16 * pb * T::RS + aoff[ks]);
                     ah[pb] = TR::mfma(sh, a, ah[pb]);
                     al[pb] = TR::mfma(sl, a, al[pb]);
+                    al[pb] = TR::mfma(sm, a, al[pb]);
                 }
             }
 #pragma unroll
@@ -365,7 +385,7 @@ __global__ __launch_bounds__(64 * (kWideCompute + kWideLoad)) void wide_scan_ker
     u16 *sA = reinterpret_cast<u16 *>(wide_smem);
     u16 *sB = sA + 2 * T::TILE, *sC = sB + 2 * T::TILE, *sO = sC + 2 * T::CTILE;
     u32x4 *sP = reinterpret_cast<u32x4 *>(sO + 2 * T::OTILE);
-    f32x4 *sX = reinterpret_cast<f32x4 *>(sP + 2 * 2 * 2 * 64);
+    f32x4 *sX = reinterpret_cast<f32x4 *>(sP + T::SCORES);
     const WorkItem wi = decode_workgroup(set.items, BH, set.xcds);
     if (wi.grp >= (SUMS ? set.G - 1 : set.G)) return;
     int which = 0, slice = wi.prob;
@@ -375,7 +395,7 @@ __global__ __launch_bounds__(64 * (kWideCompute + kWideLoad)) void wide_scan_ker
     f32x4 *slots = set.slots + ((size_t)wi.bh * set.items + wi.prob) * (set.G - 1) * wide_slot_vectors(DI);
     const int tid = threadIdx.x;
     if constexpr (!SUMS) {  // the score tiles on the other side of the diagonal are never written: zero
-        for (int x = tid; x < 2 * 2 * 2 * 64; x += 64 * (kWideCompute + kWideLoad)) sP[x] = u32x4{0u, 0u, 0u, 0u};
+        for (int x = tid; x < T::SCORES; x += 64 * (kWideCompute + kWideLoad)) sP[x] = u32x4{0u, 0u, 0u, 0u};
         __syncthreads();
     }
     const int w = __builtin_amdgcn_readfirstlane(tid >> 6);

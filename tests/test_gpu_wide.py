@@ -1,9 +1,8 @@
 """Causal ops of 16-bit heads outside the 32..128 column range (wide_scan_kernel) against the oracle.
 
-Tolerance: inputs are exact, products and sums are fp32, state and scores enter the products with 16 (bf16) or more
-significant bits, so what is left is the rounding of the output: at most half a unit in the last place of every element,
-2^-9 (bf16) and 2^-12 (fp16, away from its subnormals) of it, plus 2^-13 for the hi / lo split and the fp32 sums of
-outputs that cancel."""
+Tolerance: inputs are exact, products and sums are fp32, state and scores enter the products with all their bits, so what is
+left is the rounding of the output: at most half a unit in the last place of every element, 2^-9 (bf16) and 2^-12 (fp16,
+away from its subnormals) of it, plus 2^-13 for the fp32 sums of outputs that cancel."""
 import pytest
 import torch
 
@@ -52,6 +51,34 @@ def test_forward_and_gradients(ct, oracle, case):
         assert worst_block(got, ref, 32) <= 2 * BOUND[dt], rev
     for name, got, ref in zip(("dQ", "dK", "dV"), ct.causal_backward(*dev), oracle.causal_bwd(q, k, v, do)):
         assert rel_l2(got, ref) <= BOUND[dt], name
+
+
+@pytest.mark.parametrize("dk", [144, 192, 256])
+@pytest.mark.parametrize("dt", [BF, HF], ids=["bf16", "fp16"])
+def test_states_and_scores_take_part_with_all_their_bits(ct, oracle, dt, dk):
+    """Two fp32 numbers that differ in the last of their 24 bits cancel to that bit: state entries 1 + 2^-12 + 2^-23 and
+    1 + 2^-12 read at position 40 (the next chunk), scores of the same values at position 20 (their own chunk), against
+    values that use all the bits of their type.  Every product and partial sum is an fp32 number, so is the output: exact."""
+    q, k, v = (torch.zeros(1, 1, 64, d, dtype=dt) for d in (dk, dk, 160))
+    last = dk - 1
+    c = 1 + 2.0 ** (-7 if dt is BF else -10)
+    # columns 0..63: the state; row `last` holds all three terms, row 3 two of them
+    for t, (row, x, y) in enumerate(((last, 1, 1), (last, 2.0 ** -12, 1), (last, 2.0 ** -12, 2.0 ** -11), (3, 1, 1), (3, 2.0 ** -12, 1))):
+        k[0, 0, t, row] = x
+        v[0, 0, t, :64] = y
+    q[0, 0, 40, last], q[0, 0, 40, 3] = 4096, -4096
+    # columns 64..: the scores of positions 16 and 17 at position 20
+    q[0, 0, 20, 8:11] = torch.tensor([1, 1, 2.0 ** -11], dtype=dt)
+    k[0, 0, 16, 8:11] = torch.tensor([1, 2.0 ** -12, 2.0 ** -12], dtype=dt)
+    k[0, 0, 17, 8:10] = torch.tensor([1, 2.0 ** -12], dtype=dt)
+    v[0, 0, 16, 64:], v[0, 0, 17, 64:] = 4096 * c, -4096 * c
+    got = ct.causal_dot_product(*(t.to(DEV) for t in (q, k, v))).double().cpu()
+    assert (got[0, 0, 40, :64] == 2.0 ** -11).all()
+    assert (got[0, 0, 20, 64:] == 2.0 ** -11 * c).all()
+    assert torch.equal(got, torch.from_numpy(oracle.causal(q, k, v)))
+    # ... and summed over the future
+    rev = ct.causal_dot_product(*(t.flip(2).contiguous().to(DEV) for t in (q, k, v)), True).double().cpu()
+    assert torch.equal(rev.flip(2), got)
 
 
 @pytest.mark.parametrize("dt", [BF, HF], ids=["bf16", "fp16"])

@@ -110,8 +110,8 @@ __device__ __forceinline__ bool any_nan(f32x4 v) {
     const float s = (v[0] + v[1]) + (v[2] + v[3]);  // (also true where infinities cancel: number_or then changes nothing)
     return s != s;
 }
-// v where it is a number, else the same element of w.  An infinite state or score entry splits into hi = inf and two times
-// inf - inf; the sum formed from the hi parts alone then has the value the single-number arithmetic gives.
+// v where it is a number, else the same element of w.  An infinite state, score or (fp16) C entry splits into hi = inf and
+// inf - inf; the sum formed from the hi parts of both factors alone then has the value the single-number arithmetic gives.
 __device__ __forceinline__ f32x4 number_or(f32x4 v, f32x4 w) {
 #pragma unroll
     for (int e = 0; e < 4; ++e) v[e] = v[e] == v[e] ? v[e] : w[e];
@@ -270,11 +270,12 @@ __device__ __forceinline__ void wide_compute_role(const WideOp &op, int bh, int 
 #pragma unroll
         for (int x = 0; x < 3; ++x) p[x] = sP[((buf * 3 + x) * 2 + half) * 64 + l];
         const f32x4 other = sX[(buf * kWideCompute + (w ^ 4)) * 64 + l];
-        f32x4 hi = Bf16::mfma(ch, p[0], o + other), rest = zero;
-        if constexpr (FP16) {
-            hi = Bf16::mfma(cl, p[0], hi);
+        const f32x4 hi = Bf16::mfma(ch, p[0], o + other);
+        f32x4 rest = zero;
+        if constexpr (FP16) {  // (the lo part of an infinite C is no number either: it stays out of `hi`)
             rest = Bf16::mfma(cl, p[2], rest);
             rest = Bf16::mfma(cl, p[1], rest);
+            rest = Bf16::mfma(cl, p[0], rest);
         }
         rest = Bf16::mfma(ch, p[2], rest);
         rest = Bf16::mfma(ch, p[1], rest);

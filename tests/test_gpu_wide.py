@@ -119,6 +119,18 @@ def test_an_infinite_value_stays_in_its_column(ct, dt):
     assert not torch.isfinite(got[0, 0, 64:, 5]).any()
 
 
+@pytest.mark.parametrize("x", [float("inf"), -float("inf")])
+@pytest.mark.parametrize("dt", [BF, HF], ids=["bf16", "fp16"])
+def test_an_infinite_value_within_its_chunk(ct, dt, x):
+    """v[40, 5] infinite: from there to the end of the chunk column 5 is infinite with the sign of the score times that of x
+    (no score of these inputs is zero), in both directions: reversed, the positions of the chunk up to 40."""
+    q, k, v, _ = (t.to(DEV) for t in inputs(1, 1, 96, 256, 256, dt, seed=4))
+    v[0, 0, 40, 5] = x
+    want = torch.sign(q[0, 0].float() @ k[0, 0, 40].float()) * x
+    for rev, rows in ((False, slice(40, 64)), (True, slice(32, 41))):
+        assert torch.equal(ct.causal_dot_product(q, k, v, rev)[0, 0, rows, 5].float(), want[rows])
+
+
 def test_groups_need_no_workspace(ct):
     """Called without the workspace it asks for, the library walks the sequence whole."""
     from cottention_transformer_amd import _loader

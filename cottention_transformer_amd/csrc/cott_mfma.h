@@ -28,7 +28,9 @@ constexpr int kWaveStageStride = 64 + 8;  // elements per row of an output wavef
 // `ldc` elements (the pointers already include the first column), so a problem can own a column
 // slice of a wider tensor.  gstate: G slots of DI*DJ floats per head (G > 1 or non-causal).
 // sin / sout (either may be null): row-major fp32 [di][lds] state per head, likewise offset to the
-// first column; the scan starts from sin and its last group writes the final state to sout.
+// first column; the scan starts from sin and its last group writes the final state to sout.  They may be the same
+// memory: with more than one group the prefix pass puts sin into the groups' slots and the scan, whose last group may
+// end before another one starts, is given none (sin_in_slots).
 template <class E>
 struct ProblemT {
     const E *A, *B, *C;
@@ -79,6 +81,10 @@ struct ProblemT {
 template <class E>
 struct ProblemSetT {
     ProblemT<E> p[kMaxProblems];
+    // after the prefix pass has been launched: the scan takes the start states from the slots
+    void sin_in_slots() {
+        for (ProblemT<E> &x : p) x.sin = nullptr;
+    }
     int count;
     int xcds;  // XCDs of the device: workgroup i is dispatched to XCD i % xcds (8 on an unpartitioned MI355X)
     // 16-bit kernels: the group-state pass cuts every group of the scan into `sub` pieces, one workgroup and one
@@ -503,11 +509,14 @@ __global__ __launch_bounds__(kThreads, 2) void group_state_kernel(ProblemSet set
 
 // Over the G * sub slots of one head, element-wise.  mode 0: the first slot of group g gets the sum of all slots of
 // the groups before g (only the first `ncomputed` groups hold data), or, for an op in complement form (all groups
-// hold data), the total minus that sum.  mode 1: total into slot 0.  Slots are read in batches of independent
+// hold data), the total minus that sum; to either the problem's start state is added (sin, not in complement form).
+// mode 1: total into slot 0.  Slots are read in batches of independent
 // loads and only written after they have been read.
+// Tile t of a slot (64 float4) holds rows 16 (t / njt) and columns 16 (t % njt) onwards, or, with nit > 0 (the slots of
+// cott_mfma_f32.h), rows 16 (t % nit) and columns 16 (t / nit).
 template <class E>
 __global__ __launch_bounds__(kThreads) void state_prefix_kernel(ProblemSetT<E> set, int BH, int G, int sub, int ncomputed,
-                                                                int state_floats, int mode) {
+                                                                int state_floats, int mode, int njt, int nit = 0) {
     constexpr int BATCH = 8;
     const int sf4 = state_floats / 4;
     const int blocks_per_state = (sf4 + kThreads - 1) / kThreads;
@@ -534,6 +543,16 @@ __global__ __launch_bounds__(kThreads) void state_prefix_kernel(ProblemSetT<E> s
             return;
         }
     }
+    f32x4 start = zero;
+    if (set.p[prob].sin != nullptr) {
+        const ProblemT<E> &pr = set.p[prob];
+        const int tile = e >> 6, it = nit > 0 ? tile % nit : tile / njt, jt = nit > 0 ? tile / nit : tile % njt;
+        const int i0 = 16 * it + 4 * ((e >> 4) & 3), j = 16 * jt + (e & 15);
+        const float *src = pr.sin + ((size_t)bh * pr.di + i0) * pr.lds + j;
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+            if (i0 + q < pr.di && j < pr.dj) start[q] = src[(size_t)q * pr.lds];
+    }
     f32x4 run = zero;
     for (int s0 = 0; s0 < nslots; s0 += BATCH) {
         f32x4 t[BATCH];
@@ -542,7 +561,7 @@ __global__ __launch_bounds__(kThreads) void state_prefix_kernel(ProblemSetT<E> s
 #pragma unroll
         for (int u = 0; u < BATCH; ++u) {
             const int s = s0 + u;
-            if (s < nslots && s % sub == 0) p[(size_t)s * sf4] = comp ? total - run : run;
+            if (s < nslots && s % sub == 0) p[(size_t)s * sf4] = comp ? total - run : run + start;
             run += t[u];
         }
     }

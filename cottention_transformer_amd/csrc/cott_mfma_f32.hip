@@ -11,7 +11,7 @@ template <int DI, int DJ>
 hipError_t run_causal_split(const SetArgs &a) {
     using TL = Tiling<DI, DJ>;
     constexpr int PF = 2;
-    const ProblemSetF ps = make_set<float, DI, DJ>(a);
+    ProblemSetF ps = make_set<float, DI, DJ>(a);
     if (a.G > 1) {
         if (ps.nact > 0) {
             ProfScope prof(K_GROUP_STATE, a.stream);
@@ -21,7 +21,8 @@ hipError_t run_causal_split(const SetArgs &a) {
         const int bps = (TL::STATE_FLOATS / 4 + kThreads - 1) / kThreads;
         ProfScope prof(K_STATE_PREFIX, a.stream);
         state_prefix_kernel<float><<<dim3((unsigned)(a.BH * ps.count * bps)), dim3(kThreads), 0, a.stream>>>(
-            ps, a.BH, a.G, a.sub, a.G - 1, TL::STATE_FLOATS, 0);
+            ps, a.BH, a.G, a.sub, a.G - 1, TL::STATE_FLOATS, 0, TL::NJT);
+        ps.sin_in_slots();
     }
     ProfScope prof(a.scan_prof_id, a.stream);
     split_scan_kernel<DI, DJ, PF><<<dim3(grid_for(a.BH, a.count, a.G, a.xcds)), dim3(512), 0, a.stream>>>(
@@ -36,7 +37,7 @@ hipError_t run_causal_f32(const SetArgs &a) {
         if (split) return run_causal_split<DI, DJ>(a);
     }
     using TL = TilingF32<DI, DJ>;
-    const ProblemSetF32 ps = make_set<float, DI, DJ>(a);
+    ProblemSetF32 ps = make_set<float, DI, DJ>(a);
     if (a.G > 1) {
         {
             ProfScope prof(K_GROUP_STATE, a.stream);
@@ -46,7 +47,8 @@ hipError_t run_causal_f32(const SetArgs &a) {
         const int bps = (TL::STATE_FLOATS / 4 + kThreads - 1) / kThreads;
         ProfScope prof(K_STATE_PREFIX, a.stream);
         state_prefix_kernel<float><<<dim3((unsigned)(a.BH * a.count * bps)), dim3(kThreads), 0, a.stream>>>(
-            ps, a.BH, a.G, 1, a.G - 1, TL::STATE_FLOATS, 0);
+            ps, a.BH, a.G, 1, a.G - 1, TL::STATE_FLOATS, 0, 0, TL::NIT);
+        ps.sin_in_slots();
     }
     ProfScope prof(a.scan_prof_id, a.stream);
     scan_f32_kernel<DI, DJ, false><<<dim3(grid_for(a.BH, a.count, a.G, a.xcds)), dim3(kThreads), 0, a.stream>>>(
@@ -68,7 +70,7 @@ hipError_t run_noncausal_f32(const SetArgs &a) {
         const int bps = (TL::STATE_FLOATS / 4 + kThreads - 1) / kThreads;
         ProfScope prof(K_STATE_PREFIX, a.stream);
         state_prefix_kernel<float><<<dim3((unsigned)(a.BH * a.count * bps)), dim3(kThreads), 0, a.stream>>>(
-            ps, a.BH, a.G, 1, a.G, TL::STATE_FLOATS, 1);
+            ps, a.BH, a.G, 1, a.G, TL::STATE_FLOATS, 1, 0, TL::NIT);
     }
     ProfScope prof(K_APPLY, a.stream);
     scan_f32_kernel<DI, DJ, true><<<dim3(grid_for(a.BH, a.count, a.G, a.xcds)), dim3(kThreads), 0, a.stream>>>(

@@ -93,7 +93,8 @@ COTT_API int cott_causal_fwd_noalloc(const void *q, const void *k, const void *v
  * state (GPT_Trainer/GPTCosAttention.py:253-272; generation driver fast_infer.py:111): one call
  * over the prompt yields the outputs of cott_causal_fwd AND the state that cott_decode_step
  * continues from.  state_in / state_out: (B,H,Dk,Dv) fp32 (fp64 for COTT_F64), the layout of
- * cott_decode_step; either may be NULL (start from zero / state not wanted); they may alias.
+ * cott_decode_step; either may be NULL (start from zero / state not wanted); they may be the same memory (but not
+ * overlap in part).
  * Workspace: cott_causal_workspace_bytes().  N == 0 copies state_in to state_out. */
 COTT_API int cott_causal_fwd_state(const void *q, const void *k, const void *v, void *o,
                           const void *state_in, void *state_out,

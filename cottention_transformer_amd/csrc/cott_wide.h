@@ -45,9 +45,11 @@ struct WideSet {
     int count, items;  // ops; workgroups per head and group = all slices of all ops
     int xcds;
     // Few heads: the sequence is cut into G groups of cpg chunks (in walking order).  wide_scan_kernel<..., SUMS> leaves the
-    // sum of B^T C over each group but the last in slots [head][item][group] of wide_slot_vectors() float4; a group of the
-    // scan starts from the sum of the slots before it (and sin).
-    int G, cpg;
+    // sum of B^T C over each group but the last in slots [head][item][1 + group] of wide_slot_vectors() float4 and, where
+    // there is one, the start state in slot 0 (its workgroups `G - 1`; first_slot = 0, else 1); a group of the scan starts
+    // from the sum of the slots up to its own number.  The scan itself then reads no sin: sout may be the same memory, and
+    // the last group may write it before another one starts.
+    int G, cpg, first_slot;
     f32x4 *slots;
 };
 // One slice's state in the order of its owners: [wavefront][tile][lane].
@@ -218,10 +220,11 @@ __device__ __forceinline__ void wide_loader_role(const WideOp &op, int bh, int c
 }
 
 // Wavefront w of kWideCompute: state columns 16 (w & 3) .. + 15 of the slice, row half w >> 2.
-// slots: those of this head and item; `grp` of them precede this group (SUMS: slot `grp` receives the sum).
+// slots: those of this head and item; this group starts from the sum of slots first_slot .. grp (SUMS: slot grp + 1 receives
+// the sum, or, with an empty range of chunks, slot 0 the start state).
 template <class TR, int DI, bool SUMS>
 __device__ __forceinline__ void wide_compute_role(const WideOp &op, int bh, int c0, const WideRange &rg, f32x4 *slots, int grp,
-                                                  bool last_group, int w, int l, const u16 *sA, const u16 *sB,
+                                                  int first_slot, bool last_group, int w, int l, const u16 *sA, const u16 *sB,
                                                   const u16 *sC, u16 *sO, const u32x4 *sP, f32x4 *sX) {
     using T = WideTiling<DI>;
     constexpr bool FP16 = std::is_same<TR, Fp16>::value;
@@ -234,7 +237,8 @@ __device__ __forceinline__ void wide_compute_role(const WideOp &op, int bh, int 
 #pragma unroll
     for (int it = 0; it < 2 * KS; ++it) S[it] = zero;
     const int own = w * 2 * KS * 64 + l;
-    if (!SUMS && op.sin != nullptr && j < dj) {
+    const bool start = SUMS && rg.p0 == rg.p1;
+    if ((!SUMS || start) && op.sin != nullptr && j < dj) {
         const float *src = op.sin + (size_t)bh * di * dj + j;
 #pragma unroll
         for (int it = 0; it < 2 * KS; ++it)
@@ -244,8 +248,13 @@ __device__ __forceinline__ void wide_compute_role(const WideOp &op, int bh, int 
                 if (i < di) S[it][q] = src[(size_t)i * dj];
             }
     }
+    if (start) {
+#pragma unroll
+        for (int it = 0; it < 2 * KS; ++it) slots[own + 64 * it] = S[it];
+        return;
+    }
     if constexpr (!SUMS) {
-        for (int gp = 0; gp < grp; ++gp) {
+        for (int gp = first_slot; gp <= grp; ++gp) {
             f32x4 t[2 * KS];
 #pragma unroll
             for (int it = 0; it < 2 * KS; ++it) t[it] = slots[(size_t)gp * wide_slot_vectors(DI) + own + 64 * it];
@@ -360,7 +369,7 @@ __device__ __forceinline__ void wide_compute_role(const WideOp &op, int bh, int 
     });
     if constexpr (SUMS) {
 #pragma unroll
-        for (int it = 0; it < 2 * KS; ++it) slots[(size_t)grp * wide_slot_vectors(DI) + own + 64 * it] = S[it];
+        for (int it = 0; it < 2 * KS; ++it) slots[(size_t)(grp + 1) * wide_slot_vectors(DI) + own + 64 * it] = S[it];
         return;
     }
     finish((rg.p1 - 1 - rg.p0) & 1);
@@ -377,8 +386,8 @@ __device__ __forceinline__ void wide_compute_role(const WideOp &op, int bh, int 
     }
 }
 
-// 768 threads: wavefronts 0..7 compute, 8..11 load.  Grid: grid_for(BH, set.items, groups, set.xcds), groups = G, or G - 1 for
-// the sums, so that the slices and ops of a head and group run on one XCD and share its tiles through that L2.
+// 768 threads: wavefronts 0..7 compute, 8..11 load.  Grid: grid_for(BH, set.items, groups, set.xcds), groups = G, or for the sums
+// G - first_slot, so that the slices and ops of a head and group run on one XCD and share its tiles through that L2.
 template <class TR, int DI, bool SUMS>
 __global__ __launch_bounds__(64 * (kWideCompute + kWideLoad)) void wide_scan_kernel(WideSet set, int BH, int N, int nchunks) {
     using T = WideTiling<DI>;
@@ -388,12 +397,13 @@ __global__ __launch_bounds__(64 * (kWideCompute + kWideLoad)) void wide_scan_ker
     u32x4 *sP = reinterpret_cast<u32x4 *>(sO + 2 * T::OTILE);
     f32x4 *sX = reinterpret_cast<f32x4 *>(sP + T::SCORES);
     const WorkItem wi = decode_workgroup(set.items, BH, set.xcds);
-    if (wi.grp >= (SUMS ? set.G - 1 : set.G)) return;
+    if (wi.grp >= (SUMS ? set.G - set.first_slot : set.G)) return;
+    const bool start = SUMS && wi.grp == set.G - 1;  // this workgroup only puts the start state into slot 0
     int which = 0, slice = wi.prob;
     while (which + 1 < set.count && slice >= set.op[which].slices) slice -= set.op[which++].slices;
     const WideOp &op = set.op[which];
-    const WideRange rg = {N, nchunks, wi.grp * set.cpg, min((wi.grp + 1) * set.cpg, nchunks)};
-    f32x4 *slots = set.slots + ((size_t)wi.bh * set.items + wi.prob) * (set.G - 1) * wide_slot_vectors(DI);
+    const WideRange rg = {N, nchunks, start ? 0 : wi.grp * set.cpg, start ? 0 : min((wi.grp + 1) * set.cpg, nchunks)};
+    f32x4 *slots = set.slots + ((size_t)wi.bh * set.items + wi.prob) * set.G * wide_slot_vectors(DI);
     const int tid = threadIdx.x;
     if constexpr (!SUMS) {  // the score tiles on the other side of the diagonal are never written: zero
         for (int x = tid; x < T::SCORES; x += 64 * (kWideCompute + kWideLoad)) sP[x] = u32x4{0u, 0u, 0u, 0u};
@@ -401,9 +411,9 @@ __global__ __launch_bounds__(64 * (kWideCompute + kWideLoad)) void wide_scan_ker
     }
     const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
     if (w < kWideCompute)
-        wide_compute_role<TR, DI, SUMS>(op, wi.bh, slice * kWideSlice, rg, slots, wi.grp, wi.grp == set.G - 1, w, tid & 63, sA, sB,
-                                        sC, sO, sP, sX);
-    else
+        wide_compute_role<TR, DI, SUMS>(op, wi.bh, slice * kWideSlice, rg, slots, wi.grp, set.first_slot, wi.grp == set.G - 1, w,
+                                        tid & 63, sA, sB, sC, sO, sP, sX);
+    else if (!start)
         wide_loader_role<TR, DI, SUMS>(op, wi.bh, slice * kWideSlice, rg, tid - 64 * kWideCompute, sA, sB, sC, sO,
                                        reinterpret_cast<u32x2 *>(sP));
 }

@@ -27,18 +27,23 @@ int wide_groups(long BH, int items, int nchunks, int cus, int xcds) {
 
 int wide_chunks(int N) { return (N + kWideChunk - 1) / kWideChunk; }
 
-// Slots of one launch: BH heads, `items` slices, all groups but the last.
+// Slots of one launch in G > 1 groups: BH heads, `items` slices, the start state and all groups but the last.
 size_t wide_slot_bytes(long BH, int items, int G, int pad) {
-    return (size_t)BH * items * (G - 1) * wide_slot_vectors(pad) * sizeof(f32x4);
+    return G > 1 ? (size_t)BH * items * G * wide_slot_vectors(pad) * sizeof(f32x4) : 0;
 }
 
 template <class TR, int DI>
-hipError_t launch_set(const WideSet &set, int BH, int N, int prof_id, hipStream_t stream) {
+hipError_t launch_set(WideSet set, int BH, int N, int prof_id, hipStream_t stream) {
     const int nchunks = wide_chunks(N);
     const dim3 block(64 * (kWideCompute + kWideLoad));
+    set.first_slot = 1;
     if (set.G > 1) {
+        for (const WideOp &o : set.op)
+            if (o.sin != nullptr) set.first_slot = 0;
         ProfScope ps(K_GROUP_STATE, stream);
-        wide_scan_kernel<TR, DI, true><<<dim3(grid_for(BH, set.items, set.G - 1, set.xcds)), block, 0, stream>>>(set, BH, N, nchunks);
+        wide_scan_kernel<TR, DI, true><<<dim3(grid_for(BH, set.items, set.G - set.first_slot, set.xcds)), block, 0, stream>>>(
+            set, BH, N, nchunks);
+        for (WideOp &o : set.op) o.sin = nullptr;
     }
     ProfScope ps(prof_id, stream);
     wide_scan_kernel<TR, DI, false><<<dim3(grid_for(BH, set.items, set.G, set.xcds)), block, 0, stream>>>(set, BH, N, nchunks);

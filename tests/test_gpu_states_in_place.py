@@ -13,8 +13,9 @@ BF, HF, F32, F64 = torch.bfloat16, torch.float16, torch.float32, torch.float64
 # (heads, positions, Dk, Dv, type, cut into groups): every kernel that starts from a state; odd widths and lengths
 CASES = [(2, 4000, 64, 64, BF, True), (16, 8192, 64, 64, HF, True), (5, 3001, 48, 80, BF, True), (4, 4100, 128, 128, BF, True),
          (16, 9000, 128, 128, HF, True), (3, 2100, 112, 64, BF, True), (2, 2500, 32, 128, HF, True), (2, 3000, 64, 64, F32, True),
-         (3, 2051, 48, 64, F32, True), (2, 2500, 128, 96, F32, True), (2, 1500, 32, 64, F32, True),
-         (300, 200, 64, 64, BF, False), (2, 100, 64, 64, F64, False)]
+         (3, 2051, 48, 64, F32, True), (2, 2500, 128, 96, F32, True), (2, 1500, 32, 64, F32, True), (2, 2000, 256, 256, BF, True),
+         (1, 4100, 160, 144, HF, True), (3, 900, 64, 192, BF, True), (300, 200, 64, 64, BF, False), (2, 300, 256, 160, BF, False),
+         (2, 100, 64, 64, F64, False)]
 
 
 @pytest.mark.parametrize("case", CASES, ids=lambda c: "x".join(map(str, c[:4])) + "-" + str(c[4]).split(".")[-1])

@@ -136,12 +136,12 @@ __global__ __launch_bounds__(256) void generic_scan_kernel(const typename ST::el
 //   S[i][j] += k[i] v[j] ;  o[j] = sum_i q[i] S[i][j]
 // Thread t owns a 4-wide column strip (t % nvb) and every rg-th row starting at t / nvb.  Rows are
 // processed 16 at a time; the state loads of a pass are issued before anything else (q and k are
-// staged through LDS while they are in flight) and every load precedes the first store.
+// staged through LDS while they are in flight) and every load precedes the first store.  o may be the memory of q, k or v:
+// a head's rows are written after its workgroup has read q and k whole, and these columns of v.
 template <class ST, class SF /* state scalar: float or double */>
-__global__ __launch_bounds__(256) void decode_kernel(SF *__restrict__ S, const typename ST::elem *__restrict__ q,
-                                                     const typename ST::elem *__restrict__ k,
-                                                     const typename ST::elem *__restrict__ v,
-                                                     typename ST::elem *__restrict__ o, int dk, int dv) {
+__global__ __launch_bounds__(256) void decode_kernel(SF *__restrict__ S, const typename ST::elem *q,
+                                                     const typename ST::elem *k, const typename ST::elem *v,
+                                                     typename ST::elem *o, int dk, int dv) {
     typedef SF __attribute__((ext_vector_type(4))) sf4;
     constexpr int U = 16;
     extern __shared__ __attribute__((aligned(32))) unsigned char smem_raw[];
@@ -229,15 +229,15 @@ struct DecodePrep {
 };
 
 // 1 << strip_log2 wavefronts per head, each with its own columns of the state (1 << row_log2 lanes to a row, at least 8):
-// few heads are a serial chain of row batches in too few wavefronts otherwise.
+// few heads are a serial chain of row batches in too few wavefronts otherwise.  Every one of them reads all of q and k, so
+// with o in their memory there has to be one wavefront per head, which writes o last (run_decode).
 // NT bit 0: non-temporal state loads, bit 1: non-temporal state stores (a state far larger than the last-level
 // cache is not found there again by the next step).
 template <class ST, class SF, bool PREP, int NT = 0>
-__global__ __launch_bounds__(256) void decode_wave_kernel(SF *__restrict__ S, const typename ST::elem *__restrict__ q,
-                                                          const typename ST::elem *__restrict__ k,
-                                                          const typename ST::elem *__restrict__ v,
-                                                          typename ST::elem *__restrict__ o, int BH, int dk, int dv,
-                                                          int strip_log2, int row_log2, DecodePrep prep) {
+__global__ __launch_bounds__(256) void decode_wave_kernel(SF *__restrict__ S, const typename ST::elem *q,
+                                                          const typename ST::elem *k, const typename ST::elem *v,
+                                                          typename ST::elem *o, int BH, int dk, int dv, int strip_log2,
+                                                          int row_log2, DecodePrep prep) {
     typedef SF __attribute__((ext_vector_type(4))) sf4;
     constexpr int U = 16;
     extern __shared__ __attribute__((aligned(32))) unsigned char smem_raw[];

@@ -61,8 +61,15 @@ hipError_t run_decode(void *state, const void *q, const void *k, const void *v, 
         // 32 columns, and up to one wavefront per CU is a workgroup of its own so that they land on different CUs.  16-bit
         // tensors, state out of the caches, us per step before / after: D128 16 heads 8.9 / 3.7, 128 heads 9.9 / 5.9,
         // 256 heads 14.7 / 9.6, 512 heads 19.5 / 17.7, 1024 heads (unchanged form) 32.0; D64 16 heads 3.3 / 3.1.
+        // (o in the memory of q or k: one wavefront per head, see decode_wave_kernel.)
+        const char *const ob = static_cast<const char *>(o);
+        auto in_o = [&](const void *x) {
+            const char *const xb = static_cast<const char *>(x);
+            return xb < ob + (size_t)BH * dv * sizeof(E) && ob < xb + (size_t)BH * dk * sizeof(E);
+        };
+        const bool strips = !in_o(q) && !in_o(k);
         int strip_log2 = 0;
-        while ((nv >> strip_log2) > 8 && ((long)BH << strip_log2) < 1024) ++strip_log2;
+        while (strips && (nv >> strip_log2) > 8 && ((long)BH << strip_log2) < 1024) ++strip_log2;
         const int row_log2 = __builtin_ctz((unsigned)(nv >> strip_log2));
         const long units = (long)BH << strip_log2;
         const int waves = units <= 256 ? 1 : 4;

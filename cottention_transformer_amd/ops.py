@@ -504,10 +504,20 @@ def noncausal_backward(q, k, v, grad_out, merged_heads=False):
     return dq, dk_, dv_
 
 
+def _decode_out(out, *inputs):
+    """Where a decode step may write its output: `out` itself, also when it IS one of q, k, v, but not when it shares memory
+    with one of them in another way (heads run in any order, each reads its own rows before it writes them)."""
+    for t in inputs:
+        if _overlaps(out, t) and (out.data_ptr() != t.data_ptr() or out.shape != t.shape):
+            return torch.empty_like(out)
+    return out
+
+
 def decode_step(state, q, k, v, out=None):
     """One recurrent step, in place on `state` (B,H,Dk,Dv; fp32, or fp64 for fp64 inputs):
     state += k v^T ; returns o = q state  (GPT_Trainer/GPTCosAttention.py:264,267).
-    q,k: (B,H,Dk); v: (B,H,Dv).  The reference's `past_KV` is `state.transpose(-1,-2)`."""
+    q,k: (B,H,Dk); v: (B,H,Dv); out: may share memory with q, k or v.  The reference's `past_KV` is
+    `state.transpose(-1,-2)`."""
     _require_gpu(state=state, q=q, k=k, v=v)
     if state.dim() != 4 or q.dim() != 3 or k.dim() != 3 or v.dim() != 3:
         raise RuntimeError("decode_step: state (B,H,Dk,Dv), q/k (B,H,Dk), v (B,H,Dv)")
@@ -522,15 +532,17 @@ def decode_step(state, q, k, v, out=None):
         raise RuntimeError(f"decode_step: state must be a contiguous {want} tensor (it is updated in place)")
     q, k, v = q.contiguous(), k.contiguous(), v.contiguous()
     if out is None:
-        out = torch.empty((b, h, dv), dtype=q.dtype, device=q.device)
+        o = out = torch.empty((b, h, dv), dtype=q.dtype, device=q.device)
     elif out.shape != (b, h, dv) or out.dtype != q.dtype or not out.is_contiguous() or out.device != q.device:
         raise RuntimeError("decode_step: bad `out` tensor")
+    else:
+        o = _decode_out(out, q, k, v)
     L = _loader.lib()
     with _on(q.device):
-        rc = L.cott_decode_step(state.data_ptr(), q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), b, h, dk,
+        rc = L.cott_decode_step(state.data_ptr(), q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(), b, h, dk,
                                 dv, code, _stream(q.device))
     _check(rc, "cott_decode_step")
-    return out
+    return out if o is out else out.copy_(o)
 
 
 def decode_step_prepared(state, q, k, v, sig=None, cnt=0.0, rotary=None, out=None):
@@ -554,9 +566,11 @@ def decode_step_prepared(state, q, k, v, sig=None, cnt=0.0, rotary=None, out=Non
         raise RuntimeError(f"decode_step_prepared: state must be a contiguous {want} tensor")
     q, k, v = q.contiguous(), k.contiguous(), v.contiguous()
     if out is None:
-        out = torch.empty((b, h, dv), dtype=q.dtype, device=q.device)
+        o = out = torch.empty((b, h, dv), dtype=q.dtype, device=q.device)
     elif out.shape != (b, h, dv) or out.dtype != q.dtype or not out.is_contiguous() or out.device != q.device:
         raise RuntimeError("decode_step_prepared: bad `out` tensor")
+    else:
+        o = _decode_out(out, q, k, v)
     if sig is not None:
         if sig.shape != (h,):
             raise RuntimeError(f"sig must have shape {(h,)}")
@@ -570,12 +584,12 @@ def decode_step_prepared(state, q, k, v, sig=None, cnt=0.0, rotary=None, out=Non
         pos = int(pos)
     L = _loader.lib()
     with _on(q.device):
-        rc = L.cott_decode_step_prep(state.data_ptr(), q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(),
+        rc = L.cott_decode_step_prep(state.data_ptr(), q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(),
                                      sig.data_ptr() if sig is not None else None, float(cnt),
                                      table.data_ptr() if table is not None else None, pos, rdim, rows, b, h, dk, dv, code,
                                      _stream(q.device))
     _check(rc, "cott_decode_step_prep")
-    return out
+    return out if o is out else out.copy_(o)
 
 
 DECODE_BLOCK_ROWS = 16  # sequences up to which decode_block is built (kTokenRows, csrc/cott_launch.h)

@@ -214,7 +214,8 @@ COTT_API int cott_noncausal_bwd_bnhd(const void *q, const void *k, const void *v
  * Replaces the per-token body of GPT_Trainer/GPTCosAttention.py:262-269 (:264 update, :267 read;
  * the output uses the UPDATED state).  `state` is caller-owned, (B,H,Dk,Dv), fp32 (fp64 for
  * COTT_F64) and updated in place; the reference keeps the transposed orientation (B,H,Dv,Dk) in
- * fp64 (:80).  q,k: (B,H,Dk); v,o: (B,H,Dv) in `dtype`.  Needs no workspace. */
+ * fp64 (:80).  q,k: (B,H,Dk); v,o: (B,H,Dv) in `dtype`.  Needs no workspace.  o may be the memory of v or, with
+ * Dk == Dv, of q or k; no other overlap. */
 COTT_API int cott_decode_step(void *state, const void *q, const void *k, const void *v, void *o,
                      int B, int H, int Dk, int Dv, int dtype, void *stream);
 
@@ -224,7 +225,7 @@ COTT_API int cott_decode_step(void *state, const void *q, const void *k, const v
  * sigmoid(norm_const), NULL = no scaling; cnt = tokens so far including this one) run inside the kernel: one
  * launch per token and layer instead of the separate elementwise kernels of
  * GPT_Trainer/GPTCosAttention.py:229-248,462-476 in front of :264-267.  q, k: (B,H,Dk) = the (B,1,H,Dk)
- * projection output; Dv in {32,64,128,256}, Dk <= 256. */
+ * projection output; Dv in {32,64,128,256}, Dk <= 256; o as in cott_decode_step. */
 COTT_API int cott_decode_step_prep(void *state, const void *q, const void *k, const void *v, void *o,
                           const float *sig, float cnt, const float *rot_table, long long position,
                           int rotary_dim, int table_rows,

@@ -108,3 +108,40 @@ def test_decode_in_column_strips(ct, oracle, case):
     o = ct.decode_step(s, q.to(DEV), k.to(DEV), v.to(DEV))
     assert rel_l2(o, ref) <= 2.0 ** -9 + 2.0 ** -16   # the output's rounding
     assert rel_l2(s, ref_state) <= 2.0 ** -23         # one fp32 multiply-add per entry
+
+
+# fewer heads than strips are made of, more, and the workgroup-per-head kernel (16 columns)
+@pytest.mark.parametrize("case", [(1, 3, 128), (2, 150, 64), (1, 1025, 64), (1, 5, 256), (1, 3, 16)], ids=lambda c: "x".join(map(str, c)))
+def test_output_in_the_memory_of_an_input(ct, oracle, case):
+    """decode_step(..., out=): q, k or v themselves, or a tensor that overlaps all three of them by half a head."""
+    b, h, d = case
+    g = torch.Generator().manual_seed(h)
+    q, k, v = (torch.randn(b, h, d, generator=g).to(BF) for _ in range(3))
+    state = torch.randn(b, h, d, d, generator=g)
+    ref_state = state.double().numpy().copy()
+    ref = oracle.decode_step(ref_state, q, k, v)
+    for which in ("q", "k", "v", "part"):
+        flat = torch.empty(4, b * h * d, dtype=BF, device=DEV)
+        x = dict(zip("qkv", (row.view(b, h, d) for row in flat)))
+        for name, t in zip("qkv", (q, k, v)):
+            x[name].copy_(t)
+        out = x[which] if which != "part" else flat.view(-1)[b * h * d - d // 2:][:b * h * d].view(b, h, d)
+        s = state.to(DEV)
+        got = ct.decode_step(s, x["q"], x["k"], x["v"], out=out)
+        assert got is out and rel_l2(out, ref) <= 2.0 ** -9 + 2.0 ** -16, which   # the output's rounding
+        assert rel_l2(s, ref_state) <= 2.0 ** -23, which                          # one fp32 multiply-add per entry
+
+
+def test_prepared_output_in_the_memory_of_an_input(ct):
+    from cottention_transformer_amd import ops
+    g = torch.Generator().manual_seed(1)
+    q, k, v = (torch.randn(2, 9, 128, generator=g).to(DEV, BF) for _ in range(3))
+    state = torch.randn(2, 9, 128, 128, generator=g).to(DEV)
+    want_state = state.clone()
+    want = ops.decode_step_prepared(want_state, q, k, v)
+    for i in range(3):
+        x = [t.clone() for t in (q, k, v)]
+        s = state.clone()
+        got = ops.decode_step_prepared(s, *x, out=x[i])
+        # the same sum in one wavefront's order or in strips: half a unit each
+        assert got is x[i] and rel_l2(got, want.double().cpu().numpy()) <= 2.0 ** -8 and torch.equal(s, want_state)

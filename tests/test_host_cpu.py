@@ -391,3 +391,15 @@ def test_launch_plans_over_device_geometries(cus, xcds):
         assert seen_groups > 50 and seen_pair > 5 and seen_comp > 5
     finally:
         assert L.cott_plan_geometry(0, 0) == _loader.OK
+
+
+@pytest.mark.parametrize("which", ["apart", "same", "shifted", "other shape"])
+def test_decode_output_that_shares_memory_with_an_input(which):
+    """decode steps write into `out` itself unless it overlaps an input without being that very tensor."""
+    from cottention_transformer_amd import ops
+    flat = torch.zeros(64)
+    q = flat[:24].view(1, 3, 8)
+    out = {"apart": flat[24:48].view(1, 3, 8), "same": flat[:24].view(1, 3, 8), "shifted": flat[8:32].view(1, 3, 8),
+           "other shape": flat[:12].view(1, 3, 4)}[which]
+    direct = ops._decode_out(out, q, torch.zeros(1, 3, 8)) is out
+    assert direct == (which in ("apart", "same"))

@@ -52,8 +52,10 @@ SIGNATURES = {
     "cott_noncausal_bwd_bnhd": (_i, [_vp] * 7 + [_i] * 6 + [_vp, _sz, _vp]),
     "cott_decode_step": (_i, [_vp] * 5 + [_i] * 5 + [_vp]),
     "cott_decode_step_prep": (_i, [_vp] * 6 + [ctypes.c_float, _vp, ctypes.c_longlong] + [_i] * 7 + [_vp]),
+    "cott_decode_step_norm": (_i, [_vp] * 6 + [_i, ctypes.c_float, _vp, ctypes.c_longlong] + [_i] * 7 + [_vp]),
     "cott_decode_block_scratch_bytes": (_sz, [_i] * 4),
     "cott_decode_block": (_i, [_vp] * 8 + [ctypes.c_float, _vp, ctypes.c_longlong] + [_i] * 6 + [_vp, _sz, _vp]),
+    "cott_decode_block_norm": (_i, [_vp] * 8 + [_i, ctypes.c_float, _vp, ctypes.c_longlong] + [_i] * 6 + [_vp, _sz, _vp]),
     "cott_profile_enable": (_i, [_i]),
     "cott_profile_read": (_i, [_i, ctypes.POINTER(ctypes.c_double), ctypes.POINTER(ctypes.c_long)]),
     "cott_kernel_name": (ctypes.c_char_p, [_i]),

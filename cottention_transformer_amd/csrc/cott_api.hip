@@ -1363,10 +1363,17 @@ int cott_decode_step(void *state, const void *q, const void *k, const void *v, v
     return COTT_OK;
 }
 
-int cott_decode_step_prep(void *state, const void *q, const void *k, const void *v, void *o, const float *sig, float cnt,
-                          const float *rot_table, long long position, int rotary_dim, int table_rows, int B, int H,
+namespace {
+// The exponent of the value scaling: sig, norm (of type norm_type), or neither.
+struct Scaling {
+    const float *sig;
+    const void *norm;
+    int norm_type;
+};
+int decode_step_prep_impl(const char *fn, void *state, const void *q, const void *k, const void *v, void *o, const Scaling &sc,
+                          float cnt, const float *rot_table, long long position, int rotary_dim, int table_rows, int B, int H,
                           int Dk, int Dv, int dtype, void *stream) {
-    const char *fn = "cott_decode_step_prep";
+    if (sc.norm != nullptr && elem_size(sc.norm_type) == 0) return fail(COTT_ERR_INVALID, "%s: unknown dtype %d", fn, sc.norm_type);
     if (elem_size(dtype) == 0) return fail(COTT_ERR_INVALID, "%s: unknown dtype %d", fn, dtype);
     if (B < 0 || H < 0 || Dk < 1 || Dv < 1) return fail(COTT_ERR_INVALID, "%s: bad size", fn);
     const int nv = Dv / 4;
@@ -1385,10 +1392,25 @@ int cott_decode_step_prep(void *state, const void *q, const void *k, const void 
         if (table_rows < 1) return fail(COTT_ERR_INVALID, "%s: empty rotary table", fn);
         pos = position < 0 ? 0 : (position >= table_rows ? table_rows - 1 : position);  // clamped like the batched pass
     }
-    hipError_t e = cott::launch_decode_prep(dtype, state, q, k, v, o, (int)BH, H, Dk, Dv, sig, cnt, rot_table, pos, rotary_dim,
-                                            1e-12f, static_cast<hipStream_t>(stream));
+    hipError_t e = cott::launch_decode_prep(dtype, state, q, k, v, o, (int)BH, H, Dk, Dv, sc.sig, sc.norm, sc.norm_type, cnt,
+                                            rot_table, pos, rotary_dim, 1e-12f, static_cast<hipStream_t>(stream));
     if (e != hipSuccess) return fail(COTT_ERR_HIP, "%s: HIP launch failed: %s", fn, hipGetErrorString(e));
     return COTT_OK;
+}
+}  // namespace
+
+int cott_decode_step_prep(void *state, const void *q, const void *k, const void *v, void *o, const float *sig, float cnt,
+                          const float *rot_table, long long position, int rotary_dim, int table_rows, int B, int H,
+                          int Dk, int Dv, int dtype, void *stream) {
+    return decode_step_prep_impl("cott_decode_step_prep", state, q, k, v, o, Scaling{sig, nullptr, 0}, cnt, rot_table, position,
+                                 rotary_dim, table_rows, B, H, Dk, Dv, dtype, stream);
+}
+
+int cott_decode_step_norm(void *state, const void *q, const void *k, const void *v, void *o, const void *norm_const,
+                          int norm_dtype, float cnt, const float *rot_table, long long position, int rotary_dim, int table_rows,
+                          int B, int H, int Dk, int Dv, int dtype, void *stream) {
+    return decode_step_prep_impl("cott_decode_step_norm", state, q, k, v, o, Scaling{nullptr, norm_const, norm_dtype}, cnt,
+                                 rot_table, position, rotary_dim, table_rows, B, H, Dk, Dv, dtype, stream);
 }
 
 size_t cott_decode_block_scratch_bytes(int B, int H, int D, int dtype) {
@@ -1396,10 +1418,11 @@ size_t cott_decode_block_scratch_bytes(int B, int H, int D, int dtype) {
     return (size_t)4 * B * H * D * 2;
 }
 
-int cott_decode_block(const void *x, const void *wq, const void *wk, const void *wv, const void *wo, void *state, void *y,
-                      const float *sig, float cnt, const float *rot_table, long long position, int rotary_dim,
+namespace {
+int decode_block_impl(const char *fn, const void *x, const void *wq, const void *wk, const void *wv, const void *wo, void *state,
+                      void *y, const Scaling &sc, float cnt, const float *rot_table, long long position, int rotary_dim,
                       int table_rows, int B, int H, int D, int dtype, void *scratch, size_t scratch_bytes, void *stream) {
-    const char *fn = "cott_decode_block";
+    if (sc.norm != nullptr && elem_size(sc.norm_type) == 0) return fail(COTT_ERR_INVALID, "%s: unknown dtype %d", fn, sc.norm_type);
     if (dtype != COTT_BF16 && dtype != COTT_F16) return fail(COTT_ERR_UNSUPPORTED, "%s: needs bf16 / fp16 tensors", fn);
     if (B < 0 || H < 1 || D < 1) return fail(COTT_ERR_INVALID, "%s: bad size", fn);
     if (D != 32 && D != 64 && D != 128 && D != 256)
@@ -1426,12 +1449,28 @@ int cott_decode_block(const void *x, const void *wq, const void *wk, const void 
     void *const yin[3] = {q, k, v}, *const yout[3] = {y, nullptr, nullptr};
     hipError_t e = cott::launch_token_linear(dtype, x, win, yin, 3, B, (int)E, (int)E, st);
     if (e != hipSuccess) return fail(COTT_ERR_HIP, "%s: HIP launch failed: %s", fn, hipGetErrorString(e));
-    if (int rc = cott_decode_step_prep(state, q, k, v, o, sig, cnt, rot_table, position, rotary_dim, table_rows, B, H, D, D,
+    if (int rc = decode_step_prep_impl(fn, state, q, k, v, o, sc, cnt, rot_table, position, rotary_dim, table_rows, B, H, D, D,
                                        dtype, stream))
         return rc;
     e = cott::launch_token_linear(dtype, o, wout, yout, 1, B, (int)E, (int)E, st);
     if (e != hipSuccess) return fail(COTT_ERR_HIP, "%s: HIP launch failed: %s", fn, hipGetErrorString(e));
     return COTT_OK;
+}
+}  // namespace
+
+int cott_decode_block(const void *x, const void *wq, const void *wk, const void *wv, const void *wo, void *state, void *y,
+                      const float *sig, float cnt, const float *rot_table, long long position, int rotary_dim,
+                      int table_rows, int B, int H, int D, int dtype, void *scratch, size_t scratch_bytes, void *stream) {
+    return decode_block_impl("cott_decode_block", x, wq, wk, wv, wo, state, y, Scaling{sig, nullptr, 0}, cnt, rot_table, position,
+                             rotary_dim, table_rows, B, H, D, dtype, scratch, scratch_bytes, stream);
+}
+
+int cott_decode_block_norm(const void *x, const void *wq, const void *wk, const void *wv, const void *wo, void *state, void *y,
+                           const void *norm_const, int norm_dtype, float cnt, const float *rot_table, long long position,
+                           int rotary_dim, int table_rows, int B, int H, int D, int dtype, void *scratch, size_t scratch_bytes,
+                           void *stream) {
+    return decode_block_impl("cott_decode_block_norm", x, wq, wk, wv, wo, state, y, Scaling{nullptr, norm_const, norm_dtype}, cnt,
+                             rot_table, position, rotary_dim, table_rows, B, H, D, dtype, scratch, scratch_bytes, stream);
 }
 
 namespace {

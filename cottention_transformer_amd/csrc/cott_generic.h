@@ -221,12 +221,27 @@ __global__ __launch_bounds__(256) void decode_kernel(SF *__restrict__ S, const t
 // v / max(cnt^sig[h], 1) -- what GPT_Trainer/GPTCosAttention.py:229-248,462-476 do with separate kernels before
 // the recurrence of :264-267.  dk <= 256.
 struct DecodePrep {
-    const float *sig;  // (H) sigmoid(norm_const), or null: no value scaling
+    const float *sig;  // (H) sigmoid(norm_const), or null: no value scaling ...
+    const void *norm;  // ... unless this is given: (H) norm_const itself, of type norm_type (cott_dtype)
+    int norm_type;
     const float *rot;  // (rows, R) table [sin | cos], or null: no rotation
     long long pos;     // table row, already clamped to the table
     float cnt, eps;    // number of tokens so far including this one; norm clamp
     int R, H, on;
 };
+
+// The exponent of the value scaling from the parameter: the sigmoid in fp32 (fp64 of an fp64 parameter), rounded to the
+// parameter's type and then to fp32, as a sigmoid of the tensor followed by a conversion leaves it.
+__device__ __forceinline__ float sigmoid_as(const void *norm, int type, int h) {
+    if (type == 1) {
+        const double x = static_cast<const double *>(norm)[h];
+        return (float)(1.0 / (1.0 + exp(-x)));
+    }
+    const u16 bits = type == 0 ? (u16)0 : static_cast<const u16 *>(norm)[h];
+    const float x = type == 0 ? static_cast<const float *>(norm)[h] : type == 2 ? Fp16::to_float(bits) : Bf16::to_float(bits);
+    const float s = 1.f / (1.f + expf(-x));
+    return type == 0 ? s : type == 2 ? Fp16::to_float(Fp16::from_float(s)) : Bf16::to_float(Bf16::from_float(s));
+}
 
 // 1 << strip_log2 wavefronts per head, each with its own columns of the state (1 << row_log2 lanes to a row, at least 8):
 // few heads are a serial chain of row batches in too few wavefronts otherwise.  Every one of them reads all of q and k, so
@@ -305,8 +320,10 @@ __global__ __launch_bounds__(256) void decode_wave_kernel(SF *__restrict__ S, co
                         sk[i] = xk[t] * rk;
                     }
                 }
-                if (prep.sig != nullptr) {
-                    const SF p = prep.cnt > 0.f ? (SF)pow((SF)prep.cnt, (SF)prep.sig[bh % prep.H]) : (SF)0;
+                if (prep.sig != nullptr || prep.norm != nullptr) {
+                    const int h = bh % prep.H;
+                    const float sig = prep.norm != nullptr ? sigmoid_as(prep.norm, prep.norm_type, h) : prep.sig[h];
+                    const SF p = prep.cnt > 0.f ? (SF)pow((SF)prep.cnt, (SF)sig) : (SF)0;
                     if (p > (SF)1) vv = vv * ((SF)1 / p);
                 }
             } else {

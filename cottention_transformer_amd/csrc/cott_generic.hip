@@ -140,10 +140,12 @@ hipError_t launch_decode(int dtype, void *state, const void *q, const void *k, c
 }
 
 hipError_t launch_decode_prep(int dtype, void *state, const void *q, const void *k, const void *v, void *o, int BH, int H,
-                              int dk, int dv, const float *sig, float cnt, const float *rot, long long pos, int R,
-                              float eps, hipStream_t stream) {
+                              int dk, int dv, const float *sig, const void *norm, int norm_type, float cnt, const float *rot,
+                              long long pos, int R, float eps, hipStream_t stream) {
     DecodePrep p{};
     p.sig = sig;
+    p.norm = norm;
+    p.norm_type = norm_type;
     p.rot = rot;
     p.pos = pos;
     p.cnt = cnt;

@@ -127,8 +127,8 @@ hipError_t launch_decode(int dtype, void *state, const void *q, const void *k, c
 // normalisation of q and k, v / max(cnt^sig[h], 1) (sig null = none) happen inside the kernel.  dv / 4 in
 // {8,16,32,64} and dk <= 256, else hipErrorInvalidValue.
 hipError_t launch_decode_prep(int dtype, void *state, const void *q, const void *k, const void *v, void *o, int BH, int H,
-                              int dk, int dv, const float *sig, float cnt, const float *rot, long long pos, int R,
-                              float eps, hipStream_t stream);
+                              int dk, int dv, const float *sig, const void *norm, int norm_type, float cnt, const float *rot,
+                              long long pos, int R, float eps, hipStream_t stream);
 
 // y[i] = x w[i]^T for i < count <= 3: x (rows, in), w (out, in), y (rows, out), all 16-bit of one type, 16-byte aligned;
 // rows <= 16, in a multiple of 32, out of 16, 32 * in bytes and rows * in * 2 below 2^31.

@@ -100,23 +100,22 @@ class GPTCosAttention(nn.Module):
         if self.state is None:
             self.state = torch.zeros(b, h, d, value.shape[-1], device=query.device,
                                      dtype=torch.float64 if query.dtype == torch.float64 else torch.float32)
-        sig, table = self._decode_side_inputs(query.device)
-        out = ops.decode_step_prepared(self.state, query, key, value, sig=sig, cnt=float(self.cur_s),
+        norm_const, table = self._decode_side_inputs(query.device)
+        out = ops.decode_step_prepared(self.state, query, key, value, norm_const=norm_const, cnt=float(self.cur_s),
                                        rotary=(table, self.cur_s - 1))
         self.cur_s += 1
         return out.reshape(b, 1, h * value.shape[-1])
 
     def _decode_side_inputs(self, device):
-        """sigmoid(norm_const) per head (recomputed when the parameter was written to) and the rotary table on `device`."""
-        cached = getattr(self, "_sig_cache", None)
-        if cached is None or cached[0] != self.norm_const._version or cached[1].device != device:
-            cached = (self.norm_const._version,
-                      self.norm_const.detach().sigmoid().reshape(self.num_attention_heads).float().to(device))
-            self._sig_cache = cached
+        """norm_const as it is now (nothing derived from it is kept: the kernel forms its sigmoid) and the rotary table, both
+        on `device`."""
+        norm_const = self.norm_const
+        if norm_const.device != device or not norm_const.is_contiguous():
+            norm_const = norm_const.detach().to(device).contiguous()
         table = self.embed_positions
         if table.device != device:
             table = self.embed_positions = table.to(device)
-        return cached[1], table
+        return norm_const, table
 
     def _decode_block_weights(self, hidden_states):
         """The four projection weights when one new token can take ops.decode_block, else None.  It can when there is
@@ -239,8 +238,8 @@ class GPTCosAttention(nn.Module):
             b, dev = hidden_states.shape[0], hidden_states.device
             if self.state is None:
                 self.state = torch.zeros(b, self.num_attention_heads, self.head_dim, self.head_dim, device=dev)
-            sig, table = self._decode_side_inputs(dev)
-            out = ops.decode_block(hidden_states[:, 0], *weights, self.state, sig=sig, cnt=float(self.cur_s),
+            norm_const, table = self._decode_side_inputs(dev)
+            out = ops.decode_block(hidden_states[:, 0], *weights, self.state, norm_const=norm_const, cnt=float(self.cur_s),
                                    rotary=(table, self.cur_s - 1))
             self.cur_s += 1
             return (self.resid_dropout(out[:, None]), None)

@@ -545,11 +545,18 @@ def decode_step(state, q, k, v, out=None):
     return out if o is out else out.copy_(o)
 
 
-def decode_step_prepared(state, q, k, v, sig=None, cnt=0.0, rotary=None, out=None):
+def _check_norm_const(norm_const, sig, h, device):
+    if (sig is not None or norm_const.numel() != h or norm_const.dtype not in _DTYPES or norm_const.device != device
+            or not norm_const.is_contiguous()):
+        raise RuntimeError(f"norm_const must be a contiguous floating tensor of {h} elements on the inputs' device, in place of sig")
+
+
+def decode_step_prepared(state, q, k, v, sig=None, cnt=0.0, rotary=None, out=None, norm_const=None):
     """decode_step on the RAW projections of the new token: rotation (rotary = (table (P,R) fp32, position int)),
     L2 normalisation of q and k and v / max(cnt^sig[h], 1) run inside the kernel (one launch instead of
     prepare_inputs + decode_step).  q, k: (B,H,Dk) or the (B,1,H,Dk) projection output; v likewise; sig: (H) or
-    None; cnt: number of tokens so far including this one."""
+    None; cnt: number of tokens so far including this one.  norm_const, in place of sig: the H elements of the
+    parameter, whose sigmoid the kernel forms."""
     if q.dim() == 4 and q.shape[1] == 1:
         q, k, v = q[:, 0], k[:, 0], v[:, 0]
     _require_gpu(state=state, q=q, k=k, v=v)
@@ -575,6 +582,8 @@ def decode_step_prepared(state, q, k, v, sig=None, cnt=0.0, rotary=None, out=Non
         if sig.shape != (h,):
             raise RuntimeError(f"sig must have shape {(h,)}")
         sig = sig.detach().to(device=q.device, dtype=torch.float32).contiguous()
+    if norm_const is not None:
+        _check_norm_const(norm_const, sig, h, q.device)
     table, pos, rdim, rows = None, 0, 0, 0
     if rotary is not None:
         table, pos = rotary
@@ -584,10 +593,12 @@ def decode_step_prepared(state, q, k, v, sig=None, cnt=0.0, rotary=None, out=Non
         pos = int(pos)
     L = _loader.lib()
     with _on(q.device):
-        rc = L.cott_decode_step_prep(state.data_ptr(), q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(),
-                                     sig.data_ptr() if sig is not None else None, float(cnt),
-                                     table.data_ptr() if table is not None else None, pos, rdim, rows, b, h, dk, dv, code,
-                                     _stream(q.device))
+        rest = (float(cnt), _ptr(table), pos, rdim, rows, b, h, dk, dv, code, _stream(q.device))
+        ptrs = (state.data_ptr(), q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr())
+        if norm_const is not None:
+            rc = L.cott_decode_step_norm(*ptrs, norm_const.data_ptr(), _DTYPES[norm_const.dtype], *rest)
+        else:
+            rc = L.cott_decode_step_prep(*ptrs, _ptr(sig), *rest)
     _check(rc, "cott_decode_step_prep")
     return out if o is out else out.copy_(o)
 
@@ -595,11 +606,11 @@ def decode_step_prepared(state, q, k, v, sig=None, cnt=0.0, rotary=None, out=Non
 DECODE_BLOCK_ROWS = 16  # sequences up to which decode_block is built (kTokenRows, csrc/cott_launch.h)
 
 
-def decode_block(x, wq, wk, wv, wo, state, sig=None, cnt=0.0, rotary=None):
+def decode_block(x, wq, wk, wv, wo, state, sig=None, cnt=0.0, rotary=None, norm_const=None):
     """One new token of up to DECODE_BLOCK_ROWS sequences through a whole attention block without biases, three launches:
     q, k, v = x wq^T, x wk^T, x wv^T, then decode_step_prepared on them (state (B,H,D,D) fp32, updated in place), then
     the returned y = o wo^T.  x: (B,E) bf16 / fp16; weights (E,E), contiguous and 16-byte aligned, in x's type;
-    sig, cnt, rotary as in decode_step_prepared."""
+    sig, cnt, rotary, norm_const as in decode_step_prepared."""
     _require_gpu(x=x, wq=wq, wk=wk, wv=wv, wo=wo, state=state)
     dt = x.dtype
     code = _dtype_code(x)
@@ -614,6 +625,8 @@ def decode_block(x, wq, wk, wv, wo, state, sig=None, cnt=0.0, rotary=None):
             raise RuntimeError(f"decode_block: weights must be contiguous {(e, e)} tensors of type {dt}")
     if sig is not None and (sig.shape != (h,) or sig.dtype != torch.float32 or sig.device != x.device or not sig.is_contiguous()):
         raise RuntimeError(f"decode_block: sig must be a contiguous float32 tensor of shape {(h,)} on x's device")
+    if norm_const is not None:
+        _check_norm_const(norm_const, sig, h, x.device)
     table, pos, rdim, rows = None, 0, 0, 0
     if rotary is not None:
         table, pos = rotary
@@ -624,10 +637,13 @@ def decode_block(x, wq, wk, wv, wo, state, sig=None, cnt=0.0, rotary=None):
     scratch = torch.empty((4, b, e), dtype=x.dtype, device=x.device)
     y = torch.empty((b, e), dtype=x.dtype, device=x.device)
     with _on(x.device):
-        rc = _loader.lib().cott_decode_block(x.data_ptr(), wq.data_ptr(), wk.data_ptr(), wv.data_ptr(), wo.data_ptr(),
-                                             state.data_ptr(), y.data_ptr(), _ptr(sig), float(cnt), _ptr(table), int(pos),
-                                             rdim, rows, b, h, d, code, scratch.data_ptr(), scratch.numel() * 2,
-                                             _stream(x.device))
+        rest = (float(cnt), _ptr(table), int(pos), rdim, rows, b, h, d, code, scratch.data_ptr(), scratch.numel() * 2,
+                _stream(x.device))
+        ptrs = (x.data_ptr(), wq.data_ptr(), wk.data_ptr(), wv.data_ptr(), wo.data_ptr(), state.data_ptr(), y.data_ptr())
+        if norm_const is not None:
+            rc = _loader.lib().cott_decode_block_norm(*ptrs, norm_const.data_ptr(), _DTYPES[norm_const.dtype], *rest)
+        else:
+            rc = _loader.lib().cott_decode_block(*ptrs, _ptr(sig), *rest)
     _check(rc, "cott_decode_block")
     return y
 

@@ -230,6 +230,13 @@ COTT_API int cott_decode_step_prep(void *state, const void *q, const void *k, co
                           const float *sig, float cnt, const float *rot_table, long long position,
                           int rotary_dim, int table_rows,
                           int B, int H, int Dk, int Dv, int dtype, void *stream);
+/* ... with the parameter itself in place of sig: norm_const (H) of type norm_dtype, whose sigmoid the kernel forms (in
+ * fp32, fp64 for COTT_F64, rounded to norm_dtype and then to fp32): nothing to keep up to date between tokens.  NULL =
+ * no scaling. */
+COTT_API int cott_decode_step_norm(void *state, const void *q, const void *k, const void *v, void *o,
+                          const void *norm_const, int norm_dtype, float cnt, const float *rot_table, long long position,
+                          int rotary_dim, int table_rows,
+                          int B, int H, int Dk, int Dv, int dtype, void *stream);
 
 /* One new token through a whole attention block without biases (GPT_Trainer/GPTCosAttention.py:443-445, 229-272, 501):
  * q, k, v = x wq^T, x wk^T, x wv^T; cott_decode_step_prep on them; y = o wo^T.  Three launches.  x, y: (B, H * D), the
@@ -238,6 +245,11 @@ COTT_API int cott_decode_step_prep(void *state, const void *q, const void *k, co
 COTT_API size_t cott_decode_block_scratch_bytes(int B, int H, int D, int dtype);
 COTT_API int cott_decode_block(const void *x, const void *wq, const void *wk, const void *wv, const void *wo,
                       void *state, void *y, const float *sig, float cnt,
+                      const float *rot_table, long long position, int rotary_dim, int table_rows,
+                      int B, int H, int D, int dtype, void *scratch, size_t scratch_bytes, void *stream);
+/* ... with cott_decode_step_norm in its middle. */
+COTT_API int cott_decode_block_norm(const void *x, const void *wq, const void *wk, const void *wv, const void *wo,
+                      void *state, void *y, const void *norm_const, int norm_dtype, float cnt,
                       const float *rot_table, long long position, int rotary_dim, int table_rows,
                       int B, int H, int D, int dtype, void *scratch, size_t scratch_bytes, void *stream);
 

@@ -145,3 +145,43 @@ def test_prepared_output_in_the_memory_of_an_input(ct):
         got = ops.decode_step_prepared(s, *x, out=x[i])
         # the same sum in one wavefront's order or in strips: half a unit each
         assert got is x[i] and rel_l2(got, want.double().cpu().numpy()) <= 2.0 ** -8 and torch.equal(s, want_state)
+
+
+@pytest.mark.parametrize("dt", [torch.float32, torch.float64, HF, BF], ids=["fp32", "fp64", "fp16", "bf16"])
+def test_norm_const_in_place_of_its_sigmoid(ct, dt):
+    """The sigmoid formed in the kernel is torch's, bit for bit: same states and outputs from norm_const and from sig."""
+    from cottention_transformer_amd import ops
+    g = torch.Generator().manual_seed(5)
+    b, h, d = 3, 40, 64
+    norm = torch.linspace(-8, 8, h, device=DEV).to(dt).reshape(1, h, 1, 1)
+    sig = norm.sigmoid().reshape(h).float()
+    x = torch.float64 if dt is torch.float64 else BF
+    q, k, v = (torch.randn(b, h, d, generator=g).to(DEV, x) for _ in range(3))
+    s1 = torch.randn(b, h, d, d, generator=g).to(DEV, torch.float64 if x is torch.float64 else torch.float32)
+    s2 = s1.clone()
+    o1 = ops.decode_step_prepared(s1, q, k, v, sig=sig, cnt=37.0)
+    o2 = ops.decode_step_prepared(s2, q, k, v, norm_const=norm, cnt=37.0)
+    assert torch.equal(o1, o2) and torch.equal(s1, s2)
+    with pytest.raises(RuntimeError, match="norm_const"):
+        ops.decode_step_prepared(s2, q, k, v, norm_const=norm[:, :3], cnt=37.0)
+
+
+@pytest.mark.parametrize("grad", [False, True], ids=["one call", "separate calls"])
+def test_module_tokens_follow_norm_const(ct, grad):
+    """norm_const written through .data between two tokens counts from the next one on."""
+    from types import SimpleNamespace
+    from cottention_transformer_amd.modules import GPTCosAttention
+    cfg = SimpleNamespace(hidden_size=128, num_attention_heads=2, max_position_embeddings=64, rotary_dim=32, attn_pdrop=0.0,
+                          resid_pdrop=0.0, fast_inference=True)
+    torch.manual_seed(3)
+    m, fresh = GPTCosAttention(cfg).to(DEV, BF).eval(), GPTCosAttention(cfg).to(DEV, BF).eval()
+    fresh.load_state_dict(m.state_dict())
+    fresh.norm_const.data.fill_(-3.0)
+    tokens = torch.randn(3, 1, 1, 128, device=DEV).to(BF)
+    with torch.set_grad_enabled(grad):
+        for t in tokens[:2]:
+            m(t)
+        fresh.state, fresh.cur_s = m.state.clone(), m.cur_s
+        m.norm_const.data.fill_(-3.0)
+        got, want = m(tokens[2])[0], fresh(tokens[2])[0]
+    assert torch.equal(got, want) and torch.equal(m.state, fresh.state)

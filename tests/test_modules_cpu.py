@@ -156,3 +156,22 @@ def test_projections_call_layers_that_are_not_plain_linears():
         assert torch.allclose(got, lin(x), rtol=1e-12, atol=1e-12)
     a, b2 = project(x, plain, hooked)          # one odd layer sends the whole group through the modules
     assert torch.allclose(a, plain(x)) and torch.allclose(b2, hooked(x))
+
+
+def test_the_token_path_reads_norm_const_as_it_is():
+    """After a state dict assigned in its place, a write through .data, a new parameter and a conversion of the module."""
+    from cottention_transformer_amd.modules import GPTCosAttention
+    cfg = SimpleNamespace(hidden_size=64, num_attention_heads=2, max_position_embeddings=8, rotary_dim=16, attn_pdrop=0.0,
+                          resid_pdrop=0.0, fast_inference=True)
+    m, other = GPTCosAttention(cfg), GPTCosAttention(cfg)
+    seen = lambda: m._decode_side_inputs(torch.device("cpu"))[0]
+    assert seen().flatten().tolist() == [0.5, 0.5]
+    torch.nn.init.constant_(other.norm_const, -3.0)
+    m.load_state_dict(other.state_dict(), assign=True)
+    assert seen().flatten().tolist() == [-3.0, -3.0]
+    m.norm_const.data.fill_(2.0)
+    assert seen().flatten().tolist() == [2.0, 2.0]
+    m.norm_const = torch.nn.Parameter(torch.tensor([1.0, -1.0]).reshape(1, 2, 1, 1))
+    assert seen().flatten().tolist() == [1.0, -1.0]
+    m.to(torch.bfloat16)
+    assert seen().dtype is torch.bfloat16 and seen().flatten().tolist() == [1.0, -1.0]

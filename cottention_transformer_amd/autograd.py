@@ -293,8 +293,9 @@ def linear_hooks_installed():
 
 def _is_plain_linear(lin):
     """Whether calling the layer is nothing but x w^T + b with the parameters it holds: exactly torch.nn.Linear, no
-    forward (pre-)hooks and no parametrization.  Adapters, quantised linears and hooked layers must be CALLED."""
-    if type(lin) is not torch.nn.Linear:
+    forward (pre-)hooks, no `forward` of its own on the instance (as offloading and casting wrappers put there) and no
+    parametrization.  Adapters, quantised linears and hooked layers must be CALLED."""
+    if type(lin) is not torch.nn.Linear or "forward" in lin.__dict__:
         return False
     if lin._forward_hooks or lin._forward_pre_hooks or getattr(lin, "_forward_hooks_with_kwargs", None):
         return False

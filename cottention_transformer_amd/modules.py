@@ -136,7 +136,8 @@ class GPTCosAttention(nn.Module):
         modules = self._modules
         for name in ("q_proj", "k_proj", "v_proj", "out_proj"):
             lin = modules.get(name)
-            if type(lin) is not nn.Linear or lin._forward_hooks or lin._forward_pre_hooks or "parametrizations" in lin._modules:
+            if (type(lin) is not nn.Linear or lin._forward_hooks or lin._forward_pre_hooks or "parametrizations" in lin._modules
+                    or "forward" in lin.__dict__):
                 return None
             params = lin._parameters
             w = params.get("weight")

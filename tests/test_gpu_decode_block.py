@@ -185,3 +185,14 @@ def test_module_tokens_follow_norm_const(ct, grad):
         m.norm_const.data.fill_(-3.0)
         got, want = m(tokens[2])[0], fresh(tokens[2])[0]
     assert torch.equal(got, want) and torch.equal(m.state, fresh.state)
+
+
+def test_module_token_calls_a_projection_whose_forward_was_replaced(ct):
+    from types import SimpleNamespace
+    from cottention_transformer_amd.modules import GPTCosAttention
+    cfg = SimpleNamespace(hidden_size=128, num_attention_heads=2, max_position_embeddings=64, rotary_dim=32, attn_pdrop=0.0,
+                          resid_pdrop=0.0, fast_inference=True)
+    m = GPTCosAttention(cfg).to(DEV, BF).eval()
+    m.out_proj.forward = lambda x: torch.full_like(x, 3.0)
+    with torch.no_grad():
+        assert (m(torch.randn(1, 1, 128, device=DEV).to(BF))[0] == 3.0).all()

@@ -175,3 +175,14 @@ def test_the_token_path_reads_norm_const_as_it_is():
     assert seen().flatten().tolist() == [1.0, -1.0]
     m.to(torch.bfloat16)
     assert seen().dtype is torch.bfloat16 and seen().flatten().tolist() == [1.0, -1.0]
+
+
+def test_a_projection_whose_forward_was_replaced_is_called():
+    """Wrappers that offload or cast weights set `forward` on the instance; the layer then is not x w^T + b of what it holds."""
+    from cottention_transformer_amd.autograd import project
+    plain, wrapped = torch.nn.Linear(8, 8), torch.nn.Linear(8, 8)
+    inner = wrapped.forward
+    wrapped.forward = lambda x: inner(x) + 1.0
+    x = torch.randn(2, 8)
+    a, b = project(x, plain, wrapped)
+    assert torch.allclose(a, plain(x)) and torch.allclose(b, inner(x) + 1.0)

@@ -178,14 +178,15 @@ def causal_dot_product_as(q, k, v, dtype):
         ok = _f32in_cache.get(shape)
         if ok is None:
             ok = _remember(_f32in_cache, shape, bool(_loader.lib().cott_causal_fwd_f32in_supported(*shape)))
-        q, k, v = q.contiguous(), k.contiguous(), v.contiguous()
-        if ok and not (q.data_ptr() | k.data_ptr() | v.data_ptr()) & 15:
-            o = torch.empty((b, h, n, dv), dtype=dtype, device=q.device)
-            with _on(q.device):
-                rc = _loader.lib().cott_causal_fwd_f32in(q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(), b, h, n, dk,
-                                                         dv, _stream(q.device))
-            _check(rc, "cott_causal_fwd_f32in")
-            return o
+        if ok:
+            q, k, v = q.contiguous(), k.contiguous(), v.contiguous()
+            if not (q.data_ptr() | k.data_ptr() | v.data_ptr()) & 15:
+                o = torch.empty((b, h, n, dv), dtype=dtype, device=q.device)
+                with _on(q.device):
+                    rc = _loader.lib().cott_causal_fwd_f32in(q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(), b, h, n,
+                                                             dk, dv, _stream(q.device))
+                _check(rc, "cott_causal_fwd_f32in")
+                return o
     return causal_dot_product(q.to(dtype), k.to(dtype), v.to(dtype))
 
 
@@ -450,6 +451,7 @@ def causal_backward_from(q, k, v, grad_out):
         if ok is None:
             ok = _remember(_g16_cache, shape, bool(_loader.lib().cott_causal_bwd_g16_supported(*shape)))
         q, k, v, g = q.contiguous(), k.contiguous(), v.contiguous(), grad_out.contiguous()
+        grad_out = g
         if ok and not (q.data_ptr() | k.data_ptr() | v.data_ptr() | g.data_ptr()) & 15:
             dq, dk_, dv_ = torch.empty_like(q), torch.empty_like(k), torch.empty_like(v)
             with _on(q.device):

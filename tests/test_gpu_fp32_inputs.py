@@ -69,3 +69,16 @@ def test_backward_of_other_gradients_converts(ct):
             assert torch.equal(got, want)
     with pytest.raises(RuntimeError, match="prev_grad must have shape"):
         ops.causal_backward_from(q, k, v, do[:, :, :5].to(BF))
+
+
+def test_strided_inputs_of_other_shapes_are_converted_before_they_are_copied(ct):
+    """Transposed fp32 heads of a width the converting forward is not built for: the 16-bit copies and the output are all
+    that is allocated (three tensors converted with their strides, three made contiguous, one output)."""
+    from cottention_transformer_amd import ops
+    q, k, v = (torch.randn(4, 128, 75, 128, device=DEV).transpose(1, 2) for _ in range(3))
+    want = ct.causal_dot_product(*(t.bfloat16() for t in (q, k, v)))
+    torch.cuda.reset_peak_memory_stats()
+    held = torch.cuda.memory_allocated()
+    got = ops.causal_dot_product_as(q, k, v, torch.bfloat16)
+    assert torch.equal(got, want)
+    assert torch.cuda.max_memory_allocated() - held <= 7.5 * 2 * q.numel()

@@ -46,8 +46,27 @@ hipError_t launch_set(WideSet set, int BH, int N, int prof_id, hipStream_t strea
         for (WideOp &o : set.op) o.sin = nullptr;
     }
     ProfScope ps(prof_id, stream);
-    wide_scan_kernel<TR, DI, false><<<dim3(grid_for(BH, set.items, set.G, set.xcds)), block, 0, stream>>>(set, BH, N, nchunks);
-    return hipGetLastError();
+    // A launch holds fewer than 2^32 threads: more heads than that (whole sequences, then) take several launches.
+    const long most = ((1L << 32) - 1) / (block.x * (long)set.items) / set.G - set.xcds;
+    const int step = set.G > 1 || BH <= most ? BH : (int)most;
+    for (int bh = 0; bh < BH; bh += step) {
+        const int heads = BH - bh < step ? BH - bh : step;
+        WideSet part = set;
+        for (int i = 0; i < set.count; ++i) {
+            WideOp &o = part.op[i];
+            const size_t rows = (size_t)bh * N, state = (size_t)bh * o.di * o.dj;
+            o.A += rows * o.di;
+            o.B += rows * o.di;
+            o.C += rows * o.dj;
+            o.O += rows * o.dj;
+            if (o.sin != nullptr) o.sin += state;
+            if (o.sout != nullptr) o.sout += state;
+        }
+        wide_scan_kernel<TR, DI, false><<<dim3(grid_for(heads, set.items, set.G, set.xcds)), block, 0, stream>>>(part, heads, N, nchunks);
+        const hipError_t e = hipGetLastError();
+        if (e != hipSuccess) return e;
+    }
+    return hipSuccess;
 }
 
 template <class TR>

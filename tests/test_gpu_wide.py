@@ -152,3 +152,16 @@ def test_states_in_and_out_of_groups(ct, oracle):
     assert rel_l2(torch.cat((o1, o2), 2), oracle.causal(q, k, v)) <= BOUND[HF]
     # 4000 products summed in fp32, errors of either sign: sqrt(4000) * 2^-24 in the mean
     assert rel_l2(s2, (k.double().transpose(2, 3) @ v.double()).numpy()) <= 64 * 2.0 ** -24
+
+
+def test_more_heads_than_one_launch_holds(ct):
+    """2^19 heads of one position: twelve workgroups of 768 threads a head for the gradients, over 2^32 threads in all.  The
+    plain-FMA kernel took 3 * 2^19 * 8 * 256."""
+    h, d = 1 << 19, 256
+    q, k, v, do = (torch.randn(1, h, 1, d, device=DEV).to(BF) for _ in range(4))
+    dq, dk, dv = ct.causal_backward(q, k, v, do)
+    dot = lambda a, b: (a.float() * b.float()).sum(-1, keepdim=True)
+    for got, ref in ((dq, dot(do, v) * k.float()), (dk, dot(do, v) * q.float()), (dv, dot(q, k) * do.float())):
+        # half a unit of the output, and the fp32 sum of 256 products that cancel: 256 * 2^-24 of their absolute sum
+        assert float((got.float() - ref).norm() / ref.norm()) <= BOUND[BF]
+        assert float((got[0, -1].float() - ref[0, -1]).norm() / ref[0, -1].norm()) <= 2 * BOUND[BF]

@@ -110,7 +110,8 @@ bool generic_fits(int dtype, int di);
 // Causal ops on 16-bit tensors whose head dims lie outside the MFMA path's range (cott_wide.h): every op needs
 // wide_fits(); full tensors (ldc == dj), no layout flags.
 inline bool wide_fits(int di, int dj) { return di % 16 == 0 && dj % 16 == 0 && di >= 32 && di <= 256 && dj >= 16; }
-// The workspace (16-byte aligned) may be smaller than wide_workspace() or null: sequences are then walked whole.
+// The workspace (16-byte aligned) may be smaller than wide_workspace() or null: sequences are then walked whole, with the sums
+// in another order.
 size_t wide_workspace(const int *di, const int *dj, int n, long BH, int N, int cus, int xcds);
 hipError_t launch_wide(int dtype, const OpDesc *ops, int n, int BH, int N, int cus, int xcds, void *ws, size_t ws_bytes,
                        int prof_id, hipStream_t stream);

@@ -96,7 +96,9 @@ hipError_t launch_typed(const OpDesc *ops, int n, int BH, int N, int cus, int xc
         const int nchunks = wide_chunks(N);
         set.G = wide_groups(BH, set.items, nchunks, cus, xcds);
         const size_t need = wide_slot_bytes(BH, set.items, set.G, pad);
-        if (need > ws_bytes) set.G = 1;  // (a caller without the workspace gets the same results from whole sequences)
+        // These widths needed no workspace on the plain-FMA kernel, so calls without one stay accepted: sequences are then
+        // walked whole, the sums in another order (results equal to rounding, not bit for bit) and with few heads slower.
+        if (need > ws_bytes) set.G = 1;
         set.cpg = (nchunks + set.G - 1) / set.G;
         if (set.G > 1) {
             set.slots = reinterpret_cast<f32x4 *>(ws);

@@ -51,7 +51,9 @@ COTT_API const char *cott_last_error(void);
  * Replaces kernel_call<T> / forward_<T>, Cuda_Kernel/combined_kernel_general.cu:257-289,352-429
  * (Python: FastAttention2.kernel.<dtype>(Q,K,V,block_size,inplace,reversed), :444-454).
  * q,k: (B,H,N,Dk); v,o: (B,H,N,Dv).  The diagonal s'=s is included.  `reversed` is the flag of
- * :126-130.  Workspace: cott_causal_workspace_bytes() bytes of device memory (may be 0). */
+ * :126-130.  Workspace: cott_causal_workspace_bytes() bytes of device memory (may be 0).  Less than that is an error,
+ * except for 16-bit heads outside 32..128 columns: this call, cott_causal_fwd_state and cott_causal_bwd then walk the
+ * sequences whole, which adds the fp32 sums up in another order (results equal to rounding) and is slower for few heads. */
 COTT_API size_t cott_causal_workspace_bytes(int B, int H, int N, int Dk, int Dv, int dtype);
 COTT_API int cott_causal_fwd(const void *q, const void *k, const void *v, void *o,
                     int B, int H, int N, int Dk, int Dv, int dtype, int reversed,
@@ -74,14 +76,15 @@ COTT_API int cott_causal_fwd_may_alias_v(int B, int H, int N, int Dk, int Dv, in
  * cott_causal_fwd with the group-state slots (its workspace) kept in a device array built into the library
  * instead of caller memory.  It has no counterpart in the reference; it is for callers that cannot allocate
  * device memory around the call: code under HIP graph capture, tight serving loops, harnesses that forbid
- * hipMalloc.  Same arguments, results (bit for bit) and errors as cott_causal_fwd; a shape whose slots exceed
- * cott_noalloc_scratch_bytes() (48 MiB, enough for every plan this build makes on a part of up to 256 CUs)
- * returns COTT_ERR_WORKSPACE.
+ * hipMalloc.  Same arguments, results (bit for bit those with a full workspace) and errors as cott_causal_fwd; a shape
+ * whose slots exceed cott_noalloc_scratch_bytes() (48 MiB, enough for every plan this build makes on a part of up to
+ * 256 CUs) returns COTT_ERR_WORKSPACE.
  * The array's address is looked up once per device (hipGetSymbolAddress): by cott_noalloc_scratch_bytes() when a
  * device is current, else by the first call of the entry point on that device.  Call cott_noalloc_scratch_bytes()
  * before a stream capture starts, so that the lookup does not happen inside it.  No call allocates or frees.
  * All calls on one GPU share that GPU's array: calls that may overlap on one GPU (different streams or threads)
- * race on it and must be ordered by the caller.  Keep cott_profile_enable off (it creates HIP events). */
+ * race on it and must be ordered by the caller (heads of every width: a shape uses the array when
+ * cott_causal_workspace_bytes() is not 0 for it).  Keep cott_profile_enable off (it creates HIP events). */
 COTT_API size_t cott_noalloc_scratch_bytes(void);
 COTT_API int cott_causal_fwd_noalloc(const void *q, const void *k, const void *v, void *o,
                             int B, int H, int N, int Dk, int Dv, int dtype, int reversed, void *stream);

@@ -65,7 +65,7 @@ SIGNATURES = {
 }
 
 KERNEL_IDS = {"group_state": 0, "state_prefix": 1, "scan": 2, "apply": 3, "scan_grad": 4, "generic": 5, "decode": 6,
-              "prep": 7, "stream_probe": 8}
+              "prep": 7, "stream_probe": 8, "token_linear": 9, "wide_scan": 10, "wide_sums": 11}
 
 
 def profile_enable(on):

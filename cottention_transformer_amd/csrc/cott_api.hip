@@ -517,7 +517,7 @@ int run_ops(const char *fn, bool causal, const Op *ops, int n, long BH, int N, i
         }
         if (wide) {
             hipError_t e = cott::launch_wide(dtype, wide_ops, n, (int)BH, N, device_cus(), device_xcds(), ws,
-                                             ws != nullptr && aligned16(ws) ? ws_bytes : 0, n > 1 ? cott::K_SCAN_GRAD : cott::K_SCAN, stream);
+                                             ws != nullptr && aligned16(ws) ? ws_bytes : 0, stream);
             if (e != hipSuccess) return fail(COTT_ERR_HIP, "%s: HIP launch failed: %s", fn, hipGetErrorString(e));
         }
         return COTT_OK;
@@ -668,7 +668,8 @@ int cott_profile_read(int kernel_id, double *total_ms, long *launches) {
 const char *cott_kernel_name(int kernel_id) {
     static const char *names[cott::K_COUNT] = {"group_state_kernel", "state_prefix_kernel", "scan_kernel<causal>",
                                                "scan_kernel<apply>", "scan_kernel<causal> (dQ,dK,dV set)", "generic_scan_kernel",
-                                               "decode_kernel", "prep_kernel", "stream_probe_kernel"};
+                                               "decode_kernel", "prep_kernel", "stream_probe_kernel", "token_linear_kernel",
+                                               "wide_scan_kernel", "wide_scan_kernel (group sums)"};
     return (kernel_id >= 0 && kernel_id < cott::K_COUNT) ? names[kernel_id] : "";
 }
 

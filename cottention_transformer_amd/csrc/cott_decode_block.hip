@@ -70,6 +70,7 @@ hipError_t launch_token_linear(int dtype, const void *x, const void *const w[3],
     a.rows = rows;
     a.in = in;
     a.out = out;
+    ProfScope ps(K_TOKEN_LINEAR, stream);
     const dim3 grid((unsigned)(count * (out / 16))), block(64 * kTokenWaves);
     if (dtype == COTT_BF16)
         token_linear_kernel<Bf16><<<grid, block, 0, stream>>>(a);

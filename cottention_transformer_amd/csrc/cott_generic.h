@@ -210,10 +210,10 @@ __global__ __launch_bounds__(256) void decode_kernel(SF *__restrict__ S, const t
     }
 }
 
-// Decode step, one WAVEFRONT per (batch, head): no workgroup barrier anywhere, so the four heads of
-// a workgroup stream independently.  For dv/4 = nv in {8,16,32,64} columns of float4: lane l owns
-// column l % nv and every (64/nv)-th row starting at l / nv; q and k are staged in a per-wavefront
-// LDS slice while the first batch of state loads is in flight; the row groups are combined with
+// Decode step, one WAVEFRONT per (batch, head) or per column strip of a head: no workgroup barrier anywhere, so the
+// wavefronts of a workgroup stream independently.  Of the dv/4 = nv in {8,16,32,64} columns of float4 a strip has
+// lw = nv >> strip_log2; lane l owns the strip's column l % lw and every (64/lw)-th row starting at l / lw; q and k are
+// staged in a per-wavefront LDS slice while the first batch of state loads is in flight; the row groups are combined with
 // lane-xor shuffles.  Plain (cacheable) loads and stores: a state that fits the last-level cache is
 // then served from it on the next step.
 // Optional preparation of the raw projections of the ONE new token inside the decode step (on = 1): GPT-J

@@ -71,7 +71,8 @@ struct SetArgs {
 };
 
 // Kernel families, as reported by cott_profile_read().
-enum KernelId { K_GROUP_STATE = 0, K_STATE_PREFIX, K_SCAN, K_APPLY, K_SCAN_GRAD, K_GENERIC, K_DECODE, K_PREP, K_STREAM_PROBE, K_COUNT };
+enum KernelId { K_GROUP_STATE = 0, K_STATE_PREFIX, K_SCAN, K_APPLY, K_SCAN_GRAD, K_GENERIC, K_DECODE, K_PREP, K_STREAM_PROBE,
+                K_TOKEN_LINEAR, K_WIDE_SCAN, K_WIDE_SUMS, K_COUNT };
 
 // While profiling is enabled (cott_profile_enable), brackets the launches made in its lifetime
 // with a pair of HIP events on the launch stream; otherwise does nothing.
@@ -114,7 +115,7 @@ inline bool wide_fits(int di, int dj) { return di % 16 == 0 && dj % 16 == 0 && d
 // in another order.
 size_t wide_workspace(const int *di, const int *dj, int n, long BH, int N, int cus, int xcds);
 hipError_t launch_wide(int dtype, const OpDesc *ops, int n, int BH, int N, int cus, int xcds, void *ws, size_t ws_bytes,
-                       int prof_id, hipStream_t stream);
+                       hipStream_t stream);
 
 // Fused input preparation (backward = false) or its backward; see cott_prep.hip.
 hipError_t launch_prep(bool backward, const void *const x[3], const void *const g[3], void *const y[3],

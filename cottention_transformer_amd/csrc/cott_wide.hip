@@ -33,19 +33,19 @@ size_t wide_slot_bytes(long BH, int items, int G, int pad) {
 }
 
 template <class TR, int DI>
-hipError_t launch_set(WideSet set, int BH, int N, int prof_id, hipStream_t stream) {
+hipError_t launch_set(WideSet set, int BH, int N, hipStream_t stream) {
     const int nchunks = wide_chunks(N);
     const dim3 block(64 * (kWideCompute + kWideLoad));
     set.first_slot = 1;
     if (set.G > 1) {
         for (const WideOp &o : set.op)
             if (o.sin != nullptr) set.first_slot = 0;
-        ProfScope ps(K_GROUP_STATE, stream);
+        ProfScope ps(K_WIDE_SUMS, stream);
         wide_scan_kernel<TR, DI, true><<<dim3(grid_for(BH, set.items, set.G - set.first_slot, set.xcds)), block, 0, stream>>>(
             set, BH, N, nchunks);
         for (WideOp &o : set.op) o.sin = nullptr;
     }
-    ProfScope ps(prof_id, stream);
+    ProfScope ps(K_WIDE_SCAN, stream);
     // A launch holds fewer than 2^32 threads: more heads than that (whole sequences, then) take several launches.
     const long most = ((1L << 32) - 1) / (block.x * (long)set.items) / set.G - set.xcds;
     const int step = set.G > 1 || BH <= most ? BH : (int)most;
@@ -70,7 +70,7 @@ hipError_t launch_set(WideSet set, int BH, int N, int prof_id, hipStream_t strea
 }
 
 template <class TR>
-hipError_t launch_typed(const OpDesc *ops, int n, int BH, int N, int cus, int xcds, char *ws, size_t ws_bytes, int prof_id,
+hipError_t launch_typed(const OpDesc *ops, int n, int BH, int N, int cus, int xcds, char *ws, size_t ws_bytes,
                         hipStream_t stream) {
     // one launch per padded width of the contracted dim (the gradients of square heads are one)
     for (int pad = 128; pad <= 256; pad += 64) {
@@ -105,9 +105,9 @@ hipError_t launch_typed(const OpDesc *ops, int n, int BH, int N, int cus, int xc
             ws += need;
             ws_bytes -= need;
         }
-        const hipError_t e = pad == 128   ? launch_set<TR, 128>(set, BH, N, prof_id, stream)
-                             : pad == 192 ? launch_set<TR, 192>(set, BH, N, prof_id, stream)
-                                          : launch_set<TR, 256>(set, BH, N, prof_id, stream);
+        const hipError_t e = pad == 128   ? launch_set<TR, 128>(set, BH, N, stream)
+                             : pad == 192 ? launch_set<TR, 192>(set, BH, N, stream)
+                                          : launch_set<TR, 256>(set, BH, N, stream);
         if (e != hipSuccess) return e;
     }
     return hipSuccess;
@@ -127,10 +127,10 @@ size_t wide_workspace(const int *di, const int *dj, int n, long BH, int N, int c
 }
 
 hipError_t launch_wide(int dtype, const OpDesc *ops, int n, int BH, int N, int cus, int xcds, void *ws, size_t ws_bytes,
-                       int prof_id, hipStream_t stream) {
+                       hipStream_t stream) {
     char *w = static_cast<char *>(ws);
-    if (dtype == COTT_BF16) return launch_typed<Bf16>(ops, n, BH, N, cus, xcds, w, ws_bytes, prof_id, stream);
-    if (dtype == COTT_F16) return launch_typed<Fp16>(ops, n, BH, N, cus, xcds, w, ws_bytes, prof_id, stream);
+    if (dtype == COTT_BF16) return launch_typed<Bf16>(ops, n, BH, N, cus, xcds, w, ws_bytes, stream);
+    if (dtype == COTT_F16) return launch_typed<Fp16>(ops, n, BH, N, cus, xcds, w, ws_bytes, stream);
     return hipErrorInvalidValue;
 }
 

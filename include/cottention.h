@@ -353,7 +353,8 @@ COTT_API int cott_causal_fwd_prep_save(const void *q, const void *k, const void 
  * cott_profile_read() waits for the recorded launches of one kernel family, returns their summed
  * duration and count, and forgets them.  Kernel ids: 0 group_state, 1 state_prefix, 2 causal scan
  * (forward launch), 3 non-causal apply, 4 causal scan (the launch that computes dQ, dK and dV together),
- * 5 generic scan, 6 decode, 7 input preparation, 8 the streaming probe below.  Stands where the reference wraps
+ * 5 generic scan, 6 decode, 7 input preparation, 8 the streaming probe below, 9 the projections of cott_decode_block,
+ * 10 causal scan of wide 16-bit heads and 11 its sums over sequence groups.  Stands where the reference wraps
  * its kernel call in torch.autograd.profiler (Cuda_Kernel/Custom_Kernel.py:165-179). */
 COTT_API int cott_profile_enable(int on);
 COTT_API int cott_profile_read(int kernel_id, double *total_ms, long *launches);

@@ -196,3 +196,21 @@ def test_module_token_calls_a_projection_whose_forward_was_replaced(ct):
     m.out_proj.forward = lambda x: torch.full_like(x, 3.0)
     with torch.no_grad():
         assert (m(torch.randn(1, 1, 128, device=DEV).to(BF))[0] == 3.0).all()
+
+
+def test_every_launch_of_a_token_and_of_wide_heads_is_counted(ct):
+    from cottention_transformer_amd import _loader, ops
+    x, w, s = torch.randn(1, 64, device=DEV).to(BF), torch.randn(64, 64, device=DEV).to(BF), torch.zeros(1, 1, 64, 64, device=DEV)
+    wide = torch.randn(1, 2, 1000, 256, device=DEV).to(BF)
+    _loader.profile_enable(True)
+    try:
+        for name in _loader.KERNEL_IDS:
+            _loader.profile_read(name)
+        ops.decode_block(x, w, w, w, w, s)
+        ct.causal_dot_product(wide, wide, wide)
+        counts = {name: _loader.profile_read(name)[1] for name in _loader.KERNEL_IDS}
+    finally:
+        _loader.profile_enable(False)
+    assert {k: n for k, n in counts.items() if n} == {"token_linear": 2, "decode": 1, "wide_sums": 1, "wide_scan": 1}
+    names = [_loader.lib().cott_kernel_name(i).decode() for i in _loader.KERNEL_IDS.values()]
+    assert all(names) and len(set(names)) == len(names)

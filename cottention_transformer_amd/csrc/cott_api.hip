@@ -185,6 +185,14 @@ bool pair_eligible(const Op *ops, int n, int dtype, bool causal) {
 //   non-causal, 16-bit D64: 2 heads N512 7.9 / 6.6 forward, 8.4 / 8.2 gradients, N768 8.4 / 8.7; 12 heads N768 9.2 / 8.9, 11.3 /
 //   10.7.  D128: 2 heads N256 9.4 / 7.4, 10.2 / 9.7; 12 heads N512 13.0 / 11.7, 17.6 / 16.0; 32 heads N768 18.1 / 16.6 forward.
 //   (the fp32 non-causal form goes through the workspace in any case)
+// The limits switch at 8 heads, in us at 7 / 8 / 9 / 11 heads, cut / one group: forward D64 N1023 12.3 / 11.4, 12.6 / 11.4,
+// 11.3 / 11.5, 11.7 / 11.5; D128 N512 14.5 / 12.5, 15.2 / 12.4, 15.5 / 12.5, 16.6 / 12.5 (2 heads 12.2 / 12.4); gradients D64
+// N768 14.3 / 12.2, 14.7 / 12.2, 14.5 / 12.3, 14.9 / 12.5 (2 heads 12.5 / 12.1); D128 19.7 / 18.1, 20.4 / 18.1, 21.1 / 18.3,
+// 22.0 / 18.3 (2 heads 16.2 / 17.9).
+// One problem of 128-wide rows and at most 64 value columns in one group has no column halves to share it (the preparation
+// is not built for those) and loses sooner: D128 x 64 forward 16 heads N512 13.7 / 12.5, N640 13.8 / 14.9, 24 heads N768
+// 16.1 / 17.2, 32 heads 17.2 / 17.2; non-causal 8 heads N384 9.7 / 9.5, N512 10.4 / 11.5, 16 heads 10.3 / 9.5, 10.5 / 11.6, 24 heads
+// N512 12.6 / 11.7, 32 heads N640 13.2 / 13.8, 48 heads 16.2 / 13.9.
 int one_group_chunks(long BH, int nops, int di, int dj, int dtype, bool causal) {
     const int pi = cott::mfma_pad(di), pj = cott::mfma_pad(dj);
     if (dtype == COTT_F32) {
@@ -193,6 +201,8 @@ int one_group_chunks(long BH, int nops, int di, int dj, int dtype, bool causal) 
         return pi <= 64 && pj <= 64 ? 2 : 0;
     }
     const bool wide = pi > 64 || pj > 64, forward = nops == 1;
+    if (forward && pi == 128 && dj < 128)
+        return causal ? (BH >= 32 ? 12 : BH >= 8 ? 8 : 4) : (BH >= 48 ? 10 : BH >= 24 ? 8 : BH >= 8 ? 6 : 4);
     if (!causal) return wide ? (forward && BH >= 32 ? 12 : BH >= 8 ? 8 : 4) : (BH >= 8 ? 12 : 8);
     if (wide) return forward ? (BH >= 16 ? 12 : BH >= 8 ? 8 : 4) : (BH >= 8 ? 12 : 8);
     return forward ? (BH >= 8 ? 16 : 12) : (BH >= 8 || pi + pj == 64 ? 12 : 8);
@@ -287,12 +297,14 @@ SetPlan plan_set(long BH, int N, int nops, int di, int dj, bool causal, int dtyp
     }
     // Short sequences of few heads: one group, however few workgroups that is.  Column halves where there is room for
     // them, but not of three causal gradient problems of tiles up to 64 x 64 (whole and separate, they are lighter than a
-    // pair workgroup, see use_pair) nor halves below 64 columns beside 128-wide rows (the input preparation inside the
-    // forward is not built for those).
+    // pair workgroup, see use_pair) nor, where the sequence would be cut otherwise, halves below 64 columns beside 128-wide
+    // rows (the input preparation inside the forward is not built for those).  More heads, whose sequences are whole anyway,
+    // keep such halves (100 heads 128 x 64, forward N512: 11.1 us, 13.7 without).
     if (pol < 0 && p.nchunks <= one_group_chunks(BH, nops, di, dj, dtype, causal)) {
+        const bool whole_anyway = best_g == 1 && BH > 64;
         best_g = 1;
         best_h = can_split && BH * nops * 2 <= tgt && !(causal && nops == 3 && small_tiles) &&
-                         !(cott::mfma_pad(di) == 128 && dj < 128)
+                         !(cott::mfma_pad(di) == 128 && dj < 128 && !whole_anyway)
                      ? 2
                      : 1;
     }

@@ -1,5 +1,6 @@
 """Host-side rules that choose a launch form, swept without a GPU: workspaces stay within what the entry points without a
 caller's workspace hold, and every call that was accepted has a plan."""
+import ctypes
 import itertools
 
 import pytest
@@ -48,3 +49,23 @@ def test_preparation_inside_the_forward_keeps_its_shapes(lib):
     for h, n, dv in itertools.product((1, 2, 8, 16, 32), (1, 64, 256, 500, 768), (64, 80, 128)):
         if n <= 256:
             assert L.cott_causal_fwd_prep_supported(1, h, n, 128, dv, BF16, 64) == 1
+
+
+def test_narrow_values_beside_wide_rows(lib):
+    """128-wide rows with 64 value columns: few heads run as one group of whole problems only as long as that is the faster
+    form, and more heads, whose sequences are whole anyway, keep their column halves."""
+    L, (cus, _) = lib
+    sets, nsets = (ctypes.c_int * 64)(), ctypes.c_int(0)
+
+    def plan(which, h, n):
+        assert L.cott_plan_describe(which, 0, 1, h, n, 128, 64, BF16, sets, ctypes.byref(nsets)) == _loader.OK
+        return sets[1], sets[2]  # column halves, groups
+
+    for which, h, chunks in ((0, 2, 4), (0, 8, 8), (0, 16, 8), (2, 2, 4), (2, 8, 6), (2, 16, 6)):
+        if h * 4 > cus:
+            continue
+        assert plan(which, h, 64 * chunks) == (1, 1)
+        if h * 8 <= cus:  # (room for groups)
+            assert plan(which, h, 64 * chunks + 1)[1] > 1
+    if cus > 200:
+        assert plan(0, cus // 2 - 10, 500) == (2, 1)

@@ -25,6 +25,7 @@ SIGNATURES = {
     "cott_causal_fwd_prep": (_i, [_vp] * 12 + [ctypes.c_longlong] + [_i] * 10 + [_vp, _sz, _vp]),
     "cott_causal_fwd_prep_save": (_i, [_vp] * 12 + [ctypes.c_longlong] + [_i] * 4 + [_vp] + [_i] * 8 + [_vp, _sz, _vp]),
     "cott_noncausal_fwd_prep_supported": (_i, [_i] * 6),
+    "cott_noncausal_fwd_prep_preferred": (_i, [_i] * 6),
     "cott_noncausal_fwd_prep": (_i, [_vp] * 10 + [_i] * 8 + [_vp]),
     "cott_causal_fwd_state": (_i, [_vp] * 6 + [_i] * 6 + [_vp, _sz, _vp]),
     "cott_prep_fwd": (_i, [_vp] * 9 + [_i] * 7 + [_vp]),

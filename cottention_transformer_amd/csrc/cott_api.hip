@@ -752,6 +752,29 @@ int cott_causal_fwd_prep_supported(int B, int H, int N, int Dk, int Dv, int dtyp
     return (pk <= 64 && pk * pv <= 128 * 64) || (pk == 128 && pv >= 64);
 }
 
+namespace {
+// Few heads whose short sequences run as one group (one_group_chunks; at most half of the CUs get a workgroup): chunks up to
+// which the preparation inside the forward is the better form.  The loader wavefronts of such a launch prepare their rows
+// alone, chunk after chunk, where the separate pass spreads them over the chip; against that stands one call less on the
+// host, which bounds steps of this size (a whole block, forward and backward, in eager mode: causal 597 against 624 us,
+// non-causal 513 against 537).  One launch is taken as long as the device needs no longer for it than for the two calls
+// whose forward is cut into sequence groups; us, one launch / two calls in one group / two calls, forward in groups:
+//   causal  32 columns: 8 heads N512 11.5 / 10.2 / 12.0, N640 13.2 / 11.1 / 12.6, 32 heads N640 13.7 / 12.6 / 14.3;  64 columns:
+//     8 heads N256 11.3 / 8.9 / 13.0, N384 14.3 / 10.1 / 13.6, 16 heads N384 14.5 / 10.7 / 15.0, N512 17.4 / 12.0 / 16.2,
+//     8 heads N1023 29.0 / 16.0 / 17.3;  128 columns: 8 heads N128 14.6 / 9.6 / 15.1, N256 20.5 / 12.1 / 16.5, N512 32.2 /
+//     17.1 / 19.9;  128 rows x 64: N64 11.0 / 8.3 / 7.8.
+//   non-causal  32 columns: 8 heads N384 8.9 / 8.0 / 10.2, N512 10.6 / 8.8 / 10.3, 16 heads N512 10.8 / 9.2 / 10.8;  64 columns: 4 heads
+//     N256 9.0 / 8.0 / 10.8, N384 11.2 / 9.2 / 11.3, 16 heads N384 11.4 / 9.9 / 12.6, N640 16.1 / 12.8 / 13.9;  128 columns: 4 heads
+//     N128 11.2 / 8.6 / 12.3, N256 15.8 / 10.8 / 12.8, 8 heads N512 24.8 / 15.9 / 15.7;  128 x 64: N64 8.2 / 7.2 / 7.1.
+int few_heads_prep_chunks(long BH, int Dk, int Dv, bool causal) {
+    const int pk = cott::mfma_pad(Dk);
+    if (pk == 32) return causal ? (BH >= 32 ? 10 : 8) : (BH >= 16 ? 8 : 6);
+    if (pk == 64) return BH >= 16 ? 6 : 4;
+    return Dv <= 64 ? 0 : (causal ? 1 : 2);
+}
+bool few_heads(const SetPlan &p, long BH) { return p.G == 1 && BH * p.halves * 2 <= target_workgroups(); }
+}  // namespace
+
 int cott_causal_fwd_prep_preferred(int B, int H, int N, int Dk, int Dv, int dtype, int rotary_dim) {
     if (!cott_causal_fwd_prep_supported(B, H, N, Dk, Dv, dtype, rotary_dim)) return 0;
     if ((long)B * H * N == 0) return 1;
@@ -765,6 +788,7 @@ int cott_causal_fwd_prep_preferred(int B, int H, int N, int Dk, int Dv, int dtyp
     // halves of a head prepare its q and k rows and so does the group-state pass (B2 H12 N8192 D64 92 against 65, D128
     // 183 against 149; B1 H16 N8192 D128 112 against 92).
     const SetPlan p = plan_set((long)B * H, N, 1, Dk, Dv, true, dtype);
+    if (few_heads(p, (long)B * H)) return p.nchunks <= few_heads_prep_chunks((long)B * H, Dk, Dv, true);
     return p.G == 1 || p.halves == 1;
 }
 
@@ -860,6 +884,13 @@ int cott_noncausal_fwd_prep_supported(int B, int H, int N, int Dk, int Dv, int d
     // one workgroup (or two column halves) per head (B16 H16 N512 D128: 56 us against 60 us for the two kernels;
     // B32 H12 N512 D64: 40 against 47 us)
     return plan_set((long)B * H, N, 1, Dk, Dv, false, dtype).G == 1;
+}
+
+int cott_noncausal_fwd_prep_preferred(int B, int H, int N, int Dk, int Dv, int dtype) {
+    if (!cott_noncausal_fwd_prep_supported(B, H, N, Dk, Dv, dtype)) return 0;
+    if ((long)B * H * N == 0) return 1;
+    const SetPlan p = plan_set((long)B * H, N, 1, Dk, Dv, false, dtype);
+    return !few_heads(p, (long)B * H) || p.nchunks <= few_heads_prep_chunks((long)B * H, Dk, Dv, false);
 }
 
 int cott_noncausal_fwd_prep(const void *q, const void *k, const void *v, void *o, void *q_out, void *k_out, void *v_out,

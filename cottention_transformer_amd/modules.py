@@ -337,7 +337,7 @@ class BertCosAttention(nn.Module):
             cnt = keep.sum(-1, keepdim=True).to(torch.float32).expand(b, s).contiguous()
         dt = _autocast_target(query_layer)
         d = self.attention_head_size
-        if (query_layer.dtype == dt and ops.noncausal_fused_preparation_supported(dt, b, h, s, d, d)
+        if (query_layer.dtype == dt and ops.noncausal_fused_preparation_preferred(dt, b, h, s, d, d)
                 and ops.merged_heads_supported(dt, s, h, d, d)):
             # one forward launch: normalisation, value scaling, mask and the attention op
             context_layer = PreparedNonCausalAttention.apply(query_layer, key_layer, value_layer, keep, cnt,

@@ -255,9 +255,9 @@ def fused_preparation_supported(dtype, b, h, n, dk, dv, rotary_dim=0):
 
 
 def fused_preparation_preferred(dtype, b, h, n, dk, dv, rotary_dim=0):
-    """Whether the one launch of causal_dot_product_prepared is also the faster form for the shape (all but those planned
-    as column halves in sequence groups: cott_causal_fwd_prep_preferred); the modules take prepare_inputs +
-    causal_dot_product elsewhere."""
+    """Whether the one launch of causal_dot_product_prepared is also the better form for the shape (all but those planned
+    as column halves in sequence groups, and few heads past a short length: cott_causal_fwd_prep_preferred); the modules
+    take prepare_inputs + causal_dot_product elsewhere."""
     if dtype not in (torch.bfloat16, torch.float16):
         return False
     key = ("preferred", dtype, b, h, n, dk, dv, rotary_dim)
@@ -329,7 +329,8 @@ def causal_dot_product_prepared(q, k, v, keep=None, cnt=None, sig=None, rotary=N
 
 def noncausal_fused_preparation_supported(dtype, b, h, n, dk, dv):
     """Whether noncausal_dot_product_prepared has a kernel for the shape: bf16 / fp16, head dims 32..128 in steps of
-    16, enough heads that a head is handled by one workgroup (cott_noncausal_fwd_prep_supported)."""
+    16, enough heads, or positions few enough, that a head is handled by one workgroup
+    (cott_noncausal_fwd_prep_supported)."""
     if dtype not in (torch.bfloat16, torch.float16):
         return False
     key = ("nc", dtype, b, h, n, dk, dv)
@@ -337,6 +338,19 @@ def noncausal_fused_preparation_supported(dtype, b, h, n, dk, dv):
     if ok is None:
         ok = _remember(_prep_supported_cache, key, bool(
             _loader.lib().cott_noncausal_fwd_prep_supported(b, h, n, dk, dv, _DTYPES[dtype])))
+    return ok
+
+
+def noncausal_fused_preparation_preferred(dtype, b, h, n, dk, dv):
+    """Whether noncausal_dot_product_prepared is also the better form for the shape (cott_noncausal_fwd_prep_preferred); the
+    modules take prepare_inputs + noncausal_dot_product elsewhere."""
+    if dtype not in (torch.bfloat16, torch.float16):
+        return False
+    key = ("nc preferred", dtype, b, h, n, dk, dv)
+    ok = _prep_supported_cache.get(key)
+    if ok is None:
+        ok = _remember(_prep_supported_cache, key, bool(
+            _loader.lib().cott_noncausal_fwd_prep_preferred(b, h, n, dk, dv, _DTYPES[dtype])))
     return ok
 
 

@@ -311,8 +311,9 @@ COTT_API int cott_prep_ex_bwd(const void *q, const void *k, const void *v,
  * same shape (cott_causal_workspace_bytes; sequences cut into groups, whose group sums are then formed from rows
  * prepared the same way; NULL / 0 when that is 0). */
 COTT_API int cott_causal_fwd_prep_supported(int B, int H, int N, int Dk, int Dv, int dtype, int rotary_dim);
-/* 1 where the one launch has also measured faster than cott_prep_ex_fwd followed by cott_causal_fwd (every shape but
- * those planned as column halves in sequence groups: few heads, medium sequence lengths), else 0: the rule the
+/* 1 where the one launch is also the better form against cott_prep_ex_fwd followed by cott_causal_fwd (every shape but
+ * those planned as column halves in sequence groups, i.e. few heads, medium sequence lengths, and few heads whose short
+ * sequences are one group but longer than the one launch gains on), else 0: the rule the
  * modules of this package follow when they choose between the two forms.  Pure host function. */
 COTT_API int cott_causal_fwd_prep_preferred(int B, int H, int N, int Dk, int Dv, int dtype, int rotary_dim);
 COTT_API int cott_causal_fwd_prep(const void *q, const void *k, const void *v, void *o,
@@ -327,9 +328,10 @@ COTT_API int cott_causal_fwd_prep(const void *q, const void *k, const void *v, v
  * cnt is the number of real tokens of the batch element at every position).  q_out, k_out, v_out receive the
  * prepared tensors for the backward pass (cott_noncausal_bwd on them, then cott_prep_ex_bwd).  bf16 / fp16, head
  * dims 32..128 in steps of 16, and a head must fit one workgroup (no sequence groups: B*H at least about the number
- * of CUs): cott_noncausal_fwd_prep_supported() says whether a shape qualifies; otherwise COTT_ERR_UNSUPPORTED.
- * Needs no workspace. */
+ * of CUs, or a short sequence): cott_noncausal_fwd_prep_supported() says whether a shape qualifies; otherwise
+ * COTT_ERR_UNSUPPORTED.  cott_noncausal_fwd_prep_preferred(): as for the causal form.  Needs no workspace. */
 COTT_API int cott_noncausal_fwd_prep_supported(int B, int H, int N, int Dk, int Dv, int dtype);
+COTT_API int cott_noncausal_fwd_prep_preferred(int B, int H, int N, int Dk, int Dv, int dtype);
 COTT_API int cott_noncausal_fwd_prep(const void *q, const void *k, const void *v, void *o,
                             void *q_out, void *k_out, void *v_out,
                             const unsigned char *keep, const float *cnt, const float *sig,

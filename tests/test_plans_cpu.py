@@ -69,3 +69,21 @@ def test_narrow_values_beside_wide_rows(lib):
             assert plan(which, h, 64 * chunks + 1)[1] > 1
     if cus > 200:
         assert plan(0, cus // 2 - 10, 500) == (2, 1)
+
+
+def test_where_the_preparation_inside_the_forward_is_preferred(lib):
+    """Few heads: up to the measured lengths; many heads: as before, whatever the length; never where it is not supported."""
+    L, (cus, _) = lib
+    for causal, d, h, chunks in ((1, 32, 8, 8), (1, 64, 8, 4), (1, 64, 16, 6), (1, 128, 8, 1), (0, 32, 8, 6), (0, 64, 8, 4), (0, 64, 16, 6),
+                                 (0, 128, 8, 2)):
+        if h * 4 > cus:
+            continue
+        ask = L.cott_causal_fwd_prep_preferred if causal else L.cott_noncausal_fwd_prep_preferred
+        for n in (1, 64 * chunks, 64 * chunks + 1):
+            assert ask(1, h, n, d, d, BF16, *((0,) if causal else ())) == (n <= 64 * chunks), (causal, d, h, n)
+    for h, n, d in itertools.product((1, 8, 100, 130, 512), (1, 64, 300, 512, 1023, 4096), (32, 64, 128)):
+        sup = L.cott_noncausal_fwd_prep_supported(1, h, n, d, d, BF16)
+        assert L.cott_noncausal_fwd_prep_preferred(1, h, n, d, d, BF16) <= sup
+        if h == 512:
+            assert L.cott_noncausal_fwd_prep_preferred(1, h, n, d, d, BF16) == sup
+            assert L.cott_causal_fwd_prep_preferred(1, h, n, d, d, BF16, 0) == 1

@@ -18,10 +18,10 @@
 // every product is that of the fp32 number and what is left is the order of the fp32 sums.  fp16: the state is scaled by
 // a power of two per column first, so that neither its largest nor its small entries leave the range, and the scores and
 // C take part as bf16 triples and pairs (C exactly).
-// What bounds it: the chain of chunks, 1.5 us each at DI = 256, and in it the vector instructions of the splits (with two
+// What bounds it: the chain of chunks, 1.48 us each at DI = 256, and in it the vector instructions of the splits (with two
 // terms, 16 significant bits, it took 1.27 us).  64-column slices rather than 128: twice as many workgroups share the chip,
 // and with few heads workgroups are what is short; the rest of the chip is filled by sequence groups (wide_groups).  B1 H16
-// N1024 D256: forward 30 us, gradients (192 workgroups, whole sequences) 57 us, where the plain-FMA kernel took 18.0 ms for
+// N1024 D256: forward 31 us, gradients (192 workgroups, whole sequences) 57 us, where the plain-FMA kernel took 18.0 ms for
 // both.  Share of the outputs that are not the 16-bit number nearest to the exact result, same shape: 1.5e-4 (bf16) and
 // 1.2e-3 (fp16), plain-FMA kernel 2.9e-4 and 3.2e-3, two terms 2.4e-3 and 5.5e-3.
 #pragma once
@@ -76,10 +76,18 @@ struct WideTiling {
                                   (SCORES + 2 * kWideCompute * 64) * sizeof(u32x4);
 };
 
-// Where 16-byte piece c of row r of an A or B tile lies within the row.  Read in the order of either access, 16 pieces
-// then fall on 16 different 16-byte bank groups: piece c of rows r .. r + 15 (operands along the contracted dim), and
-// pieces 4k .. 4k+3 of rows 4r' .. 4r'+3 (the transposing reads).
-__device__ __forceinline__ int wide_piece(int r, int c) { return c ^ (4 * (r & 3) + ((r >> 2) & 3)); }
+// Where 16-byte piece c of row r of an A or B tile lies within the row.  A 16-byte read of the wavefront is served 16 lanes
+// at a time, not in lane order: 0-3, 12-15 and 20-27 together, then 4-11, 16-19 and 28-31.  Along the contracted dim (lane
+// 16g + m reads piece 4ks + g of row m) those are rows 0-3 and 12-15 of one piece and rows 4-11 of its neighbour, or the
+// reverse; with rows 4i .. 4i+3 in different groups of four pieces and the rows' upper bits turned by {0, 2, 3, 1} they
+// fall on 16 different 16-byte bank groups.  The transposing reads (pieces 4k .. 4k+3 of rows 4i .. 4i+3, one half of each
+// piece) cannot do better than two lanes to a bank.  Conflict cycles of the gradients of 16 heads N1024 D256: 2.3 of 10.6
+// million LDS cycles, without the turn 5.0 of 13.3, with rows padded by 32 bytes instead 5.4 of 13.7 (2 heads N4096 in one
+// group, forward: 190, 197 and 198 us).
+__device__ __forceinline__ int wide_piece(int r, int c) {
+    const int up = (r >> 1) & 6;  // twice the upper bits of r, carried over into {0, 2, 3, 1}
+    return c ^ (4 * (r & 3) + (up & 4 ? up ^ 7 : up));
+}
 
 // Two fp32 numbers cut to 16-bit ones of type TR towards zero (so that no finite number becomes infinite).
 template <class TR>

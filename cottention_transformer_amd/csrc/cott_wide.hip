@@ -10,9 +10,9 @@ int wide_pad(int di) { return di <= 128 ? 128 : (di <= 192 ? 192 : 256); }
 
 // Groups a sequence is cut into: as many as keep the launch at one workgroup per CU (the (head, group) units are dealt round
 // the XCDs, and the fullest XCD has to hold its units' workgroups at once), of eight chunks at least, at most 16 (a group
-// reads the slots of all groups before it).  Sequences below 24 chunks stay whole (2 heads N512 D256, forward 29 us; two
-// launches of a few us each would have to save more).  Whole / groups, us: forward 16 heads D256 N768 41.9 / 27.1, N1024
-// 53.9 / 30.2, N4096 201 / 91; 2 heads N4096 196 / 39, N16384 786 / 85; gradients 2 heads N1024 55 / 30, N4096 203 / 52.  More
+// reads the slots of all groups before it).  Sequences below 24 chunks stay whole (2 heads N512 D256, forward 28 us; two
+// launches of a few us each would have to save more).  Whole / groups, us: forward 16 heads D256 N768 40.8 / 27.4, N1024
+// 53.1 / 30.6, N4096 194 / 95; 2 heads N4096 190 / 39, N16384 760 / 83; gradients 2 heads N1024 54 / 30, N4096 197 / 52.  More
 // groups than an XCD holds at once are slower (gradients of 2 heads N4096, with the two-term splits: 10 groups 67 us, 8
 // groups 47).
 int wide_groups(long BH, int items, int nchunks, int cus, int xcds) {

@@ -78,8 +78,9 @@ hipError_t run_decode(void *state, const void *q, const void *k, const void *v, 
         // and stores then stream it 10 % faster (1 GiB: 437 -> 393 us per step); a state that fits is served from
         // that cache and keeps the plain accesses.
         const bool stream_state = !prep.on && (size_t)BH * dk * dv * sizeof(SF) >= ((size_t)384 << 20);
-        auto kern = prep.on ? decode_wave_kernel<ST, SF, true> : stream_state ? decode_wave_kernel<ST, SF, false, 3>
-                                                                              : decode_wave_kernel<ST, SF, false>;
+        auto kern = prep.on        ? (prep.norm != nullptr ? decode_wave_kernel<ST, SF, 2> : decode_wave_kernel<ST, SF, 1>)
+                    : stream_state ? decode_wave_kernel<ST, SF, 0, 3>
+                                   : decode_wave_kernel<ST, SF, 0>;
         if (lds_w > 48 * 1024) {  // (fp64 with dk = 1024: 64 KiB)
             hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(kern),
                                                hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_w);

@@ -20,8 +20,9 @@ hipError_t run_causal_split(const SetArgs &a) {
         }
         const int bps = (TL::STATE_FLOATS / 4 + kThreads - 1) / kThreads;
         ProfScope prof(K_STATE_PREFIX, a.stream);
-        state_prefix_kernel<float><<<dim3((unsigned)(a.BH * ps.count * bps)), dim3(kThreads), 0, a.stream>>>(
-            ps, a.BH, a.G, a.sub, a.G - 1, TL::STATE_FLOATS, 0, TL::NJT);
+        const auto prefix = ps.has_start() ? state_prefix_kernel<float, true> : state_prefix_kernel<float, false>;
+        prefix<<<dim3((unsigned)(a.BH * ps.count * bps)), dim3(kThreads), 0, a.stream>>>(ps, a.BH, a.G, a.sub, a.G - 1, TL::STATE_FLOATS,
+                                                                                        0, TL::NJT, 0);
         ps.sin_in_slots();
     }
     ProfScope prof(a.scan_prof_id, a.stream);
@@ -46,8 +47,9 @@ hipError_t run_causal_f32(const SetArgs &a) {
         }
         const int bps = (TL::STATE_FLOATS / 4 + kThreads - 1) / kThreads;
         ProfScope prof(K_STATE_PREFIX, a.stream);
-        state_prefix_kernel<float><<<dim3((unsigned)(a.BH * a.count * bps)), dim3(kThreads), 0, a.stream>>>(
-            ps, a.BH, a.G, 1, a.G - 1, TL::STATE_FLOATS, 0, 0, TL::NIT);
+        const auto prefix = ps.has_start() ? state_prefix_kernel<float, true> : state_prefix_kernel<float, false>;
+        prefix<<<dim3((unsigned)(a.BH * a.count * bps)), dim3(kThreads), 0, a.stream>>>(ps, a.BH, a.G, 1, a.G - 1, TL::STATE_FLOATS, 0,
+                                                                                       0, TL::NIT);
         ps.sin_in_slots();
     }
     ProfScope prof(a.scan_prof_id, a.stream);
@@ -69,7 +71,7 @@ hipError_t run_noncausal_f32(const SetArgs &a) {
     if (a.G > 1) {
         const int bps = (TL::STATE_FLOATS / 4 + kThreads - 1) / kThreads;
         ProfScope prof(K_STATE_PREFIX, a.stream);
-        state_prefix_kernel<float><<<dim3((unsigned)(a.BH * a.count * bps)), dim3(kThreads), 0, a.stream>>>(
+        state_prefix_kernel<float, false><<<dim3((unsigned)(a.BH * a.count * bps)), dim3(kThreads), 0, a.stream>>>(
             ps, a.BH, a.G, 1, a.G, TL::STATE_FLOATS, 1, 0, TL::NIT);
     }
     ProfScope prof(K_APPLY, a.stream);

@@ -109,7 +109,9 @@ class GPTCosAttention(nn.Module):
     def _decode_side_inputs(self, device):
         """norm_const as it is now (nothing derived from it is kept: the kernel forms its sigmoid) and the rotary table, both
         on `device`."""
-        norm_const = self.norm_const
+        norm_const = self._parameters.get("norm_const")
+        if norm_const is None:  # (a parametrized one)
+            norm_const = self.norm_const
         if norm_const.device != device or not norm_const.is_contiguous():
             norm_const = norm_const.detach().to(device).contiguous()
         table = self.embed_positions

@@ -609,12 +609,11 @@ def decode_step_prepared(state, q, k, v, sig=None, cnt=0.0, rotary=None, out=Non
         pos = int(pos)
     L = _loader.lib()
     with _on(q.device):
-        rest = (float(cnt), _ptr(table), pos, rdim, rows, b, h, dk, dv, code, _stream(q.device))
-        ptrs = (state.data_ptr(), q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr())
+        fn, scaling = L.cott_decode_step_prep, (_ptr(sig),)
         if norm_const is not None:
-            rc = L.cott_decode_step_norm(*ptrs, norm_const.data_ptr(), _DTYPES[norm_const.dtype], *rest)
-        else:
-            rc = L.cott_decode_step_prep(*ptrs, _ptr(sig), *rest)
+            fn, scaling = L.cott_decode_step_norm, (norm_const.data_ptr(), _DTYPES[norm_const.dtype])
+        rc = fn(state.data_ptr(), q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(), *scaling, float(cnt), _ptr(table), pos,
+                rdim, rows, b, h, dk, dv, code, _stream(q.device))
     _check(rc, "cott_decode_step_prep")
     return out if o is out else out.copy_(o)
 
@@ -653,13 +652,12 @@ def decode_block(x, wq, wk, wv, wo, state, sig=None, cnt=0.0, rotary=None, norm_
     scratch = torch.empty((4, b, e), dtype=x.dtype, device=x.device)
     y = torch.empty((b, e), dtype=x.dtype, device=x.device)
     with _on(x.device):
-        rest = (float(cnt), _ptr(table), int(pos), rdim, rows, b, h, d, code, scratch.data_ptr(), scratch.numel() * 2,
-                _stream(x.device))
-        ptrs = (x.data_ptr(), wq.data_ptr(), wk.data_ptr(), wv.data_ptr(), wo.data_ptr(), state.data_ptr(), y.data_ptr())
+        fn, scaling = _loader.lib().cott_decode_block, (_ptr(sig),)
         if norm_const is not None:
-            rc = _loader.lib().cott_decode_block_norm(*ptrs, norm_const.data_ptr(), _DTYPES[norm_const.dtype], *rest)
-        else:
-            rc = _loader.lib().cott_decode_block(*ptrs, _ptr(sig), *rest)
+            fn, scaling = _loader.lib().cott_decode_block_norm, (norm_const.data_ptr(), _DTYPES[norm_const.dtype])
+        rc = fn(x.data_ptr(), wq.data_ptr(), wk.data_ptr(), wv.data_ptr(), wo.data_ptr(), state.data_ptr(), y.data_ptr(),
+                *scaling, float(cnt), _ptr(table), int(pos), rdim, rows, b, h, d, code, scratch.data_ptr(),
+                scratch.numel() * 2, _stream(x.device))
     _check(rc, "cott_decode_block")
     return y
 

@@ -319,9 +319,9 @@ __device__ __forceinline__ void wide_compute_role(const WideOp &op, int bh, int 
                 for (int q = 0; q < 4; ++q) mx = fmaxf(mx, __builtin_fabsf(S[it][q]));
             mx = fmaxf(mx, __shfl_xor(mx, 16));
             mx = fmaxf(mx, __shfl_xor(mx, 32));
-            // exponent kept to where both the scale and its inverse are normal numbers
+            // exponent kept to where both the scale and its inverse are normal numbers, and every finite entry in range
             int e = (int)(bitcast<uint32_t>(mx) >> 23) - 127;
-            e = e < -100 ? -100 : (e > 120 ? 120 : e);
+            e = e < -100 ? -100 : (e > 127 ? 127 : e);
             up = bitcast<float>((uint32_t)(127 + 14 - e) << 23);
 #pragma unroll
             for (int q = 0; q < 4; ++q) down[q] = bitcast<float>((uint32_t)(127 - 14 + __shfl(e, 4 * g + q)) << 23);

@@ -131,6 +131,22 @@ def test_an_infinite_value_within_its_chunk(ct, dt, x):
         assert torch.equal(ct.causal_dot_product(q, k, v, rev)[0, 0, rows, 5].float(), want[rows])
 
 
+@pytest.mark.parametrize("dt", [BF, HF], ids=["bf16", "fp16"])
+def test_the_largest_start_states(ct, dt):
+    """Start states of 2^126, of either sign and 2^125 apart: the sums are fp32's, and infinite in fp16 only as outputs."""
+    q, k, v, _ = (t.to(DEV) for t in inputs(1, 1, 40, 160, 160, dt, seed=2))
+    q[0, 0, :, :2] = torch.tensor([1.0, -1.0], device=DEV).to(dt)
+    q[0, 0, :, 2:] = 0
+    state = torch.zeros(1, 1, 160, 160, device=DEV)
+    state[0, 0, 0, :80], state[0, 0, 1, :80] = 2.0 ** 126, 2.0 ** 125
+    state[0, 0, 0, 80:], state[0, 0, 1, 80:] = -(2.0 ** 126), -(2.0 ** 126)
+    o, _ = ct.causal_prefill(q, k, v, state=state)
+    want = torch.tensor(2.0 ** 125, device=DEV).to(dt)  # (fp16: infinite)
+    assert (o[..., :80] == want).all()
+    # equal entries cancel: what is left of the first chunk is the sequence's own part
+    assert torch.equal(o[..., :32, 80:], ct.causal_prefill(q, k, v)[0][..., :32, 80:])
+
+
 def test_groups_need_no_workspace(ct):
     """Called without the workspace it asks for, the library walks the sequence whole."""
     from cottention_transformer_amd import _loader

@@ -180,8 +180,11 @@ bool pair_eligible(const Op *ops, int n, int dtype, bool causal) {
 //   N768 19.0 / 17.5.
 //   gradients, 16-bit D64: 2 heads N128 10.5 / 4.9; 12 heads N256 12.0 / 6.6, N512 14.5 / 9.5; D32 12 heads N768 10.6 / 8.5;
 //   D128: 2 heads N512 14.0 / 13.1, N768 16.2 / 18.1; 12 heads N768 23.9 / 18.5.
-//   fp32 D64: 2 heads N128 12.8 / 7.9 forward, N256 13.1 / 11.3, N512 13.5 / 18.3; gradients of 16 heads N512 19.7 / 19.0.
-//   fp32 D32 (fp32 matrix pipe): gradients N128 11.5 / 9.4, N256 11.9 / 16.8; D128: always cut (N128 30.9 / 35.5).
+//   fp32 D64 (two terms, cott_split.h): 2 heads N384 17.7 / 13.7 forward, 21.3 / 14.4 gradients, N512 17.8 / 17.2, 20.7 / 17.7; 16
+//   heads N512 17.5 / 17.6, 20.6 / 18.2, N640 18.3 / 21.2, 20.9 / 21.9; 40 heads N768 20.1 / 24.6, 29.3 / 26.0.
+//   fp32 D128 (three terms): 2 heads N128 24.5 / 17.8, 24.6 / 18.3, N256 24.2 / 29.3; 16 heads N256 25.9 / 29.9, 34.3 / 31.2, N512
+//   30.8 / 53.4; 40 heads D96 N256 32.1 / 30.1, 43.0 / 32.1, N384 33.0 / 41.8; D128 x 64 2 heads N128 18.6 / 13.3, N256 18.2 / 21.6.
+//   fp32 D32 (fp32 matrix pipe): gradients N128 11.5 / 9.4, N256 11.9 / 16.8; 32 x 128: always cut.
 //   non-causal, 16-bit D64: 2 heads N512 7.9 / 6.6 forward, 8.4 / 8.2 gradients, N768 8.4 / 8.7; 12 heads N768 9.2 / 8.9, 11.3 /
 //   10.7.  D128: 2 heads N256 9.4 / 7.4, 10.2 / 9.7; 12 heads N512 13.0 / 11.7, 17.6 / 16.0; 32 heads N768 18.1 / 16.6 forward.
 //   (the fp32 non-causal form goes through the workspace in any case)
@@ -197,7 +200,9 @@ int one_group_chunks(long BH, int nops, int di, int dj, int dtype, bool causal) 
     const int pi = cott::mfma_pad(di), pj = cott::mfma_pad(dj);
     if (dtype == COTT_F32) {
         if (!causal) return 0;
-        if (pi == 64 && pj == 64) return nops == 3 && BH >= 16 ? 8 : 4;
+        const int terms = cott::f32_terms(di, dj);
+        if (terms == 2) return nops == 3 && BH >= 32 ? 12 : 8;
+        if (terms == 3) return nops == 3 && BH >= 16 ? 4 : 2;
         return pi <= 64 && pj <= 64 ? 2 : 0;
     }
     const bool wide = pi > 64 || pj > 64, forward = nops == 1;
@@ -212,11 +217,12 @@ SetPlan plan_set(long BH, int N, int nops, int di, int dj, bool causal, int dtyp
                  bool has_ext = false) {
     SetPlan p;
     // the kernels on the fp32 matrix pipe are bound by it, with four wavefronts per workgroup: two workgroups per CU
-    // overlap well.  Causal fp32 ops of padded head dims 64 x 64 run from split operands on the bf16 matrix cores,
-    // one workgroup of eight wavefronts per CU like the 16-bit kernels.
-    const bool f32_split = dtype == COTT_F32 && causal && cott::mfma_pad(di) == 64 && cott::mfma_pad(dj) == 64 &&
-                           exp_int("COTT_F32_SPLIT", 1) != 0;
-    const long tgt = target_workgroups() * ((dtype == COTT_F32 && !f32_split) ? 2 : 1);
+    // overlap well.  Causal fp32 ops on split operands (padded head dims of 64 and 128) run as one workgroup of eight
+    // wavefronts per CU like the 16-bit kernels.  (Two of them fit a CU at 64 x 64 and share it when the heads alone make that
+    // many; cutting sequences to get there costs more than it gives: 128 heads N2048 forward 64 -> 73 us, 64 heads N1024
+    // gradients 35 -> 47.)
+    const bool f32_split = dtype == COTT_F32 && causal && cott::f32_terms(di, dj) > 0;
+    const long tgt = target_workgroups() * (dtype == COTT_F32 && !f32_split ? 2 : 1);
     const bool can_split = !no_split && dtype != COTT_F32 && dj >= 64 && dj % 32 == 0 && 2 * nops <= 6;
     const int pol = split_policy();
     const long xcds = device_xcds();
@@ -386,8 +392,7 @@ SetLayout layout_set(const Op *ops, int n, const int *members, int cnt, long BH,
     // workgroups on the fullest CU the pass takes about k * (1.15 if k == 2) / pieces of its one-piece time
     // (measured at B1 H16 N65536 D128: 144 workgroups 194 us, 288: 193, 432: 158, 576: 187; 240 -> 480: 84 -> 90).
     // (fp32 ops on split operands have a group-state pass of the same kind, one 80 KiB workgroup per CU)
-    const bool split32 = dtype == COTT_F32 && causal && cott::mfma_pad(first.di) == 64 && cott::mfma_pad(first.dj) == 64 &&
-                         exp_int("COTT_F32_SPLIT", 1) != 0;
+    const bool split32 = dtype == COTT_F32 && causal && cott::f32_terms(first.di, first.dj) > 0;
     if (p.G > 1 && (half || split32)) {
         long wgs = 0;
         if (L.pair)
@@ -1052,9 +1057,8 @@ int cott_causal_bwd(const void *q, const void *k, const void *v, const void *d_o
 
 int cott_causal_bwd_g16_supported(int B, int H, int N, int Dk, int Dv) {
     if (B < 0 || H < 0 || N < 0 || Dk < 1 || Dv < 1 || (long)B * H > (1L << 22)) return 0;
-    // all three gradients on split operands: padded head dims 64 x 64
-    return use_mfma(COTT_F32, Dk, Dv, N) && cott::mfma_pad(Dk) == 64 && cott::mfma_pad(Dv) == 64 &&
-           exp_int("COTT_F32_SPLIT", 1) != 0;
+    // all three gradients on split operands, with the same padded head dims
+    return use_mfma(COTT_F32, Dk, Dv, N) && cott::mfma_pad(Dk) == cott::mfma_pad(Dv) && cott::f32_terms(Dk, Dv) > 0;
 }
 
 int cott_causal_bwd_g16(const float *q, const float *k, const float *v, const void *d_o, float *dq, float *dk, float *dv, int B,
@@ -1063,7 +1067,7 @@ int cott_causal_bwd_g16(const float *q, const float *k, const float *v, const vo
     if (int rc = check_common(fn, B, H, N, Dk, Dv, COTT_F32)) return rc;
     if (int rc = check_common(fn, B, H, N, Dv, Dk, COTT_F32)) return rc;
     if (!cott_causal_bwd_g16_supported(B, H, N, Dk, Dv))
-        return fail(COTT_ERR_UNSUPPORTED, "%s: needs head dims of 48 or 64 (cott_causal_bwd_g16_supported); convert d_o and use "
+        return fail(COTT_ERR_UNSUPPORTED, "%s: needs head dims of 48 or 64, or both of 80 to 128 (cott_causal_bwd_g16_supported); convert d_o and use "
                     "cott_causal_bwd", fn);
     if ((long)B * H * N == 0) return COTT_OK;
     if (!q || !k || !v || !d_o || !dq || !dk || !dv) return fail(COTT_ERR_INVALID, "%s: null tensor pointer", fn);

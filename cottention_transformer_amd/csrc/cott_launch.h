@@ -20,7 +20,7 @@ struct OpDesc {
     // of a position next to each other, as the projections of a transformer block produce and consume them.
     unsigned char lay[4] = {0, 0, 0, 0};
     int H = 1;  // heads per batch element; needed when any layout flag is set
-    // fp32 ops on split operands only: bit 0 / 1 / 2 = A / B / C is a bf16 tensor (its lo parts are zero)
+    // fp32 ops on split operands only: bit 0 / 1 / 2 = A / B / C is a bf16 tensor (its lower terms are zero)
     int bf16_operands = 0;
     // Complement form (16-bit causal MFMA kernels, sets with sequence groups only): the op is walked against its
     // own direction so that it reads the same tiles at the same time as the other ops of its set.
@@ -91,8 +91,14 @@ class ProfScope {
 };
 
 // Padded state size of the MFMA path (head dims padded to 32, 64 or 128).
-inline int mfma_pad(int d) { return d <= 32 ? 32 : (d <= 64 ? 64 : 128); }
+constexpr int mfma_pad(int d) { return d <= 32 ? 32 : (d <= 64 ? 64 : 128); }
 inline size_t mfma_state_floats(int di, int dj) { return (size_t)mfma_pad(di) * mfma_pad(dj); }
+
+// bf16 terms that the operands of a causal fp32 op are split into for the bf16 matrix cores (0: it runs on the fp32 ones).
+constexpr int f32_terms(int di, int dj) {
+    const int pi = mfma_pad(di), pj = mfma_pad(dj);
+    return pi < 64 || pj < 64 ? 0 : (pi + pj == 128 ? 2 : 3);
+}
 
 // 16-bit storage; every op: 32 <= di,dj <= 128, multiples of 16, same padded dims across the set.
 hipError_t launch_causal_mfma_bf16(const SetArgs &a);

@@ -6,17 +6,17 @@
 namespace cott {
 namespace {
 
-// Padded head dims 64 x 64: the products run on the bf16 matrix cores from split operands (cott_split.h).
-template <int DI, int DJ>
+// Padded head dims of 64 and 128: the products run on the bf16 matrix cores from T terms per operand (cott_split.h).
+template <int DI, int DJ, int T>
 hipError_t run_causal_split(const SetArgs &a) {
     using TL = Tiling<DI, DJ>;
-    constexpr int PF = 2;
     ProblemSetF ps = make_set<float, DI, DJ>(a);
+    const int nsteps = (a.N + kSplitChunk - 1) / kSplitChunk, spg = a.cpg * (kChunk / kSplitChunk);
     if (a.G > 1) {
-        if (ps.nact > 0) {
+        {
             ProfScope prof(K_GROUP_STATE, a.stream);
-            group_state_split_kernel<DI, DJ, PF><<<dim3(grid_for(a.BH, ps.nact * a.sub, a.G - 1, a.xcds)), dim3(kThreads), 0, a.stream>>>(
-                ps, a.BH, a.N, a.nchunks, a.cpg, a.G, a.G - 1);
+            split_scan_kernel<DI, DJ, T, true><<<dim3(grid_for(a.BH, ps.nact * a.sub, a.G - 1, a.xcds)), dim3(512), 0, a.stream>>>(
+                ps, a.BH, a.N, nsteps, spg, a.G);
         }
         const int bps = (TL::STATE_FLOATS / 4 + kThreads - 1) / kThreads;
         ProfScope prof(K_STATE_PREFIX, a.stream);
@@ -26,17 +26,14 @@ hipError_t run_causal_split(const SetArgs &a) {
         ps.sin_in_slots();
     }
     ProfScope prof(a.scan_prof_id, a.stream);
-    split_scan_kernel<DI, DJ, PF><<<dim3(grid_for(a.BH, a.count, a.G, a.xcds)), dim3(512), 0, a.stream>>>(
-        ps, a.BH, a.N, a.nchunks, a.cpg, a.G);
+    split_scan_kernel<DI, DJ, T, false><<<dim3(grid_for(a.BH, a.count, a.G, a.xcds)), dim3(512), 0, a.stream>>>(ps, a.BH, a.N, nsteps,
+                                                                                                             spg, a.G);
     return hipGetLastError();
 }
 
 template <int DI, int DJ>
 hipError_t run_causal_f32(const SetArgs &a) {
-    if constexpr (DI == 64 && DJ == 64) {
-        static const int split = exp_env("COTT_F32_SPLIT", 1);
-        if (split) return run_causal_split<DI, DJ>(a);
-    }
+    if constexpr (f32_terms(DI, DJ) > 0) return run_causal_split<DI, DJ, f32_terms(DI, DJ)>(a);
     using TL = TilingF32<DI, DJ>;
     ProblemSetF32 ps = make_set<float, DI, DJ>(a);
     if (a.G > 1) {

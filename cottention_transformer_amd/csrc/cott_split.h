@@ -1,71 +1,90 @@
-// fp32 storage on the bf16 matrix cores: every fp32 operand is split into two bf16 numbers, x = hi + lo with
-// hi = bf16(x) and lo = bf16(x - hi), and every product of the chunk recurrence is formed from three bf16 matrix
-// instructions accumulating in fp32,
-//     a b  ~  a_hi b_hi + a_hi b_lo + a_lo b_hi .
-// hi + lo carries 16 of the 24 significant bits of x and the term left out, a_lo b_lo, is 2^-16 of the product: measured
-// rel-L2 of o, dQ, dK, dV against fp64 is 6.3e-6, inside the 1e-4 bar of fp32 inputs (the fp32 matrix pipe gives
-// 2e-7).  The price is three times the bf16 matrix work; the fp32 matrix pipe is sixteen times slower than the bf16
-// one on this part and the kernels on it (cott_mfma_f32.h) are bound by it: at B8 H16 N2048 D64 forward + backward
-// takes 430 us there and 243 us here (forward 73: group sums 26, prefix 6, scan 50; three gradients 146).
-//
-// Structure: that of colscan_kernel (cott_colscan.h) -- four compute wavefronts that each own a quarter of the
-// state's columns in fp32 accumulators and produce those columns of the output, the masked scores formed once per
-// workgroup and handed round through LDS, four loader wavefronts -- with these differences:
-//   * the loaders read fp32 rows and write TWO 16-bit tiles per operand (hi and lo);
-//   * the 16-bit operand copies of the state and of the masked scores are split the same way;
-//   * the outputs leave as fp32 straight from the accumulators (16 bytes per lane and tile);
-//   * one barrier per chunk: the (scores) x C product of a chunk is finished at the start of the next one, when every
-//     wavefront's score tiles have passed the barrier anyway (a barrier in the middle of the chunk also stops the
-//     loader wavefronts, whose conversion work is a fifth of the chunk here: gradients 164 -> 146 us).
-// Where the time goes (counters at the shape above, gradient launch, 384 workgroups on 256 CUs): per workgroup and chunk
-// 5300 cycles, of which the matrix pipe is busy 1344 on each SIMD, LDS 2030, vector-ALU issue about 2600 (the hi / lo
-// conversions of loaders and compute wavefronts: 284 instructions per wavefront), waves waiting on counters a third
-// of their time: one workgroup of eight wavefronts per CU (155 KiB of LDS) leaves no second wavefront to cover them.
-// The state slots of the group-state pass use the layout of the 16-bit kernels, so state_prefix_kernel serves both.
-// Padded head dims 64 x 64 (33 .. 64 columns); other widths stay on the fp32 matrix pipe.
+// fp32 storage on the bf16 matrix cores: every fp32 operand is split into T bf16 numbers and every product of the chunk
+// recurrence
+//     out_c = ((A_c B_c^T) o mask) C_c + A_c S_c ;   S_{c+1} = S_c + B_c^T C_c          (chunks of 32 positions)
+// is formed from the products of those terms, accumulating in fp32.
+//   T = 2 (padded head dims 64 x 64): x = hi + lo with 16 of the 24 significant bits, a b from three matrix instructions,
+//     rel-L2 of o, dQ, dK, dV against fp64 6.3e-6.
+//   T = 3 (128-wide heads): x = hi + mid + lo holds all 24 bits; the six products down to 2^-16 of a b (what is left out is
+//     2^-24 of it).  Rel-L2 against fp64 1.3e-7 .. 2.0e-7, where the fp32 matrix pipe, which these widths took before, gives
+//     2.4e-7 .. 5.1e-7 (N63 .. N8192, D 80 .. 128, both directions).  That pipe is sixteen times slower than the bf16 one.
+// Structure: that of colscan_kernel (cott_colscan.h).
+//   * Four compute wavefronts each own a quarter of the state's columns, all rows, in fp32 accumulators whose row order makes
+//     them the operand of A_c S_c once they are split; they produce those columns of the output.
+//   * Four loader wavefronts move fp32 rows global -> registers -> T tiles per operand in LDS, two chunks ahead, and form
+//     the three live 16 x 16 score tiles once per workgroup.
+//   * One barrier per chunk: the product of the scores with C_c is finished at the start of the next chunk.
+// Why 32 positions: T = 3 at 128 x 128 fills LDS (156 KiB with both buffers); at T = 2 it takes 68 KiB and two workgroups fit
+// a CU, a third of the score products falls away, and the state is packed twice as often.  The group sums run the same code
+// without A, scores and outputs (SUMS).
+// What bounds it: the vector instructions of the splits, which share the issue port with the matrix ones.  Per chunk and
+// SIMD at T = 3, 128 x 128: matrix pipe 3744 cycles, splits (11 instructions per pair of numbers) 750 instructions; 7400
+// cycles in all.  Splitting with the packed dot product (one instruction per difference instead of two) is slower: it waits
+// for the matrix pipe.
+// Measured (us, forward / gradients, back to back; before: T = 3 on the fp32 matrix pipe, T = 2 in chunks of 64 positions with
+// one workgroup per CU):
+//   1 x 16 x 2048 x 128    73 / 168 -> 50 / 98       8 x 16 x 1024 x 128   175 / 418 -> 105 / 248
+//   1 x 4 x 8192 x 128     80 / 171 -> 56 / 100      2 x 16 x 1024 x 128 / 64   42 / 102 -> 35 / 81
+//   1 x 16 x 63 x 128      20 / 20 -> 12 / 12        8 x 16 x 2048 x 64 (T = 2)   67 / 160 -> 64 / 133
+//   1 x 16 x 4096 x 64 (T = 2)   33 / 57 -> 31 / 49
+// The state slots of the group sums use the layout of the 16-bit kernels, so state_prefix_kernel serves both.
 #pragma once
 #include "cott_colscan.h"
+#include "cott_terms.h"
 
 namespace cott {
 
 typedef ProblemT<float> ProblemF;
 typedef ProblemSetT<float> ProblemSetF;
 
-// eight fp32 values (two 16-byte vectors) -> their bf16 hi parts and bf16 lo parts
-__device__ __forceinline__ void split8(u32x4 a, u32x4 b, u32x4 &hi, u32x4 &lo) {
-    const float x[8] = {bitcast<float>(a[0]), bitcast<float>(a[1]), bitcast<float>(a[2]), bitcast<float>(a[3]),
-                        bitcast<float>(b[0]), bitcast<float>(b[1]), bitcast<float>(b[2]), bitcast<float>(b[3])};
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-        const uint32_t h = Bf16::pack2(x[2 * e], x[2 * e + 1]);
-        hi[e] = h;
-        lo[e] = Bf16::pack2(x[2 * e] - bitcast<float>(h << 16), x[2 * e + 1] - bitcast<float>(h & 0xffff0000u));
+constexpr int kSplitChunk = 32;  // positions per chunk
+
+template <int T>
+struct SplitPairs;  // (a term, b term) of a product, smallest first; the last pair is hi hi
+template <>
+struct SplitPairs<2> {
+    static constexpr int N = 3, A[3] = {1, 0, 0}, B[3] = {0, 1, 0};
+};
+template <>
+struct SplitPairs<3> {
+    static constexpr int N = 6, A[6] = {2, 0, 1, 1, 0, 0}, B[6] = {0, 2, 1, 0, 1, 0};
+};
+
+// One term of a [32][D] operand tile in LDS.
+template <int D>
+struct SplitTile {
+    static constexpr int RS = D == 128 ? 128 : D + 16;
+    static constexpr int SIZE = kSplitChunk * RS;
+    __device__ static __forceinline__ int piece(int r, int c) {  // element offset of 16-byte piece c of row r
+        return r * RS + 8 * (D == 128 ? wide_piece(r, c) : c);
     }
+    // the same as an LDS address, from that of piece c < 4 to piece c + 4 ks (the turned pieces differ in two bits of the
+    // address, tiles start at multiples of 256 bytes there: one instruction each time instead of a register for every ks)
+    __device__ static __forceinline__ uint32_t step(uint32_t at, int ks) { return D == 128 ? at ^ (64u * ks) : at + 64u * ks; }
+};
+
+template <int DI, int DJ, int T, bool SUMS>
+struct SplitTiling {
+    static_assert(DI % 64 == 0 && DJ % 64 == 0, "four wavefronts of whole 16-column tiles");
+    static constexpr int KS = DI / 32, NIT = DI / 16, NJT = DJ / 16, NJW = NJT / 4;
+    static constexpr int AB = SplitTile<DI>::SIZE, C = SplitTile<DJ>::SIZE;
+    static constexpr int SCORES = 2 * T * 2 * 64;  // u32x4: [2 buffers][T terms][2 position blocks][64]: keys of both key blocks
+    static constexpr size_t LDS = ((SUMS ? 1 : 2) * AB + C) * 2 * T * sizeof(u16) + (SUMS ? 0 : SCORES * sizeof(u32x4));
+    static constexpr int STATE_FLOATS = DI * DJ;
+};
+
+// LDS addresses in bytes.
+typedef const __attribute__((address_space(3))) u16 *lds_ptr;
+__device__ __forceinline__ uint32_t lds_address(const u16 *p) { return (uint32_t)(uintptr_t)(lds_ptr)p; }
+__device__ __forceinline__ u32x4 lds_read16(uint32_t at) {
+    return *reinterpret_cast<const __attribute__((address_space(3))) u32x4 *>((lds_ptr)(uintptr_t)at);
 }
-// four accumulator values -> two dwords of hi parts, two of lo parts
-__device__ __forceinline__ void split4(f32x4 v, u32x2 &hi, u32x2 &lo) {
-#pragma unroll
-    for (int e = 0; e < 2; ++e) {
-        const uint32_t h = Bf16::pack2(v[2 * e], v[2 * e + 1]);
-        hi[e] = h;
-        lo[e] = Bf16::pack2(v[2 * e] - bitcast<float>(h << 16), v[2 * e + 1] - bitcast<float>(h & 0xffff0000u));
-    }
-}
-// Term t = 0, 1, 2 of a product: a_lo b_hi, a_hi b_lo, a_hi b_hi.  Callers with several independent accumulators run term
-// 0 for all of them, then term 1, then term 2, so that a matrix instruction never follows the one it depends on.
-__device__ __forceinline__ f32x4 mfma_term(int t, u32x4 ah, u32x4 al, u32x4 bh, u32x4 bl, f32x4 c) {
-    return Bf16::mfma(t == 0 ? al : ah, t == 1 ? bl : bh, c);
-}
-// c + a b from the three leading terms of (a_hi + a_lo)(b_hi + b_lo)
-__device__ __forceinline__ f32x4 mfma3(u32x4 ah, u32x4 al, u32x4 bh, u32x4 bl, f32x4 c) {
-    c = Bf16::mfma(al, bh, c);
-    c = Bf16::mfma(ah, bl, c);
-    return Bf16::mfma(ah, bh, c);
+__device__ __forceinline__ u32x2 lds_read_tr16(uint32_t at) {
+    s16x4 v = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4 *)(uintptr_t)at);
+    return bitcast<u32x2>(v);
 }
 
 // One operand of a problem: the rows of one head, fp32, or bf16 (an upstream gradient as the consumer of a bf16 output left
-// it: exact as a hi part, so the tiles are those of the converted tensor; B8 H16 N2048 D64,
-// training step 208 -> 183 us).
+// it: exact as a hi part, so the tiles are those of the converted tensor).
 struct SplitRows {
     rsrc_t rs;
     uint32_t esz;  // bytes per element
@@ -78,147 +97,177 @@ __device__ __forceinline__ SplitRows split_rows(const float *base, size_t head, 
     s.rs = make_rsrc_uniform(reinterpret_cast<const char *>(base) + head * s.esz, ((uint32_t)(N - 1) * ld + d) * s.esz);
     return s;
 }
-// [64][D] tile, global -> registers: thread t of NT owns pieces t, t + NT, ... (eight columns of a row: two 16-byte loads,
-// of bf16 rows one and one out of range, so that the number of loads in flight is the same)
-template <int D, int NT>
-__device__ __forceinline__ void load_tile_f(u32x4 (*r)[2], const SplitRows &src, int row0, int ld, int tid) {
+
+struct SplitRange {
+    int N, nsteps, p0, p1, reversed;  // chunks of 32 positions p0 .. p1-1 in walking order
+    __device__ __forceinline__ int first_row(int p) const { return (reversed ? nsteps - 1 - p : p) * kSplitChunk; }
+};
+
+typedef __attribute__((ext_vector_type(2))) unsigned short u16x2;
+// How two fp32 numbers are split into T packed pairs of bf16 terms (T = 2: rounded, 16 significant bits; T = 3: cut, all 24,
+// with the sign of the number in every term).
+// INFINITE (T = 3): the lower terms, where they are zero, become the smallest normal number of that sign, also those of an
+// infinite number: an infinite factor then meets no exact zero among the other factor's lower terms, and every partial product
+// of inf * x is the infinity that inf * x is (and not a number, from the hi parts, for x = 0).  To finite products that adds
+// 2^-126 of a factor.
+template <int T, bool INFINITE>
+__device__ __forceinline__ void split_pair(float a, float b, uint32_t *t) {
 #pragma unroll
-    for (int u = 0; u < 8 * D / NT; ++u) {
-        const int v = tid + NT * u;
-        const uint32_t off = (uint32_t)((row0 + v / (D / 8)) * ld + (v % (D / 8)) * 8) * src.esz;
-        r[u][0] = buf_load16(src.rs, off);
-        r[u][1] = buf_load16(src.rs, src.half ? kOobOffset : off + 16u);
+    for (int x = 0; x < T; ++x) {
+        if constexpr (T == 2)
+            t[x] = Bf16::pack2(a, b);
+        else
+            t[x] = __builtin_amdgcn_perm(bitcast<uint32_t>(b), bitcast<uint32_t>(a), 0x07060302u);
+        if (x + 1 < T) {
+            if constexpr (T == 2) {
+                a -= bitcast<float>(t[x] << 16);
+                b -= bitcast<float>(t[x] & 0xffff0000u);
+            } else {
+                a -= bitcast<float>(bitcast<uint32_t>(a) & 0xffff0000u);
+                b -= bitcast<float>(bitcast<uint32_t>(b) & 0xffff0000u);
+                if (INFINITE && x == 0) {  // (inf - inf: the median of two non-numbers and zero is zero)
+                    a = __builtin_amdgcn_fmed3f(a, a, 0.f);
+                    b = __builtin_amdgcn_fmed3f(b, b, 0.f);
+                }
+            }
+        }
+        if constexpr (T == 3 && INFINITE) {
+            if (x > 0) {
+                const uint32_t some = bitcast<uint32_t>(__builtin_elementwise_max(bitcast<u16x2>(t[x]), u16x2{0x0080, 0x0080}));
+                t[x] = (some & 0x7fff7fffu) | (t[0] & 0x80008000u);
+            }
+        }
     }
 }
-// registers -> the hi tile and the lo tile in LDS; columns past the runtime width d become zero
-template <int D, int STRIDE, int NT>
-__device__ __forceinline__ void store_tile_split(u16 *th, u16 *tl, const u32x4 (*r)[2], const SplitRows &src, int d, int tid) {
+// four accumulator values -> T pairs of dwords
+template <int T>
+__device__ __forceinline__ void split_acc(f32x4 v, u32x2 *t) {
+    uint32_t a[T], b[T];
+    split_pair<T, false>(v[0], v[1], a);
+    split_pair<T, false>(v[2], v[3], b);
 #pragma unroll
-    for (int u = 0; u < 8 * D / NT; ++u) {
-        const int v = tid + NT * u;
-        const int col = (v % (D / 8)) * 8;
-        u32x4 hi = {0u, 0u, 0u, 0u}, lo = hi;
-        if (col < d) {
-            if (src.half)
-                hi = r[u][0];
-            else
-                split8(r[u][0], r[u][1], hi, lo);
-        }
-        *reinterpret_cast<u32x4 *>(th + (v / (D / 8)) * STRIDE + col) = hi;
-        *reinterpret_cast<u32x4 *>(tl + (v / (D / 8)) * STRIDE + col) = lo;
-    }
+    for (int x = 0; x < T; ++x) t[x] = u32x2{a[x], b[x]};
 }
 
-// Sum of B^T C over each group of chunks of each head, in the slot layout of group_state_kernel (cott_mfma.h):
-// float4 index (w * TPW + u) * 64 + lane of slot (bh * G + grp) * sub + piece.
-template <int DI, int DJ, int PF>
-__global__ __launch_bounds__(kThreads) void group_state_split_kernel(ProblemSetF set, int BH, int N, int nchunks, int cpg,
-                                                                     int G, int ngroups) {
-    using TL = Tiling<DI, DJ>;
-    constexpr int SB = kChunk * TL::BS, SC = kChunk * TL::CS;
-    __shared__ __attribute__((aligned(16))) u16 sBh[2 * SB];
-    __shared__ __attribute__((aligned(16))) u16 sBl[2 * SB];
-    __shared__ __attribute__((aligned(16))) u16 sCh[2 * SC];
-    __shared__ __attribute__((aligned(16))) u16 sCl[2 * SC];
-    const int tid = threadIdx.x, l = tid & 63, g = l >> 4, m = l & 15;
-    const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
-    // every group is cut into `sub` pieces, one workgroup and one slot each (slot (bh * G + grp) * sub + piece)
-    const int sub = set.sub;
-    const WorkItem wi = decode_workgroup(set.nact * sub, BH, set.xcds);
-    if (wi.grp >= ngroups) return;
-    const ProblemF &pr = set.p[set.act[wi.prob / sub]];
-    const int piece = wi.prob % sub;
-    const int di = pr.di, dj = pr.dj, ldb = pr.ldb, ldc = pr.ldc, reversed = pr.reversed;
-    const SplitRows rB = split_rows(pr.B, head_base(pr.bsB, pr.hsB, pr.H, wi.bh), pr.bf16_operands & 2, N, ldb, di);
-    const SplitRows rC = split_rows(pr.C, head_base(pr.bsC, pr.hsC, pr.H, wi.bh), pr.bf16_operands & 4, N, ldc, dj);
-    const int cps = (cpg + sub - 1) / sub;  // chunks per piece
-    const int p0 = wi.grp * cpg + piece * cps;
-    const int p1 = min(p0 + cps, min((wi.grp + 1) * cpg, nchunks));
-    f32x4 S[TL::TPW];
-#pragma unroll
-    for (int u = 0; u < TL::TPW; ++u) S[u] = f32x4{0.f, 0.f, 0.f, 0.f};
-    f32x4 *slot = reinterpret_cast<f32x4 *>(pr.gstate + (((size_t)wi.bh * G + wi.grp) * sub + piece) * TL::STATE_FLOATS);
-    if (p1 <= p0) {  // a piece past the end of its group: its slot is zero
-#pragma unroll
-        for (int u = 0; u < TL::TPW; ++u) slot[(w * TL::TPW + u) * 64 + l] = S[u];
-        return;
-    }
-    u32x4 rb[PF][DI / 32][2], rc[PF][DJ / 32][2];
-    auto load_chunk = [&](int s, int p) __attribute__((always_inline)) {
-        const int pc = min(p, p1 - 1);
-        const int row0 = (reversed ? nchunks - 1 - pc : pc) * kChunk;
-        load_tile_f<DI, kThreads>(rb[s], rB, row0, ldb, tid);
-        load_tile_f<DJ, kThreads>(rc[s], rC, row0, ldc, tid);
-    };
-    auto stage = [&](int s, int buf) __attribute__((always_inline)) {
-        store_tile_split<DI, TL::BS, kThreads>(sBh + buf * SB, sBl + buf * SB, rb[s], rB, di, tid);
-        store_tile_split<DJ, TL::CS, kThreads>(sCh + buf * SC, sCl + buf * SC, rc[s], rC, dj, tid);
-    };
-    // S[i][j] += sum over the 64 positions of B[tok][i] C[tok][j] for the tiles this wavefront owns (see state_update)
-    auto update = [&](int buf) __attribute__((always_inline)) {
-        constexpr int ROWS = (TL::TPW + TL::NJT - 1) / TL::NJT;
-        constexpr int COLS = TL::TPW < TL::NJT ? TL::TPW : TL::NJT;
-        const u16 *bh = sBh + buf * SB, *bl = sBl + buf * SB, *ch = sCh + buf * SC, *cl = sCl + buf * SC;
-#pragma unroll
-        for (int kb = 0; kb < 2; ++kb) {
-            const int k0 = 32 * kb + 8 * g;
-            u32x4 ah[ROWS], al[ROWS], xh[COLS], xl[COLS];
-#pragma unroll
-            for (int r = 0; r < ROWS; ++r) {
-                const int it = (w * TL::TPW + r * TL::NJT) / TL::NJT;
-                ah[r] = cat(lds_col4(bh, TL::BS, k0, 16 * it, m), lds_col4(bh, TL::BS, k0 + 4, 16 * it, m));
-                al[r] = cat(lds_col4(bl, TL::BS, k0, 16 * it, m), lds_col4(bl, TL::BS, k0 + 4, 16 * it, m));
-            }
-#pragma unroll
-            for (int c = 0; c < COLS; ++c) {
-                const int jt = (w * TL::TPW + c) % TL::NJT;
-                xh[c] = cat(lds_col4(ch, TL::CS, k0, 16 * jt, m), lds_col4(ch, TL::CS, k0 + 4, 16 * jt, m));
-                xl[c] = cat(lds_col4(cl, TL::CS, k0, 16 * jt, m), lds_col4(cl, TL::CS, k0 + 4, 16 * jt, m));
-            }
-#pragma unroll
-            for (int u = 0; u < TL::TPW; ++u)
-                S[u] = mfma3(ah[u / TL::NJT], al[u / TL::NJT], xh[u % COLS], xl[u % COLS], S[u]);
-        }
-    };
-#pragma unroll
-    for (int s = 0; s < PF; ++s) load_chunk(s, p0 + s);
-    stage(0, 0);
-    load_chunk(0, p0 + PF);
-    __syncthreads();
-    run_rounds<PF>(p0, p1, [&](int s, int p) __attribute__((always_inline)) {
-        const int s1 = (s + 1) % PF;
-        const int buf = (p - p0) & 1;
-        stage(s1, buf ^ 1);
-        load_chunk(s1, p + 1 + PF);
-        update(buf);
-        chunk_barrier();
-    });
-#pragma unroll
-    for (int u = 0; u < TL::TPW; ++u) slot[(w * TL::TPW + u) * 64 + l] = S[u];
-}
-
-// Loader role: LT threads move the A, B and C tiles of fp32 rows global -> registers -> hi / lo tiles in LDS, PF
-// chunks ahead.  One barrier per chunk.
-template <int DI, int DJ, int PF, int LT>
+// Loader role: 256 threads move the tiles two chunks ahead and form the scores of the chunk the compute wavefronts are at.
+template <int DI, int DJ, int T, bool SUMS>
 __device__ __forceinline__ void split_loader_role(const SplitRows &rA, const SplitRows &rB, const SplitRows &rC, int di, int dj,
-                                                  int lda, int ldb, int ldc, const ScanRange &r, int tid, u16 *sA, u16 *sB,
-                                                  u16 *sC) {
-    using TL = Tiling<DI, DJ>;
-    using CT = ColTiling<DI, DJ>;
-    static_assert((8 * DI) % LT == 0 && (8 * DJ) % LT == 0, "tile pieces divide over the loader threads");
-    u32x4 ra[PF][8 * DI / LT][2], rb[PF][8 * DI / LT][2], rc[PF][8 * DJ / LT][2];
-    auto load_chunk = [&](int s, int p) __attribute__((always_inline)) {
-        const int pc = min(p, r.p1 - 1);
-        const int row0 = (r.reversed ? r.nchunks - 1 - pc : pc) * kChunk;
-        load_tile_f<DI, LT>(ra[s], rA, row0, lda, tid);
-        load_tile_f<DI, LT>(rb[s], rB, row0, ldb, tid);
-        load_tile_f<DJ, LT>(rc[s], rC, row0, ldc, tid);
+                                                 int lda, int ldb, int ldc, const SplitRange &r, int tid, u16 *sA, u16 *sB, u16 *sC,
+                                                 u32x2 *sP) {
+    using TL = SplitTiling<DI, DJ, T, SUMS>;
+    constexpr int PF = 2, PI = kSplitChunk * DI / 8 / 256, PJ = kSplitChunk * DJ / 8 / 256;
+    static_assert(PI >= 1 && PJ >= 1, "a piece per loader thread at least");
+    const int l = tid & 63, g = l >> 4, m = l & 15;
+    const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+    u32x4 ra[PF][SUMS ? 1 : PI][2], rb[PF][PI][2], rc[PF][PJ][2];
+    // Piece u of this thread in a tile of D columns: wavefront w holds rows 8w .. 8w+7 of every operand.
+    auto piece_row = [&](int u, int D) __attribute__((always_inline)) { return 8 * w + (64 * u + l) / (D / 8); };
+    auto piece_col = [&](int D) __attribute__((always_inline)) { return l % (D / 8); };
+    // Byte offsets of the pieces within their chunk; out of range, so that they load zeros, for columns past the runtime width.
+    uint32_t offA[PI], offB[PI], offC[PJ];
+#pragma unroll
+    for (int u = 0; u < PI; ++u) {
+        const int row = piece_row(u, DI), col = 8 * piece_col(DI);
+        offA[u] = col < di ? (uint32_t)(row * lda + col) * rA.esz : kOobOffset;
+        offB[u] = col < di ? (uint32_t)(row * ldb + col) * rB.esz : kOobOffset;
+    }
+#pragma unroll
+    for (int u = 0; u < PJ; ++u) {
+        const int row = piece_row(u, DJ), col = 8 * piece_col(DJ);
+        offC[u] = col < dj ? (uint32_t)(row * ldc + col) * rC.esz : kOobOffset;
+    }
+    auto load_piece = [&](u32x4 *x, const SplitRows &src, uint32_t off) __attribute__((always_inline)) {
+        x[0] = buf_load16(src.rs, off);
+        x[1] = buf_load16(src.rs, src.half ? kOobOffset : off + 16u);  // (bf16 rows: the same number of loads in flight)
     };
-    // LDS: [hi | lo] x [2 buffers] per operand
+    auto load_chunk = [&](int s, int p) __attribute__((always_inline)) {
+        const uint32_t row0 = (uint32_t)r.first_row(min(p, r.p1 - 1));
+        const uint32_t a0 = row0 * lda * rA.esz, b0 = row0 * ldb * rB.esz, c0 = row0 * ldc * rC.esz;
+#pragma unroll
+        for (int u = 0; u < PI; ++u) {
+            if constexpr (!SUMS) load_piece(ra[s][u], rA, offA[u] + a0);
+            load_piece(rb[s][u], rB, offB[u] + b0);
+        }
+#pragma unroll
+        for (int u = 0; u < PJ; ++u) load_piece(rc[s][u], rC, offC[u] + c0);
+    };
+    // one piece -> its T tiles; largest: the largest magnitude seen so far
+    auto stage_piece = [&](u16 *tile, int term_stride, const u32x4 *x, const SplitRows &src, int at, auto infinite, float &largest)
+                           __attribute__((always_inline)) {
+        u32x4 t[T];
+        if (T == 2 && src.half) {
+            t[0] = x[0];
+            t[1] = u32x4{0u, 0u, 0u, 0u};
+        } else {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                uint32_t q[T];
+                float a = bitcast<float>(x[e >> 1][2 * (e & 1)]), b = bitcast<float>(x[e >> 1][2 * (e & 1) + 1]);
+                if (T == 3 && src.half) {
+                    a = bitcast<float>(x[0][e] << 16);
+                    b = bitcast<float>(x[0][e] & 0xffff0000u);
+                }
+                split_pair<T, decltype(infinite)::value>(a, b, q);
+#pragma unroll
+                for (int y = 0; y < T; ++y) t[y][e] = q[y];
+                if constexpr (T == 3 && !decltype(infinite)::value)
+                    largest = __builtin_fmaxf(__builtin_fmaxf(largest, __builtin_fabsf(a)), __builtin_fabsf(b));
+            }
+        }
+#pragma unroll
+        for (int e = 0; e < T; ++e) *reinterpret_cast<u32x4 *>(tile + e * term_stride + at) = t[e];
+    };
+    auto stage_bc = [&](int s, int buf, auto infinite, float &largest) __attribute__((always_inline)) {
+#pragma unroll
+        for (int u = 0; u < PI; ++u)
+            stage_piece(sB + buf * TL::AB, 2 * TL::AB, rb[s][u], rB, SplitTile<DI>::piece(piece_row(u, DI), piece_col(DI)), infinite, largest);
+#pragma unroll
+        for (int u = 0; u < PJ; ++u)
+            stage_piece(sC + buf * TL::C, 2 * TL::C, rc[s][u], rC, SplitTile<DJ>::piece(piece_row(u, DJ), piece_col(DJ)), infinite, largest);
+    };
     auto stage = [&](int s, int buf) __attribute__((always_inline)) {
-        store_tile_split<DI, TL::BS, LT>(sA + buf * CT::SA, sA + (2 + buf) * CT::SA, ra[s], rA, di, tid);
-        store_tile_split<DI, TL::BS, LT>(sB + buf * CT::SA, sB + (2 + buf) * CT::SA, rb[s], rB, di, tid);
-        store_tile_split<DJ, TL::CS, LT>(sC + buf * CT::SC, sC + (2 + buf) * CT::SC, rc[s], rC, dj, tid);
+        float largest = 0.f;
+        if constexpr (!SUMS) {
+#pragma unroll
+            for (int u = 0; u < PI; ++u)
+                stage_piece(sA + buf * TL::AB, 2 * TL::AB, ra[s][u], rA, SplitTile<DI>::piece(piece_row(u, DI), piece_col(DI)),
+                            std::false_type{}, largest);
+        }
+        largest = 0.f;  // (infinite entries of A need nothing: they enter outputs only, see add_rest)
+        stage_bc(s, buf, std::false_type{}, largest);
+        if constexpr (T == 3) {
+            // a row with an infinite entry in B or C (this wavefront holds that row of both): once more
+            if (__any(largest == __builtin_inff())) stage_bc(s, buf, std::true_type{}, largest);
+        }
+    };
+    // Score tile of this wavefront (0..2): key block kt against position block pb, transposed (a lane holds four
+    // consecutive keys of one position).  Sum over the past: (0,0) (1,0) (1,1); over the future: (0,0) (0,1) (1,1).
+    const int pb = r.reversed ? (w == 2) : (w >= 1), kt = r.reversed ? (w >= 1) : (w == 2);
+    const int dir = pb != kt ? 0 : (r.reversed ? 1 : -1), side = dir * (4 * g - m);
+    auto scores = [&](int buf) __attribute__((always_inline)) {
+        if (w >= 3) return;
+        f32x4 hi = {0.f, 0.f, 0.f, 0.f}, rest[2] = {hi, hi};
+#pragma unroll
+        for (int ks = 0; ks < TL::KS; ++ks) {
+            u32x4 a[T], b[T];
+#pragma unroll
+            for (int x = 0; x < T; ++x) {
+                a[x] = ld128(sB + (2 * x + buf) * TL::AB + 16 * kt * SplitTile<DI>::RS + SplitTile<DI>::piece(m, 4 * ks + g));
+                b[x] = ld128(sA + (2 * x + buf) * TL::AB + 16 * pb * SplitTile<DI>::RS + SplitTile<DI>::piece(m, 4 * ks + g));
+            }
+#pragma unroll
+            for (int e = 0; e + 1 < SplitPairs<T>::N; ++e)
+                rest[e & 1] = Bf16::mfma(a[SplitPairs<T>::A[e]], b[SplitPairs<T>::B[e]], rest[e & 1]);
+            hi = Bf16::mfma(a[0], b[0], hi);
+        }
+        f32x4 acc = hi + (rest[0] + rest[1]);
+        if (T == 3 && __any(any_nan(acc))) acc = number_or(acc, hi);
+#pragma unroll
+        for (int q = 0; q < 4; ++q) acc[q] = side + dir * q >= 0 ? acc[q] : 0.f;
+        u32x2 t[T];
+        split_acc<T>(acc, t);
+#pragma unroll
+        for (int x = 0; x < T; ++x) sP[((buf * T + x) * 2 + pb) * 128 + 2 * l + kt] = t[x];
     };
 #pragma unroll
     for (int s = 0; s < PF; ++s) load_chunk(s, r.p0 + s);
@@ -226,61 +275,47 @@ __device__ __forceinline__ void split_loader_role(const SplitRows &rA, const Spl
     load_chunk(0, r.p0 + PF);
     __syncthreads();
     run_rounds<PF>(r.p0, r.p1, [&](int s, int p) __attribute__((always_inline)) {
-        const int s1 = (s + 1) % PF;
-        const int buf = (p - r.p0) & 1;
+        const int s1 = (s + 1) % PF, buf = s;  // (PF = 2: the LDS buffer is the register stage)
+        if constexpr (!SUMS) scores(buf);
         stage(s1, buf ^ 1);
         load_chunk(s1, p + 1 + PF);
         chunk_barrier();
     });
 }
 
-// Compute role: col_compute_role (cott_colscan.h) with split operands and fp32 outputs.  io: seed (group prefix),
-// sin / sout; the transposed seeds and the states saved for a backward pass exist for 16-bit storage only.
-template <int DI, int DJ, bool FUT>
-__device__ __forceinline__ void split_compute_role(const ColStateIO &io, float *O_head, int ldo, int di, int dj,
-                                                   const ScanRange &r, int w, int l, const u16 *sA, const u16 *sB,
-                                                   const u16 *sC, u32x2 *sP) {
-    using TL = Tiling<DI, DJ>;
-    using CT = ColTiling<DI, DJ>;
-    constexpr int KS = TL::KS, NIT = TL::NIT, NJW = CT::NJW;
-    static_assert(NIT == 2 * KS && NIT % 4 == 0, "two row tiles per contraction step, row tiles in batches of four");
+// the bf16 matrix instruction over 16 instead of 32 contraction steps, four of them per lane
+__device__ __forceinline__ f32x4 mfma_half(u32x2 a, u32x2 b, f32x4 c) {
+    return __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(bitcast<s16x4>(a), bitcast<s16x4>(b), c, 0, 0, 0);
+}
+
+// Compute role: wavefront w of 4 owns column tiles NJW * w .. of the state (all rows, interleaved as in colscan_kernel) and
+// of the output.
+template <int DI, int DJ, int T, bool SUMS, bool FUT>
+__device__ __forceinline__ void split_compute_role(const ColStateIO &io, float *O_head, int ldo, int di, int dj, const SplitRange &r,
+                                                  int w, int l, const u16 *sA, const u16 *sB, const u16 *sC, const u32x4 *sP) {
+    using TL = SplitTiling<DI, DJ, T, SUMS>;
+    using TP = SplitPairs<T>;
+    constexpr int KS = TL::KS, NIT = TL::NIT, NJW = TL::NJW;
     const int g = l >> 4, m = l & 15;
-    const bool mask_rev = r.mask_rev != 0;
-    auto live = [&](int pb, int jt) __attribute__((always_inline)) { return FUT ? jt >= pb : jt <= pb; };
-    const rsrc_t rO = make_rsrc(O_head, ((uint32_t)(r.N - 1) * ldo + dj) * 4u);
-    int spb[3], sjt[3];  // the three score tiles of this wavefront (see col_compute_role)
-    {
-        const int fut_pb[12] = {0, 0, 0, 0, 1, 1, 1, 2, 2, 3, 3, 3}, fut_jt[12] = {0, 1, 2, 3, 1, 2, 3, 2, 3, 3, 3, 3};
-        const int pst_pb[12] = {0, 1, 1, 2, 2, 2, 3, 3, 3, 3, 3, 3}, pst_jt[12] = {0, 0, 1, 0, 1, 2, 0, 1, 2, 3, 3, 3};
-#pragma unroll
-        for (int t = 0; t < 3; ++t) {
-            int pbv = 0, jtv = 0;
-#pragma unroll
-            for (int e = 0; e < 12; ++e)
-                if (e == 3 * w + t) {
-                    pbv = FUT ? fut_pb[e] : pst_pb[e];
-                    jtv = FUT ? fut_jt[e] : pst_jt[e];
-                }
-            spb[t] = __builtin_amdgcn_readfirstlane(pbv);
-            sjt[t] = __builtin_amdgcn_readfirstlane(jtv);
-        }
-    }
+    const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
+    const rsrc_t rO = make_rsrc_uniform(O_head, SUMS ? 0u : ((uint32_t)(r.N - 1) * ldo + dj) * 4u);
     f32x4 S[NIT][NJW];
 #pragma unroll
     for (int it = 0; it < NIT; ++it)
 #pragma unroll
-        for (int jw = 0; jw < NJW; ++jw) S[it][jw] = f32x4{0.f, 0.f, 0.f, 0.f};
-    if (io.seed != nullptr) {
+        for (int jw = 0; jw < NJW; ++jw) S[it][jw] = zero;
+    // slot of the standard tile layout that holds this lane's four rows of S[it][jw]
+    auto slot_at = [&](int it, int jw) __attribute__((always_inline)) {
+        return (size_t)((2 * (it >> 1) + (g >> 1)) * TL::NJT + NJW * w + jw) * 64 + 16 * (2 * (g & 1) + (it & 1)) + m;
+    };
+    if (!SUMS && io.seed != nullptr) {
         const f32x4 *gs = reinterpret_cast<const f32x4 *>(io.seed);
 #pragma unroll
         for (int it = 0; it < NIT; ++it)
 #pragma unroll
-            for (int jw = 0; jw < NJW; ++jw) {
-                const int ks = it >> 1, t = it & 1;
-                S[it][jw] = gs[(size_t)((2 * ks + (g >> 1)) * TL::NJT + NJW * w + jw) * 64 + 16 * (2 * (g & 1) + t) + m];
-            }
+            for (int jw = 0; jw < NJW; ++jw) S[it][jw] = gs[slot_at(it, jw)];
     }
-    if (io.sin != nullptr) {
+    if (!SUMS && io.sin != nullptr) {
 #pragma unroll
         for (int it = 0; it < NIT; ++it)
 #pragma unroll
@@ -291,208 +326,217 @@ __device__ __forceinline__ void split_compute_role(const ColStateIO &io, float *
                     if (i < di && j < dj) S[it][jw][q] += io.sin[(size_t)i * io.lds + j];
                 }
     }
-    u32x4 soph[KS][NJW], sopl[KS][NJW];
-    auto pack_state = [&]() __attribute__((always_inline)) {
+    // C fragments of the chunk: keys 4g .. 4g+3 and 16+4g .. of column 16 (NJW w + jw) + m, the order of the score operands;
+    // the state update contracts in the same order.
+    u32x4 cf[NJW][T];
+    f32x4 o[2][NJW];
+    uint32_t a_at = lds_address(sA + SplitTile<DI>::piece(m, g)), b_at[2], c_at[2];
 #pragma unroll
-        for (int ks = 0; ks < KS; ++ks)
+    for (int h = 0; h < 2; ++h) {
+        const int row = 16 * h + 4 * g + (m >> 2);
+        b_at[h] = lds_address(sB + SplitTile<DI>::piece(row, m & 3));
+        c_at[h] = lds_address(sC + SplitTile<DJ>::piece(row, 2 * NJW * w + ((m >> 1) & 1)) + 4 * (m & 1));
+    }
+    // C tiles: column tile jw, two pieces on, of this wavefront (with one tile there is none)
+    auto c_step = [&](uint32_t at, int jw) __attribute__((always_inline)) { return DJ == 128 ? at ^ (32u * jw) : at; };
+    // this lane's four output columns of the first column tile in the first row of a chunk; dj is a multiple of 16, so that a
+    // column tile lies inside the width or outside as a whole
+    const uint32_t o_at = (uint32_t)(m * ldo + 16 * NJW * w + 4 * g) * 4u;
+    // v = hi + rest; T = 3: where that is no number, hi, which has the value of the single-number arithmetic (a rest of inf -
+    // inf or inf * 0).  The empty asm keeps the repair behind its branch: as selects it would take 40 instructions a chunk.
+    auto add_rest = [&](f32x4 (&v)[2][NJW], const f32x4 (&hi)[2][NJW], const f32x4 (&rest)[2][NJW]) __attribute__((always_inline)) {
+        f32x4 sum = zero;
+#pragma unroll
+        for (int pb = 0; pb < 2; ++pb)
 #pragma unroll
             for (int jw = 0; jw < NJW; ++jw) {
-                u32x2 h0, l0, h1, l1;
-                split4(S[2 * ks][jw], h0, l0);
-                split4(S[2 * ks + 1][jw], h1, l1);
-                soph[ks][jw] = cat(h0, h1);
-                sopl[ks][jw] = cat(l0, l1);
+                v[pb][jw] = hi[pb][jw] + rest[pb][jw];
+                if constexpr (T == 3) sum += v[pb][jw];
             }
-    };
-    pack_state();
-    // The (scores) x C product of a chunk is finished at the start of the NEXT chunk, after the barrier that ends this
-    // one: by then every wavefront's score tiles are in LDS, and no second barrier in the middle of a chunk is needed
-    // (which would hold the loader wavefronts as well).  Carried across the barrier: the partial outputs o (A_c S_c),
-    // the C fragments, and the score tiles in the LDS buffer of the chunk's parity.
-    u32x2 *sPh = sP, *sPl = sP + 2 * 16 * 64;  // [2 buffers][16 tiles][64 lanes], hi then lo
-    f32x4 o[4][NJW];
-    u32x4 cfh[NJW][2], cfl[NJW][2], pfh[4][2], pfl[4][2];
-    int pbuf = 0;  // score buffer written in the current chunk
-    auto read_scores_of_previous = [&]() __attribute__((always_inline)) {
-        const int base = (pbuf ^ 1) * 16 * 64;
+        if constexpr (T == 3) {
+            if (__any(any_nan(sum))) {
+                asm volatile("" ::: "memory");
 #pragma unroll
-        for (int pb = 0; pb < 4; ++pb)
+                for (int pb = 0; pb < 2; ++pb)
 #pragma unroll
-            for (int kb = 0; kb < 2; ++kb) {
-                const u32x2 z = {0u, 0u};
-                if (live(pb, 2 * kb) || live(pb, 2 * kb + 1)) {
-                    const int t0 = base + (pb * 4 + 2 * kb) * 64 + l, t1 = t0 + 64;
-                    pfh[pb][kb] = cat(live(pb, 2 * kb) ? sPh[t0] : z, live(pb, 2 * kb + 1) ? sPh[t1] : z);
-                    pfl[pb][kb] = cat(live(pb, 2 * kb) ? sPl[t0] : z, live(pb, 2 * kb + 1) ? sPl[t1] : z);
-                }
+                    for (int jw = 0; jw < NJW; ++jw) v[pb][jw] = number_or(v[pb][jw], hi[pb][jw]);
             }
+        }
     };
-    auto finish_previous = [&](int pprev) __attribute__((always_inline)) {
-        const int row0 = (r.reversed ? r.nchunks - 1 - pprev : pprev) * kChunk;
-        f32x4 acc2[4][NJW];
+    auto finish = [&](int buf, int p) __attribute__((always_inline)) {
+        const int row0 = r.first_row(p);
+        u32x4 pf[2][T];
 #pragma unroll
-        for (int pb = 0; pb < 4; ++pb)
+        for (int x = 0; x < T; ++x)
 #pragma unroll
-            for (int jw = 0; jw < NJW; ++jw) acc2[pb][jw] = f32x4{0.f, 0.f, 0.f, 0.f};
+            for (int pb = 0; pb < 2; ++pb) pf[pb][x] = sP[((buf * T + x) * 2 + pb) * 64 + l];
+        f32x4 rest[2][NJW];
 #pragma unroll
-        for (int t = 0; t < 3; ++t)
+        for (int pb = 0; pb < 2; ++pb)
 #pragma unroll
-            for (int pb = 0; pb < 4; ++pb)
+            for (int jw = 0; jw < NJW; ++jw) rest[pb][jw] = zero;
+#pragma unroll
+        for (int e = 0; e < TP::N; ++e)
+#pragma unroll
+            for (int pb = 0; pb < 2; ++pb)
 #pragma unroll
                 for (int jw = 0; jw < NJW; ++jw) {
-                    if (live(pb, 0) || live(pb, 1))
-                        o[pb][jw] = mfma_term(t, cfh[jw][0], cfl[jw][0], pfh[pb][0], pfl[pb][0], o[pb][jw]);
-                    if (live(pb, 2) || live(pb, 3))
-                        acc2[pb][jw] = mfma_term(t, cfh[jw][1], cfl[jw][1], pfh[pb][1], pfl[pb][1], acc2[pb][jw]);
+                    f32x4 &acc = e + 1 < TP::N ? rest[pb][jw] : o[pb][jw];
+                    const u32x4 c = cf[jw][TP::A[e]], q = pf[pb][TP::B[e]];
+                    // one position block has a single live key block: the other's keys stay out (a masked zero times an
+                    // infinite entry of C would be no number)
+                    if (pb == (FUT ? 1 : 0))
+                        acc = mfma_half(FUT ? u32x2{c[2], c[3]} : u32x2{c[0], c[1]}, FUT ? u32x2{q[2], q[3]} : u32x2{q[0], q[1]}, acc);
+                    else
+                        acc = Bf16::mfma(c, q, acc);
                 }
+        f32x4 v[2][NJW];
+        add_rest(v, o, rest);
 #pragma unroll
-        for (int pb = 0; pb < 4; ++pb)
-#pragma unroll
-            for (int jw = 0; jw < NJW; ++jw) {
-                const f32x4 acc = o[pb][jw] + acc2[pb][jw];
-                const int col = 16 * (NJW * w + jw) + 4 * g;
-                const uint32_t off = (col < dj) ? (uint32_t)((row0 + 16 * pb + m) * ldo + col) * 4u : kOobOffset;
-                __builtin_amdgcn_raw_buffer_store_b128(bitcast<u32x4>(acc), rO, (int)off, 0, 0);
-            }
-    };
-    __syncthreads();
-    for (int p = r.p0; p < r.p1; ++p) {
-        const int buf = (p - r.p0) & 1;
-        pbuf = buf;
-        const u16 *cAh = sA + buf * CT::SA, *cAl = sA + (2 + buf) * CT::SA;
-        const u16 *cBh = sB + buf * CT::SA, *cBl = sB + (2 + buf) * CT::SA;
-        const u16 *cCh = sC + buf * CT::SC, *cCl = sC + (2 + buf) * CT::SC;
-        u32x4 sqh[2][KS], sql[2][KS], skh[2][KS], skl[2][KS];
-        auto read_score = [&](int slot, int t) __attribute__((always_inline)) {
-#pragma unroll
-            for (int ks = 0; ks < KS; ++ks) {
-                const int qa = (16 * spb[t] + m) * TL::BS + 32 * ks + 8 * g, ka = (16 * sjt[t] + m) * TL::BS + 32 * ks + 8 * g;
-                sqh[slot][ks] = ld128(cAh + qa);
-                sql[slot][ks] = ld128(cAl + qa);
-                skh[slot][ks] = ld128(cBh + ka);
-                skl[slot][ks] = ld128(cBl + ka);
-            }
-        };
-        auto score_tile = [&](int slot, int t) __attribute__((always_inline)) {
-            f32x4 acc[KS];
-#pragma unroll
-            for (int ks = 0; ks < KS; ++ks) acc[ks] = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-            for (int t = 0; t < 3; ++t)
-#pragma unroll
-                for (int ks = 0; ks < KS; ++ks)
-                    acc[ks] = mfma_term(t, skh[slot][ks], skl[slot][ks], sqh[slot][ks], sql[slot][ks], acc[ks]);
-#pragma unroll
-            for (int ks = 1; ks < KS; ++ks) acc[0] += acc[ks];
-            const int d0 = 16 * (sjt[t] - spb[t]) + 4 * g - m;  // key position - query position at element 0
-#pragma unroll
-            for (int q = 0; q < 4; ++q) {
-                const bool keep = mask_rev ? (d0 + q >= 0) : (d0 + q <= 0);
-                acc[0][q] = keep ? acc[0][q] : 0.f;
-            }
-            u32x2 hi, lo;
-            split4(acc[0], hi, lo);
-            sPh[pbuf * 16 * 64 + (spb[t] * 4 + sjt[t]) * 64 + l] = hi;
-            sPl[pbuf * 16 * 64 + (spb[t] * 4 + sjt[t]) * 64 + l] = lo;
-        };
-        u32x4 qfh[2][KS], qfl[2][KS];
-        auto read_q = [&](int slot, int pb) __attribute__((always_inline)) {
-#pragma unroll
-            for (int ks = 0; ks < KS; ++ks) {
-                qfh[slot][ks] = ld128(cAh + (16 * pb + m) * TL::BS + 32 * ks + 8 * g);
-                qfl[slot][ks] = ld128(cAl + (16 * pb + m) * TL::BS + 32 * ks + 8 * g);
-            }
-        };
-        auto state_product = [&](int slot, int pb) __attribute__((always_inline)) {
-#pragma unroll
-            for (int jw = 0; jw < NJW; ++jw) {
-                f32x4 acc[KS];
-#pragma unroll
-                for (int ks = 0; ks < KS; ++ks) acc[ks] = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-                for (int t = 0; t < 3; ++t)
-#pragma unroll
-                    for (int ks = 0; ks < KS; ++ks)
-                        acc[ks] = mfma_term(t, soph[ks][jw], sopl[ks][jw], qfh[slot][ks], qfl[slot][ks], acc[ks]);
-#pragma unroll
-                for (int ks = 1; ks < KS; ++ks) acc[0] += acc[ks];
-                o[pb][jw] = acc[0];
-            }
-        };
-        u32x4 bfh[2][4], bfl[2][4];
-        auto read_c = [&]() __attribute__((always_inline)) {
+        for (int pb = 0; pb < 2; ++pb)
 #pragma unroll
             for (int jw = 0; jw < NJW; ++jw)
+            {
+                const uint32_t tile = 16 * (NJW * w + jw) < dj ? (uint32_t)(row0 + 16 * pb) * ldo * 4u + 64u * jw : kOobOffset;
+                __builtin_amdgcn_raw_buffer_store_b128(bitcast<u32x4>(v[pb][jw]), rO, (int)(o_at + tile), 0, 0);
+            }
+    };
+    u32x4 s[NJW][T];  // terms of the state rows of the next contraction step
+    auto pack_state = [&](int ks, int jw) __attribute__((always_inline)) {
+        u32x2 lo[T], hi[T];
+        split_acc<T>(S[2 * ks][jw], lo);
+        split_acc<T>(S[2 * ks + 1][jw], hi);
 #pragma unroll
-                for (int kb = 0; kb < 2; ++kb) {
-                    const int a0 = (32 * kb + 4 * g + (m >> 2)) * TL::CS + 16 * (NJW * w + jw) + 4 * (m & 3), a1 = a0 + 16 * TL::CS;
-                    cfh[jw][kb] = cat(lds_read_tr16(cCh + a0), lds_read_tr16(cCh + a1));
-                    cfl[jw][kb] = cat(lds_read_tr16(cCl + a0), lds_read_tr16(cCl + a1));
+        for (int x = 0; x < T; ++x) s[jw][x] = cat(lo[x], hi[x]);
+    };
+    // keeps the terms of the next chunk's first rows where they are formed, under this chunk's last products
+    auto pin_state = [&](int jw) __attribute__((always_inline)) {
+#pragma unroll
+        for (int x = 0; x < T; ++x) asm volatile("" : "+v"(s[jw][x]));
+    };
+    auto chunk = [&](int buf) __attribute__((always_inline)) {
+        f32x4 ah[2][NJW], ar[2][NJW];
+#pragma unroll
+        for (int pb = 0; pb < 2; ++pb)
+#pragma unroll
+            for (int jw = 0; jw < NJW; ++jw) ah[pb][jw] = ar[pb][jw] = zero;
+        u32x4 a[2][T], b[2][T];
+        // (else the addresses of all steps would be kept in registers)
+        asm volatile("" : "+v"(a_at), "+v"(b_at[0]), "+v"(b_at[1]), "+v"(c_at[0]), "+v"(c_at[1]));
+        auto read_a = [&](int ks) __attribute__((always_inline)) {
+#pragma unroll
+            for (int pb = 0; pb < 2; ++pb)
+#pragma unroll
+                for (int x = 0; x < T; ++x) a[pb][x] = lds_read16(SplitTile<DI>::step(a_at, ks) + 2 * ((2 * x + buf) * TL::AB + 16 * pb * SplitTile<DI>::RS));
+        };
+        auto read_b = [&](int ks) __attribute__((always_inline)) {
+#pragma unroll
+            for (int t = 0; t < 2; ++t)
+#pragma unroll
+                for (int x = 0; x < T; ++x)
+                    b[t][x] = cat(lds_read_tr16(SplitTile<DI>::step(b_at[0], ks) + 2 * ((2 * x + buf) * TL::AB + 4 * t)),
+                                  lds_read_tr16(SplitTile<DI>::step(b_at[1], ks) + 2 * ((2 * x + buf) * TL::AB + 4 * t)));
+        };
+        auto state_product = [&](int jw) __attribute__((always_inline)) {
+#pragma unroll
+            for (int e = 0; e < TP::N; ++e)
+#pragma unroll
+                for (int pb = 0; pb < 2; ++pb) {
+                    if (e + 1 < TP::N)
+                        ar[pb][jw] = Bf16::mfma(s[jw][TP::A[e]], a[pb][TP::B[e]], ar[pb][jw]);
+                    else
+                        ah[pb][jw] = Bf16::mfma(s[jw][0], a[pb][0], ah[pb][jw]);
                 }
         };
-        auto read_b = [&](int slot, int kb, int it0) __attribute__((always_inline)) {
+        // S += B^T C of one contraction step.  T = 3: the product of the chunk by itself first, one addition (rounded to
+        // nearest) to the state then; accumulating the six partial products on the state itself loses a bit over long sums.
+        auto update = [&](int ks, int t) __attribute__((always_inline)) {
+            {
+                f32x4 d[NJW];
 #pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                const int it = it0 + e;
-                const int a0 = (32 * kb + 4 * g + (m >> 2)) * TL::BS + 32 * (it >> 1) + 8 * (m & 3) + 4 * (it & 1), a1 = a0 + 16 * TL::BS;
-                bfh[slot][e] = cat(lds_read_tr16(cBh + a0), lds_read_tr16(cBh + a1));
-                bfl[slot][e] = cat(lds_read_tr16(cBl + a0), lds_read_tr16(cBl + a1));
-            }
-        };
-        auto update = [&](int slot, int kb, int it0) __attribute__((always_inline)) {
-#pragma unroll
-            for (int t = 0; t < 3; ++t)
-#pragma unroll
-                for (int e = 0; e < 4; ++e)
+                for (int e = 0; e < TP::N; ++e)
 #pragma unroll
                     for (int jw = 0; jw < NJW; ++jw)
-                        S[it0 + e][jw] = mfma_term(t, bfh[slot][e], bfl[slot][e], cfh[jw][kb], cfl[jw][kb], S[it0 + e][jw]);
-        };
-
-        read_score(0, 0);
-        if (p > r.p0) read_scores_of_previous();
-        sched_fence();
-        read_score(1, 1);
-        sched_fence();
-        if (p > r.p0) finish_previous(p - 1);  // (scores) x C of the chunk before, whose score tiles every wavefront has by now
-        sched_fence();
-        score_tile(0, 0);
-        sched_fence();
-        read_score(0, 2);
-        sched_fence();
-        score_tile(1, 1);
-        sched_fence();
-        read_q(0, 0);
-        sched_fence();
-        score_tile(0, 2);
-        sched_fence();
+                        d[jw] = Bf16::mfma(b[t][TP::A[e]], cf[jw][TP::B[e]], e > 0 ? d[jw] : (T == 3 ? zero : S[2 * ks + t][jw]));
 #pragma unroll
-        for (int pb = 0; pb < 4; ++pb) {
-            if (pb < 3) read_q((pb + 1) & 1, pb + 1);
-            else {
-                read_c();
-                read_b(0, 0, 0);
+                for (int jw = 0; jw < NJW; ++jw) S[2 * ks + t][jw] = T == 3 ? S[2 * ks + t][jw] + d[jw] : d[jw];
             }
-            sched_fence();
-            state_product(pb & 1, pb);
-            sched_fence();
+        };
+        // Under the products of one kind the operands of the other are read and split.
+        if constexpr (!SUMS) {
+            read_a(0);
+        } else {
+            read_b(0);
         }
-        constexpr int NB = 2 * (NIT / 4);
 #pragma unroll
-        for (int b = 0; b < NB; ++b) {
-            if (b + 1 < NB) read_b((b + 1) & 1, (b + 1) / (NIT / 4), 4 * ((b + 1) % (NIT / 4)));
-            sched_fence();
-            update(b & 1, b / (NIT / 4), 4 * (b % (NIT / 4)));
-            sched_fence();
+        for (int jw = 0; jw < NJW; ++jw)
+#pragma unroll
+            for (int x = 0; x < T; ++x)
+                cf[jw][x] = cat(lds_read_tr16(c_step(c_at[0], jw) + 2 * (2 * x + buf) * TL::C), lds_read_tr16(c_step(c_at[1], jw) + 2 * (2 * x + buf) * TL::C));
+        sched_fence();
+#pragma unroll
+        for (int ks = 0; ks < KS; ++ks) {
+            if constexpr (!SUMS) {
+                // a matrix instruction, and under it vector ones and a read of LDS
+                auto interleave = [&](auto n, auto vector) __attribute__((always_inline)) {
+#pragma unroll
+                    for (int e = 0; e < decltype(n)::value; ++e) {
+                        __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);
+                        __builtin_amdgcn_sched_group_barrier(0x2, decltype(vector)::value, 0);
+                        __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+                    }
+                };
+                read_b(ks);
+                state_product(0);
+                sched_fence();
+                constexpr std::integral_constant<int, NJW * TP::N> half{};
+                if constexpr (NJW == 2) {
+                    pack_state((ks + 1) % KS, 0);  // (the first step's rows are final after its own update)
+                    if (ks + 1 == KS) pin_state(0);
+                    state_product(1);
+                    interleave(half, std::integral_constant<int, 4>{});
+                    sched_fence();
+                }
+                pack_state((ks + 1) % KS, NJW - 1);
+                if (ks + 1 == KS) pin_state(NJW - 1);
+                update(ks, 0);
+                interleave(half, std::integral_constant<int, 4>{});
+                sched_fence();
+                if (ks + 1 < KS) read_a(ks + 1);
+                update(ks, 1);
+                interleave(half, std::integral_constant<int, 2>{});
+                sched_fence();
+            } else {
+                update(ks, 0);
+                update(ks, 1);
+                if (ks + 1 < KS) read_b(ks + 1);
+            }
         }
-        pack_state();
+        if constexpr (!SUMS) {
+            add_rest(o, ah, ar);
+        }
+    };
+    if constexpr (!SUMS) {
+#pragma unroll
+        for (int jw = 0; jw < NJW; ++jw) pack_state(0, jw);
+    }
+    __syncthreads();
+    run_rounds<2>(r.p0, r.p1, [&](int buf, int p) __attribute__((always_inline)) {
+        if constexpr (!SUMS) {
+            if (p > r.p0) finish(buf ^ 1, p - 1);
+        }
+        chunk(buf);
         chunk_barrier();
+    });
+    if constexpr (SUMS) {
+        f32x4 *slot = reinterpret_cast<f32x4 *>(io.sums);
+#pragma unroll
+        for (int it = 0; it < NIT; ++it)
+#pragma unroll
+            for (int jw = 0; jw < NJW; ++jw) slot[slot_at(it, jw)] = S[it][jw];
+        return;
     }
-    if (r.p1 > r.p0) {
-        pbuf = (r.p1 - r.p0) & 1;  // (finish_previous reads the other buffer: the last chunk's)
-        read_scores_of_previous();
-        finish_previous(r.p1 - 1);
-    }
+    if (r.p1 > r.p0) finish((r.p1 - 1 - r.p0) & 1, r.p1 - 1);
     if (io.sout != nullptr) {
 #pragma unroll
         for (int it = 0; it < NIT; ++it)
@@ -506,46 +550,56 @@ __device__ __forceinline__ void split_compute_role(const ColStateIO &io, float *
     }
 }
 
-// One problem per workgroup: 4 compute wavefronts, 4 loader wavefronts; grid and state slots as scan_kernel.
-template <int DI, int DJ, int PF>
-__global__ __launch_bounds__(512) void split_scan_kernel(ProblemSetF set, int BH, int N, int nchunks, int cpg, int G) {
-    using TL = Tiling<DI, DJ>;
-    using CT = ColTiling<DI, DJ>;
-    __shared__ __attribute__((aligned(16))) u16 sA[4 * CT::SA];  // [hi | lo] x [2 buffers]
-    __shared__ __attribute__((aligned(16))) u16 sB[4 * CT::SA];
-    __shared__ __attribute__((aligned(16))) u16 sC[4 * CT::SC];
-    __shared__ __attribute__((aligned(16))) u32x2 sP[2 * 2 * 16 * 64];  // masked score tiles: [hi | lo] x [2 buffers]
+// 512 threads: wavefronts 0..3 compute, 4..7 load.  Grid: grid_for(BH, count, G) for the scan, grid_for(BH, nact * sub,
+// G - 1) for the sums of the groups.  spg: chunks of 32 positions per group.
+template <int DI, int DJ, int T, bool SUMS>
+__global__ __launch_bounds__(512, T == 2 ? 4 : 2) void split_scan_kernel(ProblemSetF set, int BH, int N, int nsteps, int spg, int G) {
+    using TL = SplitTiling<DI, DJ, T, SUMS>;
+    __shared__ __attribute__((aligned(256))) unsigned char smem[TL::LDS];  // (see SplitTile::step)
+    u16 *sB = reinterpret_cast<u16 *>(smem), *sC = sB + 2 * T * TL::AB, *sA = sC + 2 * T * TL::C;
+    u32x4 *sP = reinterpret_cast<u32x4 *>(sA + (SUMS ? 0 : 2 * T * TL::AB));
     const int l = threadIdx.x & 63;
     const int wv = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
-    const WorkItem wi = decode_workgroup(set.count, BH, set.xcds);
-    if (wi.grp >= G) return;
-    const ProblemF &pr = set.p[wi.prob];
+    const int sub = set.sub;
+    const WorkItem wi = decode_workgroup(SUMS ? set.nact * sub : set.count, BH, set.xcds);
+    if (wi.grp >= (SUMS ? G - 1 : G)) return;
+    const ProblemF &pr = set.p[SUMS ? set.act[wi.prob / sub] : wi.prob];
     const int di = pr.di, dj = pr.dj;
-    ScanRange r;
+    SplitRange r;
     r.N = N;
-    r.nchunks = nchunks;
-    r.p0 = wi.grp * cpg;
-    r.p1 = min(r.p0 + cpg, nchunks);
+    r.nsteps = nsteps;
+    r.p0 = wi.grp * spg;
+    r.p1 = min(r.p0 + spg, nsteps);
     r.reversed = pr.reversed;
-    r.mask_rev = pr.mask_rev;
-    r.comp = 0;
+    ColStateIO io;
+    if constexpr (SUMS) {  // a piece of the group; one past its end leaves a zero slot
+        const int piece = wi.prob % sub, per = (spg + sub - 1) / sub;
+        r.p0 += piece * per;
+        r.p1 = min(r.p0 + per, r.p1);
+        io.sums = pr.gstate + (((size_t)wi.bh * G + wi.grp) * sub + piece) * TL::STATE_FLOATS;
+        if (r.p1 <= r.p0) {
+            for (int e = threadIdx.x; e < TL::STATE_FLOATS / 4; e += 512) reinterpret_cast<f32x4 *>(io.sums)[e] = f32x4{0.f, 0.f, 0.f, 0.f};
+            return;
+        }
+    } else {
+        if (pr.gstate != nullptr) io.seed = pr.gstate + ((size_t)wi.bh * G + wi.grp) * sub * TL::STATE_FLOATS;
+        if (pr.sin != nullptr) io.sin = pr.sin + (size_t)wi.bh * di * pr.lds;
+        if (pr.sout != nullptr && wi.grp == G - 1) io.sout = pr.sout + (size_t)wi.bh * di * pr.lds;
+        io.lds = pr.lds;
+    }
     if (wv >= 4) {
         const SplitRows rA = split_rows(pr.A, head_base(pr.bsA, pr.hsA, pr.H, wi.bh), pr.bf16_operands & 1, N, pr.lda, di);
         const SplitRows rB = split_rows(pr.B, head_base(pr.bsB, pr.hsB, pr.H, wi.bh), pr.bf16_operands & 2, N, pr.ldb, di);
         const SplitRows rC = split_rows(pr.C, head_base(pr.bsC, pr.hsC, pr.H, wi.bh), pr.bf16_operands & 4, N, pr.ldc, dj);
-        split_loader_role<DI, DJ, PF, 256>(rA, rB, rC, di, dj, pr.lda, pr.ldb, pr.ldc, r, (int)threadIdx.x - 256, sA, sB, sC);
-        return;
+        split_loader_role<DI, DJ, T, SUMS>(rA, rB, rC, di, dj, pr.lda, pr.ldb, pr.ldc, r, (int)threadIdx.x - 256, sA, sB, sC,
+                                          reinterpret_cast<u32x2 *>(sP));
+    } else {
+        float *O_head = SUMS ? nullptr : pr.O + head_base(pr.bsO, pr.hsO, pr.H, wi.bh);
+        if (!SUMS && pr.reversed)
+            split_compute_role<DI, DJ, T, SUMS, true>(io, O_head, pr.ldo, di, dj, r, wv, l, sA, sB, sC, sP);
+        else
+            split_compute_role<DI, DJ, T, SUMS, false>(io, O_head, pr.ldo, di, dj, r, wv, l, sA, sB, sC, sP);
     }
-    ColStateIO io;
-    if (pr.gstate != nullptr) io.seed = pr.gstate + ((size_t)wi.bh * G + wi.grp) * set.sub * TL::STATE_FLOATS;
-    if (pr.sin != nullptr) io.sin = pr.sin + (size_t)wi.bh * di * pr.lds;
-    if (pr.sout != nullptr && wi.grp == G - 1) io.sout = pr.sout + (size_t)wi.bh * di * pr.lds;
-    io.lds = pr.lds;
-    float *O_head = pr.O + head_base(pr.bsO, pr.hsO, pr.H, wi.bh);
-    if (pr.mask_rev != 0)
-        split_compute_role<DI, DJ, true>(io, O_head, pr.ldo, di, dj, r, wv, l, sA, sB, sC, sP);
-    else
-        split_compute_role<DI, DJ, false>(io, O_head, pr.ldo, di, dj, r, wv, l, sA, sB, sC, sP);
 }
 
 }  // namespace cott

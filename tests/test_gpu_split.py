@@ -1,0 +1,71 @@
+"""Causal fp32 ops on split operands (cott_split.h): widths below their padding, ragged lengths on either side of a chunk of 32 and
+of the one-group limits, infinite entries, bf16 upstream gradients of 128-wide heads."""
+import pytest
+import torch
+
+from util import inputs, rel_l2, worst_block
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+F32, BF = torch.float32, torch.bfloat16
+
+
+@pytest.fixture(scope="module")
+def ct():
+    import cottention_transformer_amd as ct_
+    return ct_
+
+
+# With three terms a product is exact to 2^-24 and only the fp32 sums round.  A result passes at most N / 32 additions to its
+# state and about 50 sums within a chunk and between groups; with independent roundings of 2^-25 rms that is
+# 2^-25 sqrt(4200 / 32 + 50) = 4e-7, taken twice over for the worst block.
+CASES = [(1, 1, 1, 80, 96), (1, 2, 31, 128, 64), (1, 2, 33, 64, 128), (2, 3, 65, 112, 128), (1, 2, 128, 128, 128), (1, 2, 129, 128, 128),
+         (1, 16, 256, 128, 96), (1, 16, 257, 96, 96), (2, 20, 100, 80, 48), (1, 3, 4100, 128, 128), (1, 2, 700, 48, 80)]
+
+
+@pytest.mark.parametrize("case", CASES, ids=lambda c: "x".join(map(str, c)))
+def test_three_terms_keep_fp32_precision(ct, oracle, case):
+    q, k, v, do = inputs(*case, F32, seed=case[2])
+    dev = [t.to(DEV) for t in (q, k, v, do)]
+    for rev in (False, True):
+        got, ref = ct.causal_dot_product(*dev[:3], rev), oracle.causal(q, k, v, rev)
+        assert rel_l2(got, ref) <= 4e-7 and worst_block(got, ref) <= 8e-7, rev
+    for name, got, ref in zip(("dQ", "dK", "dV"), ct.causal_backward(*dev), oracle.causal_bwd(q, k, v, do)):
+        assert rel_l2(got, ref) <= 4e-7 and worst_block(got, ref) <= 8e-7, name
+
+
+@pytest.mark.parametrize("n,at", [(70, 40), (300, 100)])  # one group; groups, so that sums and prefixes carry the infinity
+@pytest.mark.parametrize("which", ["q", "k", "v"])
+def test_infinite_entries_of_three_term_ops(ct, which, n, at):
+    """One infinite entry: its own row (q) or everything after it is infinite or no number exactly where 64-bit arithmetic has
+    it, with the same sign, and the rest is as precise as ever.  Whole numbers, whose lower terms are zero, among the others.
+    Left out: positions before an infinite value in its block of 16, where a masked score, zero, is multiplied with it."""
+    g = torch.Generator().manual_seed(n)
+    q, k = (torch.rand(1, 2, n, 128, generator=g) + 0.25 for _ in range(2))
+    v = torch.randint(1, 4, (1, 2, n, 128), generator=g).float() * torch.where(torch.rand(1, 2, 1, 128, generator=g) < 0.5, -1.0, 1.0)
+    x = {"q": q, "k": k, "v": v}[which]
+    x[0, 1, at, 5] = float("inf")
+    got = ct.causal_dot_product(q.to(DEV), k.to(DEV), v.to(DEV)).cpu().double()
+    q, k, v = q.double(), k.double(), v.double()
+    S = torch.zeros(1, 2, 128, 128, dtype=torch.float64)
+    want = torch.empty(1, 2, n, 128, dtype=torch.float64)
+    for t in range(n):
+        S = S + k[:, :, t, :, None] * v[:, :, t, None, :]
+        want[:, :, t] = (q[:, :, t, :, None] * S).sum(-2)
+    if which == "v":
+        before = slice(at // 16 * 16, at)
+        got[:, 1, before, 5] = want[:, 1, before, 5]
+    finite = torch.isfinite(want)
+    assert not finite.all() and torch.equal(torch.isnan(got), torch.isnan(want))
+    assert torch.equal(got[~finite & ~torch.isnan(want)], want[~finite & ~torch.isnan(want)])
+    assert float((got[finite] - want[finite]).norm() / want[finite].norm()) <= 4e-7
+
+
+@pytest.mark.parametrize("case", [(1, 2, 128, 128, 128), (1, 3, 700, 80, 112), (2, 20, 65, 96, 96)], ids=lambda c: "x".join(map(str, c)))
+def test_bf16_gradient_of_wide_heads(ct, case):
+    from cottention_transformer_amd import _loader, ops
+    assert _loader.lib().cott_causal_bwd_g16_supported(*case) == 1
+    q, k, v, do = (t.to(DEV) for t in inputs(*case, F32, seed=3))
+    do = do.to(BF)
+    for got, want in zip(ops.causal_backward_from(q, k, v, do), ops.causal_backward(q, k, v, do.float())):
+        assert got.dtype == F32 and torch.equal(got, want)

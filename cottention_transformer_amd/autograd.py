@@ -138,7 +138,7 @@ class PrepareInputs(torch.autograd.Function):
 
     @staticmethod
     def forward(ctx, q, k, v, keep, cnt, sig, out_dtype, rot_table=None, position_ids=None, bnhd=False):
-        q, k, v = q.contiguous(), k.contiguous(), v.contiguous()
+        q, k, v = ops.preparation_rows(q, k, v, bnhd)
         ctx.save_for_backward(q, k, v, keep, cnt, sig, rot_table, position_ids)
         ctx.bnhd = bool(bnhd)
         rotary = (rot_table, position_ids) if rot_table is not None else None
@@ -168,7 +168,7 @@ class PreparedCausalAttention(torch.autograd.Function):
 
     @staticmethod
     def forward(ctx, q, k, v, keep, cnt, sig, rot_table=None, first_position=0, bnhd=False, merged_heads=False):
-        q, k, v = q.contiguous(), k.contiguous(), v.contiguous()
+        q, k, v = ops.preparation_rows(q, k, v, bnhd)
         ids = first_position if torch.is_tensor(first_position) else None
         rotary = (rot_table, ids if ids is not None else int(first_position)) if rot_table is not None else None
         out, prepared, states = ops.causal_dot_product_prepared(q, k, v, keep, cnt, sig, rotary=rotary, bnhd=bnhd,
@@ -209,7 +209,7 @@ class PreparedNonCausalAttention(torch.autograd.Function):
 
     @staticmethod
     def forward(ctx, q, k, v, keep, cnt, sig, bnhd=False, merged_heads=False):
-        q, k, v = q.contiguous(), k.contiguous(), v.contiguous()
+        q, k, v = ops.preparation_rows(q, k, v, bnhd)
         out, prepared = ops.noncausal_dot_product_prepared(q, k, v, keep, cnt, sig, bnhd=bnhd, merged_heads=merged_heads)
         ctx.save_for_backward(q, k, v, keep, cnt, sig, *prepared)
         ctx.bnhd, ctx.merged = bool(bnhd), bool(merged_heads)
@@ -230,11 +230,15 @@ class PreparedNonCausalAttention(torch.autograd.Function):
 def _weight_gradient(gy, x):
     """gy^T x for gy (R, out), x (R, in).  With many rows and a small weight the library's single GEMM fills the
     chip with too few tiles over a long reduction (out = in = 1024, R = 16384, bf16: 109 us); the rows are cut into
-    pieces multiplied as one batched GEMM and summed in fp32 instead (8 pieces: 47 us)."""
+    pieces multiplied as one batched GEMM and summed in fp32 instead (8 pieces: 47 us).  Weights above 1 M elements (three
+    projections at once) are cut until their 256 x 128 tiles fill the chip (R = 16384: 3072 x 1024 in 1 / 2 / 4 / 8 pieces 163 /
+    132 / 105 / 112 us, 2304 x 768 125 / 88 / 92 / 77; R = 8192: 6144 x 2048 176 / 204)."""
     r = x.shape[0]
     pieces = 1
-    if x.is_cuda and x.dtype in (torch.float16, torch.bfloat16) and gy.shape[1] * x.shape[1] <= 1 << 20:
-        while pieces < 16 and r % (2 * pieces) == 0 and r // (2 * pieces) >= 2048:
+    if x.is_cuda and x.dtype in (torch.float16, torch.bfloat16):
+        out, inner = gy.shape[1], x.shape[1]
+        tiles = 0 if out * inner <= 1 << 20 else -(-out // 256) * -(-inner // 128)
+        while pieces < 16 and tiles * pieces < 256 and r % (2 * pieces) == 0 and r // (2 * pieces) >= 2048:
             pieces *= 2
     if pieces == 1:
         return gy.t() @ x
@@ -242,11 +246,32 @@ def _weight_gradient(gy, x):
     return parts.sum(0, dtype=torch.float32)
 
 
+def _joined(parts, sizes):
+    """(R, n_0), (R, n_1), ... side by side as one (R, sum n) matrix: without a copy when they are neighbouring column slices of
+    one and nothing is recorded for a second derivative (which would see a view of the first slice alone)."""
+    if torch.is_grad_enabled():
+        return torch.cat(parts, dim=1)
+    first, total, size = parts[0], sum(sizes), parts[0].element_size()
+    at, rows = first.data_ptr(), first.shape[0]
+    for t, n in zip(parts, sizes):
+        if (t.data_ptr() != at or t.dtype != first.dtype or n != 1 and t.stride(1) != 1 or rows != 1 and t.stride(0) != total
+                or t.untyped_storage().data_ptr() != first.untyped_storage().data_ptr()):
+            return torch.cat(parts, dim=1)
+        at += n * size
+    return first.as_strided((rows, total), (total, 1))
+
+
 class InputProjections(torch.autograd.Function):
     """(x, w_0, b_0, w_1, b_1, ...) -> (x w_0^T + b_0, x w_1^T + b_1, ...): the q / k / v projections of an attention
     block (GPT_Trainer/GPTCosAttention.py:443-445, BERT_Trainer/BertCosAttention.py:121,143-144 with biases) as one
     operator.  Under autocast x is converted once for all of them, the gradient of x is accumulated by the GEMMs
-    themselves and converted back once, and the weight gradients take `_weight_gradient`.  b_i may be None."""
+    themselves and converted back once, and the weight gradients take `_weight_gradient`.  b_i may be None.
+
+    Several weights that have to be converted anyway (fp32 parameters under autocast) are converted into one matrix, and all
+    the products are one GEMM each: the outputs are then column slices of one tensor, which the input preparation
+    reads, and whose gradients it writes, as such; dx leaves the GEMM in fp32.  Forward / dx / dW of three projections, us, one
+    by one and together: 16384 x 1024 98 / 124 / 157 and 94 / 91 / 105, 16384 x 768 75 / 86 / 133 and 65 / 55 / 77,
+    2048 x 512 60 / 54 / 59 and 19 / 19 / 20."""
 
     @staticmethod
     def forward(ctx, x, *wb):
@@ -255,12 +280,26 @@ class InputProjections(torch.autograd.Function):
         if x.is_cuda and x.dtype != torch.float64 and torch.is_autocast_enabled("cuda"):
             cd = torch.get_autocast_dtype("cuda")
         x2 = x.reshape(-1, x.shape[-1]).to(cd)
-        ws = [w.to(cd) for w in wb[0::2]]
-        ctx.save_for_backward(x2, *ws)
+        weights, biases = wb[0::2], wb[1::2]
         ctx.x_meta = (x.shape, x.dtype)
         ctx.wb_dtypes = [None if t is None else t.dtype for t in wb]
+        ctx.sizes = [w.shape[0] for w in weights]
+        ctx.joint = False
+        if len(weights) > 1 and weights[0].dtype != cd and x.is_cuda:
+            bias_free = biases[0] is None
+            ctx.joint = (all(w.dtype != cd and w.device == x.device for w in weights)
+                         and all((b is None) == bias_free for b in biases))
+        if ctx.joint:
+            w = torch.empty((sum(ctx.sizes), x2.shape[1]), dtype=cd, device=x.device)
+            for part, own in zip(w.split(ctx.sizes), weights):
+                part.copy_(own)
+            ctx.save_for_backward(x2, w)
+            y = torch.nn.functional.linear(x2, w, None if bias_free else torch.cat([b.to(cd) for b in biases]))
+            return tuple(part.view(x.shape[:-1] + (n,)) for part, n in zip(y.split(ctx.sizes, dim=1), ctx.sizes))
+        ws = [w.to(cd) for w in weights]
+        ctx.save_for_backward(x2, *ws)
         outs = []
-        for w, b in zip(ws, wb[1::2]):
+        for w, b in zip(ws, biases):
             y = torch.nn.functional.linear(x2, w, None if b is None else b.to(cd))
             outs.append(y.view(x.shape[:-1] + (w.shape[0],)))
         return tuple(outs)
@@ -270,18 +309,32 @@ class InputProjections(torch.autograd.Function):
         x2, *ws = ctx.saved_tensors
         shape, xdt = ctx.x_meta
         gys = [g.reshape(-1, g.shape[-1]).to(x2.dtype) for g in gys]
+        if ctx.joint:
+            gys = [_joined(gys, ctx.sizes)]
         gx = None
         if ctx.needs_input_grad[0]:
-            gx = gys[0] @ ws[0]
-            for g, w in zip(gys[1:], ws[1:]):
-                gx.addmm_(g, w)
+            # (with a second derivative to record, products that have one)
+            if (ctx.joint and xdt == torch.float32 and x2.dtype in (torch.float16, torch.bfloat16)
+                    and not torch.is_grad_enabled()):
+                gx = torch.mm(gys[0], ws[0], out_dtype=torch.float32)
+            else:
+                gx = gys[0] @ ws[0]
+                for g, w in zip(gys[1:], ws[1:]):
+                    gx.addmm_(g, w)
             gx = gx.view(shape).to(xdt)
+        column_sum = lambda g: g.sum(0, dtype=torch.promote_types(g.dtype, torch.float32))
+        want_w = [ctx.needs_input_grad[1 + 2 * i] for i in range(len(ctx.sizes))]
+        want_b = [t is not None and ctx.needs_input_grad[2 + 2 * i] for i, t in enumerate(ctx.wb_dtypes[1::2])]
+        if ctx.joint:
+            gws = _weight_gradient(gys[0], x2).split(ctx.sizes) if any(want_w) else want_w
+            gbs = column_sum(gys[0]).split(ctx.sizes) if any(want_b) else want_b
+        else:
+            gws = [_weight_gradient(g, x2) if want else None for g, want in zip(gys, want_w)]
+            gbs = [column_sum(g) if want else None for g, want in zip(gys, want_b)]
         grads = [gx]
-        for i, g in enumerate(gys):
-            wdt, bdt = ctx.wb_dtypes[2 * i], ctx.wb_dtypes[2 * i + 1]
-            grads.append(_weight_gradient(g, x2).to(wdt) if ctx.needs_input_grad[1 + 2 * i] else None)
-            grads.append(g.sum(0, dtype=torch.promote_types(g.dtype, torch.float32)).to(bdt)
-                         if bdt is not None and ctx.needs_input_grad[2 + 2 * i] else None)
+        for i in range(len(ctx.sizes)):
+            grads.append(gws[i].to(ctx.wb_dtypes[2 * i]) if want_w[i] else None)
+            grads.append(gbs[i].to(ctx.wb_dtypes[2 * i + 1]) if want_b[i] else None)
         return tuple(grads)
 
 

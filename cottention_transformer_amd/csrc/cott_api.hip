@@ -137,6 +137,7 @@ struct Op {
     void *sout = nullptr;
     unsigned char lay[4] = {0, 0, 0, 0};  // A, B, C, O given as (B,N,H,width) instead of (BH,N,width)
     int H = 1;
+    int token_stride = 0;  // > 0: elements from one position to the next of A, B, C in that layout (0: H * width)
     int bf16_operands = 0;  // fp32 op on split operands: bit 0 / 1 / 2 = A / B / C is a bf16 tensor
     bool f32_in = false;  // A, B, C are fp32 tensors of an op in bf16 (cott_causal_fwd_f32in)
     // states handed from a forward to a backward pass (cott_causal_fwd_save / cott_causal_bwd_saved)
@@ -592,6 +593,7 @@ int run_ops(const char *fn, bool causal, const Op *ops, int n, long BH, int N, i
                 d.lds = o.dj;
                 for (int x = 0; x < 4; ++x) d.lay[x] = o.lay[x];
                 d.H = o.H;
+                d.token_stride = o.token_stride;
                 d.bf16_operands = o.bf16_operands;
                 if (o.save != nullptr) {
                     if (!causal || o.reversed || dtype == COTT_F32)
@@ -632,6 +634,19 @@ int run_ops(const char *fn, bool causal, const Op *ops, int n, long BH, int N, i
             e = causal ? cott::launch_causal_mfma_fp16(a) : cott::launch_noncausal_mfma_fp16(a);
         if (e != hipSuccess) return fail(COTT_ERR_HIP, "%s: HIP launch failed: %s", fn, hipGetErrorString(e));
     }
+    return COTT_OK;
+}
+
+// Input layout argument of the preparation entry points: 0 = (B,H,N,D), other values below H * max(Dk, Dv) = (B,N,H,D), larger
+// ones = (B,N,H,D) with that many elements from one position to the next.  token: 0, 1 or that number.
+int input_layout(const char *fn, int in_bnhd, int H, int N, int Dk, int Dv, bool fused, int *token) {
+    const long packed = (long)H * (Dk > Dv ? Dk : Dv);
+    *token = in_bnhd == 0 ? 0 : ((long)in_bnhd <= packed ? 1 : in_bnhd);
+    if (*token > 1 && *token % 8 != 0)
+        return fail(COTT_ERR_INVALID, "%s: %d elements between positions: needs a multiple of 8", fn, *token);
+    const long row = *token > 1 ? (long)*token : packed;
+    if (fused && *token > 0 && (long)N * row > (1L << 30))
+        return fail(COTT_ERR_UNSUPPORTED, "%s: %ld elements of a batch element exceed 2^30", fn, (long)N * row);
     return COTT_OK;
 }
 
@@ -829,9 +844,12 @@ int fwd_prep_impl(const char *fn, const void *q, const void *k, const void *v, v
         return fail(COTT_ERR_INVALID, "%s: tensor pointers must be 16-byte aligned", fn);
     if (reinterpret_cast<uintptr_t>(pos_ids) & 7u) return fail(COTT_ERR_INVALID, "%s: position ids must be 8-byte aligned", fn);
     if ((long)N > (1L << 28)) return fail(COTT_ERR_UNSUPPORTED, "%s: N = %d exceeds 2^28", fn, N);
+    int token = 0;
+    if (int rc = input_layout(fn, in_bnhd, H, N, Dk, Dv, true, &token)) return rc;
     Op op{q, k, v, o, Dk, Dv, 0};
     op.H = H;
-    if (in_bnhd) op.lay[0] = op.lay[1] = op.lay[2] = 1;
+    if (token > 0) op.lay[0] = op.lay[1] = op.lay[2] = 1;
+    if (token > 1) op.token_stride = token;
     if (o_bnhd) op.lay[3] = 1;
     if (saved != nullptr) {
         if (chunks_per_cut < 1 || ncuts < 1 || (long)(ncuts - 1) * chunks_per_cut > (N + 63) / 64 - 1)
@@ -914,9 +932,12 @@ int cott_noncausal_fwd_prep(const void *q, const void *k, const void *v, void *o
     if (!aligned16(q) || !aligned16(k) || !aligned16(v) || !aligned16(o) || !aligned16(q_out) || !aligned16(k_out) ||
         !aligned16(v_out))
         return fail(COTT_ERR_INVALID, "%s: tensor pointers must be 16-byte aligned", fn);
+    int token = 0;
+    if (int rc = input_layout(fn, in_bnhd, H, N, Dk, Dv, true, &token)) return rc;
     Op op{q, k, v, o, Dk, Dv, 0};
     op.H = H;
-    if (in_bnhd) op.lay[0] = op.lay[1] = op.lay[2] = 1;
+    if (token > 0) op.lay[0] = op.lay[1] = op.lay[2] = 1;
+    if (token > 1) op.token_stride = token;
     if (o_bnhd) op.lay[3] = 1;
     cott::SetArgs::Prep prep;
     prep.on = true;
@@ -1552,10 +1573,12 @@ int cott_prep_ex_fwd(const void *q, const void *k, const void *v, void *q_out, v
     if (!aligned16(q) || !aligned16(k) || !aligned16(v) || !aligned16(q_out) || !aligned16(k_out) || !aligned16(v_out))
         return fail(COTT_ERR_INVALID, "%s: tensor pointers must be 16-byte aligned", fn);
     if ((cnt == nullptr) != (sig == nullptr)) return fail(COTT_ERR_INVALID, "%s: cnt and sig go together", fn);
+    int token = 0;
+    if (int rc = input_layout(fn, in_bnhd, H, N, Dk, Dv, false, &token)) return rc;
     const void *x[3] = {q, k, v};
     void *y[3] = {q_out, k_out, v_out};
     hipError_t e = cott::launch_prep(false, x, nullptr, y, keep, cnt, sig, nullptr, B, H, N, Dk, Dv, in_dtype, out_dtype,
-                                     out_dtype, 1e-12f, in_bnhd ? 1 : 0, rot_table, pos, rot_table ? rotary_dim : 0,
+                                     out_dtype, 1e-12f, token, rot_table, pos, rot_table ? rotary_dim : 0,
                                      table_rows, static_cast<hipStream_t>(stream));
     if (e != hipSuccess) return fail(COTT_ERR_HIP, "%s: HIP launch failed: %s", fn, hipGetErrorString(e));
     return COTT_OK;
@@ -1574,11 +1597,13 @@ int cott_prep_ex_bwd(const void *q, const void *k, const void *v, const void *gq
         !aligned16(dq) || !aligned16(dk) || !aligned16(dv))
         return fail(COTT_ERR_INVALID, "%s: tensor pointers must be 16-byte aligned", fn);
     if ((cnt == nullptr) != (sig == nullptr)) return fail(COTT_ERR_INVALID, "%s: cnt and sig go together", fn);
+    int token = 0;
+    if (int rc = input_layout(fn, in_bnhd, H, N, Dk, Dv, false, &token)) return rc;
     const void *x[3] = {q, k, v};
     const void *g[3] = {gq, gk, gv};
     void *y[3] = {dq, dk, dv};
     hipError_t e = cott::launch_prep(true, x, g, y, keep, cnt, sig, dsig_rows, B, H, N, Dk, Dv, in_dtype, in_dtype,
-                                     grad_dtype, 1e-12f, in_bnhd ? 1 : 0, rot_table, pos, rot_table ? rotary_dim : 0,
+                                     grad_dtype, 1e-12f, token, rot_table, pos, rot_table ? rotary_dim : 0,
                                      table_rows, static_cast<hipStream_t>(stream));
     if (e != hipSuccess) return fail(COTT_ERR_HIP, "%s: HIP launch failed: %s", fn, hipGetErrorString(e));
     return COTT_OK;

@@ -20,6 +20,7 @@ struct OpDesc {
     // of a position next to each other, as the projections of a transformer block produce and consume them.
     unsigned char lay[4] = {0, 0, 0, 0};
     int H = 1;  // heads per batch element; needed when any layout flag is set
+    int token_stride = 0;  // > 0: elements from one position to the next of the (B,N,H,width) operands among A, B, C
     // fp32 ops on split operands only: bit 0 / 1 / 2 = A / B / C is a bf16 tensor (its lower terms are zero)
     int bf16_operands = 0;
     // Complement form (16-bit causal MFMA kernels, sets with sequence groups only): the op is walked against its
@@ -126,7 +127,7 @@ hipError_t launch_wide(int dtype, const OpDesc *ops, int n, int BH, int N, int c
 // Fused input preparation (backward = false) or its backward; see cott_prep.hip.
 hipError_t launch_prep(bool backward, const void *const x[3], const void *const g[3], void *const y[3],
                        const unsigned char *keep, const float *cnt, const float *sig, float *dsig_rows, int B, int H, int N,
-                       int dk, int dv, int x_dtype, int y_dtype, int g_dtype, float eps, int x_bnhd, const float *rot,
+                       int dk, int dv, int x_dtype, int y_dtype, int g_dtype, float eps, long x_token, const float *rot,
                        const long long *pos, int R, int table_rows, hipStream_t stream);
 
 hipError_t launch_decode(int dtype, void *state, const void *q, const void *k, const void *v, void *o, int BH,

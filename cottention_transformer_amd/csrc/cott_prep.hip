@@ -118,7 +118,9 @@ struct PrepArgs {
     float eps;
     // Optional extras: q, k, v given as (B,N,H,D) (the layout the projections produce) instead of
     // (B,H,N,D), and the GPT-J rotary embedding applied to the first R columns of q and k.
-    int x_bnhd;           // 1: x (and, backward, y) are (B,N,H,D); g (backward) / y (forward) stay (B,H,N,D)
+    // > 0: x (and, backward, y) are (B,N,H,D) with this many elements from one position to the next, or H*D when 1;
+    // g (backward) / y (forward) stay (B,H,N,D)
+    long x_token;
     const float *rot;     // (P,R) table, row p = [sin(p f_0..f_{R/2-1}) | cos(...)], or null
     const long long *pos; // (B,N) row of the table per position (clamped to the table)
     int R, table_rows;
@@ -185,6 +187,7 @@ __global__ __launch_bounds__(kPrepThreads) void prep_kernel(PrepArgs a) {
               g_dtype = ALL_BF16 ? (int)COTT_BF16 : a.g_dtype;
     const int t = blockIdx.y;
     const int D = t < 2 ? a.dk : a.dv;
+    const long token = a.x_token == 1 ? (long)a.H * D : a.x_token;
     const int lpr = a.lpr[t];
     const int rpb = kPrepThreads / lpr;
     const long row0 = ((long)blockIdx.x * R) * rpb + threadIdx.x / lpr;
@@ -218,8 +221,8 @@ __global__ __launch_bounds__(kPrepThreads) void prep_kernel(PrepArgs a) {
         rr[u] = act[u] ? row : 0;
         int sq, hq, bq;  // position, head, batch element of the row
         split_row(rr[u], a, sq, hq, bq);
-        xoff[u] = a.x_bnhd ? (size_t)(((long)bq * a.N + sq) * a.H + hq) * D : (size_t)rr[u] * D;
         const long tok = (long)bq * a.N + sq;
+        xoff[u] = token > 0 ? (size_t)(tok * token + (long)hq * D) : (size_t)rr[u] * D;
         keep_in[u] = a.keep != nullptr ? a.keep[tok] : (uint8_t)1;
         pos_in[u] = rotary ? a.pos[tok] : 0;
         cnt_in[u] = side ? a.cnt[tok] : 0.f;
@@ -366,11 +369,11 @@ int lanes_per_row(int d, int nv) {
 
 hipError_t launch_prep(bool backward, const void *const x[3], const void *const g[3], void *const y[3],
                        const uint8_t *keep, const float *cnt, const float *sig, float *dsig_rows, int B, int H, int N,
-                       int dk, int dv, int x_dtype, int y_dtype, int g_dtype, float eps, int x_bnhd, const float *rot,
+                       int dk, int dv, int x_dtype, int y_dtype, int g_dtype, float eps, long x_token, const float *rot,
                        const long long *pos, int R, int table_rows, hipStream_t stream) {
     PrepArgs a;
     a.table_rows = table_rows > 0 ? table_rows : 1;
-    a.x_bnhd = x_bnhd;
+    a.x_token = x_token;
     a.rot = rot;
     a.pos = pos;
     a.R = R;
@@ -406,7 +409,7 @@ hipError_t launch_prep(bool backward, const void *const x[3], const void *const 
     const dim3 grid((unsigned)blocks, 3), blk(kPrepThreads);
     const bool f64 = x_dtype == COTT_F64;
     const bool all_bf16 = x_dtype == COTT_BF16 && y_dtype == COTT_BF16 && (!backward || g_dtype == COTT_BF16);
-    // rows whose lanes can take 16 bytes each: widths multiples of 8 (16-byte aligned rows in either layout) that fill
+    // rows whose lanes can take 16 bytes each: widths multiples of 8 (16-byte aligned rows in every layout) that fill
     // the two groups of every lane, or leave whole lanes empty
     const bool paired = dk % 8 == 0 && dv % 8 == 0;
 #define COTT_PREP(ACC, BWD) \

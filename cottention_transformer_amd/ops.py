@@ -300,7 +300,7 @@ def causal_dot_product_prepared(q, k, v, keep=None, cnt=None, sig=None, rotary=N
                 raise RuntimeError(f"position ids must be (B,N) = {(b, n)}, got {tuple(pos0.shape)}")
             pos_ids = pos0.to(device=q.device, dtype=torch.int64).expand(b, n).contiguous()
             pos0 = 0
-    q, k, v = q.contiguous(), k.contiguous(), v.contiguous()
+    q, k, v, layout = _input_layout(q, k, v, bnhd, b, h, n, dk, dv)
     o = torch.empty((b, n, h, dv) if merged_heads else (b, h, n, dv), dtype=q.dtype, device=q.device)
     prepared = None
     if want_prepared:
@@ -313,7 +313,7 @@ def causal_dot_product_prepared(q, k, v, keep=None, cnt=None, sig=None, rotary=N
     with _on(q.device):
         head = (q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(),
                 *((t.data_ptr() for t in prepared) if prepared else (None, None, None)),
-                _ptr(keep), _ptr(cnt), _ptr(sig), _ptr(table), _ptr(pos_ids), int(pos0), rdim, rows, int(bool(bnhd)),
+                _ptr(keep), _ptr(cnt), _ptr(sig), _ptr(table), _ptr(pos_ids), int(pos0), rdim, rows, layout,
                 int(bool(merged_heads)))
         ws, ws_ptr = _workspace(_ws_bytes("cott_causal_workspace_bytes", b, h, n, dk, dv, code), q.device)
         tail = (b, h, n, dk, dv, code, ws_ptr, ws.numel() if ws is not None else 0, _stream(q.device))
@@ -366,7 +366,7 @@ def noncausal_dot_product_prepared(q, k, v, keep=None, cnt=None, sig=None, bnhd=
         raise RuntimeError("Q, K and V must have the same dtype")
     code = _dtype_code(q)
     keep, cnt, sig = _prep_side_inputs(b, h, n, keep, cnt, sig, q.device)
-    q, k, v = q.contiguous(), k.contiguous(), v.contiguous()
+    q, k, v, layout = _input_layout(q, k, v, bnhd, b, h, n, dk, dv)
     o = torch.empty((b, n, h, dv) if merged_heads else (b, h, n, dv), dtype=q.dtype, device=q.device)
     prepared = (torch.empty((b, h, n, dk), dtype=q.dtype, device=q.device),
                 torch.empty((b, h, n, dk), dtype=q.dtype, device=q.device),
@@ -374,7 +374,7 @@ def noncausal_dot_product_prepared(q, k, v, keep=None, cnt=None, sig=None, bnhd=
     with _on(q.device):
         rc = _loader.lib().cott_noncausal_fwd_prep(q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(),
                                                    *(t.data_ptr() for t in prepared), _ptr(keep), _ptr(cnt), _ptr(sig),
-                                                   int(bool(bnhd)), int(bool(merged_heads)), b, h, n, dk, dv, code,
+                                                   layout, int(bool(merged_heads)), b, h, n, dk, dv, code,
                                                    _stream(q.device))
     _check(rc, "cott_noncausal_fwd_prep")
     return o, prepared
@@ -694,6 +694,41 @@ def _prep_shapes(q, k, v, bnhd):
     return _shapes(q, k, v)
 
 
+def _token_stride(q, k, v, b, h, n, dk, dv):
+    """Elements from one position to the next when q, k, v are neighbouring column slices, in that order, of one (B,N,H*(2 Dk +
+    Dv)) tensor, as `autograd.InputProjections` hands them out; else 0.  The kernels read that layout as it is."""
+    row = h * (2 * dk + dv)
+    if row % 8 or n * row > 1 << 30 or q.numel() == 0:
+        return 0
+    for t, d in ((q, dk), (k, dk), (v, dv)):
+        for size, have, want in zip((b, n, h, d), t.stride(), (n * row, row, d, 1)):
+            if size != 1 and have != want:
+                return 0
+    size = q.element_size()
+    at = q.data_ptr()
+    if (at % 16 or h * dk * size % 16 or k.data_ptr() != at + h * dk * size or v.data_ptr() != at + 2 * h * dk * size
+            or not q.untyped_storage().data_ptr() == k.untyped_storage().data_ptr() == v.untyped_storage().data_ptr()):
+        return 0
+    return row
+
+
+def preparation_rows(q, k, v, bnhd):
+    """q, k, v as the preparation takes them without a copy of its own: column slices of one tensor as they are (bnhd), anything
+    else contiguous."""
+    if bnhd and q.is_cuda and k.is_cuda and v.is_cuda and q.dtype == k.dtype == v.dtype and not q.is_contiguous():
+        if _token_stride(q, k, v, *_prep_shapes(q, k, v, bnhd)):
+            return q, k, v
+    return q.contiguous(), k.contiguous(), v.contiguous()
+
+
+def _input_layout(q, k, v, bnhd, b, h, n, dk, dv):
+    """(q, k, v, in_bnhd argument of the library)."""
+    stride = _token_stride(q, k, v, b, h, n, dk, dv) if bnhd and not q.is_contiguous() else 0
+    if stride:
+        return q, k, v, stride
+    return q.contiguous(), k.contiguous(), v.contiguous(), int(bool(bnhd))
+
+
 def _rotary_args(rotary, b, n, dk, device, check=True):
     if rotary is None:
         return None, None, 0, 0
@@ -734,13 +769,13 @@ def prepare_inputs(q, k, v, keep=None, cnt=None, sig=None, out_dtype=None, rotar
         raise ValueError("Only float32, float64, float16, and bfloat16 are supported")
     keep, cnt, sig = _prep_side_inputs(b, h, n, keep, cnt, sig, q.device)
     table, pos, rdim, rows = _rotary_args(rotary, b, n, dk, q.device, check_positions)
-    q, k, v = q.contiguous(), k.contiguous(), v.contiguous()
+    q, k, v, layout = _input_layout(q, k, v, bnhd, b, h, n, dk, dv)
     qo, ko = (torch.empty((b, h, n, dk), dtype=out_dtype, device=q.device) for _ in range(2))
     vo = torch.empty((b, h, n, dv), dtype=out_dtype, device=q.device)
     L = _loader.lib()
     with _on(q.device):
         rc = L.cott_prep_ex_fwd(q.data_ptr(), k.data_ptr(), v.data_ptr(), qo.data_ptr(), ko.data_ptr(), vo.data_ptr(),
-                                _ptr(keep), _ptr(cnt), _ptr(sig), _ptr(table), _ptr(pos), rdim, rows, int(bool(bnhd)),
+                                _ptr(keep), _ptr(cnt), _ptr(sig), _ptr(table), _ptr(pos), rdim, rows, layout,
                                 b, h, n, dk, dv, code, _DTYPES[out_dtype], _stream(q.device))
     _check(rc, "cott_prep_ex_fwd")
     return qo, ko, vo
@@ -748,7 +783,7 @@ def prepare_inputs(q, k, v, keep=None, cnt=None, sig=None, out_dtype=None, rotar
 
 def prepare_inputs_backward(q, k, v, gq, gk, gv, keep=None, cnt=None, sig=None, want_dsig=False, rotary=None,
                             bnhd=False, check_positions=True):
-    """Gradients of `prepare_inputs` with respect to q, k, v (their dtype and layout) and, if asked, to sig (H,).
+    """Gradients of `prepare_inputs` with respect to q, k, v (their dtype and layout, slices of one tensor where q, k, v are) and, if asked, to sig (H,).
     gq, gk, gv: gradients with respect to the outputs, (B,H,N,D)."""
     _require_gpu(Q=q, K=k, V=v, gq=gq, gk=gk, gv=gv)
     b, h, n, dk, dv = _prep_shapes(q, k, v, bnhd)
@@ -759,14 +794,19 @@ def prepare_inputs_backward(q, k, v, gq, gk, gv, keep=None, cnt=None, sig=None, 
     code, gcode = _dtype_code(q), _dtype_code(gq)
     keep, cnt, sig = _prep_side_inputs(b, h, n, keep, cnt, sig, q.device)
     table, pos, rdim, rows = _rotary_args(rotary, b, n, dk, q.device, check_positions)
-    q, k, v, gq, gk, gv = (t.contiguous() for t in (q, k, v, gq, gk, gv))
-    dq, dk_, dv_ = torch.empty_like(q), torch.empty_like(k), torch.empty_like(v)
+    q, k, v, layout = _input_layout(q, k, v, bnhd, b, h, n, dk, dv)
+    gq, gk, gv = gq.contiguous(), gk.contiguous(), gv.contiguous()
+    if layout > 1:  # the gradients as column slices of one tensor, too
+        dq, dk_, dv_ = (t.view(b, n, h, d) for t, d in zip(torch.empty((b, n, layout), dtype=q.dtype, device=q.device).split(
+            (h * dk, h * dk, h * dv), dim=-1), (dk, dk, dv)))
+    else:
+        dq, dk_, dv_ = torch.empty_like(q), torch.empty_like(k), torch.empty_like(v)
     drows = torch.empty((b, h, n), dtype=torch.float32, device=q.device) if (want_dsig and sig is not None) else None
     L = _loader.lib()
     with _on(q.device):
         rc = L.cott_prep_ex_bwd(q.data_ptr(), k.data_ptr(), v.data_ptr(), gq.data_ptr(), gk.data_ptr(), gv.data_ptr(),
                                 dq.data_ptr(), dk_.data_ptr(), dv_.data_ptr(), _ptr(drows), _ptr(keep), _ptr(cnt),
-                                _ptr(sig), _ptr(table), _ptr(pos), rdim, rows, int(bool(bnhd)), b, h, n, dk, dv, code,
+                                _ptr(sig), _ptr(table), _ptr(pos), rdim, rows, layout, b, h, n, dk, dv, code,
                                 gcode, _stream(q.device))
     _check(rc, "cott_prep_ex_bwd")
     dsig = drows.sum(dim=(0, 2)) if drows is not None else None

@@ -170,6 +170,8 @@ class PreparedCausalAttention(torch.autograd.Function):
     def forward(ctx, q, k, v, keep, cnt, sig, rot_table=None, first_position=0, bnhd=False, merged_heads=False):
         q, k, v = ops.preparation_rows(q, k, v, bnhd)
         ids = first_position if torch.is_tensor(first_position) else None
+        if ids is not None and bnhd and ids.dim() == 2 and ids.shape == (1, q.shape[1]):
+            ids = ids.expand(q.shape[0], -1).contiguous()  # once, not again in the backward
         rotary = (rot_table, ids if ids is not None else int(first_position)) if rot_table is not None else None
         out, prepared, states = ops.causal_dot_product_prepared(q, k, v, keep, cnt, sig, rotary=rotary, bnhd=bnhd,
                                                                 merged_heads=merged_heads, want_prepared=True,
@@ -279,7 +281,6 @@ class InputProjections(torch.autograd.Function):
         cd = x.dtype
         if x.is_cuda and x.dtype != torch.float64 and torch.is_autocast_enabled("cuda"):
             cd = torch.get_autocast_dtype("cuda")
-        x2 = x.reshape(-1, x.shape[-1]).to(cd)
         weights, biases = wb[0::2], wb[1::2]
         ctx.x_meta = (x.shape, x.dtype)
         ctx.wb_dtypes = [None if t is None else t.dtype for t in wb]
@@ -287,15 +288,24 @@ class InputProjections(torch.autograd.Function):
         ctx.joint = False
         if len(weights) > 1 and weights[0].dtype != cd and x.is_cuda:
             bias_free = biases[0] is None
-            ctx.joint = (all(w.dtype != cd and w.device == x.device for w in weights)
+            ctx.joint = (all(w.dtype != cd and w.device == x.device and w.shape[1] == x.shape[-1] for w in weights)
                          and all((b is None) == bias_free for b in biases))
         if ctx.joint:
+            x2 = x.reshape(-1, x.shape[-1])
             w = torch.empty((sum(ctx.sizes), x2.shape[1]), dtype=cd, device=x.device)
-            for part, own in zip(w.split(ctx.sizes), weights):
-                part.copy_(own)
+            convert = list(zip(weights, w.split(ctx.sizes)))
+            bias = None
+            if not bias_free:
+                bias = torch.empty(sum(ctx.sizes), dtype=cd, device=x.device)
+                convert += zip(biases, bias.split(ctx.sizes))
+            if x2.dtype != cd:
+                convert.append((x2, torch.empty(x2.shape, dtype=cd, device=x.device)))
+                x2 = convert[-1][1]
+            ops.convert_into(convert, cd)
             ctx.save_for_backward(x2, w)
-            y = torch.nn.functional.linear(x2, w, None if bias_free else torch.cat([b.to(cd) for b in biases]))
+            y = torch.nn.functional.linear(x2, w, bias)
             return tuple(part.view(x.shape[:-1] + (n,)) for part, n in zip(y.split(ctx.sizes, dim=1), ctx.sizes))
+        x2 = x.reshape(-1, x.shape[-1]).to(cd)
         ws = [w.to(cd) for w in weights]
         ctx.save_for_backward(x2, *ws)
         outs = []
@@ -322,7 +332,9 @@ class InputProjections(torch.autograd.Function):
                 for g, w in zip(gys[1:], ws[1:]):
                     gx.addmm_(g, w)
             gx = gx.view(shape).to(xdt)
-        column_sum = lambda g: g.sum(0, dtype=torch.promote_types(g.dtype, torch.float32))
+        column_sum = ops.column_sums
+        if torch.is_grad_enabled():  # (likewise)
+            column_sum = lambda g: g.sum(0, dtype=torch.promote_types(g.dtype, torch.float32))
         want_w = [ctx.needs_input_grad[1 + 2 * i] for i in range(len(ctx.sizes))]
         want_b = [t is not None and ctx.needs_input_grad[2 + 2 * i] for i, t in enumerate(ctx.wb_dtypes[1::2])]
         if ctx.joint:

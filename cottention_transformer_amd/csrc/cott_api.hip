@@ -1609,6 +1609,73 @@ int cott_prep_ex_bwd(const void *q, const void *k, const void *v, const void *gq
     return COTT_OK;
 }
 
+int cott_convert(const float *const *src, void *const *dst, const long *n, int count, int dtype, void *stream) {
+    const char *fn = "cott_convert";
+    if (dtype != COTT_BF16 && dtype != COTT_F16) return fail(COTT_ERR_INVALID, "%s: converts to bf16 or fp16", fn);
+    if (count < 0 || count > COTT_CONVERT_MAX) return fail(COTT_ERR_INVALID, "%s: %d arrays (at most %d)", fn, count, COTT_CONVERT_MAX);
+    if (count > 0 && (!src || !dst || !n)) return fail(COTT_ERR_INVALID, "%s: null argument", fn);
+    long total = 0;
+    for (int i = 0; i < count; ++i) {
+        if (n[i] < 0 || n[i] > (1L << 32) || (n[i] > 0 && (!src[i] || !dst[i])))
+            return fail(COTT_ERR_INVALID, "%s: array %d: %ld elements", fn, i, n[i]);
+        if (!aligned16(src[i]) || !aligned16(dst[i])) return fail(COTT_ERR_INVALID, "%s: pointers must be 16-byte aligned", fn);
+        total += n[i];
+    }
+    if (total > (1L << 33)) return fail(COTT_ERR_UNSUPPORTED, "%s: %ld elements exceed 2^33", fn, total);
+    hipError_t e = cott::launch_convert(dtype, src, dst, n, count, static_cast<hipStream_t>(stream));
+    if (e != hipSuccess) return fail(COTT_ERR_HIP, "%s: HIP launch failed: %s", fn, hipGetErrorString(e));
+    return COTT_OK;
+}
+
+int cott_keep_counts(const void *mask, int mask_dtype, unsigned char *keep, float *cnt, int B, int N, int running, void *stream) {
+    const char *fn = "cott_keep_counts";
+    if (mask_dtype != COTT_F32 && mask_dtype != COTT_BF16 && mask_dtype != COTT_F16)
+        return fail(COTT_ERR_INVALID, "%s: mask of dtype %d", fn, mask_dtype);
+    if (B < 0 || N < 0 || N > (1 << 24) || B > (1 << 22)) return fail(COTT_ERR_INVALID, "%s: B = %d, N = %d", fn, B, N);
+    if ((long)B * N == 0) return COTT_OK;
+    if (!mask || !keep || !cnt) return fail(COTT_ERR_INVALID, "%s: null tensor pointer", fn);
+    hipError_t e = cott::launch_keep_counts(mask, (int)elem_size(mask_dtype), keep, cnt, B, N, running != 0,
+                                            static_cast<hipStream_t>(stream));
+    if (e != hipSuccess) return fail(COTT_ERR_HIP, "%s: HIP launch failed: %s", fn, hipGetErrorString(e));
+    return COTT_OK;
+}
+
+int cott_head_sums(const float *rows, float *out, int B, int H, int N, void *stream) {
+    const char *fn = "cott_head_sums";
+    if (B < 0 || H < 0 || N < 0 || H > (1 << 22)) return fail(COTT_ERR_INVALID, "%s: B = %d, H = %d, N = %d", fn, B, H, N);
+    if ((long)B * N >= (1L << 32)) return fail(COTT_ERR_UNSUPPORTED, "%s: B * N = %ld", fn, (long)B * N);
+    if (H == 0) return COTT_OK;
+    if (!out || (!rows && (long)B * N > 0)) return fail(COTT_ERR_INVALID, "%s: null tensor pointer", fn);
+    hipError_t e = cott::launch_head_sums(rows, out, B, H, N, static_cast<hipStream_t>(stream));
+    if (e != hipSuccess) return fail(COTT_ERR_HIP, "%s: HIP launch failed: %s", fn, hipGetErrorString(e));
+    return COTT_OK;
+}
+
+size_t cott_column_sums_workspace_bytes(long rows, int cols) {
+    if (rows <= 0 || cols <= 0) return 0;
+    const int parts = cott::column_sum_parts(rows, cols, device_cus());
+    return parts > 1 ? (size_t)parts * cols * sizeof(float) : 0;
+}
+
+int cott_column_sums(const void *x, float *out, long rows, int cols, long ld, int dtype, void *workspace, size_t workspace_bytes,
+                     void *stream) {
+    const char *fn = "cott_column_sums";
+    if (dtype != COTT_BF16 && dtype != COTT_F16) return fail(COTT_ERR_INVALID, "%s: needs bf16 / fp16", fn);
+    if (rows < 0 || cols < 0 || cols % 8 != 0 || ld % 8 != 0 || ld < cols)
+        return fail(COTT_ERR_INVALID, "%s: %ld x %d, %ld elements between rows", fn, rows, cols, ld);
+    if (cols == 0) return COTT_OK;
+    if (!out || (!x && rows > 0) || !aligned16(x)) return fail(COTT_ERR_INVALID, "%s: null or unaligned pointer", fn);
+    int parts = rows > 0 ? cott::column_sum_parts(rows, cols, device_cus()) : 1;
+    if (workspace == nullptr || workspace_bytes < (size_t)parts * cols * sizeof(float)) {
+        if (parts > 1)
+            return fail(COTT_ERR_WORKSPACE, "%s: workspace of %zu bytes required", fn, (size_t)parts * cols * sizeof(float));
+    }
+    hipError_t e = cott::launch_column_sums(dtype, x, out, rows, cols, ld, parts, static_cast<float *>(workspace),
+                                            static_cast<hipStream_t>(stream));
+    if (e != hipSuccess) return fail(COTT_ERR_HIP, "%s: HIP launch failed: %s", fn, hipGetErrorString(e));
+    return COTT_OK;
+}
+
 int cott_prep_fwd(const void *q, const void *k, const void *v, void *q_out, void *k_out, void *v_out,
                   const unsigned char *keep, const float *cnt, const float *sig, int B, int H, int N, int Dk, int Dv,
                   int in_dtype, int out_dtype, void *stream) {

@@ -195,7 +195,9 @@ class GPTCosAttention(nn.Module):
         if attention_mask is None:
             keep, cnt_all = self._unmasked_side_inputs(b, s, query.device)
         else:
-            keep, cnt_all = _keep_from_additive_mask(attention_mask, b, s, query.device), None
+            # kept keys at positions <= s (:241), together with the mask
+            made = None if self.fast_inference else ops.keep_and_counts(attention_mask, b, s, running=True)
+            keep, cnt_all = made or (_keep_from_additive_mask(attention_mask, b, s, query.device), None)
         sig = self.norm_const.sigmoid().reshape(h)
         table, pos = rotary if rotary is not None else (None, None)
         if self.fast_inference:
@@ -334,9 +336,13 @@ class BertCosAttention(nn.Module):
                                                  torch.full((b, s), float(s), device=query_layer.device))
             keep, cnt = cached[1], cached[2]
         else:
-            keep = _keep_from_additive_mask(attention_mask, b, s, query_layer.device)
-            # (made contiguous here, once, rather than by the forward and again by the backward of the preparation)
-            cnt = keep.sum(-1, keepdim=True).to(torch.float32).expand(b, s).contiguous()
+            made = ops.keep_and_counts(attention_mask, b, s, running=False)
+            if made is not None:
+                keep, cnt = made
+            else:
+                keep = _keep_from_additive_mask(attention_mask, b, s, query_layer.device)
+                # (made contiguous here, once, rather than by the forward and again by the backward of the preparation)
+                cnt = keep.sum(-1, keepdim=True).to(torch.float32).expand(b, s).contiguous()
         dt = _autocast_target(query_layer)
         d = self.attention_head_size
         if (query_layer.dtype == dt and ops.noncausal_fused_preparation_preferred(dt, b, h, s, d, d)

@@ -694,6 +694,62 @@ def _prep_shapes(q, k, v, bnhd):
     return _shapes(q, k, v)
 
 
+_CONVERT_MAX = 8  # COTT_CONVERT_MAX
+
+
+def convert_into(pairs, dtype):
+    """dst.copy_(src) for every (src, dst) of `pairs`, dst contiguous of dtype `dtype`: fp32 sources become bf16 / fp16 in one
+    launch."""
+    pairs = [(src, dst) for src, dst in pairs if src.numel()]
+    if not pairs:
+        return
+    device = pairs[0][0].device
+    if (dtype not in (torch.bfloat16, torch.float16) or len(pairs) > _CONVERT_MAX
+            or any(src.dtype != torch.float32 or src.device != device or not src.is_cuda or not src.is_contiguous()
+                   or (src.data_ptr() | dst.data_ptr()) & 15 or src.numel() > 1 << 30 for src, dst in pairs)):
+        for src, dst in pairs:
+            dst.copy_(src)
+        return
+    n = len(pairs)
+    pointers = ctypes.c_void_p * n
+    with _on(device):
+        rc = _loader.lib().cott_convert(pointers(*(src.data_ptr() for src, _ in pairs)), pointers(*(dst.data_ptr() for _, dst in pairs)),
+                                        (ctypes.c_long * n)(*(src.numel() for src, _ in pairs)), n, _DTYPES[dtype], _stream(device))
+    _check(rc, "cott_convert")
+
+
+def keep_and_counts(mask, b, n, running):
+    """(keep, cnt) of the surrounding model's additive mask with b * n entries, 0 at real tokens: keep (b,n) bool = (mask == 0)
+    and cnt (b,n) fp32, the kept positions up to each one (running) or in its sequence, as one launch; None where the mask is
+    of another kind (its type, strided, on the CPU)."""
+    code = _DTYPES.get(mask.dtype)
+    if (not mask.is_cuda or code is None or code == _loader.F64 or mask.numel() != b * n or not mask.is_contiguous()
+            or n > 1 << 24):
+        return None
+    keep = torch.empty((b, n), dtype=torch.bool, device=mask.device)
+    cnt = torch.empty((b, n), dtype=torch.float32, device=mask.device)
+    with _on(mask.device):
+        rc = _loader.lib().cott_keep_counts(mask.data_ptr(), code, keep.data_ptr(), cnt.data_ptr(), b, n, int(running),
+                                            _stream(mask.device))
+    _check(rc, "cott_keep_counts")
+    return keep, cnt
+
+
+def column_sums(x):
+    """Sums over the rows of x (rows, cols), in fp32 at least."""
+    rows, cols = x.shape
+    if (not x.is_cuda or x.dtype not in (torch.bfloat16, torch.float16) or rows < 2 or cols == 0 or cols % 8 or x.stride(1) != 1
+            or x.stride(0) < cols or x.stride(0) % 8 or x.data_ptr() % 16):
+        return x.sum(0, dtype=torch.promote_types(x.dtype, torch.float32))
+    out = torch.empty(cols, dtype=torch.float32, device=x.device)
+    with _on(x.device):
+        ws, ws_ptr = _workspace(_ws_bytes("cott_column_sums_workspace_bytes", rows, cols), x.device)
+        rc = _loader.lib().cott_column_sums(x.data_ptr(), out.data_ptr(), rows, cols, x.stride(0), _DTYPES[x.dtype], ws_ptr,
+                                            ws.numel() if ws is not None else 0, _stream(x.device))
+    _check(rc, "cott_column_sums")
+    return out
+
+
 def _token_stride(q, k, v, b, h, n, dk, dv):
     """Elements from one position to the next when q, k, v are neighbouring column slices, in that order, of one (B,N,H*(2 Dk +
     Dv)) tensor, as `autograd.InputProjections` hands them out; else 0.  The kernels read that layout as it is."""
@@ -808,6 +864,11 @@ def prepare_inputs_backward(q, k, v, gq, gk, gv, keep=None, cnt=None, sig=None, 
                                 dq.data_ptr(), dk_.data_ptr(), dv_.data_ptr(), _ptr(drows), _ptr(keep), _ptr(cnt),
                                 _ptr(sig), _ptr(table), _ptr(pos), rdim, rows, layout, b, h, n, dk, dv, code,
                                 gcode, _stream(q.device))
-    _check(rc, "cott_prep_ex_bwd")
-    dsig = drows.sum(dim=(0, 2)) if drows is not None else None
+        _check(rc, "cott_prep_ex_bwd")
+        dsig = None
+        if drows is not None and b * n >= 1 << 32:
+            dsig = drows.sum(dim=(0, 2))
+        elif drows is not None:
+            dsig = torch.empty(h, dtype=torch.float32, device=q.device)
+            _check(L.cott_head_sums(drows.data_ptr(), dsig.data_ptr(), b, h, n, _stream(q.device)), "cott_head_sums")
     return dq, dk_, dv_, dsig

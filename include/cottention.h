@@ -294,6 +294,25 @@ COTT_API int cott_prep_ex_bwd(const void *q, const void *k, const void *v,
                      const float *rot_table, const long long *pos, int rotary_dim, int table_rows, int in_bnhd,
                      int B, int H, int N, int Dk, int Dv, int in_dtype, int grad_dtype, void *stream);
 
+/* ---- small passes of an attention block -----------------------------------------------------------------
+ * cott_convert: dst[i] = src[i] rounded to dtype (bf16 / fp16), n[i] elements, for up to COTT_CONVERT_MAX arrays in one launch
+ * (hidden states and weights under autocast); 16-byte aligned pointers.
+ * cott_keep_counts: the additive mask of the surrounding model, (B,N) fp32 (mask_dtype COTT_F32), bf16 or fp16, 0 at real tokens,
+ * as keep (B,N) 0 / 1 = (mask == 0) and cnt (B,N): running != 0: the kept positions up to each one
+ * (GPT_Trainer/GPTCosAttention.py:232, 241), else their number in the sequence (BERT_Trainer/BertCosAttention.py:163-175).
+ * N at most 2^24 (counts are exact in fp32).
+ * cott_head_sums: out (H) = sums of rows (B,H,N) over b and n.
+ * cott_column_sums: out (cols) fp32 = sums over the rows of x (rows, cols) bf16 / fp16 with ld elements between rows; cols and ld
+ * multiples of 8, x 16-byte aligned; workspace of cott_column_sums_workspace_bytes (may be 0). */
+#define COTT_CONVERT_MAX 8
+COTT_API int cott_convert(const float *const *src, void *const *dst, const long *n, int count, int dtype, void *stream);
+COTT_API int cott_keep_counts(const void *mask, int mask_dtype, unsigned char *keep, float *cnt, int B, int N, int running,
+                     void *stream);
+COTT_API int cott_head_sums(const float *rows, float *out, int B, int H, int N, void *stream);
+COTT_API size_t cott_column_sums_workspace_bytes(long rows, int cols);
+COTT_API int cott_column_sums(const void *x, float *out, long rows, int cols, long ld, int dtype, void *workspace,
+                     size_t workspace_bytes, void *stream);
+
 /* ---- causal forward on the RAW projections: the input preparation inside the attention kernel ------------
  *   o = cott_causal_fwd(q_hat, k_hat, v_hat)  with
  *   q_hat = keep * rot(q) / max(|rot(q)|, 1e-12),  k_hat likewise,  v_hat = keep * v / max(cnt^sig[h], 1)

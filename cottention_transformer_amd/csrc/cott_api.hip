@@ -1078,8 +1078,8 @@ int cott_causal_bwd(const void *q, const void *k, const void *v, const void *d_o
 
 int cott_causal_bwd_g16_supported(int B, int H, int N, int Dk, int Dv) {
     if (B < 0 || H < 0 || N < 0 || Dk < 1 || Dv < 1 || (long)B * H > (1L << 22)) return 0;
-    // all three gradients on split operands, with the same padded head dims
-    return use_mfma(COTT_F32, Dk, Dv, N) && cott::mfma_pad(Dk) == cott::mfma_pad(Dv) && cott::f32_terms(Dk, Dv) > 0;
+    // all three gradients on operands of two terms: padded head dims 64 x 64
+    return use_mfma(COTT_F32, Dk, Dv, N) && cott::f32_terms(Dk, Dv) == 2;
 }
 
 int cott_causal_bwd_g16(const float *q, const float *k, const float *v, const void *d_o, float *dq, float *dk, float *dv, int B,
@@ -1088,7 +1088,7 @@ int cott_causal_bwd_g16(const float *q, const float *k, const float *v, const vo
     if (int rc = check_common(fn, B, H, N, Dk, Dv, COTT_F32)) return rc;
     if (int rc = check_common(fn, B, H, N, Dv, Dk, COTT_F32)) return rc;
     if (!cott_causal_bwd_g16_supported(B, H, N, Dk, Dv))
-        return fail(COTT_ERR_UNSUPPORTED, "%s: needs head dims of 48 or 64, or both of 80 to 128 (cott_causal_bwd_g16_supported); convert d_o and use "
+        return fail(COTT_ERR_UNSUPPORTED, "%s: needs head dims of 48 or 64 (cott_causal_bwd_g16_supported); convert d_o and use "
                     "cott_causal_bwd", fn);
     if ((long)B * H * N == 0) return COTT_OK;
     if (!q || !k || !v || !d_o || !dq || !dk || !dv) return fail(COTT_ERR_INVALID, "%s: null tensor pointer", fn);

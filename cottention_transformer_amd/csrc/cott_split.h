@@ -84,7 +84,7 @@ __device__ __forceinline__ u32x2 lds_read_tr16(uint32_t at) {
 }
 
 // One operand of a problem: the rows of one head, fp32, or bf16 (an upstream gradient as the consumer of a bf16 output left
-// it: exact as a hi part, so the tiles are those of the converted tensor).
+// it: exact as a hi part, so the tiles are those of the converted tensor; T = 2 only).
 struct SplitRows {
     rsrc_t rs;
     uint32_t esz;  // bytes per element
@@ -178,7 +178,7 @@ __device__ __forceinline__ void split_loader_role(const SplitRows &rA, const Spl
     }
     auto load_piece = [&](u32x4 *x, const SplitRows &src, uint32_t off) __attribute__((always_inline)) {
         x[0] = buf_load16(src.rs, off);
-        x[1] = buf_load16(src.rs, src.half ? kOobOffset : off + 16u);  // (bf16 rows: the same number of loads in flight)
+        x[1] = buf_load16(src.rs, T == 2 && src.half ? kOobOffset : off + 16u);  // (bf16 rows: as many loads in flight)
     };
     auto load_chunk = [&](int s, int p) __attribute__((always_inline)) {
         const uint32_t row0 = (uint32_t)r.first_row(min(p, r.p1 - 1));
@@ -202,11 +202,7 @@ __device__ __forceinline__ void split_loader_role(const SplitRows &rA, const Spl
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
                 uint32_t q[T];
-                float a = bitcast<float>(x[e >> 1][2 * (e & 1)]), b = bitcast<float>(x[e >> 1][2 * (e & 1) + 1]);
-                if (T == 3 && src.half) {
-                    a = bitcast<float>(x[0][e] << 16);
-                    b = bitcast<float>(x[0][e] & 0xffff0000u);
-                }
+                const float a = bitcast<float>(x[e >> 1][2 * (e & 1)]), b = bitcast<float>(x[e >> 1][2 * (e & 1) + 1]);
                 split_pair<T, decltype(infinite)::value>(a, b, q);
 #pragma unroll
                 for (int y = 0; y < T; ++y) t[y][e] = q[y];

@@ -113,5 +113,29 @@ def lib():
     return _lib
 
 
+_native = None
+
+
+def native():
+    """The native host module (csrc/native.cpp), bound to the loaded library; built first if it is not there.  Its functions
+    answer None for calls they leave to Python."""
+    global _native
+    if _native is None:
+        import importlib.util
+        import torch
+        from . import build as _build
+        handle = lib()
+        if not os.path.exists(_build.NATIVE_PATH):
+            _build.build_native()
+        spec = importlib.util.spec_from_file_location(__package__ + "._native", _build.NATIVE_PATH)
+        module = importlib.util.module_from_spec(spec)
+        spec.loader.exec_module(module)
+        raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None) or (
+            lambda index: torch.cuda.current_stream(index).cuda_stream)
+        module.bind({name: ctypes.cast(getattr(handle, name), _vp).value for name in SIGNATURES}, raw_stream)
+        _native = module
+    return _native
+
+
 def last_error():
     return lib().cott_last_error().decode("utf-8", "replace")

@@ -11,6 +11,7 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 OBJ_DIR = os.path.join(HERE, "build", "obj")
 LIB_PATH = os.path.join(HERE, "lib", "libcottention_hip.so")
+NATIVE_PATH = os.path.join(HERE, "_native.so")
 
 SOURCES = ["cott_api.hip", "cott_mfma_bf16.hip", "cott_mfma_fp16.hip", "cott_mfma_f32.hip", "cott_generic.hip", "cott_wide.hip", "cott_decode_block.hip", "cott_prep.hip", "cott_block.hip", "cott_calib.hip"]
 
@@ -38,8 +39,27 @@ def _compile(src):
     return obj, out
 
 
+def build_native():
+    """Compile the native host module (_native, csrc/native.cpp) against the installed torch."""
+    import sysconfig
+    import torch
+    root = os.path.dirname(torch.__file__)
+    tmp = NATIVE_PATH + ".tmp"
+    cmd = ["g++", "-O2", "-std=c++17", "-shared", "-fPIC", "-fvisibility=hidden",
+           f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+           "-I" + os.path.join(root, "include"), "-I" + os.path.join(root, "include", "torch", "csrc", "api", "include"),
+           "-I" + sysconfig.get_paths()["include"], os.path.join(CSRC, "native.cpp"), "-o", tmp,
+           "-L" + os.path.join(root, "lib"), "-ltorch_python", "-ltorch_cpu", "-lc10"]
+    res = subprocess.run(cmd, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)
+    if res.returncode != 0:
+        raise RuntimeError("g++ failed on native.cpp:\n" + res.stdout)
+    os.replace(tmp, NATIVE_PATH)
+    return NATIVE_PATH
+
+
 def build(verbose=False, jobs=None):
-    """Compile all HIP sources and link the shared library; returns its path."""
+    """Compile all HIP sources and link the shared library, and the native host module; returns the library's path."""
+    build_native()
     os.makedirs(OBJ_DIR, exist_ok=True)
     os.makedirs(os.path.dirname(LIB_PATH), exist_ok=True)
     jobs = jobs or min(len(SOURCES), max(1, (os.cpu_count() or 2) // 2))

@@ -131,6 +131,10 @@ def causal_dot_product(q, k, v, reversed=False, merged_heads=False, into_v=False
     into_v: the result overwrites v and v is returned (inplace=True of Cuda_Kernel/combined_kernel_general.cu
     :403-404).  Where the library allows it (cott_causal_fwd_may_alias_v: the MFMA kernels) the kernels write
     straight into v's memory; otherwise the result is computed beside it and copied.  v must be contiguous."""
+    if not merged_heads and not into_v:
+        o = _loader.native().causal(q, k, v, reversed)
+        if o is not None:
+            return o
     _require_gpu(Q=q, K=k, V=v)
     b, h, n, dk, dv = _shapes(q, k, v)
     if not (q.dtype == k.dtype == v.dtype):
@@ -173,6 +177,9 @@ def causal_dot_product_as(q, k, v, dtype):
     (Cuda_Kernel/combined_kernel_general.cu:377-389).  fp32 tensors computed in bf16 are rounded inside the kernel where that
     is built (cott_causal_fwd_f32in_supported), bit for bit as the conversions round them."""
     if dtype is torch.bfloat16 and q.dtype == k.dtype == v.dtype == torch.float32 and q.is_cuda:
+        o = _loader.native().causal_f32in(q, k, v)
+        if o is not None:
+            return o
         _require_gpu(Q=q, K=k, V=v)
         b, h, n, dk, dv = shape = _shapes(q, k, v)
         ok = _f32in_cache.get(shape)
@@ -215,6 +222,10 @@ def causal_dot_product_saving(q, k, v, merged_heads=False):
     the (B,H,ncuts,slot) fp32 states (in the kernels' tile layout, see include/cottention.h) that causal_backward(..., saved=saved) starts dQ from instead of passing over
     k and v once more (what CustomAttention.forward keeps for backward, Cuda_Kernel/Custom_Kernel.py:16, plus this
     one small tensor).  saved is None where the plan has no cuts.  merged_heads: o as (B,N,H,Dv), see causal_dot_product."""
+    if not merged_heads:
+        pair = _loader.native().causal_saving(q, k, v)
+        if pair is not None:
+            return pair
     _require_gpu(Q=q, K=k, V=v)
     b, h, n, dk, dv = _shapes(q, k, v)
     if not (q.dtype == k.dtype == v.dtype):
@@ -414,6 +425,10 @@ def causal_backward(q, k, v, grad_out, merged_heads=False, saved=None):
     """(dQ, dK, dV) of causal_dot_product(q, k, v) for upstream gradient grad_out ((B,N,H,Dv) with merged_heads).
     saved: the states causal_dot_product_saving() (or causal_dot_product_prepared(save_states=True)) returned for
     the same q, k, v."""
+    if not merged_heads and grad_out.dtype == q.dtype:
+        grads = _loader.native().causal_backward(q, k, v, grad_out, saved)
+        if grads is not None:
+            return grads
     _require_gpu(Q=q, K=k, V=v, prev_grad=grad_out)
     b, h, n, dk, dv = _shapes(q, k, v)
     want = (b, n, h, dv) if merged_heads else tuple(v.shape)
@@ -459,6 +474,9 @@ def causal_backward_from(q, k, v, grad_out):
     kernels read the bf16 gradient as it is, with the results of the converted one."""
     if (grad_out.dtype is torch.bfloat16 and q.dtype == k.dtype == v.dtype == torch.float32 and grad_out.is_cuda
             and tuple(grad_out.shape) == tuple(v.shape)):
+        grads = _loader.native().causal_backward(q, k, v, grad_out, None)
+        if grads is not None:
+            return grads
         _require_gpu(Q=q, K=k, V=v, prev_grad=grad_out)
         b, h, n, dk, dv = shape = _shapes(q, k, v)
         ok = _g16_cache.get(shape)
@@ -481,6 +499,10 @@ def causal_backward_from(q, k, v, grad_out):
 def noncausal_dot_product(q, k, v, merged_heads=False):
     """o = q (k^T v) per (batch, head): BERT_Trainer/BertCosAttention.py:249.  merged_heads: o as (B,N,H,Dv)
     (the context-layer permute of :317 without its copy; see merged_heads_supported)."""
+    if not merged_heads:
+        o = _loader.native().noncausal(q, k, v)
+        if o is not None:
+            return o
     _require_gpu(Q=q, K=k, V=v)
     b, h, n, dk, dv = _shapes(q, k, v)
     if not (q.dtype == k.dtype == v.dtype):
@@ -500,6 +522,10 @@ def noncausal_dot_product(q, k, v, merged_heads=False):
 
 def noncausal_backward(q, k, v, grad_out, merged_heads=False):
     """(dQ, dK, dV) of noncausal_dot_product (grad_out (B,N,H,Dv) with merged_heads)."""
+    if not merged_heads:
+        grads = _loader.native().noncausal_backward(q, k, v, grad_out)
+        if grads is not None:
+            return grads
     _require_gpu(Q=q, K=k, V=v, prev_grad=grad_out)
     b, h, n, dk, dv = _shapes(q, k, v)
     want = (b, n, h, dv) if merged_heads else tuple(v.shape)
@@ -626,6 +652,10 @@ def decode_block(x, wq, wk, wv, wo, state, sig=None, cnt=0.0, rotary=None, norm_
     q, k, v = x wq^T, x wk^T, x wv^T, then decode_step_prepared on them (state (B,H,D,D) fp32, updated in place), then
     the returned y = o wo^T.  x: (B,E) bf16 / fp16; weights (E,E), contiguous and 16-byte aligned, in x's type;
     sig, cnt, rotary, norm_const as in decode_step_prepared."""
+    if sig is None and norm_const is not None and rotary is not None:
+        y = _loader.native().decode_block(x, wq, wk, wv, wo, state, norm_const, float(cnt), rotary[0], int(rotary[1]))
+        if y is not None:
+            return y
     _require_gpu(x=x, wq=wq, wk=wk, wv=wv, wo=wo, state=state)
     dt = x.dtype
     code = _dtype_code(x)

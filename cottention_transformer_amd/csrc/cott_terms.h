@@ -25,7 +25,7 @@ __device__ __forceinline__ uint32_t cut2(float a, float b) {
     if constexpr (std::is_same<TR, Fp16>::value)
         return bitcast<uint32_t>(__builtin_amdgcn_cvt_pkrtz(a, b));
     else
-        return (bitcast<uint32_t>(a) >> 16) | (bitcast<uint32_t>(b) & 0xffff0000u);
+        return __builtin_amdgcn_perm(bitcast<uint32_t>(b), bitcast<uint32_t>(a), 0x07060302u);  // the upper halves
 }
 // fp32 -> three 16-bit numbers of type TR, hi + mid + lo.  Each takes the leading bits of what the ones before it leave: 8
 // of bf16 (3 x 8 = 24, exact wherever the last one is a normal number), 11 of fp16 (exact down to 2^-24).

@@ -18,12 +18,16 @@
 // every product is that of the fp32 number and what is left is the order of the fp32 sums.  fp16: the state is scaled by
 // a power of two per column first, so that neither its largest nor its small entries leave the range, and the scores and
 // C take part as bf16 triples and pairs (C exactly).
-// What bounds it: the chain of chunks, 1.48 us each at DI = 256, and in it the vector instructions of the splits (with two
-// terms, 16 significant bits, it took 1.27 us).  64-column slices rather than 128: twice as many workgroups share the chip,
-// and with few heads workgroups are what is short; the rest of the chip is filled by sequence groups (wide_groups).  B1 H16
-// N1024 D256: forward 31 us, gradients (192 workgroups, whole sequences) 57 us, where the plain-FMA kernel took 18.0 ms for
-// both.  Share of the outputs that are not the 16-bit number nearest to the exact result, same shape: 1.5e-4 (bf16) and
-// 1.2e-3 (fp16), plain-FMA kernel 2.9e-4 and 3.2e-3, two terms 2.4e-3 and 5.5e-3.
+// What bounds it: the chain of chunks, 1.4 us each at DI = 256, and in it the vector instructions of the splits (with two
+// terms, 16 significant bits, it took 1.27 us).  Each contraction step's LDS reads and splits are issued between the matrix
+// instructions of the step before: left to itself the compiler put a step's reads, its splits and its products one after
+// the other (bf16, same results: 16 heads N1024 D256 forward 31.0 -> 30.3 us, gradients 61.5 -> 60.0; 2 heads N4096 38.4 ->
+// 37.2 and 50.5 -> 48.6; 16 heads N1000 D224 29.8 -> 28.6 and 57.5 -> 55.2; fp16 1 %).  64-column slices rather than 128:
+// twice as many workgroups share the chip, and with few heads workgroups are what is short; the rest of the chip is filled
+// by sequence groups (wide_groups).  B1 H16 N1024 D256: forward 30 us, gradients (192 workgroups, whole sequences) 60 us
+// with their passes, where the plain-FMA kernel took 18.0 ms for both.  Share of the outputs that are not the 16-bit number
+// nearest to the exact result, same shape: 1.5e-4 (bf16) and 1.2e-3 (fp16), plain-FMA kernel 2.9e-4 and 3.2e-3, two terms
+// 2.4e-3 and 5.5e-3.
 #pragma once
 #include "cott_mfma.h"
 #include "cott_terms.h"
@@ -286,33 +290,54 @@ __device__ __forceinline__ void wide_compute_role(const WideOp &op, int bh, int 
             for (int q = 0; q < 4; ++q) down[q] = bitcast<float>((uint32_t)(127 - 14 + __shfl(e, 4 * g + q)) << 23);
         }
         f32x4 ah[2] = {zero, zero}, al[2] = {zero, zero};
+        // One contraction step ahead: while the products of step ks are issued, the state rows of step ks + 1 are split and the
+        // operands of that step are on their way from LDS (a matrix instruction and up to six vector ones in turn).
+        u32x4 fa[2][2], fb[2][2], st[2][3];
+        auto read = [&](int ks) __attribute__((always_inline)) {
+#pragma unroll
+            for (int x = 0; x < 2; ++x) {
+                if constexpr (!SUMS) fa[ks & 1][x] = *reinterpret_cast<const u32x4 *>(tA + 16 * x * T::RS + aoff[ks]);
+                // rows of state tile 2ks+x: columns 32ks + 8i + 4x .. +3 of B, i = 0..3
+                fb[ks & 1][x] = cat(lds_read_tr16(tB + boff[ks][0] + 4 * x), lds_read_tr16(tB + boff[ks][1] + 4 * x));
+            }
+        };
+        auto split = [&](int ks) __attribute__((always_inline)) {
+#pragma unroll
+            for (int t = 0; t < 2; ++t)
+#pragma unroll
+                for (int q = 0; q < 2; ++q) {
+                    uint32_t h, mid, lo;
+                    split3<TR>(S[2 * ks + t][2 * q] * up, S[2 * ks + t][2 * q + 1] * up, h, mid, lo);
+                    st[ks & 1][0][2 * t + q] = h;
+                    st[ks & 1][1][2 * t + q] = mid;
+                    st[ks & 1][2][2 * t + q] = lo;
+                }
+        };
+        read(0);
+        if constexpr (!SUMS) split(0);
 #pragma unroll
         for (int ks = 0; ks < KS; ++ks) {
+            __builtin_amdgcn_sched_barrier(0);
+            if (ks + 1 < KS) read(ks + 1);
             if constexpr (!SUMS) {
-                u32x4 sh, sm, sl;
+                if (ks + 1 < KS) split(ks + 1);
 #pragma unroll
-                for (int t = 0; t < 2; ++t)
+                for (int x = 2; x >= 0; --x)
 #pragma unroll
-                    for (int q = 0; q < 2; ++q) {
-                        uint32_t h, mid, lo;
-                        split3<TR>(S[2 * ks + t][2 * q] * up, S[2 * ks + t][2 * q + 1] * up, h, mid, lo);
-                        sh[2 * t + q] = h;
-                        sm[2 * t + q] = mid;
-                        sl[2 * t + q] = lo;
+                    for (int pb = 0; pb < 2; ++pb) {
+                        f32x4 &acc = x == 0 ? ah[pb] : al[pb];
+                        acc = TR::mfma(st[ks & 1][x], fa[ks & 1][pb], acc);
                     }
-#pragma unroll
-                for (int pb = 0; pb < 2; ++pb) {
-                    const u32x4 a = *reinterpret_cast<const u32x4 *>(tA + 16 * pb * T::RS + aoff[ks]);
-                    ah[pb] = TR::mfma(sh, a, ah[pb]);
-                    al[pb] = TR::mfma(sl, a, al[pb]);
-                    al[pb] = TR::mfma(sm, a, al[pb]);
-                }
             }
 #pragma unroll
-            for (int t = 0; t < 2; ++t) {
-                // rows of state tile 2ks+t: columns 32ks + 8i + 4t .. +3 of B, i = 0..3
-                const u32x4 b = cat(lds_read_tr16(tB + boff[ks][0] + 4 * t), lds_read_tr16(tB + boff[ks][1] + 4 * t));
-                S[2 * ks + t] = TR::mfma(b, cu, S[2 * ks + t]);
+            for (int t = 0; t < 2; ++t) S[2 * ks + t] = TR::mfma(fb[ks & 1][t], cu, S[2 * ks + t]);
+            if constexpr (!SUMS) {
+#pragma unroll
+                for (int e = 0; e < 8; ++e) {
+                    __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+                    __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);
+                    __builtin_amdgcn_sched_group_barrier(0x2, 6, 0);
+                }
             }
         }
         if constexpr (!SUMS) {

@@ -378,8 +378,9 @@ SetLayout layout_set(const Op *ops, int n, const int *members, int cnt, long BH,
     L.complement = causal && !L.pair && p.G > 1 && cnt > 1 && any_rev && p.halves == 1 && half;
     // ... and when two of them are X = G(.,B,C), Y = G(.,C,B) with square padded head dims (dK and dV), their
     // states are transposes of each other: the group-state pass computes X's only.
+    const bool split32 = dtype == COTT_F32 && causal && cott::f32_terms(first.di, first.dj) > 0;
     for (int c = 0; c < 8; ++c) L.twin_of[c] = -1;
-    if (causal && !L.pair && p.G > 1 && p.halves == 1 && half && cott::mfma_pad(first.di) == cott::mfma_pad(first.dj))
+    if (causal && !L.pair && p.G > 1 && p.halves == 1 && (half || split32) && cott::mfma_pad(first.di) == cott::mfma_pad(first.dj))
         for (int c = 1; c < cnt; ++c)
             for (int e = 0; e < c && L.twin_of[c] < 0; ++e) {
                 const Op &x = ops[members[e]], &y = ops[members[c]];
@@ -393,7 +394,6 @@ SetLayout layout_set(const Op *ops, int n, const int *members, int cnt, long BH,
     // workgroups on the fullest CU the pass takes about k * (1.15 if k == 2) / pieces of its one-piece time
     // (measured at B1 H16 N65536 D128: 144 workgroups 194 us, 288: 193, 432: 158, 576: 187; 240 -> 480: 84 -> 90).
     // (fp32 ops on split operands have a group-state pass of the same kind, one 80 KiB workgroup per CU)
-    const bool split32 = dtype == COTT_F32 && causal && cott::f32_terms(first.di, first.dj) > 0;
     if (p.G > 1 && (half || split32)) {
         long wgs = 0;
         if (L.pair)

@@ -22,10 +22,14 @@
 // for the matrix pipe.
 // Measured (us, forward / gradients, back to back; before: T = 3 on the fp32 matrix pipe, T = 2 in chunks of 64 positions with
 // one workgroup per CU):
-//   1 x 16 x 2048 x 128    73 / 168 -> 50 / 98       8 x 16 x 1024 x 128   175 / 418 -> 105 / 248
-//   1 x 4 x 8192 x 128     80 / 171 -> 56 / 100      2 x 16 x 1024 x 128 / 64   42 / 102 -> 35 / 81
+//   1 x 16 x 2048 x 128    73 / 168 -> 49 / 88       8 x 16 x 1024 x 128   175 / 418 -> 103 / 246
+//   1 x 4 x 8192 x 128     80 / 171 -> 54 / 96       2 x 16 x 1024 x 128 / 64   42 / 102 -> 33 / 79
 //   1 x 16 x 63 x 128      20 / 20 -> 12 / 12        8 x 16 x 2048 x 64 (T = 2)   67 / 160 -> 64 / 133
-//   1 x 16 x 4096 x 64 (T = 2)   33 / 57 -> 31 / 49
+//   1 x 16 x 4096 x 64 (T = 2)   33 / 57 -> 30 / 45
+// dV's state is the transpose of dK's where the padded dims are square: the sums are formed once and dV's scan reads them
+// transposed, four dwords a tile and lane (gradients of 16 heads N2048 D128 96 -> 88 us, 8 heads N4096 94.5 -> 90, 8 heads N8192
+// D128 / 112 161 -> 155, 16 heads N2048 D64 33 -> 31; before, the sums of all three filled the chip with whole groups, now
+// those of two fill it with halves).
 // The state slots of the group sums use the layout of the 16-bit kernels, so state_prefix_kernel serves both.
 #pragma once
 #include "cott_colscan.h"
@@ -311,6 +315,16 @@ __device__ __forceinline__ void split_compute_role(const ColStateIO &io, float *
 #pragma unroll
             for (int jw = 0; jw < NJW; ++jw) S[it][jw] = gs[slot_at(it, jw)];
     }
+    if (!SUMS && DI == DJ && io.seed_t != nullptr) {  // the twin's slot, transposed: this lane's four rows are four of its columns
+#pragma unroll
+        for (int it = 0; it < NIT; ++it)
+#pragma unroll
+            for (int jw = 0; jw < NJW; ++jw)
+#pragma unroll
+                for (int q = 0; q < 4; ++q)
+                    S[it][jw][q] = io.seed_t[(((NJW * w + jw) * TL::NJT + 2 * (it >> 1) + (g >> 1)) * 64 + 16 * (m >> 2) +
+                                              8 * (g & 1) + 4 * (it & 1) + q) * 4 + (m & 3)];
+    }
     if (!SUMS && io.sin != nullptr) {
 #pragma unroll
         for (int it = 0; it < NIT; ++it)
@@ -578,7 +592,12 @@ __global__ __launch_bounds__(512, T == 2 ? 4 : 2) void split_scan_kernel(Problem
             return;
         }
     } else {
-        if (pr.gstate != nullptr) io.seed = pr.gstate + ((size_t)wi.bh * G + wi.grp) * sub * TL::STATE_FLOATS;
+        const size_t slot = ((size_t)wi.bh * G + wi.grp) * sub * TL::STATE_FLOATS;
+        if (pr.seed_from >= 0) {
+            if (set.p[pr.seed_from].gstate != nullptr) io.seed_t = set.p[pr.seed_from].gstate + slot;
+        } else if (pr.gstate != nullptr) {
+            io.seed = pr.gstate + slot;
+        }
         if (pr.sin != nullptr) io.sin = pr.sin + (size_t)wi.bh * di * pr.lds;
         if (pr.sout != nullptr && wi.grp == G - 1) io.sout = pr.sout + (size_t)wi.bh * di * pr.lds;
         io.lds = pr.lds;

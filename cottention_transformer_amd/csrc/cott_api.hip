@@ -393,7 +393,7 @@ SetLayout layout_set(const Op *ops, int n, const int *members, int cnt, long BH,
     // does not fill the chip, every group is cut into up to four pieces (one workgroup and one slot each).  With k
     // workgroups on the fullest CU the pass takes about k * (1.15 if k == 2) / pieces of its one-piece time
     // (measured at B1 H16 N65536 D128: 144 workgroups 194 us, 288: 193, 432: 158, 576: 187; 240 -> 480: 84 -> 90).
-    // (fp32 ops on split operands have a group-state pass of the same kind, one 80 KiB workgroup per CU)
+    // (fp32 ops on split operands have a group-state pass of the same kind, one workgroup per CU: 96 KiB of LDS at 128 x 128)
     if (p.G > 1 && (half || split32)) {
         long wgs = 0;
         if (L.pair)

@@ -181,10 +181,14 @@ bool pair_eligible(const Op *ops, int n, int dtype, bool causal) {
 //   N768 19.0 / 17.5.
 //   gradients, 16-bit D64: 2 heads N128 10.5 / 4.9; 12 heads N256 12.0 / 6.6, N512 14.5 / 9.5; D32 12 heads N768 10.6 / 8.5;
 //   D128: 2 heads N512 14.0 / 13.1, N768 16.2 / 18.1; 12 heads N768 23.9 / 18.5.
-//   fp32 D64 (two terms, cott_split.h): 2 heads N384 17.7 / 13.7 forward, 21.3 / 14.4 gradients, N512 17.8 / 17.2, 20.7 / 17.7; 16
-//   heads N512 17.5 / 17.6, 20.6 / 18.2, N640 18.3 / 21.2, 20.9 / 21.9; 40 heads N768 20.1 / 24.6, 29.3 / 26.0.
-//   fp32 D128 (three terms): 2 heads N128 24.5 / 17.8, 24.6 / 18.3, N256 24.2 / 29.3; 16 heads N256 25.9 / 29.9, 34.3 / 31.2, N512
-//   30.8 / 53.4; 40 heads D96 N256 32.1 / 30.1, 43.0 / 32.1, N384 33.0 / 41.8; D128 x 64 2 heads N128 18.6 / 13.3, N256 18.2 / 21.6.
+//   fp32 D64 (two terms, cott_split.h), forward: 2 heads N384 17.7 / 13.7, N512 17.8 / 17.2; 16 heads N512 17.5 / 17.6, N640 18.3 /
+//   21.2; 40 heads N768 20.1 / 24.6.  Gradients: 2 heads N320 14.8 / 12.4, N384 14.9 / 14.1, N448 14.9 / 15.9; 8 heads N384 15.5 /
+//   14.5, N512 16.2 / 17.8; 12 heads N448 17.7 / 16.3, N512 18.0 / 18.0, N640 18.6 / 21.2; 16 heads N512 18.7 / 17.8, N640 19.7 /
+//   21.6; 24 heads N640 24.1 / 21.3; 32 heads N768 28.2 / 24.8 (up to 8 chunks whatever the heads: below 12 heads the last two
+//   cost 1 to 2 us of device time and save two launches on the host).
+//   fp32 D128 (three terms), forward: 2 heads N128 24.5 / 17.8, N256 24.2 / 29.3; 16 heads N256 25.9 / 29.9.  Gradients: 2 heads
+//   N192 23.0 / 22.6, N256 23.1 / 28.5; 8 heads N192 25.0 / 23.3, N256 26.2 / 29.1; 16 heads N256 30.8 / 29.5, N320 33.4 / 35.2; 32
+//   heads N320 45.0 / 36.8; D128 x 64 2 heads N192 35.4 / 31.6, 16 heads N256 39.5 / 39.8.
 //   fp32 D32 (fp32 matrix pipe): gradients N128 11.5 / 9.4, N256 11.9 / 16.8; 32 x 128: always cut.
 //   non-causal, 16-bit D64: 2 heads N512 7.9 / 6.6 forward, 8.4 / 8.2 gradients, N768 8.4 / 8.7; 12 heads N768 9.2 / 8.9, 11.3 /
 //   10.7.  D128: 2 heads N256 9.4 / 7.4, 10.2 / 9.7; 12 heads N512 13.0 / 11.7, 17.6 / 16.0; 32 heads N768 18.1 / 16.6 forward.
@@ -202,8 +206,8 @@ int one_group_chunks(long BH, int nops, int di, int dj, int dtype, bool causal) 
     if (dtype == COTT_F32) {
         if (!causal) return 0;
         const int terms = cott::f32_terms(di, dj);
-        if (terms == 2) return nops == 3 && BH >= 32 ? 12 : 8;
-        if (terms == 3) return nops == 3 && BH >= 16 ? 4 : 2;
+        if (terms == 2) return nops == 1 ? 8 : BH >= 32 ? 12 : BH >= 24 ? 10 : 8;
+        if (terms == 3) return nops == 1 ? 2 : BH >= 32 ? 5 : BH >= 16 ? 4 : 3;
         return pi <= 64 && pj <= 64 ? 2 : 0;
     }
     const bool wide = pi > 64 || pj > 64, forward = nops == 1;

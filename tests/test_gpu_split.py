@@ -36,14 +36,18 @@ def test_three_terms_keep_fp32_precision(ct, oracle, case):
 
 # dV starts from the sums of dK's groups, transposed: widths that differ below the same padding, a group or two, many, last ones
 # short.  Two terms: a product misses lo lo and the rounding of both lo, 3 x 2^-18 of it, and the masked scores are split again.
-@pytest.mark.parametrize("case", [(1, 2, 2100, 80, 112), (1, 16, 300, 112, 80), (1, 3, 2100, 48, 64), (2, 4, 1030, 64, 48)],
+# A last block of one position holds gradients of one score: what its products miss is relative to their magnitudes, not their sum.
+@pytest.mark.parametrize("case", [(1, 2, 2100, 80, 112), (1, 16, 300, 112, 80), (1, 3, 2100, 48, 64), (2, 4, 1030, 64, 48),
+                                  (1, 24, 640, 64, 64), (1, 24, 641, 64, 64), (1, 2, 192, 128, 128), (1, 2, 193, 128, 128)],
                          ids=lambda c: "x".join(map(str, c)))
 def test_gradients_of_grouped_sequences(ct, oracle, case):
     q, k, v, do = inputs(*case, F32, seed=case[2])
     bar = 4e-7 if max(case[3:]) > 64 else 6 * 2.0**-18
+    own = [(x[:, :, -1] * y[:, :, -1]).double() for x, y in ((k, q), (v, do))]
+    block = max(float((p.abs().sum(-1) / p.sum(-1).abs()).max()) for p in own) if case[2] % 64 == 1 else 2
     for name, got, ref in zip(("dQ", "dK", "dV"), ct.causal_backward(*(t.to(DEV) for t in (q, k, v, do))),
                               oracle.causal_bwd(q, k, v, do)):
-        assert rel_l2(got, ref) <= bar and worst_block(got, ref) <= 2 * bar, name
+        assert rel_l2(got, ref) <= bar and worst_block(got, ref) <= block * bar, name
 
 
 @pytest.mark.parametrize("n,at", [(70, 40), (300, 100)])  # one group; groups, so that sums and prefixes carry the infinity

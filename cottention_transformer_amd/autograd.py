@@ -229,23 +229,36 @@ class PreparedNonCausalAttention(torch.autograd.Function):
         return dq, dk, dv, None, None, dsig, None, None
 
 
+def _row_pieces(rows, out, inner):
+    """Pieces that the rows of a weight gradient (out, inner) are cut into: until the pieces' 256 x 128 tiles fill the chip (no
+    limit up to 1 M elements), as long as a piece keeps 2048 rows and more than out * inner / 1024, below which forming
+    and adding an fp32 piece costs what the fuller chip gives.  bf16, us in 1 / 2 / 4 / 8 pieces with their sum: 16384 rows x 1024 x
+    1024 104 / 71 / 52 / 48, 2304 x 768 128 / 93 / 98 / 88, 1536 x 1536 153 / 122 / 92 / 108, 3072 x 1024 155 / 128 / 116 / 134, 2048 x
+    2048 162 / 144 / 139 / 161; 8192 rows: 2304 x 768 70 / 58 / 64 / 62, 2048 x 2048 88 / 84 / 87 / 107, 4608 x 1536 129 / 145;
+    4096 rows: 1536 x 1536 47 / 45, 2048 x 2048 52 / 56."""
+    tiles = 0 if out * inner <= 1 << 20 else -(-out // 256) * -(-inner // 128)
+    pieces = 1
+    while (pieces < 16 and tiles * pieces < 256 and rows % (2 * pieces) == 0 and rows // (2 * pieces) >= 2048
+           and rows // (2 * pieces) * 1024 > out * inner):
+        pieces *= 2
+    return pieces
+
+
 def _weight_gradient(gy, x):
     """gy^T x for gy (R, out), x (R, in).  With many rows and a small weight the library's single GEMM fills the
-    chip with too few tiles over a long reduction (out = in = 1024, R = 16384, bf16: 109 us); the rows are cut into
-    pieces multiplied as one batched GEMM and summed in fp32 instead (8 pieces: 47 us).  Weights above 1 M elements (three
-    projections at once) are cut until their 256 x 128 tiles fill the chip (R = 16384: 3072 x 1024 in 1 / 2 / 4 / 8 pieces 163 /
-    132 / 105 / 112 us, 2304 x 768 125 / 88 / 92 / 77; R = 8192: 6144 x 2048 176 / 204)."""
+    chip with too few tiles over a long reduction; the rows are cut into pieces (`_row_pieces`) multiplied as one batched GEMM
+    instead.  The pieces leave it in fp32 and are added in fp32, so the result has the sums of the single GEMM."""
     r = x.shape[0]
     pieces = 1
-    if x.is_cuda and x.dtype in (torch.float16, torch.bfloat16):
-        out, inner = gy.shape[1], x.shape[1]
-        tiles = 0 if out * inner <= 1 << 20 else -(-out // 256) * -(-inner // 128)
-        while pieces < 16 and tiles * pieces < 256 and r % (2 * pieces) == 0 and r // (2 * pieces) >= 2048:
-            pieces *= 2
+    recording = torch.is_grad_enabled()  # the batched product with fp32 results has no derivative
+    if x.is_cuda and x.dtype in (torch.float16, torch.bfloat16) and not (recording and gy.shape[1] * x.shape[1] > 1 << 20):
+        pieces = _row_pieces(r, gy.shape[1], x.shape[1])
     if pieces == 1:
         return gy.t() @ x
-    parts = torch.bmm(gy.view(pieces, r // pieces, -1).transpose(1, 2), x.view(pieces, r // pieces, -1))
-    return parts.sum(0, dtype=torch.float32)
+    a, b = gy.view(pieces, r // pieces, -1).transpose(1, 2), x.view(pieces, r // pieces, -1)
+    if recording:
+        return torch.bmm(a, b).sum(0, dtype=torch.float32)
+    return torch.bmm(a, b, out_dtype=torch.float32).sum(0)
 
 
 def _joined(parts, sizes):

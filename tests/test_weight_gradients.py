@@ -1,0 +1,63 @@
+"""Weight gradients of the projections: which are cut into row pieces, and that cutting keeps the sums of the single GEMM."""
+import pytest
+import torch
+
+DEV = "cuda:0"
+BF, HF = torch.bfloat16, torch.float16
+
+
+def test_row_pieces():
+    """Small weights as far as 2048 rows a piece go; larger ones only where a piece has more rows than its fp32 sum is worth."""
+    from cottention_transformer_amd.autograd import _row_pieces
+    assert [_row_pieces(r, 1024, 1024) for r in (4095, 4096, 8192, 16384, 1 << 16, 6144)] == [1, 2, 4, 8, 16, 2]
+    assert [_row_pieces(r, 3072, 1024) for r in (4096, 8192, 16384, 16383)] == [1, 2, 4, 1]
+    assert [_row_pieces(16384, out, n) for out, n in ((2304, 768), (1536, 1536), (6144, 2048))] == [8, 4, 1]
+    assert [_row_pieces(r, 2048, 2048) for r in (4096, 8192, 16384)] == [1, 1, 2]
+
+
+# single weights of either side of 1 M elements, several pieces; operands as slices of a wider matrix
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [BF, HF])
+@pytest.mark.parametrize("rows,out,inner,wide", [(4096, 64, 128, 64), (8192, 1024, 1024, 1024), (16384, 2048, 2048, 2048), (16384, 3072, 1024, 3072),
+                                                 (8192, 72, 256, 216)])
+def test_pieces_keep_fp32_sums(rows, out, inner, wide, dtype):
+    """Every second piece nearly takes back what the one before it added: a piece rounded to 16 bits would lose the difference
+    (fp16: is infinite).  Sums of R products in fp32 err by at most a few units of 2^-24 sqrt(R) of their magnitude."""
+    from cottention_transformer_amd.autograd import _row_pieces, _weight_gradient
+    pieces = _row_pieces(rows, out, inner)
+    assert pieces > 1
+    g = torch.Generator(device=DEV).manual_seed(rows + out)
+    x = torch.randn(rows, inner, generator=g, device=DEV).abs().to(dtype) * 4
+    gy = torch.randn(rows, wide, generator=g, device=DEV).abs().to(dtype) * 16
+    half = rows // pieces
+    for p in range(1, pieces, 2):
+        x[p * half:(p + 1) * half] = x[(p - 1) * half:p * half]
+        gy[p * half:(p + 1) * half] = -gy[(p - 1) * half:p * half]
+    gy[-1] += 1
+    gy = gy[:, wide - out:]
+    with torch.no_grad():
+        got = _weight_gradient(gy, x)
+    want = gy.double().t() @ x.double()
+    magnitude = gy.double().abs().t() @ x.double().abs()
+    assert got.dtype == torch.float32 and want.abs().max() > 0
+    assert ((got.double() - want).abs() / magnitude).max() <= 4 * 2.0 ** -24 * rows ** 0.5
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("e", [256, 2048])
+def test_gradients_of_16_bit_parameters_are_rounded_once(e):
+    """Parameters in bf16, 8192 and 16384 rows (cut): every gradient is the bf16 number nearest to the sum, but where the sum's own
+    error decides; and with a second derivative to record, products that have one."""
+    from cottention_transformer_amd.autograd import project
+    torch.manual_seed(e)
+    rows = 8192 if e == 256 else 16384
+    lin = torch.nn.Linear(e, e, bias=False, device=DEV, dtype=BF)
+    x = torch.randn(rows, e, device=DEV, dtype=BF, requires_grad=True)
+    y, = project(x, lin)
+    g = torch.randn_like(y)
+    got, = torch.autograd.grad(y, lin.weight, g, retain_graph=True)
+    want = g.double().t() @ x.detach().double()
+    # the share of numbers within the sum's error (about 1e-6 of its magnitude sqrt(R)) of the middle between two bf16 ones
+    assert got.dtype == BF and float((got != want.to(BF)).double().mean()) <= 2e-3
+    again, = torch.autograd.grad(y, lin.weight, g, create_graph=True)
+    assert again.requires_grad and float((again.detach().double() - want).norm() / want.norm()) <= 4e-3

@@ -276,6 +276,14 @@ def _joined(parts, sizes):
     return first.as_strided((rows, total), (total, 1))
 
 
+def _of_column_blocks(f, g, sizes, wanted):
+    """f, whose rows belong to the columns of its argument, of the column blocks of g: of the whole where all are wanted, else of
+    each wanted one by itself (16384 x 3072 x 1024: the weight gradients of all three 107 us, of one 47)."""
+    if all(wanted):
+        return f(g).split(sizes)
+    return [f(part) if want else None for part, want in zip(g.split(sizes, dim=1), wanted)]
+
+
 class InputProjections(torch.autograd.Function):
     """(x, w_0, b_0, w_1, b_1, ...) -> (x w_0^T + b_0, x w_1^T + b_1, ...): the q / k / v projections of an attention
     block (GPT_Trainer/GPTCosAttention.py:443-445, BERT_Trainer/BertCosAttention.py:121,143-144 with biases) as one
@@ -351,8 +359,8 @@ class InputProjections(torch.autograd.Function):
         want_w = [ctx.needs_input_grad[1 + 2 * i] for i in range(len(ctx.sizes))]
         want_b = [t is not None and ctx.needs_input_grad[2 + 2 * i] for i, t in enumerate(ctx.wb_dtypes[1::2])]
         if ctx.joint:
-            gws = _weight_gradient(gys[0], x2).split(ctx.sizes) if any(want_w) else want_w
-            gbs = column_sum(gys[0]).split(ctx.sizes) if any(want_b) else want_b
+            gws = _of_column_blocks(lambda g: _weight_gradient(g, x2), gys[0], ctx.sizes, want_w)
+            gbs = _of_column_blocks(column_sum, gys[0], ctx.sizes, want_b)
         else:
             gws = [_weight_gradient(g, x2) if want else None for g, want in zip(gys, want_w)]
             gbs = [column_sum(g) if want else None for g, want in zip(gys, want_b)]

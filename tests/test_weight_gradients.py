@@ -61,3 +61,32 @@ def test_gradients_of_16_bit_parameters_are_rounded_once(e):
     assert got.dtype == BF and float((got != want.to(BF)).double().mean()) <= 2e-3
     again, = torch.autograd.grad(y, lin.weight, g, create_graph=True)
     assert again.requires_grad and float((again.detach().double() - want).norm() / want.norm()) <= 4e-3
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("trained", [(0,), (1,), (2,), (0, 2), (0, 1, 2), ()])
+def test_frozen_projections_cost_no_gradient(trained, monkeypatch):
+    """Weights and biases of the joint form that need no gradient: no product and no sum of their columns, the others' unchanged."""
+    from cottention_transformer_amd import autograd, ops
+    torch.manual_seed(0)
+    rows, e, sizes = 4096, 128, (128, 64, 192)
+    lins = [torch.nn.Linear(e, n, device=DEV) for n in sizes]
+    x = torch.randn(rows, e, device=DEV)
+    gs = [torch.randn(rows, n, device=DEV, dtype=BF) for n in sizes]
+
+    def gradients():
+        params = [p for lin in lins for p in lin.parameters() if p.requires_grad]
+        with torch.autocast("cuda", dtype=BF):
+            ys = autograd.project(x, *lins)
+        return torch.autograd.grad(ys, params, gs) if params else ()
+    everything = gradients()
+    for i, lin in enumerate(lins):
+        lin.requires_grad_(i in trained)
+    columns = {"w": [], "b": []}
+    product, total = autograd._weight_gradient, ops.column_sums
+    monkeypatch.setattr(autograd, "_weight_gradient", lambda g, x: (columns["w"].append(g.shape[1]), product(g, x))[1])
+    monkeypatch.setattr(ops, "column_sums", lambda g: (columns["b"].append(g.shape[1]), total(g))[1])
+    got = gradients()
+    assert sum(columns["w"]) == sum(columns["b"]) == sum(sizes[i] for i in trained)
+    for a, c in zip(got, [everything[2 * i + j] for i in trained for j in (0, 1)]):
+        assert a.shape == c.shape and float((a - c).norm() / c.norm()) <= 1e-5  # the same fp32 sums in another order

@@ -244,21 +244,30 @@ def _row_pieces(rows, out, inner):
     return pieces
 
 
-def _weight_gradient(gy, x):
-    """gy^T x for gy (R, out), x (R, in).  With many rows and a small weight the library's single GEMM fills the
-    chip with too few tiles over a long reduction; the rows are cut into pieces (`_row_pieces`) multiplied as one batched GEMM
-    instead.  The pieces leave it in fp32 and are added in fp32, so the result has the sums of the single GEMM."""
+def _weight_gradient(gy, x, sizes=None):
+    """gy^T x for gy (R, out), x (R, in), or with `sizes` a list of its blocks of that many rows.  With many rows and a small
+    weight the library's single GEMM fills the chip with too few tiles over a long reduction; the rows are cut into pieces
+    (`_row_pieces`) multiplied as one batched GEMM instead.  The pieces leave it in fp32 and are added in fp32, each block into
+    a tensor of its own, so the result has the sums of the single GEMM."""
     r = x.shape[0]
     pieces = 1
     recording = torch.is_grad_enabled()  # the batched product with fp32 results has no derivative
     if x.is_cuda and x.dtype in (torch.float16, torch.bfloat16) and not (recording and gy.shape[1] * x.shape[1] > 1 << 20):
         pieces = _row_pieces(r, gy.shape[1], x.shape[1])
     if pieces == 1:
-        return gy.t() @ x
+        product = gy.t() @ x
+        return product if sizes is None else product.split(sizes)
     a, b = gy.view(pieces, r // pieces, -1).transpose(1, 2), x.view(pieces, r // pieces, -1)
-    if recording:
-        return torch.bmm(a, b).sum(0, dtype=torch.float32)
-    return torch.bmm(a, b, out_dtype=torch.float32).sum(0)
+    parts = torch.bmm(a, b) if recording else torch.bmm(a, b, out_dtype=torch.float32)
+    if sizes is None:
+        return parts.sum(0, dtype=torch.float32)
+    return [block.sum(0, dtype=torch.float32) for block in parts.split(sizes, dim=1)]
+
+
+def _own(t, dtype):
+    """t as `dtype`, in memory that holds nothing else: a gradient that is kept, saved or dropped by itself."""
+    out = t.to(dtype)
+    return out.clone() if out.untyped_storage().nbytes() != out.numel() * out.element_size() else out
 
 
 def _joined(parts, sizes):
@@ -277,11 +286,11 @@ def _joined(parts, sizes):
 
 
 def _of_column_blocks(f, g, sizes, wanted):
-    """f, whose rows belong to the columns of its argument, of the column blocks of g: of the whole where all are wanted, else of
-    each wanted one by itself (16384 x 3072 x 1024: the weight gradients of all three 107 us, of one 47)."""
+    """What f(g, sizes) makes of each column block of g: of the whole at once where all are wanted, else of each wanted one by
+    itself (16384 x 3072 x 1024: the weight gradients of all three 107 us, of one 47)."""
     if all(wanted):
-        return f(g).split(sizes)
-    return [f(part) if want else None for part, want in zip(g.split(sizes, dim=1), wanted)]
+        return f(g, sizes)
+    return [f(part, [part.shape[1]])[0] if want else None for part, want in zip(g.split(sizes, dim=1), wanted)]
 
 
 class InputProjections(torch.autograd.Function):
@@ -359,15 +368,15 @@ class InputProjections(torch.autograd.Function):
         want_w = [ctx.needs_input_grad[1 + 2 * i] for i in range(len(ctx.sizes))]
         want_b = [t is not None and ctx.needs_input_grad[2 + 2 * i] for i, t in enumerate(ctx.wb_dtypes[1::2])]
         if ctx.joint:
-            gws = _of_column_blocks(lambda g: _weight_gradient(g, x2), gys[0], ctx.sizes, want_w)
-            gbs = _of_column_blocks(column_sum, gys[0], ctx.sizes, want_b)
+            gws = _of_column_blocks(lambda g, sizes: _weight_gradient(g, x2, sizes), gys[0], ctx.sizes, want_w)
+            gbs = _of_column_blocks(lambda g, sizes: column_sum(g).split(sizes), gys[0], ctx.sizes, want_b)
         else:
             gws = [_weight_gradient(g, x2) if want else None for g, want in zip(gys, want_w)]
             gbs = [column_sum(g) if want else None for g, want in zip(gys, want_b)]
         grads = [gx]
         for i in range(len(ctx.sizes)):
-            grads.append(gws[i].to(ctx.wb_dtypes[2 * i]) if want_w[i] else None)
-            grads.append(gbs[i].to(ctx.wb_dtypes[2 * i + 1]) if want_b[i] else None)
+            grads.append(_own(gws[i], ctx.wb_dtypes[2 * i]) if want_w[i] else None)
+            grads.append(_own(gbs[i], ctx.wb_dtypes[2 * i + 1]) if want_b[i] else None)
         return tuple(grads)
 
 

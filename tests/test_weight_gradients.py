@@ -84,9 +84,24 @@ def test_frozen_projections_cost_no_gradient(trained, monkeypatch):
         lin.requires_grad_(i in trained)
     columns = {"w": [], "b": []}
     product, total = autograd._weight_gradient, ops.column_sums
-    monkeypatch.setattr(autograd, "_weight_gradient", lambda g, x: (columns["w"].append(g.shape[1]), product(g, x))[1])
+    monkeypatch.setattr(autograd, "_weight_gradient", lambda g, x, *a: (columns["w"].append(g.shape[1]), product(g, x, *a))[1])
     monkeypatch.setattr(ops, "column_sums", lambda g: (columns["b"].append(g.shape[1]), total(g))[1])
     got = gradients()
     assert sum(columns["w"]) == sum(columns["b"]) == sum(sizes[i] for i in trained)
     for a, c in zip(got, [everything[2 * i + j] for i in trained for j in (0, 1)]):
         assert a.shape == c.shape and float((a - c).norm() / c.norm()) <= 1e-5  # the same fp32 sums in another order
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("rows", [100, 4096])  # one GEMM; row pieces, whose sum is in the parameters' type already
+def test_parameter_gradients_own_their_memory(rows):
+    """.grad of each weight and bias of the joint form holds its own numbers and nothing else."""
+    from cottention_transformer_amd.autograd import project
+    torch.manual_seed(0)
+    lins = [torch.nn.Linear(64, n, device=DEV) for n in (64, 32, 64)]
+    with torch.autocast("cuda", dtype=BF):
+        ys = project(torch.randn(rows, 64, device=DEV), *lins)
+    torch.autograd.backward(ys, [torch.randn_like(y) for y in ys])
+    params = [p for lin in lins for p in lin.parameters()]
+    assert all(p.grad.untyped_storage().nbytes() == 4 * p.numel() and p.grad.is_contiguous() for p in params)
+    assert len({p.grad.untyped_storage().data_ptr() for p in params}) == len(params)

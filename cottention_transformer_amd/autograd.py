@@ -264,9 +264,9 @@ def _weight_gradient(gy, x, sizes=None):
     return [block.sum(0, dtype=torch.float32) for block in parts.split(sizes, dim=1)]
 
 
-def _own(t, dtype):
-    """t as `dtype`, in memory that holds nothing else: a gradient that is kept, saved or dropped by itself."""
-    out = t.to(dtype)
+def own(t, dtype=None):
+    """t as `dtype`, in memory that holds nothing else: for what is kept, saved or dropped by itself."""
+    out = t if dtype is None else t.to(dtype)
     return out.clone() if out.untyped_storage().nbytes() != out.numel() * out.element_size() else out
 
 
@@ -375,8 +375,8 @@ class InputProjections(torch.autograd.Function):
             gbs = [column_sum(g) if want else None for g, want in zip(gys, want_b)]
         grads = [gx]
         for i in range(len(ctx.sizes)):
-            grads.append(_own(gws[i], ctx.wb_dtypes[2 * i]) if want_w[i] else None)
-            grads.append(_own(gbs[i], ctx.wb_dtypes[2 * i + 1]) if want_b[i] else None)
+            grads.append(own(gws[i], ctx.wb_dtypes[2 * i]) if want_w[i] else None)
+            grads.append(own(gbs[i], ctx.wb_dtypes[2 * i + 1]) if want_b[i] else None)
         return tuple(grads)
 
 

@@ -17,7 +17,7 @@ from torch import nn
 from . import ops
 from .autograd import (CustomAttention, CustomAttentionMergedHeads, NonCausalAttention,
                        NonCausalAttentionMergedHeads, PreparedCausalAttention, PreparedNonCausalAttention, PrepareInputs,
-                       _autocast_target, linear_hooks_installed, project)
+                       _autocast_target, linear_hooks_installed, own, project)
 
 
 _DECODE_BLOCK_TYPES = (torch.bfloat16, torch.float16)
@@ -276,6 +276,8 @@ class GPTCosAttention(nn.Module):
                                                        merge_heads=not output_attentions, first_position=first_position)
         else:
             query, key = self._rotate(query, key, position_ids)
+            if use_cache is True and layer_past is None:
+                value = own(value)  # (it outlives the call: without the query and key that may lie beside it)
             key, query, value = key.permute(0, 2, 1, 3), query.permute(0, 2, 1, 3), value.permute(0, 2, 1, 3)
             if layer_past is not None:
                 key = torch.cat((layer_past[0], key), dim=-2)
@@ -316,6 +318,11 @@ class BertCosAttention(nn.Module):
     def transpose_for_scores(self, x):
         return x.view(x.size()[:-1] + (self.num_attention_heads, self.attention_head_size)).permute(0, 2, 1, 3)
 
+    @staticmethod
+    def _cached_layers(key_layer, value_layer):
+        """Key and value as a decoder's caller keeps them, (B,H,S,D), in memory that holds nothing else."""
+        return own(key_layer).permute(0, 2, 1, 3), own(value_layer).permute(0, 2, 1, 3)
+
     def forward(self, hidden_states, attention_mask=None, head_mask=None, encoder_hidden_states=None,
                 encoder_attention_mask=None, past_key_value=None, output_attentions=False):
         if encoder_hidden_states is not None or past_key_value is not None:
@@ -355,7 +362,7 @@ class BertCosAttention(nn.Module):
             context_layer = context_layer.view(context_layer.size()[:-2] + (self.all_head_size,))
             outputs = (context_layer, None) if output_attentions else (context_layer,)
             if self.is_decoder:
-                outputs = outputs + ((key_layer.permute(0, 2, 1, 3), value_layer.permute(0, 2, 1, 3)),)
+                outputs = outputs + (self._cached_layers(key_layer, value_layer),)
             return outputs
         q, k, v = PrepareInputs.apply(query_layer, key_layer, value_layer, keep, cnt, self.norm_const.sigmoid().reshape(h),
                                       dt, None, None, True)
@@ -372,5 +379,5 @@ class BertCosAttention(nn.Module):
         context_layer = context_layer.view(context_layer.size()[:-2] + (self.all_head_size,))
         outputs = (context_layer, None) if output_attentions else (context_layer,)
         if self.is_decoder:
-            outputs = outputs + ((key_layer.permute(0, 2, 1, 3), value_layer.permute(0, 2, 1, 3)),)
+            outputs = outputs + (self._cached_layers(key_layer, value_layer),)
         return outputs

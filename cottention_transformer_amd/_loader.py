@@ -103,7 +103,7 @@ def lib():
         path = lib_path()
         if not os.path.exists(path):
             from . import build as _build
-            _build.build()
+            _build.build_library()
         handle = ctypes.CDLL(path)
         for name, (restype, argtypes) in SIGNATURES.items():
             fn = getattr(handle, name)  # AttributeError here = header and library disagree
@@ -116,24 +116,42 @@ def lib():
 _native = None
 
 
+class _PythonOnly:
+    """Stands in for the native host module where there is none: leaves every call to Python."""
+
+    def __getattr__(self, name):
+        return lambda *args: None
+
+
+def _load_native(handle):
+    import importlib.util
+    import torch
+    from . import build as _build
+    path = _build.native_path()
+    if not os.path.exists(path):
+        _build.build_native()
+    spec = importlib.util.spec_from_file_location(__package__ + "._native", path)
+    module = importlib.util.module_from_spec(spec)
+    spec.loader.exec_module(module)
+    raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None) or (
+        lambda index: torch.cuda.current_stream(index).cuda_stream)
+    module.bind({name: ctypes.cast(getattr(handle, name), _vp).value for name in SIGNATURES}, raw_stream)
+    return module
+
+
 def native():
-    """The native host module (csrc/native.cpp), bound to the loaded library; built first if it is not there.  Its functions
-    answer None for calls they leave to Python."""
+    """The native host module (csrc/native.cpp), bound to the loaded library; built first if there is none for the installed torch.
+    Its functions answer None for calls they leave to Python.  It only shortens the host's part of a call: where it cannot be
+    built or loaded (no compiler, a torch without its headers) a warning says so once and Python takes every call."""
     global _native
     if _native is None:
-        import importlib.util
-        import torch
-        from . import build as _build
         handle = lib()
-        if not os.path.exists(_build.NATIVE_PATH):
-            _build.build_native()
-        spec = importlib.util.spec_from_file_location(__package__ + "._native", _build.NATIVE_PATH)
-        module = importlib.util.module_from_spec(spec)
-        spec.loader.exec_module(module)
-        raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None) or (
-            lambda index: torch.cuda.current_stream(index).cuda_stream)
-        module.bind({name: ctypes.cast(getattr(handle, name), _vp).value for name in SIGNATURES}, raw_stream)
-        _native = module
+        try:
+            _native = _load_native(handle)
+        except Exception as e:
+            import warnings
+            warnings.warn(f"no native host module, calls cost a few microseconds more: {e}", RuntimeWarning, stacklevel=2)
+            _native = _PythonOnly()
     return _native
 
 

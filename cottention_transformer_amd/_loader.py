@@ -27,11 +27,15 @@ SIGNATURES = {
     "cott_noncausal_fwd_prep_supported": (_i, [_i] * 6),
     "cott_noncausal_fwd_prep_preferred": (_i, [_i] * 6),
     "cott_noncausal_fwd_prep": (_i, [_vp] * 10 + [_i] * 8 + [_vp]),
+    "cott_causal_fwd_prep_strided": (_i, [_vp] * 12 + [ctypes.c_longlong] + [_i] * 4 + [_vp] + [_i] * 8 + [_vp, _sz, _vp]),
+    "cott_noncausal_fwd_prep_strided": (_i, [_vp] * 10 + [_i] * 8 + [_vp]),
     "cott_causal_fwd_state": (_i, [_vp] * 6 + [_i] * 6 + [_vp, _sz, _vp]),
     "cott_prep_fwd": (_i, [_vp] * 9 + [_i] * 7 + [_vp]),
     "cott_prep_bwd": (_i, [_vp] * 13 + [_i] * 7 + [_vp]),
     "cott_prep_ex_fwd": (_i, [_vp] * 11 + [_i] * 10 + [_vp]),
     "cott_prep_ex_bwd": (_i, [_vp] * 15 + [_i] * 10 + [_vp]),
+    "cott_prep_strided_fwd": (_i, [_vp] * 11 + [_i] * 10 + [_vp]),
+    "cott_prep_strided_bwd": (_i, [_vp] * 15 + [_i] * 10 + [_vp]),
     "cott_convert": (_i, [_vp, _vp, _vp, _i, _i, _vp]),
     "cott_keep_counts": (_i, [_vp, _i, _vp, _vp, _i, _i, _i, _vp]),
     "cott_head_sums": (_i, [_vp, _vp, _i, _i, _i, _vp]),

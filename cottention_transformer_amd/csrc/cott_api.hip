@@ -641,16 +641,13 @@ int run_ops(const char *fn, bool causal, const Op *ops, int n, long BH, int N, i
     return COTT_OK;
 }
 
-// Input layout argument of the preparation entry points: 0 = (B,H,N,D), other values below H * max(Dk, Dv) = (B,N,H,D), larger
-// ones = (B,N,H,D) with that many elements from one position to the next.  token: 0, 1 or that number.
-int input_layout(const char *fn, int in_bnhd, int H, int N, int Dk, int Dv, bool fused, int *token) {
+// Elements from one position to the next of the q, k, v that the strided preparation entry points take.
+int check_token_stride(const char *fn, int token_stride, int H, int N, int Dk, int Dv, bool fused) {
     const long packed = (long)H * (Dk > Dv ? Dk : Dv);
-    *token = in_bnhd == 0 ? 0 : ((long)in_bnhd <= packed ? 1 : in_bnhd);
-    if (*token > 1 && *token % 8 != 0)
-        return fail(COTT_ERR_INVALID, "%s: %d elements between positions: needs a multiple of 8", fn, *token);
-    const long row = *token > 1 ? (long)*token : packed;
-    if (fused && *token > 0 && (long)N * row > (1L << 30))
-        return fail(COTT_ERR_UNSUPPORTED, "%s: %ld elements of a batch element exceed 2^30", fn, (long)N * row);
+    if (token_stride % 8 != 0 || token_stride < packed)
+        return fail(COTT_ERR_INVALID, "%s: %d elements between positions: needs a multiple of 8, at least %ld", fn, token_stride, packed);
+    if (fused && (long)N * token_stride > (1L << 30))
+        return fail(COTT_ERR_UNSUPPORTED, "%s: %ld elements of a batch element exceed 2^30", fn, (long)N * token_stride);
     return COTT_OK;
 }
 
@@ -817,9 +814,10 @@ int cott_causal_fwd_prep_preferred(int B, int H, int N, int Dk, int Dv, int dtyp
 }
 
 namespace {
+// token: 0 = q, k, v are (B,H,N,D), 1 = (B,N,H,D), above 1 = (B,N,H,D) with that many elements between positions.
 int fwd_prep_impl(const char *fn, const void *q, const void *k, const void *v, void *o, void *q_out, void *k_out,
                   void *v_out, const unsigned char *keep, const float *cnt, const float *sig, const float *rot_table,
-                  const long long *pos_ids, long long pos0, int rotary_dim, int table_rows, int in_bnhd, int o_bnhd, float *saved, int chunks_per_cut,
+                  const long long *pos_ids, long long pos0, int rotary_dim, int table_rows, int token, int o_bnhd, float *saved, int chunks_per_cut,
                   int ncuts, int B, int H, int N, int Dk, int Dv, int dtype, void *workspace, size_t workspace_bytes,
                   void *stream) {
     if (int rc = check_common(fn, B, H, N, Dk, Dv, dtype)) return rc;
@@ -837,7 +835,7 @@ int fwd_prep_impl(const char *fn, const void *q, const void *k, const void *v, v
     if (!cott_causal_fwd_prep_supported(B, H, N, Dk, Dv, dtype, rot_table ? rotary_dim : 0))
         return fail(COTT_ERR_UNSUPPORTED, "%s: the fused preparation is not built for these head dims "
                     "(cott_causal_fwd_prep_supported); prepare the inputs with cott_prep_ex_fwd instead", fn);
-    if (in_bnhd || o_bnhd) {
+    if (token > 0 || o_bnhd) {
         const long dmax = Dk > Dv ? Dk : Dv;
         if ((long)N * H * dmax > (1L << 30))
             return fail(COTT_ERR_UNSUPPORTED, "%s: N*H*D = %ld exceeds 2^30", fn, (long)N * H * dmax);
@@ -848,8 +846,6 @@ int fwd_prep_impl(const char *fn, const void *q, const void *k, const void *v, v
         return fail(COTT_ERR_INVALID, "%s: tensor pointers must be 16-byte aligned", fn);
     if (reinterpret_cast<uintptr_t>(pos_ids) & 7u) return fail(COTT_ERR_INVALID, "%s: position ids must be 8-byte aligned", fn);
     if ((long)N > (1L << 28)) return fail(COTT_ERR_UNSUPPORTED, "%s: N = %d exceeds 2^28", fn, N);
-    int token = 0;
-    if (int rc = input_layout(fn, in_bnhd, H, N, Dk, Dv, true, &token)) return rc;
     Op op{q, k, v, o, Dk, Dv, 0};
     op.H = H;
     if (token > 0) op.lay[0] = op.lay[1] = op.lay[2] = 1;
@@ -888,7 +884,7 @@ int cott_causal_fwd_prep(const void *q, const void *k, const void *v, void *o, v
                          const long long *pos_ids, long long pos0, int rotary_dim, int table_rows, int in_bnhd, int o_bnhd, int B,
                          int H, int N, int Dk, int Dv, int dtype, void *workspace, size_t workspace_bytes, void *stream) {
     return fwd_prep_impl("cott_causal_fwd_prep", q, k, v, o, q_out, k_out, v_out, keep, cnt, sig, rot_table, pos_ids, pos0, rotary_dim,
-                         table_rows, in_bnhd, o_bnhd, nullptr, 0, 0, B, H, N, Dk, Dv, dtype, workspace, workspace_bytes, stream);
+                         table_rows, in_bnhd != 0, o_bnhd, nullptr, 0, 0, B, H, N, Dk, Dv, dtype, workspace, workspace_bytes, stream);
 }
 
 int cott_causal_fwd_prep_save(const void *q, const void *k, const void *v, void *o, void *q_out, void *k_out, void *v_out,
@@ -899,7 +895,19 @@ int cott_causal_fwd_prep_save(const void *q, const void *k, const void *v, void 
     const char *fn = "cott_causal_fwd_prep_save";
     if ((long)B * H * N != 0 && saved == nullptr) return fail(COTT_ERR_INVALID, "%s: null tensor pointer", fn);
     return fwd_prep_impl(fn, q, k, v, o, q_out, k_out, v_out, keep, cnt, sig, rot_table, pos_ids, pos0, rotary_dim, table_rows,
-                         in_bnhd, o_bnhd, saved, chunks_per_cut, ncuts, B, H, N, Dk, Dv, dtype, workspace, workspace_bytes, stream);
+                         in_bnhd != 0, o_bnhd, saved, chunks_per_cut, ncuts, B, H, N, Dk, Dv, dtype, workspace, workspace_bytes, stream);
+}
+
+int cott_causal_fwd_prep_strided(const void *q, const void *k, const void *v, void *o, void *q_out, void *k_out, void *v_out,
+                                 const unsigned char *keep, const float *cnt, const float *sig, const float *rot_table,
+                                 const long long *pos_ids, long long pos0, int rotary_dim, int table_rows, int token_stride, int o_bnhd,
+                                 float *saved, int chunks_per_cut, int ncuts, int B, int H, int N, int Dk, int Dv, int dtype,
+                                 void *workspace, size_t workspace_bytes, void *stream) {
+    const char *fn = "cott_causal_fwd_prep_strided";
+    if (int rc = check_common(fn, B, H, N, Dk, Dv, dtype)) return rc;
+    if (int rc = check_token_stride(fn, token_stride, H, N, Dk, Dv, true)) return rc;
+    return fwd_prep_impl(fn, q, k, v, o, q_out, k_out, v_out, keep, cnt, sig, rot_table, pos_ids, pos0, rotary_dim, table_rows,
+                         token_stride, o_bnhd, saved, chunks_per_cut, ncuts, B, H, N, Dk, Dv, dtype, workspace, workspace_bytes, stream);
 }
 
 int cott_noncausal_fwd_prep_supported(int B, int H, int N, int Dk, int Dv, int dtype) {
@@ -920,10 +928,11 @@ int cott_noncausal_fwd_prep_preferred(int B, int H, int N, int Dk, int Dv, int d
     return !few_heads(p, (long)B * H) || p.nchunks <= few_heads_prep_chunks((long)B * H, Dk, Dv, false);
 }
 
-int cott_noncausal_fwd_prep(const void *q, const void *k, const void *v, void *o, void *q_out, void *k_out, void *v_out,
-                            const unsigned char *keep, const float *cnt, const float *sig, int in_bnhd, int o_bnhd, int B,
-                            int H, int N, int Dk, int Dv, int dtype, void *stream) {
-    const char *fn = "cott_noncausal_fwd_prep";
+namespace {
+// token: as in fwd_prep_impl
+int noncausal_prep_impl(const char *fn, const void *q, const void *k, const void *v, void *o, void *q_out, void *k_out, void *v_out,
+                        const unsigned char *keep, const float *cnt, const float *sig, int token, int o_bnhd, int B, int H, int N,
+                        int Dk, int Dv, int dtype, void *stream) {
     if (int rc = check_common(fn, B, H, N, Dk, Dv, dtype)) return rc;
     if (dtype != COTT_BF16 && dtype != COTT_F16) return fail(COTT_ERR_UNSUPPORTED, "%s: needs bf16 / fp16 tensors", fn);
     if (!use_mfma(dtype, Dk, Dv, N)) return fail(COTT_ERR_UNSUPPORTED, "%s: needs head dims 32..128 in steps of 16", fn);
@@ -936,8 +945,6 @@ int cott_noncausal_fwd_prep(const void *q, const void *k, const void *v, void *o
     if (!aligned16(q) || !aligned16(k) || !aligned16(v) || !aligned16(o) || !aligned16(q_out) || !aligned16(k_out) ||
         !aligned16(v_out))
         return fail(COTT_ERR_INVALID, "%s: tensor pointers must be 16-byte aligned", fn);
-    int token = 0;
-    if (int rc = input_layout(fn, in_bnhd, H, N, Dk, Dv, true, &token)) return rc;
     Op op{q, k, v, o, Dk, Dv, 0};
     op.H = H;
     if (token > 0) op.lay[0] = op.lay[1] = op.lay[2] = 1;
@@ -958,6 +965,23 @@ int cott_noncausal_fwd_prep(const void *q, const void *k, const void *v, void *o
     prep.ko = k_out;
     prep.vo = v_out;
     return run_ops(fn, false, &op, 1, (long)B * H, N, dtype, nullptr, 0, static_cast<hipStream_t>(stream), &prep);
+}
+}  // namespace
+
+int cott_noncausal_fwd_prep(const void *q, const void *k, const void *v, void *o, void *q_out, void *k_out, void *v_out,
+                            const unsigned char *keep, const float *cnt, const float *sig, int in_bnhd, int o_bnhd, int B,
+                            int H, int N, int Dk, int Dv, int dtype, void *stream) {
+    return noncausal_prep_impl("cott_noncausal_fwd_prep", q, k, v, o, q_out, k_out, v_out, keep, cnt, sig, in_bnhd != 0, o_bnhd, B, H, N,
+                               Dk, Dv, dtype, stream);
+}
+
+int cott_noncausal_fwd_prep_strided(const void *q, const void *k, const void *v, void *o, void *q_out, void *k_out, void *v_out,
+                                    const unsigned char *keep, const float *cnt, const float *sig, int token_stride, int o_bnhd,
+                                    int B, int H, int N, int Dk, int Dv, int dtype, void *stream) {
+    const char *fn = "cott_noncausal_fwd_prep_strided";
+    if (int rc = check_common(fn, B, H, N, Dk, Dv, dtype)) return rc;
+    if (int rc = check_token_stride(fn, token_stride, H, N, Dk, Dv, true)) return rc;
+    return noncausal_prep_impl(fn, q, k, v, o, q_out, k_out, v_out, keep, cnt, sig, token_stride, o_bnhd, B, H, N, Dk, Dv, dtype, stream);
 }
 
 namespace {
@@ -1563,13 +1587,12 @@ int check_rotary(const char *fn, const float *table, const long long *pos, int R
     if (rows < 1) return fail(COTT_ERR_INVALID, "%s: empty rotary table", fn);
     return COTT_OK;
 }
-}  // namespace
 
-int cott_prep_ex_fwd(const void *q, const void *k, const void *v, void *q_out, void *k_out, void *v_out,
-                     const unsigned char *keep, const float *cnt, const float *sig, const float *rot_table,
-                     const long long *pos, int rotary_dim, int table_rows, int in_bnhd, int B, int H, int N, int Dk,
-                     int Dv, int in_dtype, int out_dtype, void *stream) {
-    const char *fn = "cott_prep_ex_fwd";
+// token: as in fwd_prep_impl
+int prep_fwd_impl(const char *fn, const void *q, const void *k, const void *v, void *q_out, void *k_out, void *v_out,
+                  const unsigned char *keep, const float *cnt, const float *sig, const float *rot_table, const long long *pos,
+                  int rotary_dim, int table_rows, int token, int B, int H, int N, int Dk, int Dv, int in_dtype, int out_dtype,
+                  void *stream) {
     if (int rc = check_prep(fn, B, H, N, Dk, Dv, in_dtype, out_dtype)) return rc;
     if (int rc = check_rotary(fn, rot_table, pos, rotary_dim, table_rows, Dk)) return rc;
     if ((long)B * H * N == 0) return COTT_OK;
@@ -1577,8 +1600,6 @@ int cott_prep_ex_fwd(const void *q, const void *k, const void *v, void *q_out, v
     if (!aligned16(q) || !aligned16(k) || !aligned16(v) || !aligned16(q_out) || !aligned16(k_out) || !aligned16(v_out))
         return fail(COTT_ERR_INVALID, "%s: tensor pointers must be 16-byte aligned", fn);
     if ((cnt == nullptr) != (sig == nullptr)) return fail(COTT_ERR_INVALID, "%s: cnt and sig go together", fn);
-    int token = 0;
-    if (int rc = input_layout(fn, in_bnhd, H, N, Dk, Dv, false, &token)) return rc;
     const void *x[3] = {q, k, v};
     void *y[3] = {q_out, k_out, v_out};
     hipError_t e = cott::launch_prep(false, x, nullptr, y, keep, cnt, sig, nullptr, B, H, N, Dk, Dv, in_dtype, out_dtype,
@@ -1588,11 +1609,10 @@ int cott_prep_ex_fwd(const void *q, const void *k, const void *v, void *q_out, v
     return COTT_OK;
 }
 
-int cott_prep_ex_bwd(const void *q, const void *k, const void *v, const void *gq, const void *gk, const void *gv,
-                     void *dq, void *dk, void *dv, float *dsig_rows, const unsigned char *keep, const float *cnt,
-                     const float *sig, const float *rot_table, const long long *pos, int rotary_dim, int table_rows,
-                     int in_bnhd, int B, int H, int N, int Dk, int Dv, int in_dtype, int grad_dtype, void *stream) {
-    const char *fn = "cott_prep_ex_bwd";
+int prep_bwd_impl(const char *fn, const void *q, const void *k, const void *v, const void *gq, const void *gk, const void *gv,
+                  void *dq, void *dk, void *dv, float *dsig_rows, const unsigned char *keep, const float *cnt, const float *sig,
+                  const float *rot_table, const long long *pos, int rotary_dim, int table_rows, int token, int B, int H, int N,
+                  int Dk, int Dv, int in_dtype, int grad_dtype, void *stream) {
     if (int rc = check_prep(fn, B, H, N, Dk, Dv, in_dtype, grad_dtype)) return rc;
     if (int rc = check_rotary(fn, rot_table, pos, rotary_dim, table_rows, Dk)) return rc;
     if ((long)B * H * N == 0) return COTT_OK;
@@ -1601,8 +1621,6 @@ int cott_prep_ex_bwd(const void *q, const void *k, const void *v, const void *gq
         !aligned16(dq) || !aligned16(dk) || !aligned16(dv))
         return fail(COTT_ERR_INVALID, "%s: tensor pointers must be 16-byte aligned", fn);
     if ((cnt == nullptr) != (sig == nullptr)) return fail(COTT_ERR_INVALID, "%s: cnt and sig go together", fn);
-    int token = 0;
-    if (int rc = input_layout(fn, in_bnhd, H, N, Dk, Dv, false, &token)) return rc;
     const void *x[3] = {q, k, v};
     const void *g[3] = {gq, gk, gv};
     void *y[3] = {dq, dk, dv};
@@ -1611,6 +1629,45 @@ int cott_prep_ex_bwd(const void *q, const void *k, const void *v, const void *gq
                                      table_rows, static_cast<hipStream_t>(stream));
     if (e != hipSuccess) return fail(COTT_ERR_HIP, "%s: HIP launch failed: %s", fn, hipGetErrorString(e));
     return COTT_OK;
+}
+}  // namespace
+
+int cott_prep_ex_fwd(const void *q, const void *k, const void *v, void *q_out, void *k_out, void *v_out,
+                     const unsigned char *keep, const float *cnt, const float *sig, const float *rot_table,
+                     const long long *pos, int rotary_dim, int table_rows, int in_bnhd, int B, int H, int N, int Dk,
+                     int Dv, int in_dtype, int out_dtype, void *stream) {
+    return prep_fwd_impl("cott_prep_ex_fwd", q, k, v, q_out, k_out, v_out, keep, cnt, sig, rot_table, pos, rotary_dim, table_rows,
+                         in_bnhd != 0, B, H, N, Dk, Dv, in_dtype, out_dtype, stream);
+}
+
+int cott_prep_ex_bwd(const void *q, const void *k, const void *v, const void *gq, const void *gk, const void *gv,
+                     void *dq, void *dk, void *dv, float *dsig_rows, const unsigned char *keep, const float *cnt,
+                     const float *sig, const float *rot_table, const long long *pos, int rotary_dim, int table_rows,
+                     int in_bnhd, int B, int H, int N, int Dk, int Dv, int in_dtype, int grad_dtype, void *stream) {
+    return prep_bwd_impl("cott_prep_ex_bwd", q, k, v, gq, gk, gv, dq, dk, dv, dsig_rows, keep, cnt, sig, rot_table, pos, rotary_dim,
+                         table_rows, in_bnhd != 0, B, H, N, Dk, Dv, in_dtype, grad_dtype, stream);
+}
+
+int cott_prep_strided_fwd(const void *q, const void *k, const void *v, void *q_out, void *k_out, void *v_out,
+                          const unsigned char *keep, const float *cnt, const float *sig, const float *rot_table,
+                          const long long *pos, int rotary_dim, int table_rows, int token_stride, int B, int H, int N, int Dk,
+                          int Dv, int in_dtype, int out_dtype, void *stream) {
+    const char *fn = "cott_prep_strided_fwd";
+    if (int rc = check_prep(fn, B, H, N, Dk, Dv, in_dtype, out_dtype)) return rc;
+    if (int rc = check_token_stride(fn, token_stride, H, N, Dk, Dv, false)) return rc;
+    return prep_fwd_impl(fn, q, k, v, q_out, k_out, v_out, keep, cnt, sig, rot_table, pos, rotary_dim, table_rows, token_stride, B, H, N,
+                         Dk, Dv, in_dtype, out_dtype, stream);
+}
+
+int cott_prep_strided_bwd(const void *q, const void *k, const void *v, const void *gq, const void *gk, const void *gv,
+                          void *dq, void *dk, void *dv, float *dsig_rows, const unsigned char *keep, const float *cnt,
+                          const float *sig, const float *rot_table, const long long *pos, int rotary_dim, int table_rows,
+                          int token_stride, int B, int H, int N, int Dk, int Dv, int in_dtype, int grad_dtype, void *stream) {
+    const char *fn = "cott_prep_strided_bwd";
+    if (int rc = check_prep(fn, B, H, N, Dk, Dv, in_dtype, grad_dtype)) return rc;
+    if (int rc = check_token_stride(fn, token_stride, H, N, Dk, Dv, false)) return rc;
+    return prep_bwd_impl(fn, q, k, v, gq, gk, gv, dq, dk, dv, dsig_rows, keep, cnt, sig, rot_table, pos, rotary_dim, table_rows,
+                         token_stride, B, H, N, Dk, Dv, in_dtype, grad_dtype, stream);
 }
 
 int cott_convert(const float *const *src, void *const *dst, const long *n, int count, int dtype, void *stream) {

@@ -331,6 +331,9 @@ def causal_dot_product_prepared(q, k, v, keep=None, cnt=None, sig=None, rotary=N
         if plan is not None:
             cpc, cuts, slot, _ = plan
             saved = torch.empty((b, h, cuts, slot), dtype=torch.float32, device=q.device)
+        if layout > 1:
+            rc = L.cott_causal_fwd_prep_strided(*head, _ptr(saved), *(plan[:2] if plan is not None else (0, 0)), *tail)
+        elif plan is not None:
             rc = L.cott_causal_fwd_prep_save(*head, saved.data_ptr(), cpc, cuts, *tail)
         else:
             rc = L.cott_causal_fwd_prep(*head, *tail)
@@ -383,10 +386,10 @@ def noncausal_dot_product_prepared(q, k, v, keep=None, cnt=None, sig=None, bnhd=
                 torch.empty((b, h, n, dk), dtype=q.dtype, device=q.device),
                 torch.empty((b, h, n, dv), dtype=q.dtype, device=q.device))
     with _on(q.device):
-        rc = _loader.lib().cott_noncausal_fwd_prep(q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(),
-                                                   *(t.data_ptr() for t in prepared), _ptr(keep), _ptr(cnt), _ptr(sig),
-                                                   layout, int(bool(merged_heads)), b, h, n, dk, dv, code,
-                                                   _stream(q.device))
+        L = _loader.lib()
+        rc = (L.cott_noncausal_fwd_prep_strided if layout > 1 else L.cott_noncausal_fwd_prep)(
+            q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(), *(t.data_ptr() for t in prepared), _ptr(keep), _ptr(cnt), _ptr(sig),
+            layout, int(bool(merged_heads)), b, h, n, dk, dv, code, _stream(q.device))
     _check(rc, "cott_noncausal_fwd_prep")
     return o, prepared
 
@@ -808,7 +811,7 @@ def preparation_rows(q, k, v, bnhd):
 
 
 def _input_layout(q, k, v, bnhd, b, h, n, dk, dv):
-    """(q, k, v, in_bnhd argument of the library)."""
+    """(q, k, v, layout): 0 and 1 are the library's in_bnhd, larger ones the token_stride of its strided forms."""
     stride = _token_stride(q, k, v, b, h, n, dk, dv) if bnhd and not q.is_contiguous() else 0
     if stride:
         return q, k, v, stride
@@ -860,9 +863,9 @@ def prepare_inputs(q, k, v, keep=None, cnt=None, sig=None, out_dtype=None, rotar
     vo = torch.empty((b, h, n, dv), dtype=out_dtype, device=q.device)
     L = _loader.lib()
     with _on(q.device):
-        rc = L.cott_prep_ex_fwd(q.data_ptr(), k.data_ptr(), v.data_ptr(), qo.data_ptr(), ko.data_ptr(), vo.data_ptr(),
-                                _ptr(keep), _ptr(cnt), _ptr(sig), _ptr(table), _ptr(pos), rdim, rows, layout,
-                                b, h, n, dk, dv, code, _DTYPES[out_dtype], _stream(q.device))
+        rc = (L.cott_prep_strided_fwd if layout > 1 else L.cott_prep_ex_fwd)(
+            q.data_ptr(), k.data_ptr(), v.data_ptr(), qo.data_ptr(), ko.data_ptr(), vo.data_ptr(), _ptr(keep), _ptr(cnt), _ptr(sig),
+            _ptr(table), _ptr(pos), rdim, rows, layout, b, h, n, dk, dv, code, _DTYPES[out_dtype], _stream(q.device))
     _check(rc, "cott_prep_ex_fwd")
     return qo, ko, vo
 
@@ -890,10 +893,10 @@ def prepare_inputs_backward(q, k, v, gq, gk, gv, keep=None, cnt=None, sig=None, 
     drows = torch.empty((b, h, n), dtype=torch.float32, device=q.device) if (want_dsig and sig is not None) else None
     L = _loader.lib()
     with _on(q.device):
-        rc = L.cott_prep_ex_bwd(q.data_ptr(), k.data_ptr(), v.data_ptr(), gq.data_ptr(), gk.data_ptr(), gv.data_ptr(),
-                                dq.data_ptr(), dk_.data_ptr(), dv_.data_ptr(), _ptr(drows), _ptr(keep), _ptr(cnt),
-                                _ptr(sig), _ptr(table), _ptr(pos), rdim, rows, layout, b, h, n, dk, dv, code,
-                                gcode, _stream(q.device))
+        rc = (L.cott_prep_strided_bwd if layout > 1 else L.cott_prep_ex_bwd)(
+            q.data_ptr(), k.data_ptr(), v.data_ptr(), gq.data_ptr(), gk.data_ptr(), gv.data_ptr(), dq.data_ptr(), dk_.data_ptr(),
+            dv_.data_ptr(), _ptr(drows), _ptr(keep), _ptr(cnt), _ptr(sig), _ptr(table), _ptr(pos), rdim, rows, layout, b, h, n, dk, dv, code,
+            gcode, _stream(q.device))
         _check(rc, "cott_prep_ex_bwd")
         dsig = None
         if drows is not None and b * n >= 1 << 32:

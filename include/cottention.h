@@ -277,9 +277,8 @@ COTT_API int cott_prep_bwd(const void *q, const void *k, const void *v,
                   int B, int H, int N, int Dk, int Dv, int in_dtype, int grad_dtype, void *stream);
 
 /* The same with the two steps that surround it in the GPT block folded in (GPTCosAttention.py:444-479):
- * in_bnhd != 0: q, k, v (and, backward, dq, dk, dv) are laid out (B,N,H,D), as the projections produce them; a value
- * above H * max(Dk, Dv) is the number of elements from one position to the next, a multiple of 8, of all of them (column
- * slices of one wider tensor, as one GEMM for the three projections leaves them).  (The outputs / incoming gradients stay (B,H,N,D).)  This removes the permute + contiguous copies of :478-479 and
+ * in_bnhd != 0: q, k, v (and, backward, dq, dk, dv) are laid out (B,N,H,D), as the projections produce them
+ * (the outputs / incoming gradients stay (B,H,N,D)), which removes the permute + contiguous copies of :478-479 and
  * Custom_Kernel.py:11-13;  rot_table != NULL: the GPT-J rotary embedding (apply_rotary_pos_emb, :462-476) is
  * applied to the first rotary_dim columns of q and k before normalisation.  rot_table: (table_rows, rotary_dim)
  * fp32, row p = [sin(p f_i) | cos(p f_i)]; pos: (B,N) int64 row index per position; an index outside [0, table_rows) is clamped
@@ -292,6 +291,18 @@ COTT_API int cott_prep_ex_bwd(const void *q, const void *k, const void *v,
                      const void *gq, const void *gk, const void *gv, void *dq, void *dk, void *dv,
                      float *dsig_rows, const unsigned char *keep, const float *cnt, const float *sig,
                      const float *rot_table, const long long *pos, int rotary_dim, int table_rows, int in_bnhd,
+                     int B, int H, int N, int Dk, int Dv, int in_dtype, int grad_dtype, void *stream);
+/* The same on q, k, v (and, backward, dq, dk, dv) that are (B,N,H,D) with token_stride elements from one position to the next
+ * and N * token_stride from one batch element to the next: column slices of one wider tensor, as one GEMM for the three
+ * projections leaves them.  token_stride: a multiple of 8, at least H * max(Dk, Dv). */
+COTT_API int cott_prep_strided_fwd(const void *q, const void *k, const void *v, void *q_out, void *k_out, void *v_out,
+                     const unsigned char *keep, const float *cnt, const float *sig,
+                     const float *rot_table, const long long *pos, int rotary_dim, int table_rows, int token_stride,
+                     int B, int H, int N, int Dk, int Dv, int in_dtype, int out_dtype, void *stream);
+COTT_API int cott_prep_strided_bwd(const void *q, const void *k, const void *v,
+                     const void *gq, const void *gk, const void *gv, void *dq, void *dk, void *dv,
+                     float *dsig_rows, const unsigned char *keep, const float *cnt, const float *sig,
+                     const float *rot_table, const long long *pos, int rotary_dim, int table_rows, int token_stride,
                      int B, int H, int N, int Dk, int Dv, int in_dtype, int grad_dtype, void *stream);
 
 /* ---- small passes of an attention block -----------------------------------------------------------------
@@ -324,7 +335,7 @@ COTT_API int cott_column_sums(const void *x, float *out, long rows, int cols, lo
  * rotary_dim) fp32 as in cott_prep_ex_fwd, rotary_dim a multiple of 8, or NULL; the table row of position s of batch
  * element b is pos_ids[b * N + s] (position_ids of GPT_Trainer/GPTCosAttention.py:458: int64, (B,N), any values) or,
  * with pos_ids NULL, pos0 + s; rows outside the table are clamped to it.  in_bnhd: q, k, v
- * are (B,N,H,D), with its values as in cott_prep_ex_fwd; o_bnhd: o is (B,N,H,Dv).  bf16 / fp16; head dims 32..128 in steps of 16 (with Dk above 64 the value
+ * are (B,N,H,D); o_bnhd: o is (B,N,H,Dv).  bf16 / fp16; head dims 32..128 in steps of 16 (with Dk above 64 the value
  * tiles must be 64 or 128 columns wide after any split into column halves, i.e. Dv above 32 resp. 64):
  * cott_causal_fwd_prep_supported() says (1 / 0) whether a shape qualifies; otherwise the call returns
  * COTT_ERR_UNSUPPORTED and the caller prepares the inputs with cott_prep_ex_fwd.  workspace: as cott_causal_fwd for the
@@ -368,6 +379,21 @@ COTT_API int cott_causal_fwd_prep_save(const void *q, const void *k, const void 
                               float *saved, int chunks_per_cut, int ncuts,
                               int B, int H, int N, int Dk, int Dv, int dtype,
                               void *workspace, size_t workspace_bytes, void *stream);
+/* The causal (saved NULL: no states are written) and the non-causal form on column slices of one tensor: token_stride as in
+ * cott_prep_strided_fwd, N * token_stride at most 2^30. */
+COTT_API int cott_causal_fwd_prep_strided(const void *q, const void *k, const void *v, void *o,
+                              void *q_out, void *k_out, void *v_out,
+                              const unsigned char *keep, const float *cnt, const float *sig,
+                              const float *rot_table, const long long *pos_ids, long long pos0, int rotary_dim,
+                              int table_rows, int token_stride, int o_bnhd,
+                              float *saved, int chunks_per_cut, int ncuts,
+                              int B, int H, int N, int Dk, int Dv, int dtype,
+                              void *workspace, size_t workspace_bytes, void *stream);
+COTT_API int cott_noncausal_fwd_prep_strided(const void *q, const void *k, const void *v, void *o,
+                            void *q_out, void *k_out, void *v_out,
+                            const unsigned char *keep, const float *cnt, const float *sig,
+                            int token_stride, int o_bnhd,
+                            int B, int H, int N, int Dk, int Dv, int dtype, void *stream);
 
 /* ---- per-kernel timing -----------------------------------------------------------------------
  * While enabled, every kernel launch made by the entry points above is bracketed by a pair of HIP

@@ -196,7 +196,9 @@ class GPTCosAttention(nn.Module):
             keep, cnt_all = self._unmasked_side_inputs(b, s, query.device)
         else:
             # kept keys at positions <= s (:241), together with the mask
-            made = None if self.fast_inference else ops.keep_and_counts(attention_mask, b, s, running=True)
+            made = None
+            if not self.fast_inference and ops.keep_and_counts_preferred(b, s, True):
+                made = ops.keep_and_counts(attention_mask, b, s, running=True)
             keep, cnt_all = made or (_keep_from_additive_mask(attention_mask, b, s, query.device), None)
         sig = self.norm_const.sigmoid().reshape(h)
         table, pos = rotary if rotary is not None else (None, None)
@@ -343,7 +345,7 @@ class BertCosAttention(nn.Module):
                                                  torch.full((b, s), float(s), device=query_layer.device))
             keep, cnt = cached[1], cached[2]
         else:
-            made = ops.keep_and_counts(attention_mask, b, s, running=False)
+            made = ops.keep_and_counts(attention_mask, b, s, running=False) if ops.keep_and_counts_preferred(b, s, False) else None
             if made is not None:
                 keep, cnt = made
             else:

@@ -768,6 +768,37 @@ def keep_and_counts(mask, b, n, running):
     return keep, cnt
 
 
+def keep_and_counts_preferred(b, n, running):
+    """Whether keep_and_counts, one workgroup per sequence, is the better form against `mask == 0` and torch's reductions: not for
+    long sequences that are too few to fill the chip.  us, this kernel / torch: running, 1 sequence N 16384 18 / 21, 20000 21 / 21,
+    32768 33 / 21; 2 sequences N 16384 18 / 44, 131072 129 / 298; totals, 1 sequence N 32768 21 / 28, 49152 30 / 27, 64 sequences N
+    65536 43 / 47."""
+    few, longest = (b < 2, 1 << 14) if running else (b < 64, 1 << 15)
+    return not few or n <= longest
+
+
+def head_sums(rows):
+    """Sums of rows (B,H,N) fp32, contiguous, over B and N.  One workgroup per head adds up to 32768 rows; more are added by one
+    workgroup per head and sequence, or piece of a sequence, first (us, 16 heads, in one step / in two, of which 13 host / torch: 8 x
+    2048 5 / - / 8, 32 x 2048 15 / 13 / 17, 64 x 2048 27 / 13 / 13, 64 x 8192 103 / 14 / 18, 256 x 4096 215 / 24 / 28)."""
+    b, h, n = rows.shape
+    if b * n > 1 << 15:
+        pieces = 1
+        while n % (2 * pieces) == 0 and n // (2 * pieces) >= 4096:
+            pieces *= 2
+        if not 512 <= n // pieces <= 1 << 15 or b * h * pieces > 1 << 22:  # too little or too much for one workgroup
+            return rows.sum(dim=(0, 2))
+        return head_sums(_head_sums(rows, 1, b * h * pieces, n // pieces).view(b, h, pieces))
+    return _head_sums(rows, b, h, n)
+
+
+def _head_sums(rows, b, h, n):
+    out = torch.empty(h, dtype=torch.float32, device=rows.device)
+    with _on(rows.device):
+        _check(_loader.lib().cott_head_sums(rows.data_ptr(), out.data_ptr(), b, h, n, _stream(rows.device)), "cott_head_sums")
+    return out
+
+
 def column_sums(x):
     """Sums over the rows of x (rows, cols), in fp32 at least."""
     rows, cols = x.shape
@@ -897,11 +928,6 @@ def prepare_inputs_backward(q, k, v, gq, gk, gv, keep=None, cnt=None, sig=None, 
             q.data_ptr(), k.data_ptr(), v.data_ptr(), gq.data_ptr(), gk.data_ptr(), gv.data_ptr(), dq.data_ptr(), dk_.data_ptr(),
             dv_.data_ptr(), _ptr(drows), _ptr(keep), _ptr(cnt), _ptr(sig), _ptr(table), _ptr(pos), rdim, rows, layout, b, h, n, dk, dv, code,
             gcode, _stream(q.device))
-        _check(rc, "cott_prep_ex_bwd")
-        dsig = None
-        if drows is not None and b * n >= 1 << 32:
-            dsig = drows.sum(dim=(0, 2))
-        elif drows is not None:
-            dsig = torch.empty(h, dtype=torch.float32, device=q.device)
-            _check(L.cott_head_sums(drows.data_ptr(), dsig.data_ptr(), b, h, n, _stream(q.device)), "cott_head_sums")
+    _check(rc, "cott_prep_ex_bwd")
+    dsig = head_sums(drows) if drows is not None else None
     return dq, dk_, dv_, dsig

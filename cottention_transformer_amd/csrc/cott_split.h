@@ -4,9 +4,12 @@
 // is formed from the products of those terms, accumulating in fp32.
 //   T = 2 (padded head dims 64 x 64): x = hi + lo with 16 of the 24 significant bits, a b from three matrix instructions,
 //     rel-L2 of o, dQ, dK, dV against fp64 6.3e-6.
-//   T = 3 (128-wide heads): x = hi + mid + lo holds all 24 bits; the six products down to 2^-16 of a b (what is left out is
-//     2^-24 of it).  Rel-L2 against fp64 1.3e-7 .. 2.0e-7, where the fp32 matrix pipe, which these widths took before, gives
-//     2.4e-7 .. 5.1e-7 (N63 .. N8192, D 80 .. 128, both directions).  That pipe is sixteen times slower than the bf16 one.
+//   T = 3 (128-wide heads): x = hi + mid + lo holds all 24 bits; the six products down to 2^-16 of a b.  What is left out, mid lo
+//     + lo mid, is of either sign and at most 2^-24 of a product of two operands, 1.5 2^-23 of one with the state or a score
+//     (SplitMode).  Rel-L2 against fp64 7.0e-8 .. 2.1e-7, where the fp32 matrix pipe, which these widths took before, gives
+//     1.9e-7 .. 3.7e-7 and terms that are all cut 1.2e-7 .. 2.3e-7 (N63 .. N8192, D 80 .. 128, forward and gradients); every
+//     entry 1.0078, the worst of cut terms, N1 .. N128: at most 4.7e-8, 1.2e-7 and 4.8e-7.  Rounding costs 1 to 3 % of the
+//     times below.  The fp32 pipe is sixteen times slower than the bf16 one.
 // Structure: that of colscan_kernel (cott_colscan.h).
 //   * Four compute wavefronts each own a quarter of the state's columns, all rows, in fp32 accumulators whose row order makes
 //     them the operand of A_c S_c once they are split; they produce those columns of the output.
@@ -22,10 +25,10 @@
 // for the matrix pipe.
 // Measured (us, forward / gradients, back to back; before: T = 3 on the fp32 matrix pipe, T = 2 in chunks of 64 positions with
 // one workgroup per CU):
-//   1 x 16 x 2048 x 128    73 / 168 -> 49 / 88       8 x 16 x 1024 x 128   175 / 418 -> 103 / 246
-//   1 x 4 x 8192 x 128     80 / 171 -> 54 / 96       2 x 16 x 1024 x 128 / 64   42 / 102 -> 33 / 79
-//   1 x 16 x 63 x 128      20 / 20 -> 12 / 12        8 x 16 x 2048 x 64 (T = 2)   67 / 160 -> 64 / 133
-//   1 x 16 x 4096 x 64 (T = 2)   33 / 57 -> 30 / 45
+//   1 x 16 x 2048 x 128    73 / 168 -> 48 / 79       8 x 16 x 1024 x 128   175 / 418 -> 97 / 219
+//   1 x 4 x 8192 x 128     80 / 171 -> 51 / 83       2 x 16 x 1024 x 128 / 64   42 / 102 -> 31 / 74
+//   1 x 16 x 63 x 128      20 / 20 -> 11 / 11        8 x 16 x 2048 x 64 (T = 2)   67 / 160 -> 63 / 132
+//   1 x 16 x 4096 x 64 (T = 2)   33 / 57 -> 27 / 43
 // dV's state is the transpose of dK's where the padded dims are square: the sums are formed once and dV's scan reads them
 // transposed, four dwords a tile and lane (gradients of 16 heads N2048 D128 96 -> 88 us, 8 heads N4096 94.5 -> 90, 8 heads N8192
 // D128 / 112 161 -> 155, 16 heads N2048 D64 33 -> 31; before, the sums of all three filled the chip with whole groups, now
@@ -108,36 +111,44 @@ struct SplitRange {
 };
 
 typedef __attribute__((ext_vector_type(2))) unsigned short u16x2;
-// How two fp32 numbers are split into T packed pairs of bf16 terms (T = 2: rounded, 16 significant bits; T = 3: cut, all 24,
-// with the sign of the number in every term).
-// INFINITE (T = 3): the lower terms, where they are zero, become the smallest normal number of that sign, also those of an
-// infinite number: an infinite factor then meets no exact zero among the other factor's lower terms, and every partial product
-// of inf * x is the infinity that inf * x is (and not a number, from the hi parts, for x = 0).  To finite products that adds
-// 2^-126 of a factor.
-template <int T, bool INFINITE>
-__device__ __forceinline__ void split_pair(float a, float b, uint32_t *t) {
+// How two fp32 numbers are split into T packed pairs of bf16 terms.  T = 2: rounded to nearest, 16 significant bits.  T = 3: the
+// terms hold all 24 bits however they are chosen; what the six products leave out, mid lo + lo mid, is of either sign and
+// below 2^-24 of a product of two rounded numbers, 1.5 2^-23 of a rounded and a cut one (two cut ones: 2^-21, always of the
+// product's sign).  Every product has an operand from memory:
+//   ROUNDED  operands from memory, each term the nearest bf16 number.
+//   CUT      accumulators (state, scores), whose first term must not round up to infinity at the largest numbers.  (Rounding the
+//            second one leaves the error as it is: 1.3e-7 at 1 x 4 x 2048 x 128.)
+//   GUARDED  operand rows with a number whose nearest bf16 number is infinite: all terms cut, with the sign of the number.
+//            `least` 0x0080, for rows with an infinite number: lower terms that are zero become the smallest normal number of that
+//            sign, also those of the infinite number: an infinite factor then meets no exact zero among the other factor's lower
+//            terms, and every partial product of inf * x is the infinity that inf * x is (and not a number, from the hi parts,
+//            for x = 0).  To finite products that adds 2^-126 of a factor.
+enum SplitMode { ROUNDED, CUT, GUARDED };
+template <int T, SplitMode M>
+__device__ __forceinline__ void split_pair(float a, float b, uint32_t *t, unsigned short least = 0) {
 #pragma unroll
     for (int x = 0; x < T; ++x) {
-        if constexpr (T == 2)
+        if ((T == 2 || M == ROUNDED) && x < 2)  // (the third is exact)
             t[x] = Bf16::pack2(a, b);
         else
             t[x] = __builtin_amdgcn_perm(bitcast<uint32_t>(b), bitcast<uint32_t>(a), 0x07060302u);
         if (x + 1 < T) {
-            if constexpr (T == 2) {
+            if constexpr (T == 2 || M == ROUNDED) {
+                asm("" : "+v"(t[x]));  // (else the compiler rounds a once more by itself)
                 a -= bitcast<float>(t[x] << 16);
                 b -= bitcast<float>(t[x] & 0xffff0000u);
             } else {
                 a -= bitcast<float>(bitcast<uint32_t>(a) & 0xffff0000u);
                 b -= bitcast<float>(bitcast<uint32_t>(b) & 0xffff0000u);
-                if (INFINITE && x == 0) {  // (inf - inf: the median of two non-numbers and zero is zero)
+                if (M == GUARDED && x == 0) {  // (inf - inf: the median of two non-numbers and zero is zero)
                     a = __builtin_amdgcn_fmed3f(a, a, 0.f);
                     b = __builtin_amdgcn_fmed3f(b, b, 0.f);
                 }
             }
         }
-        if constexpr (T == 3 && INFINITE) {
+        if constexpr (T == 3 && M == GUARDED) {
             if (x > 0) {
-                const uint32_t some = bitcast<uint32_t>(__builtin_elementwise_max(bitcast<u16x2>(t[x]), u16x2{0x0080, 0x0080}));
+                const uint32_t some = bitcast<uint32_t>(__builtin_elementwise_max(bitcast<u16x2>(t[x]), u16x2{least, least}));
                 t[x] = (some & 0x7fff7fffu) | (t[0] & 0x80008000u);
             }
         }
@@ -147,8 +158,8 @@ __device__ __forceinline__ void split_pair(float a, float b, uint32_t *t) {
 template <int T>
 __device__ __forceinline__ void split_acc(f32x4 v, u32x2 *t) {
     uint32_t a[T], b[T];
-    split_pair<T, false>(v[0], v[1], a);
-    split_pair<T, false>(v[2], v[3], b);
+    split_pair<T, CUT>(v[0], v[1], a);
+    split_pair<T, CUT>(v[2], v[3], b);
 #pragma unroll
     for (int x = 0; x < T; ++x) t[x] = u32x2{a[x], b[x]};
 }
@@ -196,8 +207,9 @@ __device__ __forceinline__ void split_loader_role(const SplitRows &rA, const Spl
         for (int u = 0; u < PJ; ++u) load_piece(rc[s][u], rC, offC[u] + c0);
     };
     // one piece -> its T tiles; largest: the largest magnitude seen so far
-    auto stage_piece = [&](u16 *tile, int term_stride, const u32x4 *x, const SplitRows &src, int at, auto infinite, float &largest)
-                           __attribute__((always_inline)) {
+    auto stage_piece = [&](u16 *tile, int term_stride, const u32x4 *x, const SplitRows &src, int at, auto mode, unsigned short least,
+                           float &largest) __attribute__((always_inline)) {
+        constexpr SplitMode M = decltype(mode)::value;
         u32x4 t[T];
         if (T == 2 && src.half) {
             t[0] = x[0];
@@ -207,37 +219,51 @@ __device__ __forceinline__ void split_loader_role(const SplitRows &rA, const Spl
             for (int e = 0; e < 4; ++e) {
                 uint32_t q[T];
                 const float a = bitcast<float>(x[e >> 1][2 * (e & 1)]), b = bitcast<float>(x[e >> 1][2 * (e & 1) + 1]);
-                split_pair<T, decltype(infinite)::value>(a, b, q);
+                split_pair<T, M>(a, b, q, least);
 #pragma unroll
                 for (int y = 0; y < T; ++y) t[y][e] = q[y];
-                if constexpr (T == 3 && !decltype(infinite)::value)
+                if constexpr (T == 3 && M == ROUNDED)
                     largest = __builtin_fmaxf(__builtin_fmaxf(largest, __builtin_fabsf(a)), __builtin_fabsf(b));
             }
         }
 #pragma unroll
         for (int e = 0; e < T; ++e) *reinterpret_cast<u32x4 *>(tile + e * term_stride + at) = t[e];
     };
-    auto stage_bc = [&](int s, int buf, auto infinite, float &largest) __attribute__((always_inline)) {
+    auto stage_a = [&](int s, int buf, auto mode, float &largest) __attribute__((always_inline)) {
 #pragma unroll
         for (int u = 0; u < PI; ++u)
-            stage_piece(sB + buf * TL::AB, 2 * TL::AB, rb[s][u], rB, SplitTile<DI>::piece(piece_row(u, DI), piece_col(DI)), infinite, largest);
+            stage_piece(sA + buf * TL::AB, 2 * TL::AB, ra[s][u], rA, SplitTile<DI>::piece(piece_row(u, DI), piece_col(DI)), mode, 0, largest);
+    };
+    auto stage_bc = [&](int s, int buf, auto mode, unsigned short least, float &largest) __attribute__((always_inline)) {
+#pragma unroll
+        for (int u = 0; u < PI; ++u)
+            stage_piece(sB + buf * TL::AB, 2 * TL::AB, rb[s][u], rB, SplitTile<DI>::piece(piece_row(u, DI), piece_col(DI)), mode, least, largest);
 #pragma unroll
         for (int u = 0; u < PJ; ++u)
-            stage_piece(sC + buf * TL::C, 2 * TL::C, rc[s][u], rC, SplitTile<DJ>::piece(piece_row(u, DJ), piece_col(DJ)), infinite, largest);
+            stage_piece(sC + buf * TL::C, 2 * TL::C, rc[s][u], rC, SplitTile<DJ>::piece(piece_row(u, DJ), piece_col(DJ)), mode, least, largest);
     };
     auto stage = [&](int s, int buf) __attribute__((always_inline)) {
+        constexpr std::integral_constant<SplitMode, ROUNDED> rounded{};
+        constexpr std::integral_constant<SplitMode, GUARDED> guarded{};
         float largest = 0.f;
-        if constexpr (!SUMS) {
-#pragma unroll
-            for (int u = 0; u < PI; ++u)
-                stage_piece(sA + buf * TL::AB, 2 * TL::AB, ra[s][u], rA, SplitTile<DI>::piece(piece_row(u, DI), piece_col(DI)),
-                            std::false_type{}, largest);
-        }
-        largest = 0.f;  // (infinite entries of A need nothing: they enter outputs only, see add_rest)
-        stage_bc(s, buf, std::false_type{}, largest);
+        if constexpr (!SUMS) stage_a(s, buf, rounded, largest);
+        stage_bc(s, buf, rounded, 0, largest);
         if constexpr (T == 3) {
-            // a row with an infinite entry in B or C (this wavefront holds that row of both): once more
-            if (__any(largest == __builtin_inff())) stage_bc(s, buf, std::true_type{}, largest);
+            // a number that the nearest bf16 one to is infinite (this wavefront holds the same rows of all operands): once more
+            if (__any(largest >= bitcast<float>(0x7f7f8000u))) {
+                if constexpr (!SUMS) stage_a(s, buf, guarded, largest);
+                // (infinite entries of A need nothing else: they enter outputs only, see add_rest)
+                bool inf = false;
+                auto look = [&](const u32x4 *x) __attribute__((always_inline)) {
+#pragma unroll
+                    for (int e = 0; e < 8; ++e) inf |= (x[e >> 2][e & 3] & 0x7fffffffu) == 0x7f800000u;
+                };
+#pragma unroll
+                for (int u = 0; u < PI; ++u) look(rb[s][u]);
+#pragma unroll
+                for (int u = 0; u < PJ; ++u) look(rc[s][u]);
+                stage_bc(s, buf, guarded, __any(inf) ? 0x0080 : 0, largest);
+            }
         }
     };
     // Score tile of this wavefront (0..2): key block kt against position block pb, transposed (a lane holds four
@@ -246,9 +272,11 @@ __device__ __forceinline__ void split_loader_role(const SplitRows &rA, const Spl
     const int dir = pb != kt ? 0 : (r.reversed ? 1 : -1), side = dir * (4 * g - m);
     auto scores = [&](int buf) __attribute__((always_inline)) {
         if (w >= 3) return;
-        f32x4 hi = {0.f, 0.f, 0.f, 0.f}, rest[2] = {hi, hi};
+        // Two accumulators each: half the chain of sums that are cut to fp32.  (From the last columns to the first: the order is free
+        // and decides how nearly cancelling scores round; with this one those that the tests look at by themselves keep to 8e-7.)
+        f32x4 hi[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}}, rest[2] = {hi[0], hi[0]};
 #pragma unroll
-        for (int ks = 0; ks < TL::KS; ++ks) {
+        for (int ks = TL::KS - 1; ks >= 0; --ks) {
             u32x4 a[T], b[T];
 #pragma unroll
             for (int x = 0; x < T; ++x) {
@@ -258,10 +286,11 @@ __device__ __forceinline__ void split_loader_role(const SplitRows &rA, const Spl
 #pragma unroll
             for (int e = 0; e + 1 < SplitPairs<T>::N; ++e)
                 rest[e & 1] = Bf16::mfma(a[SplitPairs<T>::A[e]], b[SplitPairs<T>::B[e]], rest[e & 1]);
-            hi = Bf16::mfma(a[0], b[0], hi);
+            hi[ks & 1] = Bf16::mfma(a[0], b[0], hi[ks & 1]);
         }
-        f32x4 acc = hi + (rest[0] + rest[1]);
-        if (T == 3 && __any(any_nan(acc))) acc = number_or(acc, hi);
+        f32x4 main = hi[0] + hi[1];
+        f32x4 acc = main + (rest[0] + rest[1]);
+        if (T == 3 && __any(any_nan(acc))) acc = number_or(acc, main);
 #pragma unroll
         for (int q = 0; q < 4; ++q) acc[q] = side + dir * q >= 0 ? acc[q] : 0.f;
         u32x2 t[T];

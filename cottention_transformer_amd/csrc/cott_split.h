@@ -272,11 +272,17 @@ __device__ __forceinline__ void split_loader_role(const SplitRows &rA, const Spl
     const int dir = pb != kt ? 0 : (r.reversed ? 1 : -1), side = dir * (4 * g - m);
     auto scores = [&](int buf) __attribute__((always_inline)) {
         if (w >= 3) return;
-        // Two accumulators each: half the chain of sums that are cut to fp32.  (From the last columns to the first: the order is free
-        // and decides how nearly cancelling scores round; with this one those that the tests look at by themselves keep to 8e-7.)
-        f32x4 hi[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}}, rest[2] = {hi[0], hi[0]};
+        // T = 3: two accumulators for the leading products, half the chain of sums that are cut to fp32.  (From the last columns to
+        // the first: the order is free and decides how nearly cancelling scores round; with this one those that the tests look
+        // at by themselves keep to 8e-7.)
+        constexpr int CH = T == 3 ? 2 : 1;
+        const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
+        f32x4 hi[CH], rest[2] = {zero, zero};
 #pragma unroll
-        for (int ks = TL::KS - 1; ks >= 0; --ks) {
+        for (int c = 0; c < CH; ++c) hi[c] = zero;
+#pragma unroll
+        for (int step = 0; step < TL::KS; ++step) {
+            const int ks = T == 3 ? TL::KS - 1 - step : step;
             u32x4 a[T], b[T];
 #pragma unroll
             for (int x = 0; x < T; ++x) {
@@ -286,9 +292,10 @@ __device__ __forceinline__ void split_loader_role(const SplitRows &rA, const Spl
 #pragma unroll
             for (int e = 0; e + 1 < SplitPairs<T>::N; ++e)
                 rest[e & 1] = Bf16::mfma(a[SplitPairs<T>::A[e]], b[SplitPairs<T>::B[e]], rest[e & 1]);
-            hi[ks & 1] = Bf16::mfma(a[0], b[0], hi[ks & 1]);
+            hi[ks % CH] = Bf16::mfma(a[0], b[0], hi[ks % CH]);
         }
-        f32x4 main = hi[0] + hi[1];
+        f32x4 main = hi[0];
+        if constexpr (CH == 2) main += hi[1];
         f32x4 acc = main + (rest[0] + rest[1]);
         if (T == 3 && __any(any_nan(acc))) acc = number_or(acc, main);
 #pragma unroll

@@ -41,6 +41,8 @@ SIGNATURES = {
     "cott_head_sums": (_i, [_vp, _vp, _i, _i, _i, _vp]),
     "cott_column_sums_workspace_bytes": (_sz, [ctypes.c_long, _i]),
     "cott_column_sums": (_i, [_vp, _vp, ctypes.c_long, _i, ctypes.c_long, _i, _vp, _sz, _vp]),
+    "cott_column_sums_blocks": (_i, [_vp, _vp, _vp, _i, ctypes.c_long, ctypes.c_long, _i, _vp, _sz, _vp]),
+    "cott_add_pieces": (_i, [_vp, _vp, _vp, _i, _i, _vp]),
     "cott_causal_fwd_f32in_supported": (_i, [_i] * 5),
     "cott_causal_fwd_f32in": (_i, [_vp] * 4 + [_i] * 5 + [_vp]),
     "cott_causal_fwd_may_alias_v": (_i, [_i] * 6),

@@ -258,10 +258,11 @@ def _weight_gradient(gy, x, sizes=None):
         product = gy.t() @ x
         return product if sizes is None else product.split(sizes)
     a, b = gy.view(pieces, r // pieces, -1).transpose(1, 2), x.view(pieces, r // pieces, -1)
-    parts = torch.bmm(a, b) if recording else torch.bmm(a, b, out_dtype=torch.float32)
-    if sizes is None:
-        return parts.sum(0, dtype=torch.float32)
-    return [block.sum(0, dtype=torch.float32) for block in parts.split(sizes, dim=1)]
+    if recording:
+        sums = torch.bmm(a, b).sum(0, dtype=torch.float32)
+        return sums if sizes is None else sums.split(sizes)
+    blocks = ops.add_pieces(torch.bmm(a, b, out_dtype=torch.float32), [gy.shape[1]] if sizes is None else sizes)
+    return blocks[0] if sizes is None else blocks
 
 
 def own(t, dtype=None):
@@ -362,17 +363,19 @@ class InputProjections(torch.autograd.Function):
                 for g, w in zip(gys[1:], ws[1:]):
                     gx.addmm_(g, w)
             gx = gx.view(shape).to(xdt)
-        column_sum = ops.column_sums
+        column_sums = ops.column_sums
         if torch.is_grad_enabled():  # (likewise)
-            column_sum = lambda g: g.sum(0, dtype=torch.promote_types(g.dtype, torch.float32))
+            def column_sums(g, sizes=None):
+                total = g.sum(0, dtype=torch.promote_types(g.dtype, torch.float32))
+                return total if sizes is None else total.split(sizes)
         want_w = [ctx.needs_input_grad[1 + 2 * i] for i in range(len(ctx.sizes))]
         want_b = [t is not None and ctx.needs_input_grad[2 + 2 * i] for i, t in enumerate(ctx.wb_dtypes[1::2])]
         if ctx.joint:
             gws = _of_column_blocks(lambda g, sizes: _weight_gradient(g, x2, sizes), gys[0], ctx.sizes, want_w)
-            gbs = _of_column_blocks(lambda g, sizes: column_sum(g).split(sizes), gys[0], ctx.sizes, want_b)
+            gbs = _of_column_blocks(column_sums, gys[0], ctx.sizes, want_b)
         else:
             gws = [_weight_gradient(g, x2) if want else None for g, want in zip(gys, want_w)]
-            gbs = [column_sum(g) if want else None for g, want in zip(gys, want_b)]
+            gbs = [column_sums(g) if want else None for g, want in zip(gys, want_b)]
         grads = [gx]
         for i in range(len(ctx.sizes)):
             grads.append(own(gws[i], ctx.wb_dtypes[2 * i]) if want_w[i] else None)

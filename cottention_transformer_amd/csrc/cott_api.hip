@@ -1718,21 +1718,55 @@ size_t cott_column_sums_workspace_bytes(long rows, int cols) {
     return parts > 1 ? (size_t)parts * cols * sizeof(float) : 0;
 }
 
+namespace {
+int check_blocks(const char *fn, float *const *out, const long *n, int count, int multiple, long *total) {
+    *total = 0;
+    if (count < 0 || count > COTT_CONVERT_MAX) return fail(COTT_ERR_INVALID, "%s: %d arrays (at most %d)", fn, count, COTT_CONVERT_MAX);
+    if (count > 0 && (!out || !n)) return fail(COTT_ERR_INVALID, "%s: null argument", fn);
+    for (int i = 0; i < count; ++i) {
+        if (n[i] < 0 || n[i] % multiple != 0 || n[i] > (1L << 31) || (n[i] > 0 && !out[i]))
+            return fail(COTT_ERR_INVALID, "%s: array %d: %ld elements (a multiple of %d)", fn, i, n[i], multiple);
+        *total += n[i];
+    }
+    return COTT_OK;
+}
+}  // namespace
+
+int cott_column_sums_blocks(const void *x, float *const *out, const long *n, int count, long rows, long ld, int dtype, void *workspace,
+                            size_t workspace_bytes, void *stream) {
+    const char *fn = "cott_column_sums";
+    long cols = 0;
+    if (dtype != COTT_BF16 && dtype != COTT_F16) return fail(COTT_ERR_INVALID, "%s: needs bf16 / fp16", fn);
+    if (int rc = check_blocks(fn, out, n, count, 8, &cols)) return rc;
+    if (rows < 0 || ld % 8 != 0 || ld < cols || cols > (1L << 30))
+        return fail(COTT_ERR_INVALID, "%s: %ld x %ld, %ld elements between rows", fn, rows, cols, ld);
+    if (cols == 0) return COTT_OK;
+    if ((!x && rows > 0) || !aligned16(x)) return fail(COTT_ERR_INVALID, "%s: null or unaligned pointer", fn);
+    const int parts = rows > 0 ? cott::column_sum_parts(rows, (int)cols, device_cus()) : 1;
+    if (parts > 1 && (workspace == nullptr || workspace_bytes < (size_t)parts * cols * sizeof(float)))
+        return fail(COTT_ERR_WORKSPACE, "%s: workspace of %zu bytes required", fn, (size_t)parts * cols * sizeof(float));
+    hipError_t e = cott::launch_column_sums(dtype, x, out, n, count, rows, (int)cols, ld, parts, static_cast<float *>(workspace),
+                                            static_cast<hipStream_t>(stream));
+    if (e != hipSuccess) return fail(COTT_ERR_HIP, "%s: HIP launch failed: %s", fn, hipGetErrorString(e));
+    return COTT_OK;
+}
+
 int cott_column_sums(const void *x, float *out, long rows, int cols, long ld, int dtype, void *workspace, size_t workspace_bytes,
                      void *stream) {
-    const char *fn = "cott_column_sums";
-    if (dtype != COTT_BF16 && dtype != COTT_F16) return fail(COTT_ERR_INVALID, "%s: needs bf16 / fp16", fn);
-    if (rows < 0 || cols < 0 || cols % 8 != 0 || ld % 8 != 0 || ld < cols)
-        return fail(COTT_ERR_INVALID, "%s: %ld x %d, %ld elements between rows", fn, rows, cols, ld);
-    if (cols == 0) return COTT_OK;
-    if (!out || (!x && rows > 0) || !aligned16(x)) return fail(COTT_ERR_INVALID, "%s: null or unaligned pointer", fn);
-    int parts = rows > 0 ? cott::column_sum_parts(rows, cols, device_cus()) : 1;
-    if (workspace == nullptr || workspace_bytes < (size_t)parts * cols * sizeof(float)) {
-        if (parts > 1)
-            return fail(COTT_ERR_WORKSPACE, "%s: workspace of %zu bytes required", fn, (size_t)parts * cols * sizeof(float));
-    }
-    hipError_t e = cott::launch_column_sums(dtype, x, out, rows, cols, ld, parts, static_cast<float *>(workspace),
-                                            static_cast<hipStream_t>(stream));
+    const long n = cols;
+    return cott_column_sums_blocks(x, &out, &n, 1, rows, ld, dtype, workspace, workspace_bytes, stream);
+}
+
+int cott_add_pieces(const float *parts, float *const *out, const long *n, int count, int pieces, void *stream) {
+    const char *fn = "cott_add_pieces";
+    long total = 0;
+    if (int rc = check_blocks(fn, out, n, count, 4, &total)) return rc;
+    if (pieces < 1) return fail(COTT_ERR_INVALID, "%s: %d pieces", fn, pieces);
+    if (total == 0) return COTT_OK;
+    bool aligned = parts != nullptr && aligned16(parts);
+    for (int i = 0; i < count; ++i) aligned = aligned && aligned16(out[i]);
+    if (!aligned) return fail(COTT_ERR_INVALID, "%s: null or unaligned pointer", fn);
+    hipError_t e = cott::launch_add_pieces(parts, out, n, count, pieces, static_cast<hipStream_t>(stream));
     if (e != hipSuccess) return fail(COTT_ERR_HIP, "%s: HIP launch failed: %s", fn, hipGetErrorString(e));
     return COTT_OK;
 }

@@ -132,14 +132,15 @@ hipError_t launch_prep(bool backward, const void *const x[3], const void *const 
 
 // The small passes of a block, see cott_block.hip.  convert: fp32 -> 16-bit arrays, 16-byte aligned; keep_counts: `bytes` per mask
 // entry, 4 (fp32) or 2 (bf16 / fp16); column_sums: cols and ld multiples of 8, x 16-byte aligned, ws of parts * cols floats
-// (parts > 1).
+// (parts > 1); add_pieces: all sizes multiples of 4, 16-byte aligned.  Their sums go to `count` arrays of n[i] one after the other.
 hipError_t launch_convert(int dtype, const float *const *src, void *const *dst, const long *n, int count, hipStream_t stream);
 hipError_t launch_keep_counts(const void *mask, int bytes, unsigned char *keep, float *cnt, int B, int N, bool running,
                               hipStream_t stream);
 hipError_t launch_head_sums(const float *rows, float *out, int B, int H, int N, hipStream_t stream);
 int column_sum_parts(long rows, int cols, int cus);
-hipError_t launch_column_sums(int dtype, const void *x, float *out, long rows, int cols, long ld, int parts, float *ws,
-                              hipStream_t stream);
+hipError_t launch_column_sums(int dtype, const void *x, float *const *out, const long *n, int count, long rows, int cols, long ld,
+                              int parts, float *ws, hipStream_t stream);
+hipError_t launch_add_pieces(const float *parts, float *const *out, const long *n, int count, int pieces, hipStream_t stream);
 
 hipError_t launch_decode(int dtype, void *state, const void *q, const void *k, const void *v, void *o, int BH,
                          int dk, int dv, hipStream_t stream);

@@ -799,19 +799,40 @@ def _head_sums(rows, b, h, n):
     return out
 
 
-def column_sums(x):
-    """Sums over the rows of x (rows, cols), in fp32 at least."""
+def column_sums(x, sizes=None):
+    """Sums over the rows of x (rows, cols), in fp32 at least; with `sizes` a list of tensors of their own with that many of them."""
     rows, cols = x.shape
     if (not x.is_cuda or x.dtype not in (torch.bfloat16, torch.float16) or rows < 2 or cols == 0 or cols % 8 or x.stride(1) != 1
-            or x.stride(0) < cols or x.stride(0) % 8 or x.data_ptr() % 16):
-        return x.sum(0, dtype=torch.promote_types(x.dtype, torch.float32))
-    out = torch.empty(cols, dtype=torch.float32, device=x.device)
+            or x.stride(0) < cols or x.stride(0) % 8 or x.data_ptr() % 16
+            or sizes is not None and (len(sizes) > _CONVERT_MAX or any(n % 8 for n in sizes))):
+        total = x.sum(0, dtype=torch.promote_types(x.dtype, torch.float32))
+        return total if sizes is None else [block.clone() for block in total.split(sizes)]
+    outs, count, where, lengths = _blocks([cols] if sizes is None else sizes, 1, x.device)
     with _on(x.device):
         ws, ws_ptr = _workspace(_ws_bytes("cott_column_sums_workspace_bytes", rows, cols), x.device)
-        rc = _loader.lib().cott_column_sums(x.data_ptr(), out.data_ptr(), rows, cols, x.stride(0), _DTYPES[x.dtype], ws_ptr,
-                                            ws.numel() if ws is not None else 0, _stream(x.device))
+        rc = _loader.lib().cott_column_sums_blocks(x.data_ptr(), where, lengths, count, rows, x.stride(0), _DTYPES[x.dtype], ws_ptr,
+                                                   ws.numel() if ws is not None else 0, _stream(x.device))
     _check(rc, "cott_column_sums")
-    return out
+    return outs[0].view(cols) if sizes is None else [out.view(-1) for out in outs]
+
+
+def _blocks(sizes, width, device):
+    """(tensors (size, width) fp32, their number, and the arrays of their addresses and lengths) for the library."""
+    outs = [torch.empty((n, width), dtype=torch.float32, device=device) for n in sizes]
+    n = len(outs)
+    return outs, n, (ctypes.c_void_p * n)(*(out.data_ptr() for out in outs)), (ctypes.c_long * n)(*(out.numel() for out in outs))
+
+
+def add_pieces(parts, sizes):
+    """Sums over the first dimension of parts (pieces, rows, width) fp32, as tensors of their own with `sizes` rows each."""
+    if (not parts.is_cuda or parts.dtype != torch.float32 or not parts.is_contiguous() or parts.shape[2] % 4 or parts.data_ptr() % 16
+            or len(sizes) > _CONVERT_MAX or parts.numel() == 0):
+        return [block.sum(0) for block in parts.split(sizes, dim=1)]
+    outs, count, where, lengths = _blocks(sizes, parts.shape[2], parts.device)
+    with _on(parts.device):
+        rc = _loader.lib().cott_add_pieces(parts.data_ptr(), where, lengths, count, parts.shape[0], _stream(parts.device))
+    _check(rc, "cott_add_pieces")
+    return outs
 
 
 def _token_stride(q, k, v, b, h, n, dk, dv):

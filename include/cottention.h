@@ -314,7 +314,11 @@ COTT_API int cott_prep_strided_bwd(const void *q, const void *k, const void *v,
  * N at most 2^24 (counts are exact in fp32).
  * cott_head_sums: out (H) = sums of rows (B,H,N) over b and n.
  * cott_column_sums: out (cols) fp32 = sums over the rows of x (rows, cols) bf16 / fp16 with ld elements between rows; cols and ld
- * multiples of 8, x 16-byte aligned; workspace of cott_column_sums_workspace_bytes (may be 0). */
+ * multiples of 8, x 16-byte aligned; workspace of cott_column_sums_workspace_bytes (may be 0).
+ * cott_column_sums_blocks: the same for cols = the sum of n[0 .. count-1], each a multiple of 8, at most COTT_CONVERT_MAX of them:
+ * the sums of consecutive blocks of n[i] columns go to arrays out[i] of their own (bias gradients of several projections).
+ * cott_add_pieces: out[i] (n[i] elements, a multiple of 4) = sums over the pieces of consecutive blocks of parts (pieces, sum of
+ * n) fp32 (weight gradients of several projections from row pieces); 16-byte aligned pointers. */
 #define COTT_CONVERT_MAX 8
 COTT_API int cott_convert(const float *const *src, void *const *dst, const long *n, int count, int dtype, void *stream);
 COTT_API int cott_keep_counts(const void *mask, int mask_dtype, unsigned char *keep, float *cnt, int B, int N, int running,
@@ -323,6 +327,9 @@ COTT_API int cott_head_sums(const float *rows, float *out, int B, int H, int N, 
 COTT_API size_t cott_column_sums_workspace_bytes(long rows, int cols);
 COTT_API int cott_column_sums(const void *x, float *out, long rows, int cols, long ld, int dtype, void *workspace,
                      size_t workspace_bytes, void *stream);
+COTT_API int cott_column_sums_blocks(const void *x, float *const *out, const long *n, int count, long rows, long ld, int dtype,
+                     void *workspace, size_t workspace_bytes, void *stream);
+COTT_API int cott_add_pieces(const float *parts, float *const *out, const long *n, int count, int pieces, void *stream);
 
 /* ---- causal forward on the RAW projections: the input preparation inside the attention kernel ------------
  *   o = cott_causal_fwd(q_hat, k_hat, v_hat)  with

@@ -85,7 +85,7 @@ def test_frozen_projections_cost_no_gradient(trained, monkeypatch):
     columns = {"w": [], "b": []}
     product, total = autograd._weight_gradient, ops.column_sums
     monkeypatch.setattr(autograd, "_weight_gradient", lambda g, x, *a: (columns["w"].append(g.shape[1]), product(g, x, *a))[1])
-    monkeypatch.setattr(ops, "column_sums", lambda g: (columns["b"].append(g.shape[1]), total(g))[1])
+    monkeypatch.setattr(ops, "column_sums", lambda g, *a: (columns["b"].append(g.shape[1]), total(g, *a))[1])
     got = gradients()
     assert sum(columns["w"]) == sum(columns["b"]) == sum(sizes[i] for i in trained)
     for a, c in zip(got, [everything[2 * i + j] for i in trained for j in (0, 1)]):
@@ -105,3 +105,54 @@ def test_parameter_gradients_own_their_memory(rows):
     params = [p for lin in lins for p in lin.parameters()]
     assert all(p.grad.untyped_storage().nbytes() == 4 * p.numel() and p.grad.is_contiguous() for p in params)
     assert len({p.grad.untyped_storage().data_ptr() for p in params}) == len(params)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("pieces,sizes,width", [(1, [1], 4), (2, [3, 5, 1], 12), (3, [64, 0, 7], 1028), (16, [100], 36), (8, [1024, 1024, 1024], 1024),
+                                                (2, [1, 2, 3, 4, 5, 6, 7, 8], 4), (2, [1] * 9, 4), (2, [5], 6)])
+def test_add_pieces(pieces, sizes, width):
+    """Each block's sum in memory of its own; edges of a thread's four elements and a workgroup's 1024, empty blocks, more blocks or
+    odder widths than the kernel takes."""
+    from cottention_transformer_amd import ops
+    parts = torch.randn(pieces, sum(sizes), width, generator=torch.Generator().manual_seed(pieces)).to(DEV)
+    got = ops.add_pieces(parts, sizes)
+    assert [tuple(t.shape) for t in got] == [(n, width) for n in sizes]
+    for t, block in zip(got, parts.split(sizes, dim=1)):
+        # at most 15 additions in fp32
+        assert t.untyped_storage().nbytes() == 4 * t.numel()
+        assert (t.double() - block.double().sum(0)).abs().le(block.double().abs().sum(0) * 2.0 ** -24 * pieces).all()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("rows,sizes,ld", [(2, [8], 8), (100, [8, 16, 264], 288), (129, [768, 768, 768], 2304), (5000, [48, 0, 8], 64), (300, [12, 4], 16),
+                                           (300, [8] * 9, 72)])
+def test_column_sums_in_blocks(rows, sizes, ld):
+    """The sums of one array, block by block in memory of their own: few rows (one launch a block), parts, what torch adds."""
+    from cottention_transformer_amd import ops
+    x = torch.randn(rows, ld, generator=torch.Generator().manual_seed(rows)).to(DEV, BF)[:, :sum(sizes)]
+    got, whole = ops.column_sums(x, sizes), ops.column_sums(x)
+    assert all(t.untyped_storage().nbytes() == 4 * t.numel() and t.shape == (n,) for t, n in zip(got, sizes))
+    bound = x.double().abs().sum(0) * 2.0 ** -24 * 8 + 1e-30  # (as for the whole)
+    for t, block, b in zip(got, x.double().sum(0).split(sizes), bound.split(sizes)):
+        assert (t.double() - block).abs().le(b).all()
+    if rows >= 128 and sum(sizes) % 8 == 0 and len(sizes) <= 8 and all(n % 8 == 0 for n in sizes):
+        assert torch.equal(torch.cat(got), whole)
+
+
+def test_refused_blocks():
+    import ctypes
+    from cottention_transformer_amd import _loader
+    L = _loader.lib()
+
+    def call(f, sizes, *tail, out=0x1000):
+        n = len(sizes)
+        return f((ctypes.c_void_p * n)(*[out] * n), (ctypes.c_long * n)(*sizes), n, *tail)
+    pieces = lambda sizes, p=2, **kw: call(lambda *a: L.cott_add_pieces(0x1000, *a), sizes, p, None, **kw)
+    columns = lambda sizes, ld=64, **kw: call(lambda *a: L.cott_column_sums_blocks(0x1000, *a), sizes, 1000, ld, _loader.BF16, None, 0, None, **kw)
+    for bad in ([6], [-4], [4] * 9, [4, 2]):
+        assert pieces(bad) == _loader.ERR_INVALID
+    assert pieces([4], 0) == _loader.ERR_INVALID and pieces([4], out=0x1004) == _loader.ERR_INVALID and pieces([4], out=None) == _loader.ERR_INVALID
+    for bad in ([12], [-8], [8] * 9, [72]):
+        assert columns(bad) == _loader.ERR_INVALID
+    assert columns([8], 12) == _loader.ERR_INVALID and columns([8, 8]) == _loader.ERR_WORKSPACE
+    assert pieces([]) == pieces([0]) == columns([]) == _loader.OK

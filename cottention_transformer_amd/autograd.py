@@ -231,15 +231,15 @@ class PreparedNonCausalAttention(torch.autograd.Function):
 
 def _row_pieces(rows, out, inner):
     """Pieces that the rows of a weight gradient (out, inner) are cut into: until the pieces' 256 x 128 tiles fill the chip (no
-    limit up to 1 M elements), as long as a piece keeps 2048 rows and more than out * inner / 1024, below which forming
+    limit up to 1 M elements), as long as a piece keeps 2048 rows and more than out * inner / 2048, below which forming
     and adding an fp32 piece costs what the fuller chip gives.  bf16, us in 1 / 2 / 4 / 8 pieces with their sum: 16384 rows x 1024 x
-    1024 104 / 71 / 52 / 48, 2304 x 768 128 / 93 / 98 / 88, 1536 x 1536 153 / 122 / 92 / 108, 3072 x 1024 155 / 128 / 116 / 134, 2048 x
-    2048 162 / 144 / 139 / 161; 8192 rows: 2304 x 768 70 / 58 / 64 / 62, 2048 x 2048 88 / 84 / 87 / 107, 4608 x 1536 129 / 145;
-    4096 rows: 1536 x 1536 47 / 45, 2048 x 2048 52 / 56."""
+    1024 104 / 69 / 50 / 46, 2304 x 768 128 / 85 / 90 / 78, 1536 x 1536 152 / 119 / 90 / 106, 3072 x 1024 156 / 121 / 106 / 121, 2048 x
+    2048 160 / 138 / 135 / 159; 8192 rows: 2304 x 768 71 / 49 / 56 / 52, 3072 x 1024 86 / 69 / 66, 2048 x 2048 86 / 80 / 84, 4608 x
+    1536 126 / 129; 4096 rows: 3072 x 1024 50 / 43, 2048 x 2048 50 / 51, 4608 x 1536 72 / 79."""
     tiles = 0 if out * inner <= 1 << 20 else -(-out // 256) * -(-inner // 128)
     pieces = 1
     while (pieces < 16 and tiles * pieces < 256 and rows % (2 * pieces) == 0 and rows // (2 * pieces) >= 2048
-           and rows // (2 * pieces) * 1024 > out * inner):
+           and rows // (2 * pieces) * 2048 > out * inner):
         pieces *= 2
     return pieces
 
@@ -288,7 +288,7 @@ def _joined(parts, sizes):
 
 def _of_column_blocks(f, g, sizes, wanted):
     """What f(g, sizes) makes of each column block of g: of the whole at once where all are wanted, else of each wanted one by
-    itself (16384 x 3072 x 1024: the weight gradients of all three 107 us, of one 47)."""
+    itself (16384 x 3072 x 1024: the weight gradients of all three 106 us, of one 46)."""
     if all(wanted):
         return f(g, sizes)
     return [f(part, [part.shape[1]])[0] if want else None for part, want in zip(g.split(sizes, dim=1), wanted)]
@@ -303,7 +303,7 @@ class InputProjections(torch.autograd.Function):
     Several weights that have to be converted anyway (fp32 parameters under autocast) are converted into one matrix, and all
     the products are one GEMM each: the outputs are then column slices of one tensor, which the input preparation
     reads, and whose gradients it writes, as such; dx leaves the GEMM in fp32.  Forward / dx / dW of three projections, us, one
-    by one and together: 16384 x 1024 98 / 124 / 157 and 94 / 91 / 105, 16384 x 768 75 / 86 / 133 and 65 / 55 / 77,
+    by one and together: 16384 x 1024 98 / 124 / 157 and 94 / 91 / 106, 16384 x 768 75 / 86 / 133 and 65 / 55 / 78,
     2048 x 512 60 / 54 / 59 and 19 / 19 / 20."""
 
     @staticmethod

@@ -10,9 +10,10 @@ def test_row_pieces():
     """Small weights as far as 2048 rows a piece go; larger ones only where a piece has more rows than its fp32 sum is worth."""
     from cottention_transformer_amd.autograd import _row_pieces
     assert [_row_pieces(r, 1024, 1024) for r in (4095, 4096, 8192, 16384, 1 << 16, 6144)] == [1, 2, 4, 8, 16, 2]
-    assert [_row_pieces(r, 3072, 1024) for r in (4096, 8192, 16384, 16383)] == [1, 2, 4, 1]
+    assert [_row_pieces(r, 3072, 1024) for r in (4096, 8192, 16384, 16383)] == [2, 4, 4, 1]
     assert [_row_pieces(16384, out, n) for out, n in ((2304, 768), (1536, 1536), (6144, 2048))] == [8, 4, 1]
-    assert [_row_pieces(r, 2048, 2048) for r in (4096, 8192, 16384)] == [1, 1, 2]
+    assert [_row_pieces(r, 2048, 2048) for r in (4096, 8192, 16384)] == [1, 2, 2]
+    assert [_row_pieces(r, 4608, 1536) for r in (4096, 8192, 16384)] == [1, 2, 2]
 
 
 # single weights of either side of 1 M elements, several pieces; operands as slices of a wider matrix

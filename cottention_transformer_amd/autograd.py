@@ -251,16 +251,14 @@ def _weight_gradient(gy, x, sizes=None):
     a tensor of its own, so the result has the sums of the single GEMM."""
     r = x.shape[0]
     pieces = 1
-    recording = torch.is_grad_enabled()  # the batched product with fp32 results has no derivative
-    if x.is_cuda and x.dtype in (torch.float16, torch.bfloat16) and not (recording and gy.shape[1] * x.shape[1] > 1 << 20):
+    # (with a second derivative to record, the single product: the batched one has none with fp32 results, and its own
+    # backward would multiply by transposed views, which has faulted in 16 bits; contiguous() for the same reason)
+    if x.is_cuda and x.dtype in (torch.float16, torch.bfloat16) and not torch.is_grad_enabled():
         pieces = _row_pieces(r, gy.shape[1], x.shape[1])
     if pieces == 1:
         product = gy.t() @ x
         return product if sizes is None else product.split(sizes)
-    a, b = gy.view(pieces, r // pieces, -1).transpose(1, 2), x.view(pieces, r // pieces, -1)
-    if recording:
-        sums = torch.bmm(a, b).sum(0, dtype=torch.float32)
-        return sums if sizes is None else sums.split(sizes)
+    a, b = gy.view(pieces, r // pieces, -1).transpose(1, 2), x.contiguous().view(pieces, r // pieces, -1)
     blocks = ops.add_pieces(torch.bmm(a, b, out_dtype=torch.float32), [gy.shape[1]] if sizes is None else sizes)
     return blocks[0] if sizes is None else blocks
 

@@ -157,3 +157,26 @@ def test_refused_blocks():
         assert columns(bad) == _loader.ERR_INVALID
     assert columns([8], 12) == _loader.ERR_INVALID and columns([8, 8]) == _loader.ERR_WORKSPACE
     assert pieces([]) == pieces([0]) == columns([]) == _loader.OK
+
+
+@pytest.mark.parametrize("recording", [False, True])
+def test_batched_products_get_no_transposed_right_operand(recording, monkeypatch):
+    """Column-major hidden states (one sequence, transposed), and products whose own backward would multiply by such: on the CPU,
+    with the batched product replaced."""
+    from cottention_transformer_amd import autograd
+
+    class OnGpu(torch.Tensor):
+        is_cuda = True
+    seen = []
+
+    def bmm(a, b, out_dtype=None):
+        seen.append(b.is_contiguous())
+        return torch.matmul(a.as_subclass(torch.Tensor).float(), b.as_subclass(torch.Tensor).float())
+    monkeypatch.setattr(autograd.torch, "bmm", bmm)
+    gy = torch.randn(4096, 8)
+    x = torch.randn(16, 4096).t()
+    with torch.set_grad_enabled(recording):
+        got = autograd._weight_gradient(gy.to(BF), x.to(BF).as_subclass(OnGpu))
+    want = gy.to(BF).float().t() @ x.to(BF).float()
+    assert seen == ([] if recording else [True])
+    assert float((got.float() - want).norm() / want.norm()) <= 4e-3

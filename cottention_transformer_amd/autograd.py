@@ -253,7 +253,8 @@ def _weight_gradient(gy, x, sizes=None):
     pieces = 1
     # (with a second derivative to record, the single product: the batched one has none with fp32 results, and its own
     # backward would multiply by transposed views, which has faulted in 16 bits; contiguous() for the same reason)
-    if x.is_cuda and x.dtype in (torch.float16, torch.bfloat16) and not torch.is_grad_enabled():
+    recording = torch.is_grad_enabled() and (gy.requires_grad or x.requires_grad)
+    if x.is_cuda and x.dtype in (torch.float16, torch.bfloat16) and not recording:
         pieces = _row_pieces(r, gy.shape[1], x.shape[1])
     if pieces == 1:
         product = gy.t() @ x

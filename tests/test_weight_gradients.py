@@ -176,7 +176,7 @@ def test_batched_products_get_no_transposed_right_operand(recording, monkeypatch
     gy = torch.randn(4096, 8)
     x = torch.randn(16, 4096).t()
     with torch.set_grad_enabled(recording):
-        got = autograd._weight_gradient(gy.to(BF), x.to(BF).as_subclass(OnGpu))
+        got = autograd._weight_gradient(gy.to(BF).requires_grad_(recording), x.to(BF).as_subclass(OnGpu)).detach()
     want = gy.to(BF).float().t() @ x.to(BF).float()
     assert seen == ([] if recording else [True])
     assert float((got.float() - want).norm() / want.norm()) <= 4e-3

@@ -375,10 +375,13 @@ class InputProjections(torch.autograd.Function):
         else:
             gws = [_weight_gradient(g, x2) if want else None for g, want in zip(gys, want_w)]
             gbs = [column_sums(g) if want else None for g, want in zip(gys, want_b)]
+        # (in memory of their own, each a gradient that is kept, saved or dropped by itself: blocks of a joint 16-bit product are
+        # by their conversion, sums as they come but for recorded ones)
+        convert = own if torch.is_grad_enabled() else torch.Tensor.to
         grads = [gx]
         for i in range(len(ctx.sizes)):
-            grads.append(own(gws[i], ctx.wb_dtypes[2 * i]) if want_w[i] else None)
-            grads.append(own(gbs[i], ctx.wb_dtypes[2 * i + 1]) if want_b[i] else None)
+            grads.append(convert(gws[i], ctx.wb_dtypes[2 * i]) if want_w[i] else None)
+            grads.append(convert(gbs[i], ctx.wb_dtypes[2 * i + 1]) if want_b[i] else None)
         return tuple(grads)
 
 

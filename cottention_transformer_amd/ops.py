@@ -820,7 +820,7 @@ def _blocks(sizes, width, device):
     """(tensors (size, width) fp32, their number, and the arrays of their addresses and lengths) for the library."""
     outs = [torch.empty((n, width), dtype=torch.float32, device=device) for n in sizes]
     n = len(outs)
-    return outs, n, (ctypes.c_void_p * n)(*(out.data_ptr() for out in outs)), (ctypes.c_long * n)(*(out.numel() for out in outs))
+    return outs, n, (ctypes.c_void_p * n)(*[out.data_ptr() for out in outs]), (ctypes.c_long * n)(*[width * rows for rows in sizes])
 
 
 def add_pieces(parts, sizes):

@@ -53,7 +53,8 @@ __device__ __forceinline__ bool is_zero<u16>(u16 x) {  // bf16 and fp16 alike: +
 // One workgroup of 16 wavefronts per batch element walks the positions in tiles of 8192, eight consecutive ones per thread.
 // RUNNING: cnt[s] = kept positions up to and with s, else their number in the whole sequence.  The counts inside a thread and
 // a wavefront come from bit counts of ballots; one exchange through LDS per tile.  8 x 2048: 4.9 us, where the comparison,
-// the conversion to numbers and the cumulative sum took 23 in three launches.
+// the conversion to numbers and the cumulative sum took 23 in three launches.  Bound by the one workgroup's walk, 1 us per 1000
+// positions: callers with a few long sequences do better with a reduction over the whole chip (ops.keep_and_counts_preferred).
 template <class E, bool RUNNING>
 __global__ __launch_bounds__(1024) void keep_counts_kernel(const E *mask, unsigned char *keep, float *cnt, int N) {
     __shared__ int totals[16];
@@ -115,7 +116,7 @@ __device__ __forceinline__ float block_sum(float v, float *part) {
 
 // out[h] = sum over b and s of rows[b][h][s]: one workgroup per head, eight loads in flight per thread whatever the split into b
 // and s (a loop over b with one load each took 10 us at 32 x 12 x 512).  5.6 us there and at 8 x 16 x 2048, where a general
-// reduction takes 10.4 and 11.0.
+// reduction takes 10.4 and 11.0.  Bound by the one workgroup, 20 us per 100000 rows: ops.head_sums adds longer ones in two steps.
 __global__ __launch_bounds__(1024) void head_sums_kernel(const float *rows, float *out, int B, int H, int N) {
     __shared__ float part[16];
     const float *head = rows + (size_t)blockIdx.x * N;

@@ -9,7 +9,8 @@
 //     (SplitMode).  Rel-L2 against fp64 7.0e-8 .. 2.1e-7, where the fp32 matrix pipe, which these widths took before, gives
 //     1.9e-7 .. 3.7e-7 and terms that are all cut 1.2e-7 .. 2.3e-7 (N63 .. N8192, D 80 .. 128, forward and gradients); every
 //     entry 1.0078, the worst of cut terms, N1 .. N128: at most 4.7e-8, 1.2e-7 and 4.8e-7.  Rounding costs 1 to 3 % of the
-//     times below.  The fp32 pipe is sixteen times slower than the bf16 one.
+//     times below.  A product within 2^-8 of the largest fp32 number may come out infinite.  The fp32 pipe is sixteen times
+//     slower than the bf16 one.
 // Structure: that of colscan_kernel (cott_colscan.h).
 //   * Four compute wavefronts each own a quarter of the state's columns, all rows, in fp32 accumulators whose row order makes
 //     them the operand of A_c S_c once they are split; they produce those columns of the output.

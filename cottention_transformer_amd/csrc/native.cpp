@@ -1,6 +1,7 @@
 // The host side of the hot operators in native code: for ordinary calls (plain contiguous tensors of one type on the current
 // device, shapes that agree) the tensors' pointers, the outputs, the workspace and the launch in one step each.  Anything
-// else is answered with None, and the Python of ops.py, which knows all forms and their errors, takes the call.  A call costs
+// else is answered with None, and the Python of ops.py, which knows all forms and their errors, takes the call; so is every call
+// while a function or dispatch mode is on (torch.set_default_device is one).  A call costs
 // about 6 us instead of 11, of which the launch is 3.5 (one launch; 128 positions of 2 heads).
 // Nothing is kept between calls but the library's entry points.
 #include <Python.h>

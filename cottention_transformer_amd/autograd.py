@@ -293,6 +293,19 @@ def _of_column_blocks(f, g, sizes, wanted):
     return [f(part, [part.shape[1]])[0] if want else None for part, want in zip(g.split(sizes, dim=1), wanted)]
 
 
+def _joint_form(x, weights, biases, cd):
+    """Whether the weights, and the biases if there are any, can be converted to `cd` into one matrix and one vector: all of them have
+    to be converted, are ordinary tensors on x's device, fit x, and a bias has an entry for every output (nn.functional.linear would
+    also spread one of another shape)."""
+    if len(weights) < 2 or not ops.plain(x, *weights):
+        return False
+    if any(w.dtype == cd or w.device != x.device or w.dim() != 2 or w.shape[1] != x.shape[-1] for w in weights):
+        return False
+    if all(b is None for b in biases):
+        return True
+    return all(b is not None and ops.plain(b) and b.device == x.device and b.shape == w.shape[:1] for w, b in zip(weights, biases))
+
+
 class InputProjections(torch.autograd.Function):
     """(x, w_0, b_0, w_1, b_1, ...) -> (x w_0^T + b_0, x w_1^T + b_1, ...): the q / k / v projections of an attention
     block (GPT_Trainer/GPTCosAttention.py:443-445, BERT_Trainer/BertCosAttention.py:121,143-144 with biases) as one
@@ -315,17 +328,13 @@ class InputProjections(torch.autograd.Function):
         ctx.x_meta = (x.shape, x.dtype)
         ctx.wb_dtypes = [None if t is None else t.dtype for t in wb]
         ctx.sizes = [w.shape[0] for w in weights]
-        ctx.joint = False
-        if len(weights) > 1 and weights[0].dtype != cd and x.is_cuda:
-            bias_free = biases[0] is None
-            ctx.joint = (all(w.dtype != cd and w.device == x.device and w.shape[1] == x.shape[-1] for w in weights)
-                         and all((b is None) == bias_free for b in biases))
+        ctx.joint = x.is_cuda and _joint_form(x, weights, biases, cd)
         if ctx.joint:
             x2 = x.reshape(-1, x.shape[-1])
             w = torch.empty((sum(ctx.sizes), x2.shape[1]), dtype=cd, device=x.device)
             convert = list(zip(weights, w.split(ctx.sizes)))
             bias = None
-            if not bias_free:
+            if biases[0] is not None:
                 bias = torch.empty(sum(ctx.sizes), dtype=cd, device=x.device)
                 convert += zip(biases, bias.split(ctx.sizes))
             if x2.dtype != cd:

@@ -728,6 +728,12 @@ def _prep_shapes(q, k, v, bnhd):
 
 
 _CONVERT_MAX = 8  # COTT_CONVERT_MAX
+_PLAIN = (torch.Tensor, torch.nn.Parameter)
+
+
+def plain(*tensors):
+    """Whether all are ordinary tensors, whose numbers lie at their data pointer (a subclass may keep them elsewhere)."""
+    return all(type(t) in _PLAIN for t in tensors)
 
 
 def convert_into(pairs, dtype):
@@ -738,8 +744,9 @@ def convert_into(pairs, dtype):
         return
     device = pairs[0][0].device
     if (dtype not in (torch.bfloat16, torch.float16) or len(pairs) > _CONVERT_MAX
-            or any(src.dtype != torch.float32 or src.device != device or not src.is_cuda or not src.is_contiguous()
-                   or (src.data_ptr() | dst.data_ptr()) & 15 or src.numel() > 1 << 30 for src, dst in pairs)):
+            or any(src.dtype != torch.float32 or src.device != device or not src.is_cuda or not plain(src, dst)
+                   or src.shape != dst.shape or not src.is_contiguous() or (src.data_ptr() | dst.data_ptr()) & 15
+                   or src.numel() > 1 << 30 for src, dst in pairs)):
         for src, dst in pairs:
             dst.copy_(src)
         return
@@ -756,7 +763,7 @@ def keep_and_counts(mask, b, n, running):
     and cnt (b,n) fp32, the kept positions up to each one (running) or in its sequence, as one launch; None where the mask is
     of another kind (its type, strided, on the CPU)."""
     code = _DTYPES.get(mask.dtype)
-    if (not mask.is_cuda or code is None or code == _loader.F64 or mask.numel() != b * n or not mask.is_contiguous()
+    if (not mask.is_cuda or not plain(mask) or code is None or code == _loader.F64 or mask.numel() != b * n or not mask.is_contiguous()
             or n > 1 << 24):
         return None
     keep = torch.empty((b, n), dtype=torch.bool, device=mask.device)
@@ -802,7 +809,7 @@ def _head_sums(rows, b, h, n):
 def column_sums(x, sizes=None):
     """Sums over the rows of x (rows, cols), in fp32 at least; with `sizes` a list of tensors of their own with that many of them."""
     rows, cols = x.shape
-    if (not x.is_cuda or x.dtype not in (torch.bfloat16, torch.float16) or rows < 2 or cols == 0 or cols % 8 or x.stride(1) != 1
+    if (not x.is_cuda or not plain(x) or x.dtype not in (torch.bfloat16, torch.float16) or rows < 2 or cols == 0 or cols % 8 or x.stride(1) != 1
             or x.stride(0) < cols or x.stride(0) % 8 or x.data_ptr() % 16
             or sizes is not None and (len(sizes) > _CONVERT_MAX or any(n % 8 for n in sizes))):
         total = x.sum(0, dtype=torch.promote_types(x.dtype, torch.float32))
@@ -825,7 +832,7 @@ def _blocks(sizes, width, device):
 
 def add_pieces(parts, sizes):
     """Sums over the first dimension of parts (pieces, rows, width) fp32, as tensors of their own with `sizes` rows each."""
-    if (not parts.is_cuda or parts.dtype != torch.float32 or not parts.is_contiguous() or parts.shape[2] % 4 or parts.data_ptr() % 16
+    if (not parts.is_cuda or not plain(parts) or parts.dtype != torch.float32 or not parts.is_contiguous() or parts.shape[2] % 4 or parts.data_ptr() % 16
             or len(sizes) > _CONVERT_MAX or parts.numel() == 0):
         return [block.sum(0) for block in parts.split(sizes, dim=1)]
     outs, count, where, lengths = _blocks(sizes, parts.shape[2], parts.device)
